@@ -526,6 +526,25 @@ int plh_layer_norm_backward(const void *grad_output, const void *x, int32_t dtyp
                             int64_t n_size, int64_t dimsize, int64_t m_size,
                             float eps, void *stream);
 
+/* The same with a weight and a bias per channel (dimsize elements of `dtype` each), which the reference's module applies
+ * with torch operations (pytorch_loss/layer_norm.py:125-137): forward weight * normalised + bias; backward
+ * grad_x from grad_output * weight, grad_weight[c] = sum of grad_output * normalised and grad_bias[c] = sum of grad_output
+ * over (n, m), added up in a fixed order (both NULL: not wanted). plh_layer_norm_affine_workspace_bytes: scratch for the
+ * backward's sums; 0 where a shape has no such form (m_size == 1, dimsize > 1024, an empty tensor), and the two entry
+ * points then return PLH_ERR_BAD_SIZE (an empty tensor: PLH_OK).
+ */
+int64_t plh_layer_norm_affine_workspace_bytes(int64_t n_size, int64_t dimsize, int64_t m_size);
+
+int plh_layer_norm_affine_forward(const void *x, int32_t dtype, const void *weight, const void *bias, void *out,
+                                  int64_t n_size, int64_t dimsize, int64_t m_size,
+                                  float eps, void *stream);
+
+int plh_layer_norm_affine_backward(const void *grad_output, const void *x, int32_t dtype, const void *weight,
+                                   void *grad_x, void *grad_weight, void *grad_bias,
+                                   void *workspace, int64_t workspace_bytes,
+                                   int64_t n_size, int64_t dimsize, int64_t m_size,
+                                   float eps, void *stream);
+
 /* ---- measurement aid ----------------------------------------------------------------
  * Plain fp32 device-to-device copy kernel of known traffic (4*numel bytes read,
  * 4*numel written), used to calibrate hardware byte counters and to measure the

@@ -1,0 +1,6 @@
+// layer norm kernels with weight and bias for bf16 elements (see layernorm_kernels.hpp).
+#include "layernorm_kernels.hpp"
+
+namespace plh {
+PLH_LN_INSTANTIATE_AFFINE(bf16)
+}  // namespace plh

@@ -23,9 +23,62 @@ struct LnParams {
     int C;
     int per_wave;       // channels per wave when the waves of a block share a pixel group
     float eps;
+    // affine forms only: per-channel weight and bias (elements of x's type; the backward has no use for the bias),
+    // the number of pixel groups, and the backward's per-block sums [blocks][C][2] (nullptr: not wanted)
+    const void *weight, *bias;
+    int64_t groups;
+    float *partials;
 };
 
 constexpr int kLnBlock = 256;
+
+// Wavefronts per SIMD that a kernel's registers have to leave room for: the affine backward's sums would take the slices
+// of up to 32 slots past 128 registers, and a CU would hold one block of 512 threads where it holds two.
+
+constexpr int ln_waves(int slots, bool sums) { return (sums && slots <= 32) ? 4 : 1; }
+
+// The affine forms' parameters and where the backward leaves their gradients (partials = nullptr: not wanted).
+template <class T>
+struct LnAffine {
+    const T *weight = nullptr, *bias = nullptr;
+    float *partials = nullptr;
+    T *grad_weight = nullptr, *grad_bias = nullptr;
+};
+
+// Sums of N values (8 or 16) over the 64 lanes of a wave: every step adds two values at once, each half of the lanes
+// keeping one of them, so that N values cost 2 N + 2 instructions where N separate sums would cost 7 N.
+// Lane i returns the sum of value i / (64 / N).
+template <int N>
+__device__ __forceinline__ float ln_transpose_sum(float (&v)[N], int lane) {
+    static_assert(N == 8 || N == 16, "chunks of 4 or 8 channels");
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {                  // lanes 32..63 go on with the upper half of the values
+        const auto s = __builtin_amdgcn_permlane32_swap(f32_bits(v[i]), f32_bits(v[i + N / 2]), false, false);
+        v[i] = bits_f32(s[0]) + bits_f32(s[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) {                  // odd rows of 16 lanes with the upper half of what is left
+        const auto s = __builtin_amdgcn_permlane16_swap(f32_bits(v[i]), f32_bits(v[i + N / 4]), false, false);
+        v[i] = bits_f32(s[0]) + bits_f32(s[1]);
+    }
+#pragma unroll
+    for (int i = 0; i < N / 8; ++i) {
+        const bool up = lane & 8;
+        const float keep = up ? v[i + N / 8] : v[i], give = up ? v[i] : v[i + N / 8];
+        v[i] = keep + dpp_move<0x128>(give);           // row_ror:8
+    }
+    float r = v[0];
+    if constexpr (N == 16) {
+        const bool up = lane & 4;
+        const float keep = up ? v[1] : v[0], give = up ? v[0] : v[1];
+        r = keep + dpp_move<0x141>(give);              // row_half_mirror: lane ^ 7
+    } else {
+        r += dpp_move<0x141>(r);
+    }
+    r += dpp_move<0xB1>(r);                            // quad_perm [1,0,3,2]
+    r += dpp_move<0x4E>(r);                            // quad_perm [2,3,0,1]
+    return r;
+}
 
 // KW = channel slots per wave (>= the channels it holds), V = pixels per lane, WS = waves sharing a
 // pixel group (1: each of a block's four waves has its own group and all channels; 4 or 8: the block
@@ -33,36 +86,61 @@ constexpr int kLnBlock = 256;
 // PerImage: pixel groups that never straddle two images (groups = images x groups per image), for channel planes
 // that start on element boundaries only (odd lengths): a lane's V pixels are moved with accesses of the same
 // width from element boundaries; the last lane of an image may hold fewer and goes pixel by pixel.
-template <class T, int KW, int V, int WS, bool Bwd, bool PerImage = false>
-__global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *__restrict__ x, const T *__restrict__ g,
+// Affine: out = weight * normalised + bias in the forward; in the backward the upstream gradient is multiplied by the
+// weight on its way in, and the sums of grad * normalised and of grad over the pixels (the gradients of weight and bias)
+// are left per block. HBM-bound like the plain forms: the module's two torch passes over the tensor after the forward
+// and six before the backward fall away. The backward's blocks loop over pixel groups (ln_grid) so that there are
+// few rows of sums; the cross-lane sums of a chunk of channels cost about 5 vector instructions per channel and group
+// (ln_transpose_sum), against some 25 for the gradient itself. Module step at (16,256,128,128) fp32: 0.849 -> 0.241 ms
+// (its four tensor passes of the plain forms, 5.6 TB/s).
+template <class T, int KW, int V, int WS, bool Bwd, bool PerImage = false, bool Affine = false>
+__global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock, ln_waves(KW, Affine && Bwd)) void ln_regs(const T *__restrict__ x, const T *__restrict__ g,
                                                     T *__restrict__ out, const LnParams p) {
     using PK = Pack<T, V>;
-    __shared__ float ex[WS][2][V][64];
+    constexpr bool kSums = Affine && Bwd;
+    constexpr int kChunk = KW % 8 == 0 ? 8 : 4;        // channels of the backward in flight per trip
+    // the blocks that loop write the next group's statistics while a slower wave may still read this one's
+    __shared__ float ex[kSums ? 2 : 1][WS][2][V][64];
+    __shared__ float wb[Affine ? (Bwd ? 1 : 2) : 1][Affine ? 1024 : 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t group = WS > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
-    bool live;
-    int nv = V;                                        // pixels this lane has
-    int64_t pc, n;
-    if constexpr (PerImage) {
-        const int64_t per_image = ceil_div_dev(p.m_size, (int64_t)64 * V);
-        n = group / per_image;
-        const int64_t local = ((group - n * per_image) * 64 + lane) * V;
-        const int64_t left = p.m_size - local;
-        nv = left >= V ? V : (left > 0 ? (int)left : 0);
-        live = nv > 0 && n * p.m_size < p.P;
-        if (!live) { n = 0; nv = V; }                  // dead lanes read pixel 0 and store nothing
-        pc = live ? n * p.m_size + local : 0;
-    } else {
-        const int64_t pix = (group * 64 + lane) * V;
-        live = pix < p.P;
-        pc = live ? pix : 0;                           // dead lanes read pixel 0 and store nothing
-        n = pc / p.m_size;
-    }
     const int c0 = WS > 1 ? wave * p.per_wave : 0;
     int cnt = WS > 1 ? p.C - c0 : p.C;
     cnt = cnt < 1 ? 1 : (WS > 1 && cnt > p.per_wave ? p.per_wave : cnt);   // a split always leaves every wave >= 1 channel
     cnt = __builtin_amdgcn_readfirstlane(cnt);
-    const int64_t base = pc + n * (int64_t)(p.C - 1) * p.m_size + (int64_t)c0 * p.m_size;
+    if constexpr (Affine) {
+        for (int i = threadIdx.x; i < p.C; i += blockDim.x) {
+            wb[0][i] = load_one(static_cast<const T *>(p.weight) + i);
+            if constexpr (!Bwd) wb[1][i] = load_one(static_cast<const T *>(p.bias) + i);
+        }
+        __syncthreads();
+    }
+    float sums[kSums ? KW / kChunk : 1] = {};
+    int turn = 0;
+    for (int64_t group = WS > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;
+         !kSums || group < p.groups; group += WS > 1 ? (int64_t)gridDim.x : (int64_t)gridDim.x * 4) {
+    int held = cnt;
+    int64_t plane = p.m_size;
+    // hidden from the loop: every slot's test and plane offset, taken out of it, would be 300 spilled scalar registers
+    if constexpr (kSums) asm volatile("" : "+s"(held), "+s"(plane));
+    bool live;
+    int nv = V;                                        // pixels this lane has
+    int64_t pc, n;
+    if constexpr (PerImage) {
+        const int64_t per_image = ceil_div_dev(plane, (int64_t)64 * V);
+        n = group / per_image;
+        const int64_t local = ((group - n * per_image) * 64 + lane) * V;
+        const int64_t left = plane - local;
+        nv = left >= V ? V : (left > 0 ? (int)left : 0);
+        live = nv > 0 && n * plane < p.P;
+        if (!live) { n = 0; nv = V; }                  // dead lanes read pixel 0 and store nothing
+        pc = live ? n * plane + local : 0;
+    } else {
+        const int64_t pix = (group * 64 + lane) * V;
+        live = pix < p.P;
+        pc = live ? pix : 0;                           // dead lanes read pixel 0 and store nothing
+        n = pc / plane;
+    }
+    const int64_t base = pc + n * (int64_t)(p.C - 1) * plane + (int64_t)c0 * plane;
     auto fetch = [&](const T *at) {
         if constexpr (PerImage) {
             if (nv < V) {
@@ -94,7 +172,7 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *
     // weighted out of the sums: straight-line code, no per-slot control flow.
     typename PK::Raw raw[KW];
 #pragma unroll
-    for (int j = 0; j < KW; ++j) raw[j] = fetch(x + base + (int64_t)(j < cnt ? j : cnt - 1) * p.m_size);
+    for (int j = 0; j < KW; ++j) raw[j] = fetch(x + base + (int64_t)(j < held ? j : held - 1) * plane);
 
     const float inv_c = 1.f / (float)p.C;
     float mean[V], v[V];
@@ -102,8 +180,8 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *
     for (int k = 0; k < V; ++k) {
         float s = 0.f;
 #pragma unroll
-        for (int j = 0; j < KW; ++j) s += j < cnt ? PK::get(raw[j], k) : 0.f;
-        const float mw = s / (float)cnt;
+        for (int j = 0; j < KW; ++j) s += j < held ? PK::get(raw[j], k) : 0.f;
+        const float mw = s / (float)held;
         // every sweep widens the packed slice again: kept apart for the optimiser, which would
         // otherwise hold all widened values of the first sweep in registers for the later ones
 #pragma unroll
@@ -111,12 +189,12 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *
         float q = 0.f;
 #pragma unroll
         for (int j = 0; j < KW; ++j) {
-            const float d = j < cnt ? PK::get(raw[j], k) - mw : 0.f;
+            const float d = j < held ? PK::get(raw[j], k) - mw : 0.f;
             q = __builtin_fmaf(d, d, q);
         }
         if constexpr (WS > 1) {
-            ex[wave][0][k][lane] = mw;
-            ex[wave][1][k][lane] = q;
+            ex[turn][wave][0][k][lane] = mw;
+            ex[turn][wave][1][k][lane] = q;
         } else {
             mean[k] = mw;
             v[k] = q * inv_c + p.eps;
@@ -132,7 +210,7 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *
                 int c = p.C - w * p.per_wave;
                 c = c < 0 ? 0 : (c > p.per_wave ? p.per_wave : c);
                 cw[w] = (float)c;
-                mw[w] = ex[w][0][k][lane];
+                mw[w] = ex[turn][w][0][k][lane];
                 tot = __builtin_fmaf(cw[w], mw[w], tot);
             }
             const float m = tot * inv_c;
@@ -140,7 +218,7 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *
 #pragma unroll
             for (int w = 0; w < WS; ++w) {
                 const float d = mw[w] - m;
-                m2 += ex[w][1][k][lane] + cw[w] * d * d;
+                m2 += ex[turn][w][1][k][lane] + cw[w] * d * d;
             }
             mean[k] = m;
             v[k] = m2 * inv_c + p.eps;
@@ -160,28 +238,69 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock) void ln_regs(const T *
         for (int j = 0; j < KW; ++j) {
             float r[V];
 #pragma unroll
-            for (int k = 0; k < V; ++k) r[k] = (PK::get(raw[j], k) - mean[k]) * rstd[k];
-            if (live && j < cnt) put_back(out + base + (int64_t)j * p.m_size, r);
+            for (int k = 0; k < V; ++k) {
+                r[k] = (PK::get(raw[j], k) - mean[k]) * rstd[k];
+                if constexpr (Affine) r[k] = __builtin_fmaf(wb[0][c0 + (j < held ? j : 0)], r[k], wb[1][c0 + (j < held ? j : 0)]);
+            }
+            if (live && j < held) put_back(out + base + (int64_t)j * plane, r);
         }
     } else {
-        constexpr int kChunk = KW < 8 ? KW : 8;        // gradient slices in flight per trip
 #pragma unroll
         for (int j0 = 0; j0 < KW; j0 += kChunk) {
             typename PK::Raw graw[kChunk];
+            float part[2 * kChunk];                    // per channel: grad * normalised, grad (this lane's pixels)
 #pragma unroll
             for (int jj = 0; jj < kChunk; ++jj)
-                graw[jj] = fetch(g + base + (int64_t)(j0 + jj < cnt ? j0 + jj : cnt - 1) * p.m_size);
+                graw[jj] = fetch(g + base + (int64_t)(j0 + jj < held ? j0 + jj : held - 1) * plane);
 #pragma unroll
             for (int jj = 0; jj < kChunk; ++jj) {
                 float r[V];
+                float sg = 0.f, sgy = 0.f;
+                const float w = Affine ? wb[0][c0 + (j0 + jj < held ? j0 + jj : 0)] : 1.f;
 #pragma unroll
                 for (int k = 0; k < V; ++k) {
                     const float val = PK::get(raw[j0 + jj], k);
+                    float gv = PK::get(graw[jj], k);
                     const float inner = __builtin_fmaf((val - mean[k]) * (val - inv_c), mv[k], inv_c);
-                    r[k] = -rstd[k] * inner * PK::get(graw[jj], k);
+                    if constexpr (Affine) {
+                        sg += gv;
+                        sgy = __builtin_fmaf((val - mean[k]) * rstd[k], gv, sgy);
+                        gv *= w;
+                    }
+                    r[k] = -rstd[k] * inner * gv;
                 }
-                if (live && j0 + jj < cnt) put_back(out + base + (int64_t)(j0 + jj) * p.m_size, r);
+                if (live && j0 + jj < held) put_back(out + base + (int64_t)(j0 + jj) * plane, r);
+                if constexpr (kSums) {
+                    part[2 * jj] = live ? sgy : 0.f;
+                    part[2 * jj + 1] = live ? sg : 0.f;
+                }
             }
+            if constexpr (kSums) {
+                if (p.partials) sums[j0 / kChunk] += ln_transpose_sum<2 * kChunk>(part, lane);
+            }
+        }
+    }
+    if constexpr (!kSums) return;
+    turn ^= 1;
+    }
+    if constexpr (kSums) {
+        if (!p.partials) return;                       // grid-uniform
+        // lane i of a wave holds value i / (64 / (2 * kChunk)) of every chunk; rows of sums are [C][2]
+        constexpr int kSpan = 64 / (2 * kChunk);
+        float *row = p.partials + (int64_t)blockIdx.x * 2 * p.C;
+        if constexpr (WS > 1) {
+#pragma unroll
+            for (int h = 0; h < KW / kChunk; ++h) {
+                const int ch = h * kChunk + lane / kSpan / 2;
+                if (lane % kSpan == 0 && ch < cnt) row[2 * (c0 + ch) + ((lane / kSpan) & 1)] = sums[h];
+            }
+        } else {
+            __shared__ float all[4][2 * KW];           // the four waves of the block hold all channels each
+#pragma unroll
+            for (int h = 0; h < KW / kChunk; ++h)
+                if (lane % kSpan == 0) all[wave][h * 2 * kChunk + lane / kSpan] = sums[h];
+            __syncthreads();
+            for (int i = threadIdx.x; i < 2 * p.C; i += kLnBlock) row[i] = (all[0][i] + all[1][i]) + (all[2][i] + all[3][i]);
         }
     }
 }
@@ -251,11 +370,45 @@ __global__ __launch_bounds__(256) void ln_group(const T *__restrict__ x, const T
     }
 }
 
-template <class T, bool Bwd>
+// Rows of sums in the affine backward: column by column in a fixed order, in the parameters' type. A block takes 16
+// columns (64 bytes of every row) with 64 rows in flight.
+template <class T>
+__global__ __launch_bounds__(1024) void ln_finish_sums(const float *__restrict__ partials, int rows, int C,
+                                                       T *__restrict__ grad_weight, T *__restrict__ grad_bias) {
+    __shared__ float part[64][17];
+    const int col = blockIdx.x * 16 + (threadIdx.x & 15), first = threadIdx.x >> 4;
+    float s = 0.f;
+    if (col < 2 * C) {
+#pragma unroll 8
+        for (int r = first; r < rows; r += 64) s += partials[(int64_t)r * 2 * C + col];
+    }
+    part[first][threadIdx.x & 15] = s;
+    __syncthreads();
+#pragma unroll
+    for (int half = 32; half > 0; half >>= 1) {
+        if (first < half) part[first][threadIdx.x & 15] += part[first + half][threadIdx.x & 15];
+        __syncthreads();
+    }
+    if (first == 0 && col < 2 * C) store_one((col & 1 ? grad_bias : grad_weight) + (col >> 1), part[0][threadIdx.x & 15]);
+}
+
+// The shapes that have an affine form: what ln_regs serves.
+inline bool ln_has_affine(int64_t dimsize, int64_t m_size) { return m_size > 1 && dimsize <= 1024; }
+
+// Blocks of the affine backward, which loop over the pixel groups: enough to fill the chip with the blocks that fit it
+// at once (two of 512 threads per CU, eight of 256), twice over.
+inline unsigned ln_sum_blocks(int64_t dimsize, int64_t blocks) {
+    const int64_t cap = dimsize > 64 ? 1024 : 2048;
+    return (unsigned)(blocks < cap ? blocks : cap);
+}
+
+template <class T, bool Bwd, bool Affine>
 void ln_launch(const T *x, const T *g, T *out, int64_t n_size, int64_t dimsize, int64_t m_size, float eps,
-               hipStream_t st) {
+               const LnAffine<T> &af, hipStream_t st) {
     constexpr int VT = ElemTraits<T>::kVec;
-    LnParams p;
+    LnParams p = {};
+    p.weight = af.weight;
+    p.bias = af.bias;
     p.P = n_size * m_size;
     p.m_size = m_size;
     p.C = (int)dimsize;
@@ -265,7 +418,8 @@ void ln_launch(const T *x, const T *g, T *out, int64_t n_size, int64_t dimsize, 
     // With 4 waves and C > 32, or 8 waves and C > 64, every wave holds at least one channel.
     const int ws = dimsize > 64 ? 8 : (dimsize > 32 ? 4 : 1);
     p.per_wave = (int)ceil_div(dimsize, ws);
-    if (m_size == 1 || dimsize > 1024) {
+    if (!ln_has_affine(dimsize, m_size)) {
+        if constexpr (Affine) return;
         if (m_size == 1) {
             hipLaunchKernelGGL((ln_group<T, 64, Bwd>), dim3(group_grid(p.P, 4)), dim3(256), 0, st, x, g, out, p);
         } else {
@@ -288,17 +442,22 @@ void ln_launch(const T *x, const T *g, T *out, int64_t n_size, int64_t dimsize, 
                         (image || (vec && std::is_same<T, f16>::value && slots > 64));
     const int vv = narrow ? VN : VT;
     const int64_t groups = image ? n_size * ceil_div(m_size, 64 * vv) : ceil_div(p.P, 64 * (vec ? vv : 1));
-    const unsigned grid = (unsigned)(ws > 1 ? groups : ceil_div(groups, 4));
+    p.groups = groups;
+    unsigned grid = (unsigned)(ws > 1 ? groups : ceil_div(groups, 4));
+    if constexpr (Affine && Bwd) {
+        grid = ln_sum_blocks(dimsize, grid);
+        p.partials = af.partials;
+    }
 #define PLH_LN(KW, VV, WS) \
-    hipLaunchKernelGGL((ln_regs<T, KW, VV, WS, Bwd>), dim3(grid), dim3(WS > 4 ? 64 * WS : kLnBlock), 0, st, x, g, out, p)
+    hipLaunchKernelGGL((ln_regs<T, KW, VV, WS, Bwd, false, Affine>), dim3(grid), dim3(WS > 4 ? 64 * WS : kLnBlock), 0, st, x, g, out, p)
 #define PLH_LN_IMAGE(KW, WS) \
-    hipLaunchKernelGGL((ln_regs<T, KW, VT, WS, Bwd, true>), dim3(grid), dim3(WS > 4 ? 64 * WS : kLnBlock), 0, st, x, g, out, p)
+    hipLaunchKernelGGL((ln_regs<T, KW, VT, WS, Bwd, true, Affine>), dim3(grid), dim3(WS > 4 ? 64 * WS : kLnBlock), 0, st, x, g, out, p)
 #define PLH_LN_V(KW, WS) do { if (vec) PLH_LN(KW, VT, WS); else if (image) PLH_LN_IMAGE(KW, WS); else PLH_LN(KW, 1, WS); } while (0)
 #define PLH_LN_NARROW(KW, WS)                                                                                              \
     do {                                                                                                                   \
         if (vec) PLH_LN(KW, VN, WS);                                                                                       \
         else if (image)                                                                                                    \
-            hipLaunchKernelGGL((ln_regs<T, KW, VN, WS, Bwd, true>), dim3(grid), dim3(64 * WS), 0, st, x, g, out, p);       \
+            hipLaunchKernelGGL((ln_regs<T, KW, VN, WS, Bwd, true, Affine>), dim3(grid), dim3(64 * WS), 0, st, x, g, out, p);       \
         else PLH_LN(KW, 1, WS);                                                                                            \
     } while (0)
     // Slot counts in steps of about 1.5x: a wave whose channels fall short of its slots re-reads its last
@@ -324,18 +483,32 @@ void ln_launch(const T *x, const T *g, T *out, int64_t n_size, int64_t dimsize, 
 #undef PLH_LN_V
 #undef PLH_LN_IMAGE
 #undef PLH_LN
+    if constexpr (Affine && Bwd) {
+        if (af.partials)
+            hipLaunchKernelGGL(ln_finish_sums<T>, dim3((unsigned)ceil_div(2 * dimsize, 16)), dim3(1024), 0, st, af.partials, (int)grid,
+                               p.C, af.grad_weight, af.grad_bias);
+    }
 }
 
-// Per-dtype entry, instantiated in layernorm_f32.hip / layernorm_f16.hip / layernorm_bf16.hip.
+// Per-dtype entries, instantiated in layernorm_{f32,f16,bf16}.hip (plain) and layernorm_{f32,f16,bf16}_affine.hip.
 template <class T>
 void ln_run_typed(bool bwd, const T *x, const T *g, T *out, int64_t n_size, int64_t dimsize, int64_t m_size, float eps,
                   hipStream_t st) {
-    if (bwd) ln_launch<T, true>(x, g, out, n_size, dimsize, m_size, eps, st);
-    else ln_launch<T, false>(x, g, out, n_size, dimsize, m_size, eps, st);
+    if (bwd) ln_launch<T, true, false>(x, g, out, n_size, dimsize, m_size, eps, LnAffine<T>{}, st);
+    else ln_launch<T, false, false>(x, g, out, n_size, dimsize, m_size, eps, LnAffine<T>{}, st);
+}
+template <class T>
+void ln_run_affine(bool bwd, const T *x, const T *g, T *out, int64_t n_size, int64_t dimsize, int64_t m_size, float eps,
+                   const LnAffine<T> &af, hipStream_t st) {
+    if (bwd) ln_launch<T, true, true>(x, g, out, n_size, dimsize, m_size, eps, af, st);
+    else ln_launch<T, false, true>(x, g, out, n_size, dimsize, m_size, eps, af, st);
 }
 
 #define PLH_LN_SIGNATURE(T) void ln_run_typed<T>(bool, const T *, const T *, T *, int64_t, int64_t, int64_t, float, hipStream_t);
-#define PLH_LN_EXTERN(T) extern template PLH_LN_SIGNATURE(T)
+#define PLH_LN_AFFINE_SIGNATURE(T) \
+    void ln_run_affine<T>(bool, const T *, const T *, T *, int64_t, int64_t, int64_t, float, const LnAffine<T> &, hipStream_t);
+#define PLH_LN_EXTERN(T) extern template PLH_LN_SIGNATURE(T) extern template PLH_LN_AFFINE_SIGNATURE(T)
 #define PLH_LN_INSTANTIATE(T) template PLH_LN_SIGNATURE(T)
+#define PLH_LN_INSTANTIATE_AFFINE(T) template PLH_LN_AFFINE_SIGNATURE(T)
 
 }  // namespace plh

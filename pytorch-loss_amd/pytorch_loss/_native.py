@@ -88,6 +88,9 @@ _SIGNATURES = {
     "plh_soft_dice_backward": (ctypes.c_int, [_p, _p, _i32, _p, _p, _p, _i64, _i64, _f32, _p]),
     "plh_layer_norm_forward": (ctypes.c_int, [_p, _i32, _p, _i64, _i64, _i64, _f32, _p]),
     "plh_layer_norm_backward": (ctypes.c_int, [_p, _p, _i32, _p, _i64, _i64, _i64, _f32, _p]),
+    "plh_layer_norm_affine_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "plh_layer_norm_affine_forward": (ctypes.c_int, [_p, _i32, _p, _p, _p, _i64, _i64, _i64, _f32, _p]),
+    "plh_layer_norm_affine_backward": (ctypes.c_int, [_p, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_onehot": (ctypes.c_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_stream_copy": (ctypes.c_int, [_p, _p, _i64, _p]),
 }
@@ -894,3 +897,36 @@ def layer_norm_backward(grad_output, xc, tag, eps, dtype):
         n, c, m = xc.shape
         _call(xc, "plh_layer_norm_backward", _ptr(g), _ptr(xc), tag, _ptr(out), n, c, m, float(eps))
     return out if out.dtype == dtype else out.to(dtype)
+
+
+def layer_norm_has_affine(x, weight, bias):
+    """Whether the kernels with weight and bias serve these tensors: one element type for all three, and a shape that the
+    register-resident kernels take (see plh_layer_norm_affine_workspace_bytes)."""
+    return (x.is_cuda and weight.is_cuda and bias.is_cuda and x.dtype == weight.dtype == bias.dtype and x.dtype in _DTYPE_TAGS
+            and weight.numel() == bias.numel() == x.shape[1]
+            and load().plh_layer_norm_affine_workspace_bytes(*x.shape) > 0)
+
+
+def layer_norm_affine_forward(x, weight, bias, eps):
+    """(N, C, M) normalised over C, times weight, plus bias. -> (out, the contiguous input and weight for the backward)."""
+    _require_gpu("layernorm loss", x, weight, bias)
+    (xc, tag), wc = _logits(x), weight.contiguous()
+    out = torch.empty_like(xc)
+    _call(xc, "plh_layer_norm_affine_forward", _ptr(xc), tag, _ptr(wc), _ptr(bias.contiguous()), _ptr(out), *xc.shape,
+          float(eps))
+    return out, xc, wc
+
+
+def layer_norm_affine_backward(grad_output, xc, wc, eps, sums):
+    """-> (grad of x, grad of weight, grad of bias); the last two are None unless `sums`."""
+    g = (grad_output if grad_output.dtype == xc.dtype else grad_output.to(xc.dtype)).expand(xc.shape).contiguous()
+    grad = torch.empty_like(xc)
+    grad_w = grad_b = ws = None
+    nbytes = 0
+    if sums:
+        grad_w, grad_b = torch.empty_like(wc), torch.empty_like(wc)
+        nbytes = int(load().plh_layer_norm_affine_workspace_bytes(*xc.shape))
+        ws = torch.empty((nbytes,), dtype=torch.uint8, device=xc.device)
+    _call(xc, "plh_layer_norm_affine_backward", _ptr(g), _ptr(xc), _DTYPE_TAGS[xc.dtype], _ptr(wc), _ptr(grad), _ptr(grad_w),
+          _ptr(grad_b), _ptr(ws), nbytes, *xc.shape, float(eps))
+    return grad, grad_w, grad_b

@@ -1,0 +1,94 @@
+"""The layer-norm module's kernels with weight and bias against the same module in 64 bits (its formulas in torch, on the
+CPU): every slot count and form on both sides of its limits, loops of several pixel groups per block, and what the
+gradients of weight and bias are when only some are asked for.
+Outputs and grad_x as in test_gpu_layernorm; a sum over P pixels of fp32 terms t may be off by about
+sqrt(P) * 2^-24 * max|t| (16-bit: one more rounding of the result)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pl():
+    import pytorch_loss
+    from pytorch_loss import _native
+    _native.load()
+    return pytorch_loss
+
+
+# (N, C, H, W): one wave (C <= 32), four waves, eight waves with every slot count up to 128; ragged pixel counts, one pixel per
+# lane, planes of odd length, more groups than blocks (the last two)
+SHAPES = [(2, 1, 8, 8), (1, 5, 7, 7), (2, 8, 5, 13), (3, 12, 8, 9), (1, 20, 20, 20), (2, 32, 10, 33), (2, 33, 8, 8),
+          (1, 64, 15, 20), (2, 65, 8, 16), (1, 100, 7, 11), (1, 160, 8, 8), (1, 256, 10, 13), (1, 384, 8, 8), (1, 512, 7, 7),
+          (1, 600, 8, 8), (1, 768, 7, 10), (1, 1000, 8, 9), (2, 19, 65, 65), (2, 100, 64, 65), (1, 700, 65, 65),
+          (5, 8, 513, 513), (5, 72, 256, 161)]
+
+
+def ref64(x, w, b, g, eps):
+    n, c = x.shape[:2]
+    x3, g3 = x.double().reshape(n, c, -1), g.double().reshape(n, c, -1)
+    w, b = w.double().reshape(1, c, 1), b.double().reshape(1, c, 1)
+    mean = x3.mean(1, keepdim=True)
+    v = x3.var(1, keepdim=True, unbiased=False) + eps
+    y = (x3 - mean) * v.rsqrt()
+    gx = -v.rsqrt() * (1 / c + (x3 - mean) * (x3 - 1 / c) * mean * v) * (g3 * w)       # csrc/layer_norm.cu:212-216
+    return w * y + b, gx, g3 * y, g3
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_module_matches_64_bits(pl, shape, dtype):
+    gen = torch.Generator().manual_seed(sum(shape))
+    n, c = shape[:2]
+    x = (torch.randn(shape, generator=gen) * 1.5 + 0.3).to(dtype)
+    g = torch.randn(shape, generator=gen).to(dtype)
+    m = pl.LayerNormV3(c).to("cuda", dtype)
+    with torch.no_grad():
+        m.weight.copy_(1 + 0.2 * torch.randn((1, c, 1), generator=gen))
+        m.bias.copy_(0.2 * torch.randn((1, c, 1), generator=gen))
+    xt = x.cuda().requires_grad_()
+    out = m(xt)
+    out.backward(g.cuda())
+    want, want_x, gy, g3 = ref64(x, m.weight.detach().cpu(), m.bias.detach().cpu(), g, 1e-6)
+    step = {torch.float32: 0.0, torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    assert out.dtype == dtype and xt.grad.dtype == dtype and m.weight.grad.dtype == dtype
+    flat = lambda t: t.detach().cpu().double().reshape(n, c, -1)
+    assert ((flat(out) - want).abs() <= 1e-5 + step * want.abs()).all()
+    assert ((flat(xt.grad) - want_x).abs() <= 1e-5 * want_x.abs().max() + step * want_x.abs()).all()
+    pixels = x.numel() // c
+    for got, terms in ((m.weight.grad, gy), (m.bias.grad, g3)):
+        assert got.shape == (1, c, 1)
+        total = terms.sum((0, 2))
+        bound = (8 + np.sqrt(pixels)) * 2.0 ** -24 * terms.abs().max() + step * total.abs() + 1e-30
+        # the normalised value itself is good to about 1e-6
+        bound = bound + (np.sqrt(pixels) * 1e-6 if terms is gy else 0.0)
+        assert ((got.detach().cpu().double().reshape(c) - total).abs() <= bound).all()
+
+
+def test_partial_gradients_and_fallbacks(pl):
+    x = torch.randn(2, 16, 9, 10, device="cuda", requires_grad=True)
+    m = pl.LayerNormV3(16).cuda()
+    g = torch.randn(2, 16, 9, 10, device="cuda")
+    m(x).backward(g)
+    full = [t.grad.clone() for t in (x, m.weight, m.bias)]
+    for frozen in (0, 1, 2):
+        leaves = [t.detach().requires_grad_(i != frozen) for i, t in enumerate((x, m.weight, m.bias))]
+        m2 = pl.LayerNormV3(16).cuda()
+        m2.weight, m2.bias = torch.nn.Parameter(leaves[1], leaves[1].requires_grad), torch.nn.Parameter(leaves[2], leaves[2].requires_grad)
+        m2(leaves[0]).backward(g)
+        for i, (t, want) in enumerate(zip((leaves[0], m2.weight, m2.bias), full)):
+            assert (t.grad is None) if i == frozen else torch.equal(t.grad, want)
+    # create_graph: the gradient of weight stays differentiable with respect to the upstream gradient
+    up = g.clone().requires_grad_()
+    gw, = torch.autograd.grad(m(x), m.weight, up, create_graph=True)
+    assert torch.allclose(gw, full[1], rtol=1e-4, atol=1e-4)
+    gw.sum().backward()
+    assert up.grad is not None and up.grad.abs().sum() > 0
+    # fp32 parameters on a 16-bit tensor, one pixel per row, more channels than the kernels hold: torch's operations
+    half = m(x.detach().bfloat16())
+    assert half.dtype == torch.float32
+    wide = pl.LayerNormV3(1100).cuda()
+    assert wide(torch.randn(1, 1100, 8, 8, device="cuda")).shape == (1, 1100, 8, 8)
+    assert m(torch.randn(4, 16, 1, 1, device="cuda")).shape == (4, 16, 1, 1)
