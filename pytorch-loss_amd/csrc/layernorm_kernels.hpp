@@ -264,7 +264,9 @@ __global__ __launch_bounds__(WS > 4 ? 64 * WS : kLnBlock, ln_waves(KW, Affine &&
                     const float inner = __builtin_fmaf((val - mean[k]) * (val - inv_c), mv[k], inv_c);
                     if constexpr (Affine) {
                         sg += gv;
-                        sgy = __builtin_fmaf((val - mean[k]) * rstd[k], gv, sgy);
+                        // a partly filled lane's missing pixels are zeros, normalised to NaN where eps is 0
+                        const float y = (val - mean[k]) * rstd[k];
+                        sgy = __builtin_fmaf(PerImage && k >= nv ? 0.f : y, gv, sgy);
                         gv *= w;
                     }
                     r[k] = -rstd[k] * inner * gv;

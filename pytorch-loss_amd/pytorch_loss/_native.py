@@ -900,25 +900,27 @@ def layer_norm_backward(grad_output, xc, tag, eps, dtype):
 
 
 def layer_norm_has_affine(x, weight, bias):
-    """Whether the kernels with weight and bias serve these tensors: one element type for all three, and a shape that the
-    register-resident kernels take (see plh_layer_norm_affine_workspace_bytes)."""
+    """Whether the kernels with weight and bias serve these tensors: one element type for all three, one value per channel, a
+    shape that the register-resident kernels take (see plh_layer_norm_affine_workspace_bytes), and no forward-mode tangents."""
+    per_channel = (1, x.shape[1], 1)
     return (x.is_cuda and weight.is_cuda and bias.is_cuda and x.dtype == weight.dtype == bias.dtype and x.dtype in _DTYPE_TAGS
-            and weight.numel() == bias.numel() == x.shape[1]
+            and weight.shape == per_channel and bias.shape == per_channel
+            and not any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in (x, weight, bias))
             and load().plh_layer_norm_affine_workspace_bytes(*x.shape) > 0)
 
 
 def layer_norm_affine_forward(x, weight, bias, eps):
-    """(N, C, M) normalised over C, times weight, plus bias. -> (out, the contiguous input and weight for the backward)."""
+    """(N, C, M) normalised over C, times weight, plus bias. -> (out, the contiguous input for the backward)."""
     _require_gpu("layernorm loss", x, weight, bias)
-    (xc, tag), wc = _logits(x), weight.contiguous()
+    (xc, tag), wc, bc = _logits(x), weight.contiguous(), bias.contiguous()
     out = torch.empty_like(xc)
-    _call(xc, "plh_layer_norm_affine_forward", _ptr(xc), tag, _ptr(wc), _ptr(bias.contiguous()), _ptr(out), *xc.shape,
-          float(eps))
-    return out, xc, wc
+    _call(xc, "plh_layer_norm_affine_forward", _ptr(xc), tag, _ptr(wc), _ptr(bc), _ptr(out), *xc.shape, float(eps))
+    return out, xc
 
 
-def layer_norm_affine_backward(grad_output, xc, wc, eps, sums):
+def layer_norm_affine_backward(grad_output, xc, weight, eps, sums):
     """-> (grad of x, grad of weight, grad of bias); the last two are None unless `sums`."""
+    wc = weight.contiguous()
     g = (grad_output if grad_output.dtype == xc.dtype else grad_output.to(xc.dtype)).expand(xc.shape).contiguous()
     grad = torch.empty_like(xc)
     grad_w = grad_b = ws = None

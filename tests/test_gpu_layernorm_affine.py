@@ -92,3 +92,48 @@ def test_partial_gradients_and_fallbacks(pl):
     wide = pl.LayerNormV3(1100).cuda()
     assert wide(torch.randn(1, 1100, 8, 8, device="cuda")).shape == (1, 1100, 8, 8)
     assert m(torch.randn(4, 16, 1, 1, device="cuda")).shape == (4, 16, 1, 1)
+
+
+def test_eps_zero_on_planes_of_odd_length(pl):
+    """The last lane of an image holds fewer pixels than the others: its missing ones have no variance, and with eps = 0 no
+    finite normalised value either. Bounds as above."""
+    gen = torch.Generator().manual_seed(5)
+    shape = (2, 19, 65, 65)
+    x, g = torch.randn(shape, generator=gen), torch.randn(shape, generator=gen)
+    m = pl.LayerNormV3(19, eps=0.0).cuda()
+    xt = x.cuda().requires_grad_()
+    m(xt).backward(g.cuda())
+    _, _, gy, g3 = ref64(x, m.weight.detach().cpu(), m.bias.detach().cpu(), g, 0.0)
+    for got, terms in ((m.weight.grad, gy), (m.bias.grad, g3)):
+        pixels = 2 * 65 * 65
+        bound = (8 + np.sqrt(pixels)) * 2.0 ** -24 * terms.abs().max() + np.sqrt(pixels) * 1e-6
+        assert ((got.cpu().double().reshape(19) - terms.sum((0, 2))).abs() <= bound).all()
+
+
+def test_what_torch_refuses_stays_refused(pl):
+    """A weight changed in place between the passes, a second backward through freed buffers; forward mode through the weight
+    alone keeps working, and parameters of another shape broadcast as torch broadcasts them."""
+    x = torch.randn(2, 8, 9, 10, device="cuda", requires_grad=True)
+    m = pl.LayerNormV3(8).cuda()
+    out = m(x)
+    with torch.no_grad():
+        m.weight.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+    out = m(x).sum()
+    out.backward()
+    with pytest.raises(RuntimeError, match="second time"):
+        out.backward()
+    from torch.autograd import forward_ad
+    plain = pl.LayerNormV3(8, affine=False)(x.detach())
+    weight, bias = m.weight.detach(), m.bias.detach()
+    tangent = torch.randn_like(weight)
+    with forward_ad.dual_level():
+        del m.weight, m.bias
+        m.weight, m.bias = forward_ad.make_dual(weight, tangent), bias
+        got = forward_ad.unpack_dual(m(x.detach())).tangent
+    assert torch.allclose(got, tangent.view(1, 8, 1, 1) * plain)
+    square = torch.randn(1, 8, 2, 4, device="cuda")
+    m.weight, m.bias = torch.arange(8.0, device="cuda"), torch.zeros(8, device="cuda")      # along the pixels
+    want = (pl.LayerNormV3(8, affine=False)(square).view(1, 8, 8) * m.weight).view_as(square)
+    assert torch.equal(m(square), want)
