@@ -15,6 +15,8 @@
 //                     pattern is monotone), ignored pixel = 0x7FFFFFFF (sorts last). Also the
 //                     largest positive key per class (per-block table + lov_class_max): keys
 //                     beyond it have dJ = 0 exactly and are left out of the sort (keep_key).
+//   2.-4. for rows of up to kBkMaxRow pixels: by value buckets, see lovasz_buckets.hpp. Otherwise, and in the look-back
+//                     variant, with the same results bit for bit:
 //   2. 3 x (tile_hist, row_scan, scatter): stable LSD radix passes, 8 bits each, batched over
 //                     classes with blockIdx.y. Ranking inside a tile is done per wavefront with
 //                     ballot-built match masks, tiles are re-ordered in LDS so that the global
@@ -26,8 +28,7 @@
 //                     so J, dJ and the tile's share of the loss follow at once; dJ goes to
 //                     pixel order through region-binned staging (final) and an in-LDS permute
 //                     per region (unbin), which also writes the zeros of the keys left out.
-//   4. loss per class fixed-order sum of the per-tile partials (no floating-point atomics, so
-//                     results are deterministic): by the first unbin block of the class, or by
+//   4. loss per class sum of the per-tile partials, whose terms are multiples of 2^-51 and add exactly (loss_term): by the first unbin block of the class, or by
 //                     reduce_loss when the rows are too long for the staging regions.
 // A 4096-key tile is handled by 512 threads with 8 keys each; neighbouring tiles of a class row run
 // on the same XCD (sort_tile) so that the sectors they share merge in one L2.
@@ -788,6 +789,10 @@ __global__ __launch_bounds__(kSortThreads) void lov_scatter(const SortArgs a) {
     }
 }
 
+}  // namespace plh
+#include "lovasz_buckets.hpp"
+namespace plh {
+
 // ----------------------------- 3. last radix pass fused with the Jaccard step ----
 // The last pass knows every key's final position k (its scatter destination) and, with the
 // positives counted the same way as the keys, the number of positives sorted before it. That is
@@ -808,7 +813,7 @@ constexpr int kMaxRegions = 1024;             // per class row; larger rows take
 
 template <bool Binned, bool LookBack = false>
 __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, float *__restrict__ jacc,
-                                                          float *__restrict__ tile_loss,
+                                                          double *__restrict__ tile_loss,
                                                           uint32_t *__restrict__ cursors, int regions, int region_bits) {
     __shared__ uint32_t region_cnt[Binned ? kMaxRegions : 1];    // keys of this tile per region
     __shared__ uint16_t region_start[Binned ? kMaxRegions : 1];  // first position of the region in the re-ordered tile (< 4096)
@@ -820,14 +825,14 @@ __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, floa
     __shared__ uint32_t out_base[kRadix];     // global position of the tile's first key with digit d
     __shared__ uint32_t hot_base[kRadix];     // positives sorted before that position
     __shared__ uint32_t scan_tmp[2 * kSortWaves];
-    __shared__ float wave_loss[kSortWaves];
+    __shared__ double wave_loss[kSortWaves];
 
     const int c = blockIdx.y, tile = LookBack ? lov_take_ticket(a.tickets, c) : sort_tile(row_items(a, c));
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int begin = tile * kSortTile;
     const int count = min(kSortTile, row_items(a, c) - begin);
     if (count <= 0) {                           // block-uniform: the row ends before this tile
-        if (threadIdx.x == 0) tile_loss[(int64_t)c * a.tiles + tile] = 0.f;
+        if (threadIdx.x == 0) tile_loss[(int64_t)c * a.tiles + tile] = 0.0;
         return;
     }
     const DigitPlan dp = digit_plan(a.key_bits[c], kLastPass);
@@ -932,7 +937,7 @@ __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, floa
     __syncthreads();
 
     const float npos = (float)n_pos_u;
-    float part = 0.f;
+    double part = 0.0;
 #pragma unroll
     for (int r = 0; r < kSortItems; ++r) {
         const int li = wave * (kSortItems * kWave) + r * kWave + lane;
@@ -944,12 +949,8 @@ __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, floa
             if ((k & 0x7FFFFFFFu) != kIgnoredKey) {
                 const uint32_t pos = out_base[d] + counts[wave][d] + rank[r];            // rank in the descending order
                 const uint32_t cs = hot_base[d] + counts_hot[wave][d] + hrank[r];      // positives before it
-                const float inter_prev = npos - (float)cs;                             // csrc/lovasz_softmax.cu:124-127
-                const float inter = npos - (float)(cs + hot);
-                const float j_now = 1.f - inter / (inter + (float)(pos + 1));
-                const float j_prev = (pos == 0) ? 0.f : 1.f - inter_prev / (inter_prev + (float)pos);
-                dj = j_now - j_prev;                                                   // csrc/lovasz_softmax.cu:141-147
-                part += key_error(k) * dj;
+                dj = jaccard_step(npos, pos, cs, hot);
+                part += loss_term(key_error(k), dj);
             }
             if constexpr (Binned) {
                 const uint32_t lp = region_start[val[r] >> region_bits] + slot[r];
@@ -960,11 +961,11 @@ __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, floa
             }
         }
     }
-    part = group_reduce<64>(part, OpSum());
+    part = wave_sum_f64(part);
     if (lane == 0) wave_loss[wave] = part;
     __syncthreads();
     if (threadIdx.x == 0) {
-        float s = 0.f;
+        double s = 0.0;
 #pragma unroll
         for (int w = 0; w < kSortWaves; ++w) s += wave_loss[w];
         tile_loss[(int64_t)c * a.tiles + tile] = s;
@@ -987,7 +988,7 @@ constexpr int kUnbinThreads = 1024;
 template <int kRegionBits>
 __global__ __launch_bounds__(kUnbinThreads) void lov_unbin(float *__restrict__ jacc, const SortArgs a,
                                                            const uint32_t *__restrict__ cursors, int regions, int P,
-                                                           const float *__restrict__ tile_loss, float *__restrict__ losses,
+                                                           const double *__restrict__ tile_loss, float *__restrict__ losses,
                                                            int tiles) {
     typedef unsigned plh_u4 __attribute__((ext_vector_type(4)));
     constexpr int kRegion = 1 << kRegionBits;
@@ -1022,14 +1023,16 @@ __global__ __launch_bounds__(kUnbinThreads) void lov_unbin(float *__restrict__ j
     if (blockIdx.x != 0) return;
     __syncthreads();                                // `sorted` is free again
     const int c = blockIdx.y;
-    float sum = 0.f;
+    double *sums = reinterpret_cast<double *>(sorted);
+    double sum = 0.0;
     for (int i = threadIdx.x; i < tiles; i += kUnbinThreads) sum += tile_loss[(int64_t)c * tiles + i];
-    sum = group_reduce<64>(sum, OpSum());
-    if ((threadIdx.x & 63) == 0) sorted[threadIdx.x >> 6] = sum;
+    sum = wave_sum_f64(sum);
+    if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = sum;
     __syncthreads();
     if (threadIdx.x == 0) {
-        float total = 0.f;
-        for (int w = 0; w < kUnbinThreads / 64; ++w) total += sorted[w];
+        double all = 0.0;
+        for (int w = 0; w < kUnbinThreads / 64; ++w) all += sums[w];
+        float total = (float)all;
         if (a.timed_out && *a.timed_out) total = __builtin_nanf("");        // look-back variant: a wait ran out
         losses[c] = total;
     }
@@ -1039,16 +1042,16 @@ __global__ __launch_bounds__(256) void lov_zero_f32(float *p, int64_t n) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) p[i] = 0.f;
 }
 
-__global__ __launch_bounds__(256) void lov_reduce_loss(const float *__restrict__ tile_loss, float *__restrict__ losses,
+__global__ __launch_bounds__(256) void lov_reduce_loss(const double *__restrict__ tile_loss, float *__restrict__ losses,
                                                        int tiles) {
-    __shared__ float wave_sum[4];
+    __shared__ double wave_sum[4];
     const int c = blockIdx.x;
-    float s = 0.f;
+    double s = 0.0;
     for (int i = threadIdx.x; i < tiles; i += 256) s += tile_loss[(int64_t)c * tiles + i];
-    s = group_reduce<64>(s, OpSum());
+    s = wave_sum_f64(s);
     if ((threadIdx.x & 63) == 0) wave_sum[threadIdx.x >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) losses[c] = (wave_sum[0] + wave_sum[1]) + (wave_sum[2] + wave_sum[3]);
+    if (threadIdx.x == 0) losses[c] = (float)((wave_sum[0] + wave_sum[1]) + (wave_sum[2] + wave_sum[3]));
 }
 
 // ------------------------------------------------------------ backward ----
@@ -1147,6 +1150,12 @@ struct LovaszPlan {
         off_tile_loss, off_cursors, off_class, off_block_max, bytes;
     // look-back variant: tickets + time-out word + descriptors (cleared per call), totals, per-block tables
     bool look_back;
+    // value buckets (lovasz_buckets.hpp): tiles of kBkTile keys, log2 of the buckets a class may have (0: rows that one block
+    // ranks whole)
+    bool buckets;
+    int bk_tiles, bk_bits;
+    int64_t off_sorted, off_dj, off_tile_count, off_count, off_bounds, off_buckets, off_fine, off_loss_part,
+        off_crowded, off_bucket, off_tile_hot, off_bk_tile_loss;
     int hist_blocks;
     int64_t off_lb_clear, lb_clear_bytes, off_lb_totals, off_lb_partial;
 };
@@ -1163,6 +1172,36 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
     pl.tiles = (int)ceil_div(pl.P, kSortTile);
     pl.tiles_pad = (int)round_up(pl.tiles, kSortWaves);
     int64_t off = 0;
+    pl.off_class = off;       off += round_up(4 * dimsize * 4, 256);      // pos_max[C], kept[C], all_min[C], key_bits[C]
+    pl.off_block_max = off;   off += round_up(4 * dimsize * ceil_div(pl.P, 256), 256);   // [key blocks][C]
+    // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
+    // 8 keys of a tile. At 2048 buckets (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
+    // and two classes took 0.63 ms against 0.39 of the radix passes.
+    pl.look_back = false;
+    pl.regions = 0;
+    pl.buckets = !look_back && pl.P <= kBkMaxRow;
+    if (pl.buckets) {
+        pl.bk_tiles = (int)ceil_div(pl.P, kBkTile);
+        const int64_t most = ceil_div(pl.P, kBkTarget);
+        pl.bk_bits = pl.P <= kBkCap ? 0 : (most <= 64 ? 6 : (most <= 256 ? 8 : 10));
+        const int64_t cells = dimsize << pl.bk_bits;
+        pl.off_crowded = off;        off += round_up(4 * cells, 256);
+        if (pl.bk_bits) {
+            pl.off_sorted = off;     off += round_up(4 * pl.E, 256);
+            pl.off_dj = off;         off += round_up(4 * pl.E, 256);
+            pl.off_bucket = off;     off += round_up(2 * pl.E, 256);
+            pl.off_tile_count = off; off += round_up(4 * cells * pl.bk_tiles, 256);
+            pl.off_tile_hot = off;   off += round_up(4 * cells * pl.bk_tiles, 256);
+            pl.off_bk_tile_loss = off; off += round_up(8 * dimsize * pl.bk_tiles, 256);
+            pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // count, hot, base, hot_base, runs
+            pl.off_bounds = off;     off += round_up(4 * cells, 256);
+            pl.off_buckets = off;    off += round_up(4 * 5 * dimsize, 256);
+            pl.off_fine = off;       off += round_up(2 * dimsize * (kBkFine + 2), 256);
+            pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
+        }
+        pl.bytes = off;
+        return PLH_OK;
+    }
     pl.off_keys_a = off;      off += round_up(4 * pl.E, 256);
     pl.off_keys_c = off;      off += round_up(4 * pl.E, 256);
     pl.off_vals_a = off;      off += round_up(4 * pl.E, 256);
@@ -1171,15 +1210,13 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
     pl.off_hot = off;         off += round_up(4 * dimsize * kRadix * pl.tiles_pad, 256);
     pl.off_digit_total = off; off += round_up(4 * dimsize * kRadix, 256);
     pl.off_hot_total = off;   off += round_up(4 * dimsize * kRadix, 256);
-    pl.off_tile_loss = off;   off += round_up(4 * dimsize * pl.tiles, 256);
+    pl.off_tile_loss = off;   off += round_up(8 * dimsize * pl.tiles, 256);
     // the smallest region size that keeps a row within 256 regions (runs of >= 16 values per tile and region)
     pl.region_bits = kMinRegionBits;
     while (pl.region_bits < kMaxRegionBits && ceil_div(pl.P, (int64_t)1 << pl.region_bits) > 256) ++pl.region_bits;
     const int64_t regions = ceil_div(pl.P, (int64_t)1 << pl.region_bits);
     pl.regions = (regions <= kMaxRegions) ? (int)regions : 0;
     pl.off_cursors = off;     off += round_up(4 * dimsize * kMaxRegions, 256);
-    pl.off_class = off;       off += round_up(4 * dimsize * 4, 256);      // pos_max[C], kept[C], all_min[C], key_bits[C]
-    pl.off_block_max = off;   off += round_up(4 * dimsize * ceil_div(pl.P, 256), 256);   // [key blocks][C]
     // the look-back descriptors carry a count in 30 bits next to their 2 state bits
     if (look_back && pl.P >= ((int64_t)1 << 30)) return PLH_ERR_BAD_SIZE;
     pl.look_back = look_back && pl.regions > 0;
@@ -1211,6 +1248,61 @@ extern "C" int64_t plh_lovasz_lookback_workspace_bytes(int64_t n_size, int64_t d
     return rc == PLH_OK ? pl.bytes : (int64_t)rc;
 }
 
+// 2. and 3. by value buckets: ranks of the keys in keys_0 (jacc's memory), which becomes the Jaccard differences.
+static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, const uint32_t *pos_max, float *losses, int C,
+                          hipStream_t st) {
+    BucketArgs a = {};
+    a.keys = keys_0;
+    a.pos_max = pos_max;
+    a.P = (int)pl.P;
+    a.C = C;
+    a.crowded = reinterpret_cast<uint32_t *>(ws + pl.off_crowded);
+    if (pl.bk_bits == 0) {
+        hipLaunchKernelGGL(bk_rank<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);
+        hipLaunchKernelGGL(bk_rank_crowded<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);
+        return check_launch();
+    }
+    a.tiles = pl.bk_tiles;
+    a.stride = 1 << pl.bk_bits;
+    const int64_t step = round_up(4 * (((int64_t)C << pl.bk_bits) + C), 256);
+    a.sorted = reinterpret_cast<uint32_t *>(ws + pl.off_sorted);
+    a.dj = reinterpret_cast<float *>(ws + pl.off_dj);
+    a.bucket = reinterpret_cast<uint16_t *>(ws + pl.off_bucket);
+    a.tile_hot = reinterpret_cast<uint32_t *>(ws + pl.off_tile_hot);
+    a.tile_loss = reinterpret_cast<double *>(ws + pl.off_bk_tile_loss);
+    a.tile_count = reinterpret_cast<uint32_t *>(ws + pl.off_tile_count);
+    a.count = reinterpret_cast<uint32_t *>(ws + pl.off_count);
+    a.hot = reinterpret_cast<uint32_t *>(ws + pl.off_count + step);
+    a.base = reinterpret_cast<uint32_t *>(ws + pl.off_count + 2 * step);
+    a.hot_base = reinterpret_cast<uint32_t *>(ws + pl.off_count + 3 * step);
+    a.runs = reinterpret_cast<uint32_t *>(ws + pl.off_count + 4 * step);
+    a.bounds = reinterpret_cast<uint32_t *>(ws + pl.off_bounds);
+    a.numbers = reinterpret_cast<uint32_t *>(ws + pl.off_buckets);
+    a.fine = reinterpret_cast<uint16_t *>(ws + pl.off_fine);
+    a.loss_part = reinterpret_cast<double *>(ws + pl.off_loss_part);
+    const dim3 tiles((unsigned)pl.bk_tiles, (unsigned)C), threads(kBkThreads);
+    const unsigned most = (unsigned)ceil_div(pl.P, kBkTarget);      // buckets a class can have
+    // two blocks fit a CU; each looks at every so many of the class's runs
+    const unsigned crowded_blocks = (unsigned)(ceil_div(2048, C) < most ? ceil_div(2048, C) : most);
+    hipLaunchKernelGGL(bk_split, dim3((unsigned)C), threads, 0, st, a);
+    switch (pl.bk_bits) {
+#define PLH_BUCKETS(B)                                                                                               \
+    case B:                                                                                                          \
+        hipLaunchKernelGGL(bk_hist<1 << B>, tiles, threads, 0, st, a);                                               \
+        hipLaunchKernelGGL(bk_scan, dim3((unsigned)ceil_div(most, 64), (unsigned)C), dim3(1024), 0, st, a);          \
+        hipLaunchKernelGGL(bk_group, dim3((unsigned)C), threads, 0, st, a);                                          \
+        hipLaunchKernelGGL(bk_scatter<B>, tiles, threads, 0, st, a);                                                 \
+        hipLaunchKernelGGL(bk_rank<false>, dim3(most, (unsigned)C), threads, 0, st, a, losses);                      \
+        hipLaunchKernelGGL(bk_rank_crowded<false>, dim3(crowded_blocks, (unsigned)C), threads, 0, st, a, losses);    \
+        hipLaunchKernelGGL(bk_rank_wide, dim3(kBkWideBlocks, (unsigned)C), threads, 0, st, a);                       \
+        hipLaunchKernelGGL(bk_gather<B>, tiles, threads, 0, st, a, losses);                                          \
+        break;
+        PLH_BUCKETS(6) PLH_BUCKETS(8) PLH_BUCKETS(10)
+#undef PLH_BUCKETS
+    }
+    return check_launch();
+}
+
 static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labels, float *losses, float *jacc,
                           void *workspace, int64_t workspace_bytes, int64_t n_size, int64_t dimsize, int64_t m_size,
                           int64_t ignore_index, void *stream, bool look_back) {
@@ -1235,7 +1327,7 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
     uint32_t *hot = reinterpret_cast<uint32_t *>(ws + pl.off_hot);
     uint32_t *digit_total = reinterpret_cast<uint32_t *>(ws + pl.off_digit_total);
     uint32_t *hot_total = reinterpret_cast<uint32_t *>(ws + pl.off_hot_total);
-    float *tile_loss = reinterpret_cast<float *>(ws + pl.off_tile_loss);
+    double *tile_loss = reinterpret_cast<double *>(ws + pl.off_tile_loss);
     uint32_t *pos_max = reinterpret_cast<uint32_t *>(ws + pl.off_class);
     uint32_t *kept = pos_max + dimsize;
     uint32_t *all_min = pos_max + 2 * dimsize;
@@ -1277,6 +1369,8 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
                        reinterpret_cast<uint32_t *>(ws + pl.off_cursors), pl.regions);
     hipLaunchKernelGGL(lov_absent_min, dim3(kAbsentBlocks, (unsigned)C), dim3(256), 0, st, keys_0, pos_max, all_min,
                        (int)pl.P);
+
+    if (pl.buckets) return lovasz_buckets(pl, ws, keys_0, pos_max, losses, C, st);
 
     // 2. up to three stable scatter passes: (keys_0, -) -> (keys_a, vals_a) -> (keys_c, vals_b) -> (keys_a, vals_a);
     //    how many a class takes follows from the width of its keys (DigitPlan), the blocks of a pass

@@ -1,0 +1,1206 @@
+// The sort of the Lovasz forward by value buckets (included by lovasz.hip, after the keys and the rank primitives).
+//
+// A radix sort moves every (key, pixel) pair three times before its rank is known. Here a key moves once: the class row
+// is cut into buckets of neighbouring key values, and what fits a block's LDS is sorted there.
+//   bk_split      a block per class sorts a sample of the row's keys; every n-th of them starts a bucket
+//   bk_hist       keys (and positives) per tile and bucket
+//   bk_scan       the tiles' counts to exclusive sums per bucket
+//   bk_group      where every bucket starts in the row, and runs of buckets that a block can sort at once
+//   bk_scatter    keys to their buckets, in pixel order inside a bucket (stable ranks from match masks); the tile's order is
+//                 left in the place of its keys
+//   bk_rank       a block per run of buckets: sorted in LDS, Jaccard difference of every key at its place
+//   bk_rank_crowded  the same for runs whose values crowd
+//   bk_rank_wide  the same for buckets that outgrew the LDS
+//   bk_gather     Jaccard differences back to pixel order, tile by tile
+// Sampled bounds follow any distribution; a value that fills several buckets by itself gets one of its own, which
+// needs no sort (flat: bk_scatter knows the ranks), and a bucket that outgrew the LDS all the same is taken in value ranges
+// that fit.
+// Bound by vector instructions (scatter and rank: some 80 and 110 per 64 keys at 16 waves per CU) and short runs, not by
+// the 36 bytes a key moves. Forward and backward, against the radix passes: (8,21,513,513) bf16 trained 1.22 -> 0.87 ms,
+// (4,19,512,1024) fp32 0.74 -> 0.64, (1,150,256,256) 0.51 -> 0.37; near-uniform predictions, whose keys need two
+// radix passes only, take the same time as before ((4,19,512,1024) 0.42 -> 0.43).
+#pragma once
+
+namespace plh {
+
+constexpr int kBkThreads = 512;
+constexpr int kBkItems = 15;
+constexpr int kBkCap = kBkThreads * kBkItems;       // keys a block sorts at once: 8 bytes each, two blocks per CU
+constexpr int kBkTileItems = 16;
+constexpr int kBkTile = kBkThreads * kBkTileItems;  // keys of a tile
+constexpr int kBkWaves = kBkThreads / kWave;
+constexpr int kBkChunk = 16;                        // neighbours in the order that one thread sorts
+constexpr int kBkBins = 4096;                       // bins of a run's value range
+constexpr int kBkFineBits = 11;                     // table from a key's top bits to the first bucket it can be in
+constexpr int kBkFine = 1 << kBkFineBits;
+constexpr int kBkTarget = 2560;                     // mean keys per bucket: sampled bounds leave few above kBkCap
+constexpr int kBkSlab = 6144;                       // buckets that start in one such part of the row are sorted together
+constexpr int kBkMax = 1024;                        // buckets per class
+constexpr int64_t kBkMaxRow = (int64_t)kBkTarget * kBkMax;
+constexpr uint32_t kBkCrowd = 65;                   // keys in one bin up to which merges between chunks put them in order
+constexpr uint32_t kBkFlat = 0x80000000u;
+constexpr uint16_t kBkNowhere = 0xFFFFu;            // place of a pixel that takes no part
+
+struct BucketArgs {
+    uint32_t *keys;             // [C][P] in pixel order; bk_scatter leaves the tile's order there (jacc's memory)
+    const uint32_t *pos_max;    // pos_max[C], kept[C], all_min[C], key_bits[C] (see keep_key, lov_class_max)
+    uint32_t *sorted;           // [C][P] keys by bucket
+    float *dj;                  // [C][P] Jaccard differences by bucket
+    uint16_t *bucket;           // [C][P] bucket of every pixel
+    uint32_t *tile_count;       // [C][tiles][stride]: keys | positives << 16, exclusive sums over the tiles, start of the
+                                // tile's keys of the bucket in the row less their start in the tile
+    uint32_t *tile_hot;         // [C][tiles][stride] positives in the tiles before, of buckets with more than kBkCap keys
+    uint32_t *count, *hot;      // [C][stride] keys (kBkFlat: and a single value), positives per bucket
+    uint32_t *base, *hot_base;  // [C][stride + 1] the same before the bucket
+    uint32_t *bounds;           // [C][stride] least key of buckets 1, 2, ...
+    uint32_t *runs;             // [C][stride + 1] first bucket of every run, and the end
+    uint32_t *crowded;          // [C][stride] runs (rows of one block: [C]) whose values crowd
+    uint32_t *numbers;          // [5][C]: buckets, runs, positives, least key of the sample, flat buckets
+    uint16_t *fine;             // [C][kBkFine + 2]
+    double *loss_part;          // [C][2 * stride]: runs, wide buckets
+    double *tile_loss;          // [C][tiles] of the flat buckets, where there are any
+    int P, C, tiles, stride;
+};
+
+__device__ __forceinline__ uint32_t bk_limit(const BucketArgs &a, int c) {
+    const uint32_t m = a.pos_max[c];
+    if (m) return m - 1u;
+    const uint32_t lowest = a.pos_max[2 * a.C + c];
+    return lowest <= kOne ? lowest : kOne;
+}
+
+// A term of a class's loss, rounded to a multiple of 2^-51: such terms, and their sums below 4 (a loss is at most 1), are
+// exact in double, so that the sum does not depend on the order of its terms.
+__device__ __forceinline__ double loss_term(float e, float dj) {
+    const double t = (double)(e * dj);
+    return (t + 3.0) - 3.0;
+}
+__device__ __forceinline__ double wave_sum_f64(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// Jaccard difference of the key at rank `pos`, with `cs` of the class's npos positives before it.
+__device__ __forceinline__ float jaccard_step(float npos, uint32_t pos, uint32_t cs, uint32_t hot) {
+    const float inter_prev = npos - (float)cs;                             // csrc/lovasz_softmax.cu:124-127
+    const float inter = npos - (float)(cs + hot);
+    const float j_now = 1.f - inter / (inter + (float)(pos + 1));
+    const float j_prev = (pos == 0) ? 0.f : 1.f - inter_prev / (inter_prev + (float)pos);
+    return j_now - j_prev;                                                 // csrc/lovasz_softmax.cu:141-147
+}
+
+// A key, its place among the block's items and its positive flag, ordered as the stable sort orders them, as a double in
+// [1, 2): the smaller and the larger of two are one instruction each.
+typedef double BkPair;
+__device__ __forceinline__ BkPair bk_pair(uint32_t key, uint32_t item) {
+    const uint32_t k = key & 0x7FFFFFFFu;
+    const uint64_t bits = (uint64_t)(0x3FF00000u | (k >> 18)) << 32 | (k << 14 | item << 1 | key >> 31);
+    return __builtin_bit_cast(double, bits);
+}
+__device__ __forceinline__ uint32_t bk_item_of(BkPair p) { return ((uint32_t)__builtin_bit_cast(uint64_t, p) >> 1) & 0x1FFFu; }
+__device__ __forceinline__ uint32_t bk_hot_of(BkPair p) { return (uint32_t)__builtin_bit_cast(uint64_t, p) & 1u; }
+__device__ __forceinline__ uint32_t bk_key_of(BkPair p) {              // below 2^30: the exponent's bits fall out
+    return (uint32_t)(__builtin_bit_cast(uint64_t, p) >> 14);
+}
+__device__ __forceinline__ BkPair bk_last() { return __builtin_bit_cast(double, (uint64_t)0x3FFFFFFFFFFFFFFFull); }
+static_assert(kBkCap <= 1 << 13 && kOne < 1u << 30, "13 bits of a pair name the item, 30 hold the key");
+
+__device__ __forceinline__ void bk_order(BkPair &a, BkPair &b) {
+    double lo, hi;                              // asm: fmin and fmax would quiet signalling NaNs first
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
+}
+// Batcher's odd-even merges of a chunk's runs of kFrom, 2 kFrom, ... pairs (kFrom = 1: the sort, 63 pairs ordered;
+// kFrom = 8: the merge of its halves, 25).
+template <int kFrom>
+__device__ __forceinline__ void bk_merge(BkPair (&v)[kBkChunk]) {
+#pragma unroll
+    for (int p = kFrom; p < kBkChunk; p *= 2)
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+            for (int i = 0; i < kBkChunk; ++i) {
+                // i and i + k: not across the runs being merged, and only the pairs of this step
+                const bool pair = i >= k % p && ((i - k % p) / k) % 2 == 0 && i + k < kBkChunk && i / (2 * p) == (i + k) / (2 * p);
+                if (pair) bk_order(v[i], v[i + k]);
+            }
+}
+
+struct BkShared {
+    // the pairs, 16 neighbours in the order of thread t in row t; the crowded path's keys and items; the results by item
+    __align__(16) BkPair pair[kBkCap + kBkChunk];
+    __align__(16) uint32_t bin[kBkBins];
+    uint32_t scan[2 * kSortWaves];
+    uint32_t least[kBkWaves], most[kBkWaves], crowd[kBkWaves];
+    __device__ uint32_t *key() { return reinterpret_cast<uint32_t *>(pair); }
+    __device__ uint16_t *src() { return reinterpret_cast<uint16_t *>(pair) + 2 * kBkCap; }
+    // place p of the order: the 16 pairs of a row are turned by half the row's number, so that the rows of 32 lanes
+    // reading one column each fall into different banks
+    __device__ __forceinline__ BkPair &at(uint32_t p) { return pair[p ^ ((p >> 5) & 15u)]; }
+};
+
+// Least and largest of the block's valid keys (least > largest: none).
+__device__ __forceinline__ void bk_range(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, uint32_t &least,
+                                         uint32_t &most) {
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        if (!((valid >> r) & 1u)) continue;
+        const uint32_t k = key[r] & 0x7FFFFFFFu;
+        lo = min(lo, k);
+        hi = max(hi, k);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, off, 64));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, off, 64));
+    }
+    __syncthreads();                            // an earlier use of the words is over
+    if ((threadIdx.x & 63) == 0) {
+        s.least[threadIdx.x >> 6] = lo;
+        s.most[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    least = s.least[0];
+    most = s.most[0];
+#pragma unroll
+    for (int w = 1; w < kBkWaves; ++w) {
+        least = min(least, s.least[w]);
+        most = max(most, s.most[w]);
+    }
+}
+
+// Where item r of this thread stands in the block's order of `rounds` x 512 items: a wave's items are neighbours.
+__device__ __forceinline__ int bk_item(int rounds, int r) {
+    return ((int)(threadIdx.x >> 6) * rounds + r) * kWave + (int)(threadIdx.x & 63);
+}
+
+// Sorts the block's valid keys (n of them in all, in `rounds` x 512 items): v[e] becomes the pair at place 16 t + e of the
+// order for thread t, bk_last() past the end. False (block-uniform) where values crowd: then bk_ranks_crowded has to do it.
+// from: no valid key is below it, except that such keys share the first bin; scale: bins per unit of key, below
+// kBkBins / (largest key - from + 1).
+//
+// Counting the keys into 4096 bins of their range puts them in order but for the one or two per bin; those are sorted by
+// the threads, 16 places each, then across the chunks' borders (8 places of either side) and within the chunks in turn:
+// odd-even transposition of halves of 8, of which a bin of L keys touches at most 2 + (L - 2) / 8.
+__device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds, uint32_t from,
+                                        float scale, uint32_t &n, BkPair (&v)[kBkChunk]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // monotone in the key, and at most kBkBins - 1 by the choice of scale
+    auto bin_of = [&](uint32_t k) {
+        k &= 0x7FFFFFFFu;
+        return (uint32_t)((float)(max(k, from) - from) * scale);
+    };
+    {
+        uint4 *b4 = reinterpret_cast<uint4 *>(s.bin);
+#pragma unroll
+        for (int i = 0; i < kBkBins / 4 / kBkThreads; ++i) b4[i * kBkThreads + threadIdx.x] = make_uint4(0, 0, 0, 0);
+    }
+    __syncthreads();
+    uint32_t slot[kBkItems];                    // bin << 16 | arrival
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        slot[r] = 0;
+        if (r < rounds && ((valid >> r) & 1u)) {
+            const uint32_t b = min(bin_of(key[r]), (uint32_t)kBkBins - 1u);
+            slot[r] = b << 16 | atomicAdd(&s.bin[b], 1u);
+        }
+    }
+    __syncthreads();
+    constexpr int kPer = kBkBins / kBkThreads;
+    uint32_t mine[kPer], sum = 0, crowd = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        mine[i] = s.bin[threadIdx.x * kPer + i];
+        sum += mine[i];
+        crowd = max(crowd, mine[i]);
+    }
+    const float wave_crowd = group_reduce<64>((float)crowd, OpMax());
+    if (lane == 0) s.crowd[wave] = (uint32_t)wave_crowd;
+    uint32_t run = block_excl_scan(sum, s.scan, n);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        s.bin[threadIdx.x * kPer + i] = run;
+        run += mine[i];
+    }
+#pragma unroll
+    for (int w = 0; w < kBkWaves; ++w) crowd = max(crowd, s.crowd[w]); // written before the scan's barriers
+    crowd = (uint32_t)__builtin_amdgcn_readfirstlane((int)crowd);
+    __syncthreads();
+    if (crowd > kBkCrowd) return false;
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r)
+        if (r < rounds && ((valid >> r) & 1u))
+            s.at(s.bin[slot[r] >> 16] + (slot[r] & 0xFFFFu)) = bk_pair(key[r], (uint32_t)bk_item(rounds, r));
+    __syncthreads();
+    const uint32_t p0 = threadIdx.x * kBkChunk;
+    const bool busy = p0 < n;
+    if (busy) {
+#pragma unroll
+        for (int e = 0; e < kBkChunk; ++e) v[e] = p0 + e < n ? s.at(p0 + e) : bk_last();
+        bk_merge<1>(v);
+    }
+    const bool next = p0 + kBkChunk < n;        // the thread above holds places too
+    int left = crowd < 2u ? 0 : 1 + (int)(crowd - 2u) / 8;             // steps after the first
+#pragma unroll 1
+    while (left > 0) {                          // block-uniform
+        uint32_t p0 = threadIdx.x * kBkChunk;
+        asm volatile("" : "+v"(p0));            // the places' addresses stay in the loop, not in 24 registers
+        if (busy) {
+#pragma unroll
+            for (int e = 0; e < kBkChunk / 2; ++e) s.at(p0 + e) = v[e];
+        }
+        __syncthreads();
+        if (next) {
+            BkPair w[kBkChunk];
+#pragma unroll
+            for (int e = 0; e < kBkChunk / 2; ++e) {
+                w[e] = v[kBkChunk / 2 + e];
+                w[kBkChunk / 2 + e] = s.at(p0 + kBkChunk + e);
+            }
+            bk_merge<kBkChunk / 2>(w);
+#pragma unroll
+            for (int e = 0; e < kBkChunk / 2; ++e) {
+                v[kBkChunk / 2 + e] = w[e];
+                s.at(p0 + kBkChunk + e) = w[kBkChunk / 2 + e];
+            }
+        }
+        __syncthreads();
+        if (busy && p0) {
+#pragma unroll
+            for (int e = 0; e < kBkChunk / 2; ++e) v[e] = s.at(p0 + e);
+        }
+        if (busy && left > 1) bk_merge<kBkChunk / 2>(v);
+        left -= 2;
+    }
+    __syncthreads();                            // s.pair is free again
+    return true;
+}
+
+__device__ __forceinline__ float bk_scale(uint32_t from, uint32_t to) {       // bins for the keys from..to
+    return (float)(kBkBins - 1) / (float)(to - from + 1u);
+}
+
+// rank[r] = valid keys of the block that sort before key[r] (equal keys in item order) | positives among them << 16, for
+// values that crowd (ties, clusters): a stable radix sort in LDS, 6 bits a pass over the bits of the range least..most.
+__device__ __forceinline__ void bk_ranks_crowded(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds, uint32_t least,
+                                 uint32_t most, uint32_t (&rank)[kBkItems]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t span = most - least + 1u;    // valid keys exist; keys are below 2^30
+    uint32_t slot[kBkItems];
+    // items without a key take the value after the largest
+    uint32_t k2[kBkItems], it[kBkItems];
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        const bool v = r < rounds && ((valid >> r) & 1u);
+        k2[r] = v ? (key[r] & 0x80000000u) | ((key[r] & 0x7FFFFFFFu) - least) : span;
+        it[r] = (uint32_t)bk_item(rounds, r);
+    }
+    uint16_t *counts = reinterpret_cast<uint16_t *>(s.bin);        // [kBkWaves][64], then their exclusive sums
+    const int bits = 32 - __builtin_clz(span);
+    for (int shift = 0; shift < bits; shift += 6) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < kBkWaves * 64 / 2; i += kBkThreads) s.bin[i] = 0;
+        __syncthreads();
+        const int width = min(6, bits - shift);
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            slot[r] = 0;
+            if (r < rounds) {
+                const uint32_t digit = ((k2[r] & 0x7FFFFFFFu) >> shift) & 63u;
+                uint32_t unused;
+                wave_rank_of<false>(wave_peers_n(digit, true, width), digit, true, false, counts + wave * 64, nullptr, slot[r], unused);
+            }
+        }
+        __syncthreads();
+        const int d = threadIdx.x >> 3, w = threadIdx.x & 7;       // order: digit, then wave
+        const uint32_t n = counts[w * 64 + d];
+        uint32_t all;
+        const uint32_t start = block_excl_scan(n, s.scan, all);
+        counts[w * 64 + d] = (uint16_t)start;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            if (r < rounds) {
+                const uint32_t at = counts[wave * 64 + (((k2[r] & 0x7FFFFFFFu) >> shift) & 63u)] + slot[r];
+                s.key()[at] = k2[r];
+                s.src()[at] = (uint16_t)it[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            if (r < rounds) {
+                k2[r] = s.key()[bk_item(rounds, r)];
+                it[r] = s.src()[bk_item(rounds, r)];
+            }
+        }
+    }
+    // positives before each place, then back to the items
+    uint32_t hot_here[kBkItems], wave_hot = 0;
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        hot_here[r] = 0;
+        if (r < rounds) {
+            const uint64_t vote = __builtin_amdgcn_ballot_w64(k2[r] >> 31);
+            hot_here[r] = wave_hot + peers_below(vote);
+            wave_hot += (uint32_t)__builtin_popcountll(vote);
+        }
+    }
+    __syncthreads();
+    uint32_t all;
+    const uint32_t before = block_excl_scan(lane == 0 ? wave_hot : 0u, s.scan, all);
+    const uint32_t wave_before = (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r)
+        if (r < rounds) s.key()[it[r]] = (uint32_t)bk_item(rounds, r) | (wave_before + hot_here[r]) << 16;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) rank[r] = r < rounds ? s.key()[bk_item(rounds, r)] : 0u;
+    __syncthreads();
+}
+
+// Bounds of a class's buckets from kBkCap sampled keys, one from each of as many equal parts of the row: every
+// (sample / buckets)-th key in their order. A value that would bound two buckets gets one to itself: (v, v + 1).
+__global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
+    __shared__ BkShared s;
+    const int c = blockIdx.x;
+    const uint32_t limit = bk_limit(a, c);
+    const uint32_t *row = a.keys + (int64_t)c * a.P;
+    uint32_t key[kBkItems], valid = 0, mine = 0;
+    const uint32_t part = (uint32_t)a.P / kBkCap;           // >= 1: shorter rows are not cut
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        const uint32_t i = (uint32_t)bk_item(kBkItems, r);
+        uint32_t h = i * 0x9E3779B1u;                       // somewhere in the part, so that no stride meets the image's
+        h = (h ^ (h >> 15)) * 0x85EBCA6Bu;
+        key[r] = row[(uint32_t)((uint64_t)i * (uint32_t)a.P / kBkCap) + __umulhi(h, part)];
+    }
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r)
+        if (keep_key(key[r], limit)) {
+            valid |= 1u << r;
+            ++mine;
+        }
+    uint32_t n;
+    block_excl_scan(mine, s.scan, n);
+    uint32_t want = 1, least, most;
+    bk_range(s, key, valid, least, most);
+    uint32_t *sorted = s.key();
+    if (n > 0) {                                            // block-uniform
+        BkPair v[kBkChunk];
+        uint32_t m;
+        if (bk_sort(s, key, valid, kBkItems, least, bk_scale(least, most), m, v)) {
+#pragma unroll
+            for (int e = 0; e < kBkChunk; ++e)
+                if (threadIdx.x * kBkChunk + e < n) sorted[threadIdx.x * kBkChunk + e] = bk_key_of(v[e]);
+        } else {
+            uint32_t rank[kBkItems];
+            bk_ranks_crowded(s, key, valid, kBkItems, least, most, rank);
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r)
+                if ((valid >> r) & 1u) sorted[rank[r] & 0xFFFFu] = key[r] & 0x7FFFFFFFu;
+        }
+        const uint64_t keys = (uint64_t)n * (uint32_t)a.P / kBkCap;
+        want = (uint32_t)((keys + kBkTarget - 1) / kBkTarget);
+        want = min(max(want, 1u), (uint32_t)a.stride);
+    }
+    __syncthreads();
+    // candidates 1..want-1, a run of neighbours per thread; the bounds are collected where the bins were
+    const int per = kBkMax / kBkThreads;
+    auto candidate = [&](uint32_t j) { return sorted[j * n / want]; };         // below 2^24
+    uint32_t out = 0;
+    for (int u = 0; u < per; ++u) {
+        const uint32_t j = 1u + threadIdx.x * per + u;
+        if (j >= want) break;
+        const uint32_t v = candidate(j);
+        if (j > 1 && candidate(j - 1) == v) continue;
+        out += (j + 1 < want && candidate(j + 1) == v) ? 2u : 1u;
+    }
+    uint32_t bounds;
+    uint32_t at = block_excl_scan(out, s.scan, bounds);
+    for (int u = 0; u < per; ++u) {
+        const uint32_t j = 1u + threadIdx.x * per + u;
+        if (j >= want) break;
+        const uint32_t v = candidate(j);
+        if (j > 1 && candidate(j - 1) == v) continue;
+        s.bin[at++] = v;
+        if (j + 1 < want && candidate(j + 1) == v) s.bin[at++] = v + 1u;
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < bounds; i += kBkThreads) a.bounds[(int64_t)c * a.stride + i] = s.bin[i];
+    if (threadIdx.x == 0) {
+        a.numbers[c] = bounds + 1u;
+        a.numbers[3 * a.C + c] = n ? least : 0u;
+    }
+    // the bucket of the least key with each pattern of the top bits
+    const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
+    for (int f = threadIdx.x; f <= kBkFine; f += kBkThreads) {
+        const uint32_t k = (uint32_t)f << shift;
+        uint32_t lo = 0, hi = bounds;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (s.bin[mid] <= k) lo = mid + 1;
+            else hi = mid;
+        }
+        a.fine[(int64_t)c * (kBkFine + 2) + f] = (uint16_t)lo;
+    }
+}
+
+// The bounds and the table in LDS.
+template <int kStride>
+struct BkLookup {
+    uint32_t bounds[kStride];
+    uint32_t fine2[kBkFine / 2 + 1];
+    __device__ void fetch(const BucketArgs &a, int c, uint32_t buckets) {
+        for (uint32_t i = threadIdx.x; i + 1 < buckets; i += kBkThreads) bounds[i] = a.bounds[(int64_t)c * kStride + i];
+        const uint32_t *f = reinterpret_cast<const uint32_t *>(a.fine + (int64_t)c * (kBkFine + 2));
+        for (int i = threadIdx.x; i <= kBkFine / 2; i += kBkThreads) fine2[i] = f[i];
+    }
+    // bucket of a key that takes part (key bits below 2^bits)
+    __device__ __forceinline__ uint32_t find(uint32_t key, int shift) const {
+        const uint16_t *fine = reinterpret_cast<const uint16_t *>(fine2);
+        const uint32_t f = key >> shift;
+        uint32_t lo = fine[f], hi = fine[f + 1];
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (bounds[mid] <= key) lo = mid + 1;
+            else hi = mid;
+        }
+        return lo;
+    }
+};
+
+template <int kStride>
+__global__ __launch_bounds__(kBkThreads) void bk_hist(const BucketArgs a) {
+    __shared__ BkLookup<kStride> look;
+    __shared__ uint32_t counts[kStride];
+    const int c = blockIdx.y, tile = blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
+    const uint32_t *kin = a.keys + (int64_t)c * a.P + begin;
+    uint32_t key[kBkTileItems];
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int li = bk_item(kBkTileItems, r);
+        key[r] = li < n ? kin[li] : kIgnoredKey;
+    }
+    const uint32_t buckets = a.numbers[c], limit = bk_limit(a, c);
+    const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
+    look.fetch(a, c, buckets);
+    for (uint32_t i = threadIdx.x; i < buckets; i += kBkThreads) counts[i] = 0;
+    __syncthreads();
+    uint16_t *bucket = a.bucket + (int64_t)c * a.P + begin;
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int li = bk_item(kBkTileItems, r);
+        const bool valid = keep_key(key[r], limit);
+        const uint64_t vmask = __builtin_amdgcn_ballot_w64(valid);
+        uint32_t b = kBkNowhere;
+        if (valid) b = look.find(key[r] & 0x7FFFFFFFu, shift);
+        if (li < n) bucket[li] = (uint16_t)b;
+        if (vmask == 0) continue;                           // wave-uniform
+        const uint32_t one = (uint32_t)__builtin_amdgcn_readlane((int)b, __builtin_ctzll(vmask));
+        if (__builtin_amdgcn_ballot_w64(valid && b == one) == vmask) {          // one bucket for the whole round
+            const uint64_t hot = __builtin_amdgcn_ballot_w64(valid && (key[r] >> 31));
+            if (lane == 0)
+                atomicAdd(&counts[one], (uint32_t)__builtin_popcountll(vmask) | (uint32_t)__builtin_popcountll(hot) << 16);
+        } else if (valid) {
+            atomicAdd(&counts[b], 1u | (key[r] >> 31) << 16);
+        }
+    }
+    __syncthreads();
+    uint32_t *out = a.tile_count + ((int64_t)c * a.tiles + tile) * kStride;
+    for (uint32_t i = threadIdx.x; i < buckets; i += kBkThreads) out[i] = counts[i];
+}
+
+// 64 buckets x 16 groups of tiles per block: the group's sums first, then the exclusive sums in place.
+__global__ __launch_bounds__(1024) void bk_scan(const BucketArgs a) {
+    __shared__ uint32_t sums[16][64], hots[16][64];
+    const int c = blockIdx.y, b = blockIdx.x * 64 + (threadIdx.x & 63), group = threadIdx.x >> 6;
+    const int buckets = (int)a.numbers[c];
+    if ((int)blockIdx.x * 64 >= buckets) return;            // block-uniform
+    const int per = (a.tiles + 15) / 16, first = group * per, last = min(a.tiles, first + per);
+    uint32_t *at = a.tile_count + (int64_t)c * a.tiles * a.stride + b;
+    uint32_t n = 0, h = 0;
+    if (b < buckets) {
+#pragma unroll 8
+        for (int t = first; t < last; ++t) {
+            const uint32_t v = at[(int64_t)t * a.stride];
+            n += v & 0xFFFFu;
+            h += v >> 16;
+        }
+    }
+    sums[group][threadIdx.x & 63] = n;
+    hots[group][threadIdx.x & 63] = h;
+    __syncthreads();
+    if (b >= buckets) return;
+    uint32_t before = 0, total = 0, hot = 0;
+#pragma unroll
+    for (int g = 0; g < 16; ++g) {
+        const uint32_t v = sums[g][threadIdx.x & 63];
+        before += g < group ? v : 0u;
+        total += v;
+        hot += hots[g][threadIdx.x & 63];
+    }
+    if (total > (uint32_t)kBkCap) {
+        uint32_t *hot_at = a.tile_hot + (int64_t)c * a.tiles * a.stride + b;
+        uint32_t hot_before = 0;
+        for (int g = 0; g < group; ++g) hot_before += hots[g][threadIdx.x & 63];
+        for (int t = first; t < last; ++t) {
+            hot_at[(int64_t)t * a.stride] = hot_before;
+            hot_before += at[(int64_t)t * a.stride] >> 16;
+        }
+    }
+#pragma unroll 8
+    for (int t = first; t < last; ++t) {
+        const uint32_t v = at[(int64_t)t * a.stride];
+        at[(int64_t)t * a.stride] = before;
+        before += v & 0xFFFFu;
+    }
+    if (group == 0) {
+        a.count[(int64_t)c * a.stride + b] = total;
+        a.hot[(int64_t)c * a.stride + b] = hot;
+    }
+}
+
+// Where the buckets start, and the runs of them that one block sorts: neighbours that start in the same kBkSlab keys of the
+// row, unless they come to more than kBkCap, or lie so differently dense that bins of one width would not do.
+__global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
+    __shared__ uint32_t base[kBkMax + 1], bound[kBkMax + 1], scan_tmp[2 * kSortWaves];
+    constexpr int kPer = kBkMax / kBkThreads;
+    const int c = blockIdx.x, buckets = (int)a.numbers[c], b0 = threadIdx.x * kPer;
+    uint32_t n[kPer], h[kPer], n_sum = 0, h_sum = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const bool is = b0 + i < buckets;
+        n[i] = is ? a.count[(int64_t)c * a.stride + b0 + i] : 0u;
+        h[i] = is ? a.hot[(int64_t)c * a.stride + b0 + i] : 0u;
+        bound[b0 + i] = b0 + i + 1 < buckets ? a.bounds[(int64_t)c * a.stride + b0 + i] : bk_limit(a, c) + 1u;  // of the next bucket
+        n_sum += n[i];
+        h_sum += h[i];
+    }
+    uint32_t at, n_all, at_hot, n_hot;
+    block_excl_scan2(n_sum, h_sum, scan_tmp, at, n_all, at_hot, n_hot);
+    const int64_t row = (int64_t)c * (a.stride + 1);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        base[b0 + i] = at;
+        if (b0 + i <= buckets) {
+            a.base[row + b0 + i] = at;
+            a.hot_base[row + b0 + i] = at_hot;
+        }
+        at += n[i];
+        at_hot += h[i];
+    }
+    if (threadIdx.x == kBkThreads - 1) {
+        base[kBkMax] = at;
+        if (buckets == kBkMax) {
+            a.base[row + kBkMax] = at;
+            a.hot_base[row + kBkMax] = at_hot;
+        }
+    }
+    __syncthreads();
+    const uint32_t least = a.numbers[3 * a.C + c];
+    auto width = [&](int b) { return (float)(bound[b] - (b ? bound[b - 1] : min(least, bound[0]))) / (float)(base[b + 1] - base[b] + 1u); };
+    bool start[kPer];
+    uint32_t starts = 0, flats = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int b = b0 + i;
+        start[i] = false;
+        if (b >= buckets) continue;
+        if (n[i] > (uint32_t)kBkCap && b && bound[b] - bound[b - 1] == 1u) {
+            a.count[(int64_t)c * a.stride + b] = n[i] | kBkFlat;
+            flats = 1;
+        }
+        const uint32_t slab = base[b] / kBkSlab;
+        start[i] = b == 0 || base[b - 1] / kBkSlab != slab;
+        if (!start[i]) {
+            int f = b - 1;                      // first bucket of the slab: few are empty or small
+            while (f > 0 && base[f - 1] / kBkSlab == slab) --f;
+            const float w = width(b), w1 = width(b - 1);
+            // only a slab's last bucket can take it past kBkCap, or past it alone
+            start[i] = base[b + 1] - base[f] > (uint32_t)kBkCap || w > 4.f * w1 || w1 > 4.f * w;
+        }
+        starts += start[i] ? 1u : 0u;
+    }
+    uint32_t runs, any_flat, unused;
+    uint32_t k;
+    block_excl_scan2(starts, flats, scan_tmp, k, runs, unused, any_flat);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+        if (start[i]) a.runs[row + k++] = (uint32_t)(b0 + i);
+    if (threadIdx.x == 0) {
+        a.runs[row + runs] = (uint32_t)buckets;
+        a.numbers[a.C + c] = runs;
+        a.numbers[2 * a.C + c] = n_hot;
+        a.numbers[4 * a.C + c] = any_flat;
+    }
+}
+
+template <int kBits>
+__device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
+    uint32_t diff_lo = 0, diff_hi = 0;
+#pragma unroll
+    for (int b = 0; b < kBits; ++b) {
+        uint32_t splat = (uint32_t)((int32_t)(digit << (31 - b)) >> 31);
+        asm("" : "+v"(splat));
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(splat != 0u);
+        diff_lo |= (uint32_t)vote ^ splat;
+        diff_hi |= (uint32_t)(vote >> 32) ^ splat;
+    }
+    const uint64_t diff = ((uint64_t)diff_hi << 32) | diff_lo;
+    return __builtin_amdgcn_ballot_w64(valid) & ~diff;
+}
+
+// The tile's keys by bucket, written out in runs. In the place of the tile's keys it leaves, in 16 bits each, every pixel's
+// place in the tile's order, then the bucket of every place.
+template <int kBits>
+__global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
+    constexpr int kStride = 1 << kBits, kPer = (kStride + kBkThreads - 1) / kBkThreads;
+    __shared__ uint32_t s_key[kBkTile];                     // the tile by bucket
+    __shared__ uint16_t s_bucket[kBkTile];
+    __shared__ __align__(4) uint16_t counts[kBkWaves][kStride];
+    __shared__ uint32_t start[kStride], out_base[kStride];
+    __shared__ uint32_t scan_tmp[kSortWaves];
+    const int c = blockIdx.y, wave = threadIdx.x >> 6;
+    const int tile = sort_tile(a.P, kBkTile);
+    const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
+    uint32_t *kin = a.keys + (int64_t)c * a.P + begin;
+    uint32_t key[kBkTileItems], b[kBkTileItems], rank[kBkTileItems];
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int li = bk_item(kBkTileItems, r);
+        key[r] = li < n ? kin[li] : 0u;
+        b[r] = li < n ? a.bucket[(int64_t)c * a.P + begin + li] : kBkNowhere;
+    }
+    const uint32_t buckets = a.numbers[c];
+    uint32_t first[kPer];
+    uint32_t *table = a.tile_count + ((int64_t)c * a.tiles + tile) * kStride;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = threadIdx.x * kPer + i;
+        first[i] = d < buckets ? table[d] + a.base[(int64_t)c * (kStride + 1) + d] : 0u;
+    }
+    for (int i = threadIdx.x; i < kBkWaves * kStride / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(&counts[0][0])[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const bool valid = b[r] != kBkNowhere;
+        rank[r] = 0;
+        if (__builtin_amdgcn_ballot_w64(valid) == 0) continue;      // wave-uniform
+        uint32_t unused;
+        wave_rank_of<false>(bk_peers<kBits>(b[r], valid), b[r], valid, false, counts[wave], nullptr, rank[r], unused);
+    }
+    __syncthreads();
+    uint32_t mine[kPer], n_mine = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = threadIdx.x * kPer + i;
+        mine[i] = 0;
+        if (d < buckets) {
+#pragma unroll
+            for (int w = 0; w < kBkWaves; ++w) {
+                const uint32_t t = counts[w][d];
+                counts[w][d] = (uint16_t)mine[i];
+                mine[i] += t;
+            }
+        }
+        n_mine += mine[i];
+    }
+    uint32_t n_here;
+    uint32_t at = block_excl_scan(n_mine, scan_tmp, n_here);
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = threadIdx.x * kPer + i;
+        if (d < buckets) {
+            start[d] = at;
+            out_base[d] = first[i] - at;
+            table[d] = first[i] - at;
+        }
+        at += mine[i];
+    }
+    __syncthreads();
+    uint16_t *places = reinterpret_cast<uint16_t *>(kin);
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int li = bk_item(kBkTileItems, r);
+        if (li >= n) continue;
+        uint32_t pos = kBkNowhere;
+        if (b[r] != kBkNowhere) {
+            pos = start[b[r]] + counts[wave][b[r]] + rank[r];
+            s_key[pos] = key[r];
+            s_bucket[pos] = (uint16_t)b[r];
+        }
+        places[li] = (uint16_t)pos;
+    }
+    __syncthreads();
+    uint32_t *kout = a.sorted + (int64_t)c * a.P;
+    for (int i = threadIdx.x; i < (int)n_here; i += kBkThreads) {
+        const uint32_t d = s_bucket[i];
+        kout[out_base[d] + (uint32_t)i] = s_key[i];
+        places[n + i] = (uint16_t)d;
+    }
+    if (a.numbers[4 * a.C + c] == 0) return;                // block-uniform
+    // Buckets of a single value that no block would hold: their keys are in order, so the place is the rank; the positives
+    // before it are those of the buckets before, of the tiles before and of the places before. A thread takes 16 neighbours.
+    __shared__ double wave_loss[kBkWaves];
+    uint32_t *hot_start = reinterpret_cast<uint32_t *>(counts);       // positives of the tile before each bucket
+    const uint32_t p0 = threadIdx.x * kBkTileItems;
+    uint32_t hots = 0, all;
+#pragma unroll
+    for (int e = 0; e < kBkTileItems; ++e) hots += p0 + e < n_here ? s_key[p0 + e] >> 31 : 0u;
+    uint32_t cs = block_excl_scan(hots, scan_tmp, all);
+    {
+        uint32_t before = cs;
+#pragma unroll
+        for (int e = 0; e < kBkTileItems; ++e) {
+            if (p0 + e < n_here) {
+                const uint32_t d = s_bucket[p0 + e];
+                if (start[d] == p0 + e) hot_start[d] = before;
+                before += s_key[p0 + e] >> 31;
+            }
+        }
+    }
+    __syncthreads();
+    const float npos = (float)a.numbers[2 * a.C + c];
+    double part = 0.0;
+    for (int e = 0; e < kBkTileItems; ++e) {
+        if (p0 + e >= n_here) break;
+        const uint32_t d = s_bucket[p0 + e], k = s_key[p0 + e];
+        if (a.count[(int64_t)c * kStride + d] & kBkFlat) {
+            const uint32_t pos = out_base[d] + p0 + e;
+            const uint32_t hot_before = a.hot_base[(int64_t)c * (kStride + 1) + d] +
+                                        a.tile_hot[((int64_t)c * a.tiles + tile) * kStride + d] + (cs - hot_start[d]);
+            const float dj = jaccard_step(npos, pos, hot_before, k >> 31);
+            part += loss_term(key_error(k), dj);
+            a.dj[(int64_t)c * a.P + pos] = dj;
+        }
+        cs += k >> 31;
+    }
+    part = wave_sum_f64(part);
+    if ((threadIdx.x & 63) == 0) wave_loss[wave] = part;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
+        a.tile_loss[(int64_t)c * a.tiles + tile] = sum;
+    }
+}
+
+// One run of buckets (or, Direct: a whole row of at most kBkCap pixels, straight from the keys in pixel order, with the
+// Jaccard differences left in their place and the loss complete).
+// Time goes into vector instructions, about 110 per 64 keys: a thread's places of the order are neighbours, so that a
+// difference is one new quotient less the one before, and the positives before a place are a sum over the block's threads.
+template <bool Direct>
+__global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, float *__restrict__ losses) {
+    __shared__ BkShared s;
+    __shared__ double wave_loss[kBkWaves];
+    const int c = Direct ? blockIdx.x : blockIdx.y, g = Direct ? 0 : blockIdx.x;
+    const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
+    if (!Direct && g >= (int)a.numbers[a.C + c]) return;    // block-uniform
+    const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
+    const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
+    const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
+    if (!Direct && (n > kBkCap || n == 0)) {                // block-uniform; too many are bk_rank_wide's
+        if (threadIdx.x == 0) {
+            a.loss_part[2 * (int64_t)c * a.stride + g] = 0.0;
+            a.crowded[(int64_t)c * a.stride + g] = 0u;
+        }
+        return;
+    }
+    const uint32_t *kin = Direct ? a.keys + row : a.sorted + row + rank0;
+    float *out = Direct ? reinterpret_cast<float *>(a.keys) + row : a.dj + row + rank0;
+    const uint32_t limit = bk_limit(a, c);
+    float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
+
+    uint32_t key[kBkItems], valid = 0, least, most;
+    const int rounds = (n + kBkThreads - 1) / kBkThreads;
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        const int li = bk_item(rounds, r);
+        key[r] = 0;
+        if (r < rounds && li < n) {
+            key[r] = kin[li];
+            if (!Direct || keep_key(key[r], limit)) valid |= 1u << r;
+        }
+    }
+    if constexpr (Direct) {
+        bk_range(s, key, valid, least, most);
+        uint32_t hot = 0, all;
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) hot += ((valid >> r) & 1u) ? key[r] >> 31 : 0u;
+        block_excl_scan(hot, s.scan, all);
+        npos = (float)all;
+        most = max(least, most);                            // no valid key: nothing below looks at the range
+    } else {
+        const uint32_t *bound = a.bounds + (int64_t)c * a.stride;
+        most = b1 < a.numbers[c] ? bound[b1 - 1] - 1u : limit;
+        if (b0) least = bound[b0 - 1];
+        else bk_range(s, key, valid, least, most);          // below the least of the sample lie a few more
+    }
+    double part = 0.0;
+    BkPair v[kBkChunk];
+    uint32_t kept;
+    float *result = reinterpret_cast<float *>(s.pair);      // by item
+    if (bk_sort(s, key, valid, rounds, least, bk_scale(least, most), kept, v)) {       // block-uniform
+        const uint32_t p0 = threadIdx.x * kBkChunk;
+        uint32_t hot = 0, all;
+#pragma unroll
+        for (int e = 0; e < kBkChunk; ++e) hot += p0 + e < kept ? bk_hot_of(v[e]) : 0u;
+        uint32_t cs = hot0 + block_excl_scan(hot, s.scan, all);
+        if (p0 < kept) {
+            uint32_t pos = rank0 + p0;
+            float inter = npos - (float)cs;                                            // csrc/lovasz_softmax.cu:124-127
+            float j_prev = pos == 0 ? 0.f : 1.f - inter / (inter + (float)pos);
+#pragma unroll
+            for (int e = 0; e < kBkChunk; ++e) {
+                if (p0 + e < kept) {
+                    cs += bk_hot_of(v[e]);
+                    inter = npos - (float)cs;
+                    const float j_now = 1.f - inter / (inter + (float)(pos + 1u + e));
+                    const float dj = j_now - j_prev;                                   // csrc/lovasz_softmax.cu:141-147
+                    j_prev = j_now;
+                    part += loss_term(key_error(bk_key_of(v[e])), dj);
+                    result[bk_item_of(v[e])] = dj;
+                }
+            }
+        }
+    } else {                                                // bk_rank_crowded's
+        if (threadIdx.x == 0) a.crowded[Direct ? c : (int64_t)c * a.stride + g] = 1u;
+        return;
+    }
+    part = wave_sum_f64(part);
+    if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        const int li = bk_item(rounds, r);
+        if (r < rounds && li < n) out[li] = (!Direct || ((valid >> r) & 1u)) ? result[li] : 0.f;
+    }
+    if (threadIdx.x == 0) {
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
+        if constexpr (Direct) losses[c] = (float)sum;
+        else a.loss_part[2 * (int64_t)c * a.stride + g] = sum;
+        a.crowded[Direct ? c : (int64_t)c * a.stride + g] = 0u;
+    }
+}
+
+// The runs (Direct: rows of one block) whose values crowd.
+template <bool Direct>
+__global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArgs a, float *__restrict__ losses) {
+    __shared__ BkShared s;
+    __shared__ double wave_loss[kBkWaves];
+    const int c = Direct ? blockIdx.x : blockIdx.y;
+    const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
+    const int runs = Direct ? 1 : (int)a.numbers[a.C + c];
+    for (int g = Direct ? 0 : blockIdx.x; g < runs; g += gridDim.x) {       // block-uniform
+        if (!a.crowded[Direct ? c : (int64_t)c * a.stride + g]) {
+            if (Direct) return;
+            continue;
+        }
+        const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
+        const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
+        const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
+        const uint32_t *kin = Direct ? a.keys + row : a.sorted + row + rank0;
+        float *out = Direct ? reinterpret_cast<float *>(a.keys) + row : a.dj + row + rank0;
+        const uint32_t limit = bk_limit(a, c);
+        const int rounds = (n + kBkThreads - 1) / kBkThreads;
+        uint32_t key[kBkItems], rank[kBkItems], valid = 0, hot = 0, least, most;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            const int li = bk_item(rounds, r);
+            key[r] = r < rounds && li < n ? kin[li] : kIgnoredKey;
+            if (keep_key(key[r], limit)) {
+                valid |= 1u << r;
+                hot += key[r] >> 31;
+            }
+        }
+        float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
+        if constexpr (Direct) {
+            uint32_t all;
+            block_excl_scan(hot, s.scan, all);
+            npos = (float)all;
+        }
+        bk_range(s, key, valid, least, most);
+        bk_ranks_crowded(s, key, valid, rounds, least, most, rank);    // keys crowd, so there are some
+        double part = 0.0;
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            const int li = bk_item(rounds, r);
+            if (r < rounds && li < n) {
+                float dj = 0.f;
+                if ((valid >> r) & 1u) {
+                    const uint32_t k = Direct ? key[r] : kin[li];       // read again: not held across the sort
+                    dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), k >> 31);
+                    part += loss_term(key_error(k), dj);
+                }
+                out[li] = dj;
+            }
+        }
+        part = wave_sum_f64(part);
+        if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
+            if constexpr (Direct) losses[c] = (float)sum;
+            else a.loss_part[2 * (int64_t)c * a.stride + g] = sum;
+        }
+        if (Direct) return;
+    }
+}
+
+// n keys from rank `rank0` on, with hot0 positives before them, whatever their number and values: ranges of values
+// [from, end) with at most kBkCap keys, one after the other, collected in order; a single value that more keys share is
+// ranked by position. n is at most a few times kBkCap unless one value makes it up.
+__device__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, int n) {
+    const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
+    float *out = a.dj + (int64_t)c * a.P + rank0;
+    const float npos = (float)a.numbers[2 * a.C + c];
+    double part = 0.0;
+    uint32_t key[kBkItems], rank[kBkItems], valid = 0, least, most;
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+            for (int i = threadIdx.x; i < n; i += kBkThreads) {
+                const uint32_t k = kin[i] & 0x7FFFFFFFu;
+                lo = min(lo, k);
+                hi = max(hi, k);
+            }
+            key[0] = lo;
+            bk_range(s, key, 1u, least, most);
+            uint32_t unused;
+            key[0] = hi;
+            bk_range(s, key, 1u, unused, most);
+            uint32_t from = least, done = 0;
+            int shift = 32 - (int)__builtin_clz((most - from) | 1u);
+            shift = shift > 12 ? shift - 12 : 0;
+            while (done < (uint32_t)n) {                        // a turn takes keys or narrows the bins (shift falls)
+                __syncthreads();
+                for (int i = threadIdx.x; i < kBkBins; i += kBkThreads) s.bin[i] = 0;
+                __syncthreads();
+                for (int i = threadIdx.x; i < n; i += kBkThreads) {
+                    const uint32_t k = kin[i] & 0x7FFFFFFFu;
+                    if (k >= from && ((k - from) >> shift) < (uint32_t)kBkBins) atomicAdd(&s.bin[(k - from) >> shift], 1u);
+                }
+                __syncthreads();
+                constexpr int kPer = kBkBins / kBkThreads;
+                uint32_t sum = 0, total;
+                for (int i = 0; i < kPer; ++i) sum += s.bin[threadIdx.x * kPer + i];
+                uint32_t run = block_excl_scan(sum, s.scan, total);
+                uint32_t bins = 0, keys = 0;                    // leading bins that fit together, and their keys
+                for (int i = 0; i < kPer; ++i) {
+                    run += s.bin[threadIdx.x * kPer + i];
+                    if (run <= (uint32_t)kBkCap) {
+                        ++bins;
+                        keys = run;
+                    }
+                }
+                uint32_t take, take_keys, d0, d1;
+                block_excl_scan2(bins, 0u, s.scan, d0, take, d1, unused);
+                {
+                    uint32_t m = keys;
+    #pragma unroll
+                    for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+                    if ((threadIdx.x & 63) == 0) s.crowd[threadIdx.x >> 6] = m;
+                    __syncthreads();
+                    take_keys = 0;
+                    for (int w = 0; w < kBkWaves; ++w) take_keys = max(take_keys, s.crowd[w]);
+                    __syncthreads();
+                }
+                if (take_keys == 0 && take < (uint32_t)kBkBins && shift > 0) {       // the first bin with keys is too full
+                    from += take << shift;
+                    shift = shift > 12 ? shift - 12 : 0;
+                    continue;
+                }
+                const bool single = take_keys == 0;             // ... and holds a single value
+                // 64 bits: the last range may end past 2^32
+                const uint64_t first = (uint64_t)from + (single ? take : 0u);
+                const uint64_t end = single ? first + 1u : first + ((uint64_t)take << shift);
+                const int turns = (n + kBkCap - 1) / kBkCap;
+                uint32_t seen = 0, seen_hot = 0;
+                uint32_t place[kBkItems];
+                // keys of the range in their order: into LDS, or (single) ranked as they come; then their places the same way
+                for (int what = 0; what < (single ? 1 : 2); ++what) {
+                    seen = 0;
+                    for (int t = 0; t < turns; ++t) {
+                        uint32_t k[kBkItems], mine = 0, hot = 0;
+    #pragma unroll
+                        for (int r = 0; r < kBkItems; ++r) {    // a thread's keys are neighbours here
+                            const int i = t * kBkCap + (int)threadIdx.x * kBkItems + r;
+                            k[r] = i < n ? kin[i] : kIgnoredKey;
+                            const uint32_t bits = k[r] & 0x7FFFFFFFu;
+                            if (i < n && bits >= first && bits < end) {
+                                ++mine;
+                                hot += k[r] >> 31;
+                            }
+                        }
+                        uint32_t at, all, at_hot, all_hot;
+                        block_excl_scan2(mine, hot, s.scan, at, all, at_hot, all_hot);
+                        at += seen;
+                        at_hot += seen_hot;
+    #pragma unroll
+                        for (int r = 0; r < kBkItems; ++r) {
+                            const int i = t * kBkCap + (int)threadIdx.x * kBkItems + r;
+                            const uint32_t bits = k[r] & 0x7FFFFFFFu;
+                            if (i < n && bits >= first && bits < end) {
+                                if (single) {
+                                    const float dj = jaccard_step(npos, rank0 + at, hot0 + at_hot, k[r] >> 31);
+                                    part += loss_term(key_error(k[r]), dj);
+                                    out[i] = dj;
+                                } else {
+                                    s.key()[at] = what == 0 ? k[r] : (uint32_t)i;
+                                }
+                                ++at;
+                                at_hot += k[r] >> 31;
+                            }
+                        }
+                        seen += all;
+                        seen_hot += what == 0 ? all_hot : 0u;
+                    }
+                    if (single) break;
+                    __syncthreads();
+                    const int rounds = (int)(take_keys + kBkThreads - 1) / kBkThreads;
+                    valid = 0;
+    #pragma unroll
+                    for (int r = 0; r < kBkItems; ++r) {
+                        const int li = bk_item(rounds, r);
+                        if (r < rounds && li < (int)take_keys) {
+                            if (what == 0) key[r] = s.key()[li];
+                            else place[r] = s.key()[li];
+                            valid |= 1u << r;
+                        }
+                    }
+                    __syncthreads();
+                    if (what == 1) {
+                        bk_range(s, key, valid, least, unused);
+                        uint32_t largest;
+                        bk_range(s, key, valid, unused, largest);
+                        bk_ranks_crowded(s, key, valid, rounds, least, largest, rank);
+    #pragma unroll
+                        for (int r = 0; r < kBkItems; ++r) {
+                            if ((valid >> r) & 1u) {
+                                const float dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), key[r] >> 31);
+                                part += loss_term(key_error(key[r]), dj);
+                                out[place[r]] = dj;
+                            }
+                        }
+                    }
+                }
+                done += seen;
+                rank0 += seen;
+                hot0 += seen_hot;
+                if (done >= (uint32_t)n || seen == 0) break;        // every turn takes keys
+                from = (uint32_t)end;                           // keys are left, so it is below 2^31
+                shift = 32 - (int)__builtin_clz((most - from) | 1u);
+                shift = shift > 12 ? shift - 12 : 0;
+            }
+    return part;
+}
+
+constexpr int kBkWideBlocks = 32;               // per class: one bucket at a time each
+__global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
+    __shared__ BkShared s;
+    __shared__ double wave_loss[kBkWaves];
+    __shared__ int todo[kBkMax / kBkWideBlocks + 1], found;
+    const int c = blockIdx.y, buckets = (int)a.numbers[c];
+    const int64_t cells = (int64_t)c * (a.stride + 1), row = (int64_t)c * a.stride;
+    if (threadIdx.x == 0) found = 0;
+    __syncthreads();
+    for (int i = (int)blockIdx.x + kBkWideBlocks * (int)threadIdx.x; i < buckets; i += kBkWideBlocks * kBkThreads) {
+        const uint32_t n = a.count[row + i];
+        if (n > (uint32_t)kBkCap && !(n & kBkFlat)) todo[atomicAdd(&found, 1)] = i;    // in any order: each has a sum of its own
+        else a.loss_part[2 * row + a.stride + i] = 0.0;
+    }
+    __syncthreads();
+    const int n_todo = found;
+    for (int i = 0; i < n_todo; ++i) {
+        const int b = todo[i];
+        double part = bk_wide_keys(s, a, c, a.base[cells + b], a.hot_base[cells + b], (int)a.count[row + b]);
+        part = wave_sum_f64(part);
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
+            a.loss_part[2 * row + a.stride + b] = sum;
+        }
+    }
+}
+
+// The tile's Jaccard differences in pixel order in the place of what bk_scatter left there: read in the runs that it wrote, put
+// in order in LDS. The first block of a class adds up its loss.
+template <int kBits>
+__global__ __launch_bounds__(kBkThreads) void bk_gather(const BucketArgs a, float *__restrict__ losses) {
+    constexpr int kStride = 1 << kBits;
+    __shared__ float dj[kBkTile];
+    __shared__ uint32_t from[kStride];
+    __shared__ uint32_t here[kBkWaves];
+    const int c = blockIdx.y, tile = sort_tile(a.P, kBkTile), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
+    uint32_t *row = a.keys + (int64_t)c * a.P + begin;
+    const uint16_t *places = reinterpret_cast<const uint16_t *>(row);
+    const uint32_t *table = a.tile_count + ((int64_t)c * a.tiles + tile) * kStride;
+    uint32_t place[kBkTileItems], bucket[kBkTileItems], kept = 0;
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int li = bk_item(kBkTileItems, r);
+        place[r] = li < n ? places[li] : kBkNowhere;
+        bucket[r] = li < n ? places[n + li] : 0u;           // past the kept ones: keys that were never overwritten, unused
+    }
+    const int buckets = (int)a.numbers[c];
+    for (int i = threadIdx.x; i < buckets; i += kBkThreads) from[i] = table[i];
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) kept += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(place[r] != kBkNowhere));
+    if (lane == 0) here[wave] = kept;
+    __syncthreads();
+    int n_here = 0;
+#pragma unroll
+    for (int w = 0; w < kBkWaves; ++w) n_here += (int)here[w];
+    const float *src = a.dj + (int64_t)c * a.P;
+    float v[kBkTileItems];
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int i = bk_item(kBkTileItems, r);
+        v[r] = 0.f;
+        if (i < n_here) v[r] = src[from[bucket[r]] + (uint32_t)i];
+    }
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) dj[bk_item(kBkTileItems, r)] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const int li = bk_item(kBkTileItems, r);
+        if (li < n) row[li] = place[r] != kBkNowhere ? __builtin_bit_cast(uint32_t, dj[place[r]]) : 0u;
+    }
+    if (tile != 0) return;
+    __shared__ double wave_sum[kBkWaves];
+    const int runs = (int)a.numbers[a.C + c];
+    const double *sums = a.loss_part + 2 * (int64_t)c * a.stride;
+    double sum = 0.0;
+    for (int i = threadIdx.x; i < runs; i += kBkThreads) sum += sums[i];
+    for (int i = threadIdx.x; i < buckets; i += kBkThreads) sum += sums[a.stride + i];
+    if (a.numbers[4 * a.C + c])
+        for (int i = threadIdx.x; i < a.tiles; i += kBkThreads) sum += a.tile_loss[(int64_t)c * a.tiles + i];
+    sum = wave_sum_f64(sum);
+    if (lane == 0) wave_sum[wave] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double all = 0.0;
+#pragma unroll
+        for (int w = 0; w < kBkWaves; ++w) all += wave_sum[w];
+        losses[c] = (float)all;
+    }
+}
+
+}  // namespace plh

@@ -1,0 +1,101 @@
+"""The Lovasz forward's sort by value buckets against the look-back variant, which sorts the same keys by radix passes: the
+Jaccard differences have to be the same bit for bit (same ranks, equal keys in pixel order), and so do the losses, whose
+terms are added exactly. Rows at the limits of the paths (one block, each number of buckets), values that crowd: ties,
+clusters, one value only, rows without positives, and buckets that outgrow a block because the sampled bounds miss them."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def native():
+    from pytorch_loss import _native
+    _native.load()
+    return _native
+
+
+def labels(rng, shape, n_cls, ignored=0.1):
+    y = rng.integers(0, n_cls, shape)
+    y[rng.random(shape) < ignored] = 255
+    return y
+
+
+def compare(native, x, y):
+    xt, yt = torch.as_tensor(x).cuda(), torch.as_tensor(y).cuda()
+    want_l, want_j = native.lovasz_forward(xt, yt, 255, look_back=True)
+    for _ in range(2):
+        losses, jacc = native.lovasz_forward(xt, yt, 255)
+        assert torch.equal(jacc.view(torch.int32), want_j.view(torch.int32))
+        assert torch.equal(losses, want_l) and not torch.isnan(losses).any()
+    return losses
+
+
+# pixels: one block's limit, 64 / 256 / 1024 buckets, the longest row that is cut into buckets and the first that is not
+@pytest.mark.parametrize("pixels", [1, 63, 512, 513, 7679, 7680, 7681, 8193, 20011, 2560 * 64, 2560 * 64 + 1, 2560 * 256 + 7])
+@pytest.mark.parametrize("boost", [0.0, 10.0])
+def test_row_lengths(native, pixels, boost):
+    rng = np.random.default_rng(pixels)
+    x = rng.standard_normal((1, 3, 1, pixels), dtype=np.float32) * 2
+    y = labels(rng, (1, 1, pixels), 3)
+    x += np.float32(boost) * (np.arange(3)[None, :, None, None] == y[:, None])
+    losses = compare(native, x, y)
+    if pixels < 10000 and not boost:
+        want, _ = oracle.lovasz_forward(x.astype(np.float64), y, 255)
+        np.testing.assert_allclose(losses.cpu().numpy(), want, rtol=1e-5)
+
+
+@pytest.mark.parametrize("pixels", [1024 * 2560, 1024 * 2560 + 1])
+def test_longest_rows(native, pixels):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((1, 2, 1, pixels), device="cuda", generator=g)
+    y = torch.randint(0, 2, (1, 1, pixels), device="cuda", generator=g)
+    compare(native, x, y)
+
+
+@pytest.mark.parametrize("pixels", [5000, 40000, 300000])
+@pytest.mark.parametrize("kind", ["constant", "few values", "half steps", "cluster", "two clusters", "certain", "absent"])
+def test_crowded_values(native, pixels, kind):
+    rng = np.random.default_rng(len(kind) + pixels)
+    n_cls = 2 if kind in ("few values", "half steps") else 4
+    x = rng.standard_normal((1, n_cls, 1, pixels), dtype=np.float32)
+    y = labels(rng, (1, 1, pixels), n_cls)
+    if kind == "constant":              # every error the same
+        x[:] = 0
+    elif kind == "few values":          # ties by the thousand
+        x = np.round(x)
+    elif kind == "half steps":
+        x = np.round(x * 64) / 64
+    elif kind == "cluster":             # a new network: probabilities within 1e-5 of each other
+        x *= np.float32(1e-5)
+    elif kind == "two clusters":
+        x = x * np.float32(1e-6) + np.float32(3) * (rng.random(x.shape) < 0.5)
+    elif kind == "certain":             # probabilities of exactly 1, and the steps of 2^-24 below
+        x += np.float32(17) * (np.arange(n_cls)[None, :, None, None] == y[:, None])
+    else:                               # classes that no pixel has
+        y[:] = np.where(y == 255, 255, 1)
+    compare(native, x.astype(np.float32), y)
+
+
+def sampled(pixels):
+    """The positions that the bucket bounds are chosen from (csrc/lovasz_buckets.hpp, bk_split)."""
+    i = np.arange(7680, dtype=np.uint64)
+    h = (i * 0x9E3779B1) & 0xFFFFFFFF
+    h = ((h ^ (h >> 15)) * 0x85EBCA6B) & 0xFFFFFFFF
+    return i * pixels // 7680 + ((h * (pixels // 7680)) >> 32)
+
+
+@pytest.mark.parametrize("pixels", [70000, 500000])
+@pytest.mark.parametrize("kind", ["spread", "one value", "both"])
+def test_buckets_that_the_sample_misses(native, pixels, kind):
+    rng = np.random.default_rng(pixels)
+    d = rng.random(pixels) * (0.0 if kind == "one value" else 1e-2)
+    if kind == "both":
+        d[rng.random(pixels) < 0.5] = 5e-3
+    at = sampled(pixels).astype(np.int64)
+    d[at] = 1 + rng.random(at.size)
+    x = np.stack([d, np.zeros(pixels)])[None, :, None, :].astype(np.float32)
+    compare(native, x, labels(rng, (1, 1, pixels), 2))
