@@ -1186,19 +1186,18 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
         pl.bk_bits = pl.P <= kBkCap ? 0 : (most <= 64 ? 6 : (most <= 256 ? 8 : 10));
         const int64_t cells = dimsize << pl.bk_bits;
         pl.off_crowded = off;        off += round_up(4 * cells, 256);
-        if (pl.bk_bits) {
-            pl.off_sorted = off;     off += round_up(4 * pl.E, 256);
-            pl.off_dj = off;         off += round_up(4 * pl.E, 256);
-            pl.off_bucket = off;     off += round_up(2 * pl.E, 256);
-            pl.off_tile_count = off; off += round_up(4 * cells * pl.bk_tiles, 256);
-            pl.off_tile_hot = off;   off += round_up(4 * cells * pl.bk_tiles, 256);
-            pl.off_bk_tile_loss = off; off += round_up(8 * dimsize * pl.bk_tiles, 256);
-            pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // count, hot, base, hot_base, runs
-            pl.off_bounds = off;     off += round_up(4 * cells, 256);
-            pl.off_buckets = off;    off += round_up(4 * 5 * dimsize, 256);
-            pl.off_fine = off;       off += round_up(2 * dimsize * (kBkFine + 2), 256);
-            pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
-        }
+        // one layout for every row length, also where one block ranks the row
+        pl.off_sorted = off;     off += round_up(4 * pl.E, 256);
+        pl.off_dj = off;         off += round_up(4 * pl.E, 256);
+        pl.off_bucket = off;     off += round_up(2 * pl.E, 256);
+        pl.off_tile_count = off; off += round_up(4 * cells * pl.bk_tiles, 256);
+        pl.off_tile_hot = off;   off += round_up(4 * cells * pl.bk_tiles, 256);
+        pl.off_bk_tile_loss = off; off += round_up(8 * dimsize * pl.bk_tiles, 256);
+        pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // count, hot, base, hot_base, runs
+        pl.off_bounds = off;     off += round_up(4 * cells, 256);
+        pl.off_buckets = off;    off += round_up(4 * 5 * dimsize, 256);
+        pl.off_fine = off;       off += round_up(2 * dimsize * (kBkFine + 2), 256);
+        pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
         pl.bytes = off;
         return PLH_OK;
     }
