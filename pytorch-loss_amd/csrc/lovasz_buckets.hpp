@@ -37,7 +37,7 @@ constexpr int kBkTarget = 2560;                     // mean keys per bucket: sam
 constexpr int kBkSlab = 6144;                       // buckets that start in one such part of the row are sorted together
 constexpr int kBkMax = 1024;                        // buckets per class
 constexpr int64_t kBkMaxRow = (int64_t)kBkTarget * kBkMax;
-constexpr uint32_t kBkCrowd = 65;                   // keys in one bin up to which merges between chunks put them in order
+constexpr uint32_t kBkCrowd = 97;                   // keys in one bin up to which merges between chunks put them in order
 constexpr uint32_t kBkFlat = 0x80000000u;
 constexpr uint16_t kBkNowhere = 0xFFFFu;            // place of a pixel that takes no part
 
@@ -186,13 +186,21 @@ __device__ __forceinline__ int bk_item(int rounds, int r) {
 // Counting the keys into 4096 bins of their range puts them in order but for the one or two per bin; those are sorted by
 // the threads, 16 places each, then across the chunks' borders (8 places of either side) and within the chunks in turn:
 // odd-even transposition of halves of 8, of which a bin of L keys touches at most 2 + (L - 2) / 8.
+//
+// Knee: a whole row's values rather than a run's, which crowd at its least keys (errors near 1, of a class that the
+// network misses): a quarter of the bins for the first 64th of the range.
+template <bool Knee = false>
 __device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds, uint32_t from,
                                         float scale, uint32_t &n, BkPair (&v)[kBkChunk]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     // monotone in the key, and at most kBkBins - 1 by the choice of scale
+    constexpr float kKnee = kBkBins / 64.f;     // the knee, in bins of one width
     auto bin_of = [&](uint32_t k) {
         k &= 0x7FFFFFFFu;
-        return (uint32_t)((float)(max(k, from) - from) * scale);
+        const float at = (float)(max(k, from) - from) * scale;
+        // 16 times as many bins below the knee, the other 3 of 4 above: both halves reach 1024 there
+        if constexpr (Knee) return (uint32_t)(at < kKnee ? at * 16.f : __builtin_fmaf(at - kKnee, 3072.f / (kBkBins - kKnee), 1024.f));
+        return (uint32_t)at;
     };
     {
         uint4 *b4 = reinterpret_cast<uint4 *>(s.bin);
@@ -393,7 +401,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
     if (n > 0) {                                            // block-uniform
         BkPair v[kBkChunk];
         uint32_t m;
-        if (bk_sort(s, key, valid, kBkItems, least, bk_scale(least, most), m, v)) {
+        if (bk_sort<true>(s, key, valid, kBkItems, least, bk_scale(least, most), m, v)) {
 #pragma unroll
             for (int e = 0; e < kBkChunk; ++e)
                 if (threadIdx.x * kBkChunk + e < n) sorted[threadIdx.x * kBkChunk + e] = bk_key_of(v[e]);
@@ -660,13 +668,15 @@ __device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
 // The tile's keys by bucket, written out in runs. In the place of the tile's keys it leaves, in 16 bits each, every pixel's
 // place in the tile's order, then the bucket of every place.
 template <int kBits>
-__global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
+__global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) {
     constexpr int kStride = 1 << kBits, kPer = (kStride + kBkThreads - 1) / kBkThreads;
+    // 52 KiB, three blocks per CU: the buckets by place take the counters' memory
     __shared__ uint32_t s_key[kBkTile];                     // the tile by bucket
-    __shared__ uint16_t s_bucket[kBkTile];
-    __shared__ __align__(4) uint16_t counts[kBkWaves][kStride];
-    __shared__ uint32_t start[kStride], out_base[kStride];
+    __shared__ __align__(4) uint16_t s_counts[kBkTile > kBkWaves * kStride ? kBkTile : kBkWaves * kStride];
+    __shared__ uint32_t out_base[kStride];
     __shared__ uint32_t scan_tmp[kSortWaves];
+    uint16_t *s_bucket = s_counts;
+    uint16_t(*counts)[kStride] = reinterpret_cast<uint16_t(*)[kStride]>(s_counts);
     const int c = blockIdx.y, wave = threadIdx.x >> 6;
     const int tile = sort_tile(a.P, kBkTile);
     const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
@@ -686,7 +696,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
         const uint32_t d = threadIdx.x * kPer + i;
         first[i] = d < buckets ? table[d] + a.base[(int64_t)c * (kStride + 1) + d] : 0u;
     }
-    for (int i = threadIdx.x; i < kBkWaves * kStride / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(&counts[0][0])[i] = 0;
+    for (int i = threadIdx.x; i < kBkWaves * kStride / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(s_counts)[i] = 0;
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) {
@@ -718,7 +728,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
     for (int i = 0; i < kPer; ++i) {
         const uint32_t d = threadIdx.x * kPer + i;
         if (d < buckets) {
-            start[d] = at;
+#pragma unroll
+            for (int w = 0; w < kBkWaves; ++w) counts[w][d] = (uint16_t)(counts[w][d] + at);
             out_base[d] = first[i] - at;
             table[d] = first[i] - at;
         }
@@ -727,16 +738,18 @@ __global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
     __syncthreads();
     uint16_t *places = reinterpret_cast<uint16_t *>(kin);
 #pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r)
+        rank[r] = b[r] != kBkNowhere ? counts[wave][b[r]] + rank[r] : kBkNowhere;
+    __syncthreads();
+#pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) {
         const int li = bk_item(kBkTileItems, r);
         if (li >= n) continue;
-        uint32_t pos = kBkNowhere;
         if (b[r] != kBkNowhere) {
-            pos = start[b[r]] + counts[wave][b[r]] + rank[r];
-            s_key[pos] = key[r];
-            s_bucket[pos] = (uint16_t)b[r];
+            s_key[rank[r]] = key[r];
+            s_bucket[rank[r]] = (uint16_t)b[r];
         }
-        places[li] = (uint16_t)pos;
+        places[li] = (uint16_t)rank[r];
     }
     __syncthreads();
     uint32_t *kout = a.sorted + (int64_t)c * a.P;
@@ -749,7 +762,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
     // Buckets of a single value that no block would hold: their keys are in order, so the place is the rank; the positives
     // before it are those of the buckets before, of the tiles before and of the places before. A thread takes 16 neighbours.
     __shared__ double wave_loss[kBkWaves];
-    uint32_t *hot_start = reinterpret_cast<uint32_t *>(counts);       // positives of the tile before each bucket
+    // positives before the bucket's first place, less those of the tile before it
+    uint32_t *hot_start = a.tile_hot + ((int64_t)c * a.tiles + tile) * kStride;
     const uint32_t p0 = threadIdx.x * kBkTileItems;
     uint32_t hots = 0, all;
 #pragma unroll
@@ -761,7 +775,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
         for (int e = 0; e < kBkTileItems; ++e) {
             if (p0 + e < n_here) {
                 const uint32_t d = s_bucket[p0 + e];
-                if (start[d] == p0 + e) hot_start[d] = before;
+                if ((p0 + e == 0 || s_bucket[p0 + e - 1] != d) && (a.count[(int64_t)c * kStride + d] & kBkFlat))
+                    hot_start[d] += a.hot_base[(int64_t)c * (kStride + 1) + d] - before;
                 before += s_key[p0 + e] >> 31;
             }
         }
@@ -774,9 +789,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_scatter(const BucketArgs a) {
         const uint32_t d = s_bucket[p0 + e], k = s_key[p0 + e];
         if (a.count[(int64_t)c * kStride + d] & kBkFlat) {
             const uint32_t pos = out_base[d] + p0 + e;
-            const uint32_t hot_before = a.hot_base[(int64_t)c * (kStride + 1) + d] +
-                                        a.tile_hot[((int64_t)c * a.tiles + tile) * kStride + d] + (cs - hot_start[d]);
-            const float dj = jaccard_step(npos, pos, hot_before, k >> 31);
+            const float dj = jaccard_step(npos, pos, hot_start[d] + cs, k >> 31);
             part += loss_term(key_error(k), dj);
             a.dj[(int64_t)c * a.P + pos] = dj;
         }
