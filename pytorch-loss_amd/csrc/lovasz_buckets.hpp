@@ -698,13 +698,37 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) 
     }
     for (int i = threadIdx.x; i < kBkWaves * kStride / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(s_counts)[i] = 0;
     __syncthreads();
+    // Four rounds at a time: their masks first, then a read of the counter and the leader's addition to it per round. LDS
+    // takes a wave's operations in their order, so no addition waits for what a read returns.
+    constexpr int kGroup = 2;
 #pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) {
-        const bool valid = b[r] != kBkNowhere;
-        rank[r] = 0;
-        if (__builtin_amdgcn_ballot_w64(valid) == 0) continue;      // wave-uniform
-        uint32_t unused;
-        wave_rank_of<false>(bk_peers<kBits>(b[r], valid), b[r], valid, false, counts[wave], nullptr, rank[r], unused);
+    for (int r0 = 0; r0 < kBkTileItems; r0 += kGroup) {
+        uint64_t peers[kGroup];
+        uint32_t seen[kGroup];
+        bool any = false;
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) {
+            rank[r0 + h] = 0;
+            any = any || b[r0 + h] != kBkNowhere;
+        }
+        if (__builtin_amdgcn_ballot_w64(any) == 0) continue;        // wave-uniform
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) peers[h] = bk_peers<kBits>(b[r0 + h], b[r0 + h] != kBkNowhere);
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) {
+            const uint32_t d = b[r0 + h], before = peers_below(peers[h]);
+            const bool valid = d != kBkNowhere;
+            seen[h] = 0;
+            if (valid) seen[h] = counts[wave][d];
+            asm volatile("" ::: "memory");
+            if (valid && before == 0u)
+                atomicAdd(reinterpret_cast<uint32_t *>(counts[wave]) + (d >> 1),
+                          (uint32_t)__builtin_popcountll(peers[h]) << (16u * (d & 1u)));
+            asm volatile("" ::: "memory");
+            rank[r0 + h] = before;
+        }
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) rank[r0 + h] += seen[h];
     }
     __syncthreads();
     uint32_t mine[kPer], n_mine = 0;
