@@ -73,21 +73,23 @@ __device__ __forceinline__ void publish_block_max(const uint32_t *block_max, uin
 
 // It also leaves, per class, the number of key bits the sort has to look at: keys that take part are
 // not above the limit, so the bits above the limit's highest set bit are zero in every one of them.
-__global__ __launch_bounds__(256) void lov_class_max(const uint32_t *__restrict__ block_table, int blocks, int C,
+__global__ __launch_bounds__(1024) void lov_class_max(const uint32_t *__restrict__ block_table, int blocks, int C,
                                                      uint32_t *__restrict__ pos_max, uint32_t *__restrict__ cursors,
                                                      int regions) {
-    __shared__ uint32_t wave_max[4];
+    __shared__ uint32_t wave_max[16];
     const int c = blockIdx.x;
     // the class's staging cursors start at zero (they are first used by the last pass)
-    for (int i = threadIdx.x; i < regions; i += 256) cursors[(int64_t)c * regions + i] = 0;
+    for (int i = threadIdx.x; i < regions; i += 1024) cursors[(int64_t)c * regions + i] = 0;
     uint32_t m = 0;
-    for (int b = threadIdx.x; b < blocks; b += 256) m = max(m, block_table[(int64_t)b * C + c]);
+    for (int b = threadIdx.x; b < blocks; b += 1024) m = max(m, block_table[(int64_t)b * C + c]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
     if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t top = max(max(wave_max[0], wave_max[1]), max(wave_max[2], wave_max[3]));
+        uint32_t top = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) top = max(top, wave_max[w]);
         pos_max[c] = top;
         pos_max[2 * C + c] = 0xFFFFFFFFu;       // all_min[c], for lov_absent_min
         // key_bits[c]: a class without positives keeps a single key value, wherever it lies
@@ -1195,7 +1197,7 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
         pl.off_bk_tile_loss = off; off += round_up(8 * dimsize * pl.bk_tiles, 256);
         pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // count, hot, base, hot_base, runs
         pl.off_bounds = off;     off += round_up(4 * cells, 256);
-        pl.off_buckets = off;    off += round_up(4 * 5 * dimsize, 256);
+        pl.off_buckets = off;    off += round_up(4 * 6 * dimsize, 256);
         pl.off_fine = off;       off += round_up(2 * dimsize * (kBkFine + 2), 256);
         pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
         pl.bytes = off;
@@ -1280,7 +1282,7 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
     a.fine = reinterpret_cast<uint16_t *>(ws + pl.off_fine);
     a.loss_part = reinterpret_cast<double *>(ws + pl.off_loss_part);
     const dim3 tiles((unsigned)pl.bk_tiles, (unsigned)C), threads(kBkThreads);
-    const unsigned most = (unsigned)ceil_div(pl.P, kBkTarget);      // buckets a class can have
+    const unsigned most = (unsigned)ceil_div(pl.P, kBkTarget) + 1;  // buckets a class can have
     // two blocks fit a CU; each looks at every so many of the class's runs
     const unsigned crowded_blocks = (unsigned)(ceil_div(2048, C) < most ? ceil_div(2048, C) : most);
     hipLaunchKernelGGL(bk_split, dim3((unsigned)C), threads, 0, st, a);
@@ -1364,7 +1366,7 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
                                pl.P, m_size, C, ignore_index);
         }
     });
-    hipLaunchKernelGGL(lov_class_max, dim3((unsigned)C), dim3(256), 0, st, block_table, (int)key_blocks, C, pos_max,
+    hipLaunchKernelGGL(lov_class_max, dim3((unsigned)C), dim3(1024), 0, st, block_table, (int)key_blocks, C, pos_max,
                        reinterpret_cast<uint32_t *>(ws + pl.off_cursors), pl.regions);
     hipLaunchKernelGGL(lov_absent_min, dim3(kAbsentBlocks, (unsigned)C), dim3(256), 0, st, keys_0, pos_max, all_min,
                        (int)pl.P);

@@ -55,7 +55,8 @@ struct BucketArgs {
     uint32_t *bounds;           // [C][stride] least key of buckets 1, 2, ...
     uint32_t *runs;             // [C][stride + 1] first bucket of every run, and the end
     uint32_t *crowded;          // [C][stride] runs (rows of one block: [C]) whose values crowd
-    uint32_t *numbers;          // [5][C]: buckets, runs, positives, least key of the sample, flat buckets
+    uint32_t *numbers;          // [6][C]: buckets, runs, positives, least key of the sample, flat buckets,
+                                // largest key of the sample below the limit
     uint16_t *fine;             // [C][kBkFine + 2]
     double *loss_part;          // [C][2 * stride]: runs, wide buckets
     double *tile_loss;          // [C][tiles] of the flat buckets, where there are any
@@ -178,30 +179,34 @@ __device__ __forceinline__ int bk_item(int rounds, int r) {
     return ((int)(threadIdx.x >> 6) * rounds + r) * kWave + (int)(threadIdx.x & 63);
 }
 
+// The bins of the values from..to: one width for all, or another below `knee`, which then gets the first `share` of them.
+// Monotone in the key, and below kBkBins (or rounded to kBkBins itself).
+struct BkBinning {
+    uint32_t from, knee;
+    float below, above, start;
+    bool bent;                                  // wave-uniform
+    __device__ BkBinning(uint32_t from_, uint32_t knee_, uint32_t to, float share) : from(from_), knee(knee_) {
+        bent = __builtin_amdgcn_readfirstlane(knee > from && knee <= to);
+        start = bent ? share * kBkBins : 0.f;
+        below = bent ? (start - 1.f) / (float)(knee - from) : 0.f;
+        above = ((float)(kBkBins - 1) - start) / (float)(to - (bent ? knee : from) + 1u);
+    }
+    __device__ __forceinline__ uint32_t of(uint32_t key) const {
+        const uint32_t k = max(key & 0x7FFFFFFFu, from);
+        if (!bent) return (uint32_t)((float)(k - from) * above);
+        return k < knee ? (uint32_t)((float)(k - from) * below) : (uint32_t)__builtin_fmaf((float)(k - knee), above, start);
+    }
+};
+
 // Sorts the block's valid keys (n of them in all, in `rounds` x 512 items): v[e] becomes the pair at place 16 t + e of the
 // order for thread t, bk_last() past the end. False (block-uniform) where values crowd: then bk_ranks_crowded has to do it.
-// from: no valid key is below it, except that such keys share the first bin; scale: bins per unit of key, below
-// kBkBins / (largest key - from + 1).
 //
 // Counting the keys into 4096 bins of their range puts them in order but for the one or two per bin; those are sorted by
 // the threads, 16 places each, then across the chunks' borders (8 places of either side) and within the chunks in turn:
 // odd-even transposition of halves of 8, of which a bin of L keys touches at most 2 + (L - 2) / 8.
-//
-// Knee: a whole row's values rather than a run's, which crowd at its least keys (errors near 1, of a class that the
-// network misses): a quarter of the bins for the first 64th of the range.
-template <bool Knee = false>
-__device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds, uint32_t from,
-                                        float scale, uint32_t &n, BkPair (&v)[kBkChunk]) {
+__device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds,
+                                        const BkBinning bins, uint32_t &n, BkPair (&v)[kBkChunk]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // monotone in the key, and at most kBkBins - 1 by the choice of scale
-    constexpr float kKnee = kBkBins / 64.f;     // the knee, in bins of one width
-    auto bin_of = [&](uint32_t k) {
-        k &= 0x7FFFFFFFu;
-        const float at = (float)(max(k, from) - from) * scale;
-        // 16 times as many bins below the knee, the other 3 of 4 above: both halves reach 1024 there
-        if constexpr (Knee) return (uint32_t)(at < kKnee ? at * 16.f : __builtin_fmaf(at - kKnee, 3072.f / (kBkBins - kKnee), 1024.f));
-        return (uint32_t)at;
-    };
     {
         uint4 *b4 = reinterpret_cast<uint4 *>(s.bin);
 #pragma unroll
@@ -213,7 +218,7 @@ __device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkIt
     for (int r = 0; r < kBkItems; ++r) {
         slot[r] = 0;
         if (r < rounds && ((valid >> r) & 1u)) {
-            const uint32_t b = min(bin_of(key[r]), (uint32_t)kBkBins - 1u);
+            const uint32_t b = min(bins.of(key[r]), (uint32_t)kBkBins - 1u);
             slot[r] = b << 16 | atomicAdd(&s.bin[b], 1u);
         }
     }
@@ -286,10 +291,6 @@ __device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkIt
     }
     __syncthreads();                            // s.pair is free again
     return true;
-}
-
-__device__ __forceinline__ float bk_scale(uint32_t from, uint32_t to) {       // bins for the keys from..to
-    return (float)(kBkBins - 1) / (float)(to - from + 1u);
 }
 
 // rank[r] = valid keys of the block that sort before key[r] (equal keys in item order) | positives among them << 16, for
@@ -401,7 +402,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
     if (n > 0) {                                            // block-uniform
         BkPair v[kBkChunk];
         uint32_t m;
-        if (bk_sort<true>(s, key, valid, kBkItems, least, bk_scale(least, most), m, v)) {
+        // errors near 1 crowd in classes that the network misses: a quarter of the bins for the first 64th of the range
+        if (bk_sort(s, key, valid, kBkItems, BkBinning(least, least + (most - least) / 64u, most, 0.25f), m, v)) {
 #pragma unroll
             for (int e = 0; e < kBkChunk; ++e)
                 if (threadIdx.x * kBkChunk + e < n) sorted[threadIdx.x * kBkChunk + e] = bk_key_of(v[e]);
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
         }
         const uint64_t keys = (uint64_t)n * (uint32_t)a.P / kBkCap;
         want = (uint32_t)((keys + kBkTarget - 1) / kBkTarget);
-        want = min(max(want, 1u), (uint32_t)a.stride);
+        want = min(max(want, 1u), (uint32_t)a.stride - 1u);
     }
     __syncthreads();
     // candidates 1..want-1, a run of neighbours per thread; the bounds are collected where the bins were
@@ -439,10 +441,25 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
         if (j + 1 < want && candidate(j + 1) == v) s.bin[at++] = v + 1u;
     }
     __syncthreads();
+    // The largest key that takes part, the lowest-ranked positive's, has a bucket too: where the network is sure, that is an
+    // error of exactly 0, shared by many and far from the next.
+    if (n > 0 && limit > (bounds ? s.bin[bounds - 1] : 0u)) {
+        __syncthreads();
+        if (threadIdx.x == 0) s.bin[bounds] = limit;
+        ++bounds;
+        __syncthreads();
+    }
     for (uint32_t i = threadIdx.x; i < bounds; i += kBkThreads) a.bounds[(int64_t)c * a.stride + i] = s.bin[i];
     if (threadIdx.x == 0) {
         a.numbers[c] = bounds + 1u;
         a.numbers[3 * a.C + c] = n ? least : 0u;
+        uint32_t lo = 0, hi = n;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (sorted[mid] < limit) lo = mid + 1;
+            else hi = mid;
+        }
+        a.numbers[5 * a.C + c] = lo ? sorted[lo - 1] : 0u;
     }
     // the bucket of the least key with each pattern of the top bits
     const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
@@ -856,7 +873,9 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
     const uint32_t limit = bk_limit(a, c);
     float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
 
-    uint32_t key[kBkItems], valid = 0, least, most;
+    uint32_t key[kBkItems], valid = 0, least, most, knee = 0;
+    float share = 0.25f;
+    bool flat = false;                                      // block-uniform: one value, in order as it stands
     const int rounds = (n + kBkThreads - 1) / kBkThreads;
 #pragma unroll
     for (int r = 0; r < kBkItems; ++r) {
@@ -877,15 +896,38 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
         most = max(least, most);                            // no valid key: nothing below looks at the range
     } else {
         const uint32_t *bound = a.bounds + (int64_t)c * a.stride;
-        most = b1 < a.numbers[c] ? bound[b1 - 1] - 1u : limit;
-        if (b0) least = bound[b0 - 1];
-        else bk_range(s, key, valid, least, most);          // below the least of the sample lie a few more
+        const uint32_t buckets = a.numbers[c];
+        most = b1 < buckets ? bound[b1 - 1] - 1u : limit;
+        least = b0 ? bound[b0 - 1] : 0u;
+        flat = least == most;
+        if (!flat && (b0 == 0 || b1 + 1u >= buckets)) {
+            // beyond the sample lie a few more, far apart: their own bins
+            bk_range(s, key, valid, least, most);
+            knee = b0 ? a.numbers[5 * a.C + c] + 1u : a.numbers[3 * a.C + c];
+            share = b0 ? 0.75f : 0.25f;
+        }
     }
     double part = 0.0;
     BkPair v[kBkChunk];
     uint32_t kept;
     float *result = reinterpret_cast<float *>(s.pair);      // by item
-    if (bk_sort(s, key, valid, rounds, least, bk_scale(least, most), kept, v)) {       // block-uniform
+    bool in_order = flat;
+    if (flat) {
+        kept = (uint32_t)n;
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r)
+            if ((valid >> r) & 1u) s.at((uint32_t)bk_item(rounds, r)) = bk_pair(key[r], (uint32_t)bk_item(rounds, r));
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kBkChunk; ++e) {
+            const uint32_t p = threadIdx.x * kBkChunk + e;
+            if (p < kept) v[e] = s.at(p);
+        }
+        __syncthreads();
+    } else {
+        in_order = bk_sort(s, key, valid, rounds, BkBinning(least, knee, most, share), kept, v);
+    }
+    if (in_order) {                                         // block-uniform
         const uint32_t p0 = threadIdx.x * kBkChunk;
         uint32_t hot = 0, all;
 #pragma unroll
