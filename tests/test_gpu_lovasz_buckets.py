@@ -99,3 +99,26 @@ def test_buckets_that_the_sample_misses(native, pixels, kind):
     d[at] = 1 + rng.random(at.size)
     x = np.stack([d, np.zeros(pixels)])[None, :, None, :].astype(np.float32)
     compare(native, x, labels(rng, (1, 1, pixels), 2))
+
+
+@pytest.mark.parametrize("n_cls", [2, 19, 24, 32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("plane", [(65, 67), (64, 65), (85, 121)])
+def test_planes_of_odd_length(native, n_cls, dtype, plane):
+    """Planes that start on element boundaries: the same as the pixels of four images side by side in one, whose planes start
+    on the vector accesses' boundaries."""
+    import pytorch_loss
+    g = torch.Generator(device="cuda").manual_seed(n_cls + plane[0])
+    x = (torch.randn((4, n_cls) + plane, device="cuda", generator=g) * 2).to(dtype)
+    y = torch.randint(0, n_cls, (4,) + plane, device="cuda", generator=g)
+    y[torch.rand(y.shape, device="cuda", generator=g) < 0.1] = 255
+    side_x = x.flatten(2).transpose(0, 1).contiguous().unsqueeze(0)        # (1, C, 4, pixels of an image)
+    side_y = y.flatten(1).unsqueeze(0)
+    out = []
+    for a, b in ((x, y), (side_x, side_y)):
+        losses, jacc = native.lovasz_forward(a, b, 255)
+        a = a.detach().requires_grad_()
+        pytorch_loss.LovaszSoftmaxV3(ignore_index=255)(a, b).backward()
+        out.append((losses, jacc, a.grad))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert torch.equal(out[0][2], out[1][2][0].transpose(0, 1).reshape(x.shape))
