@@ -933,22 +933,25 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
 #pragma unroll
         for (int e = 0; e < kBkChunk; ++e) hot += p0 + e < kept ? bk_hot_of(v[e]) : 0u;
         uint32_t cs = hot0 + block_excl_scan(hot, s.scan, all);
-        if (p0 < kept) {
-            uint32_t pos = rank0 + p0;
-            float inter = npos - (float)cs;                                            // csrc/lovasz_softmax.cu:124-127
-            float j_prev = pos == 0 ? 0.f : 1.f - inter / (inter + (float)pos);
+        const uint32_t pos = rank0 + p0;
+        float inter = npos - (float)cs;                                                // csrc/lovasz_softmax.cu:124-127
+        float j_prev = pos == 0 ? 0.f : 1.f - inter / (inter + (float)pos);
+        auto step = [&](int e) {
+            cs += bk_hot_of(v[e]);
+            inter = npos - (float)cs;
+            const float j_now = 1.f - inter / (inter + (float)(pos + 1u + e));
+            const float dj = j_now - j_prev;                                           // csrc/lovasz_softmax.cu:141-147
+            j_prev = j_now;
+            part += loss_term(key_error(bk_key_of(v[e])), dj);
+            result[bk_item_of(v[e])] = dj;
+        };
+        if (p0 + kBkChunk <= kept) {
 #pragma unroll
-            for (int e = 0; e < kBkChunk; ++e) {
-                if (p0 + e < kept) {
-                    cs += bk_hot_of(v[e]);
-                    inter = npos - (float)cs;
-                    const float j_now = 1.f - inter / (inter + (float)(pos + 1u + e));
-                    const float dj = j_now - j_prev;                                   // csrc/lovasz_softmax.cu:141-147
-                    j_prev = j_now;
-                    part += loss_term(key_error(bk_key_of(v[e])), dj);
-                    result[bk_item_of(v[e])] = dj;
-                }
-            }
+            for (int e = 0; e < kBkChunk; ++e) step(e);
+        } else {
+#pragma unroll
+            for (int e = 0; e < kBkChunk; ++e)
+                if (p0 + e < kept) step(e);
         }
     } else {                                                // bk_rank_crowded's
         if (threadIdx.x == 0) a.crowded[Direct ? c : (int64_t)c * a.stride + g] = 1u;
