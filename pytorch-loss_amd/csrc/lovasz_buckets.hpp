@@ -16,9 +16,9 @@
 // needs no sort (flat: bk_scatter knows the ranks), and a bucket that outgrew the LDS all the same is taken in value ranges
 // that fit.
 // Bound by vector instructions (scatter and rank: some 80 and 110 per 64 keys at 16 waves per CU) and short runs, not by
-// the 36 bytes a key moves. Forward and backward, against the radix passes: (8,21,513,513) bf16 trained 1.22 -> 0.87 ms,
-// (4,19,512,1024) fp32 0.74 -> 0.64, (1,150,256,256) 0.51 -> 0.37; near-uniform predictions, whose keys need two
-// radix passes only, take the same time as before ((4,19,512,1024) 0.42 -> 0.43).
+// the 40 bytes a key moves. Forward and backward, against the radix passes: (8,21,513,513) bf16 trained 1.21 -> 0.82 ms,
+// (4,19,512,1024) fp32 0.72 -> 0.56, (1,150,256,256) 0.51 -> 0.37; near-uniform predictions, whose keys need two
+// radix passes only, take the same time as before ((4,19,512,1024) 0.42 both ways).
 #pragma once
 
 namespace plh {
@@ -37,7 +37,8 @@ constexpr int kBkTarget = 2560;                     // mean keys per bucket: sam
 constexpr int kBkSlab = 6144;                       // buckets that start in one such part of the row are sorted together
 constexpr int kBkMax = 1024;                        // buckets per class
 constexpr int64_t kBkMaxRow = (int64_t)kBkTarget * kBkMax;
-constexpr uint32_t kBkCrowd = 97;                   // keys in one bin up to which merges between chunks put them in order
+constexpr uint32_t kBkCrowd = 257;                  // keys in one bin up to which merges between chunks put them in order: 97 left
+                                                    // lumps of bf16 logits to bk_rank_crowded (227 + 37 -> 231 + 9 us)
 constexpr uint32_t kBkFlat = 0x80000000u;
 constexpr uint16_t kBkNowhere = 0xFFFFu;            // place of a pixel that takes no part
 
