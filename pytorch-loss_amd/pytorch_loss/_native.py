@@ -910,17 +910,17 @@ def layer_norm_has_affine(x, weight, bias):
 
 
 def layer_norm_affine_forward(x, weight, bias, eps):
-    """(N, C, M) normalised over C, times weight, plus bias. -> (out, the contiguous input for the backward)."""
+    """(N, C, M), contiguous, normalised over C, times weight, plus bias."""
     _require_gpu("layernorm loss", x, weight, bias)
     (xc, tag), wc, bc = _logits(x), weight.contiguous(), bias.contiguous()
     out = torch.empty_like(xc)
     _call(xc, "plh_layer_norm_affine_forward", _ptr(xc), tag, _ptr(wc), _ptr(bc), _ptr(out), *xc.shape, float(eps))
-    return out, xc
+    return out
 
 
-def layer_norm_affine_backward(grad_output, xc, weight, eps, sums):
+def layer_norm_affine_backward(grad_output, x, weight, eps, sums):
     """-> (grad of x, grad of weight, grad of bias); the last two are None unless `sums`."""
-    wc = weight.contiguous()
+    xc, wc = x.contiguous(), weight.contiguous()
     g = (grad_output if grad_output.dtype == xc.dtype else grad_output.to(xc.dtype)).expand(xc.shape).contiguous()
     grad = torch.empty_like(xc)
     grad_w = grad_b = ws = None

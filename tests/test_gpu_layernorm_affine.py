@@ -137,3 +137,69 @@ def test_what_torch_refuses_stays_refused(pl):
     m.weight, m.bias = torch.arange(8.0, device="cuda"), torch.zeros(8, device="cuda")      # along the pixels
     want = (pl.LayerNormV3(8, affine=False)(square).view(1, 8, 8) * m.weight).view_as(square)
     assert torch.equal(m(square), want)
+
+
+def test_input_changed_in_place_before_the_backward(pl):
+    """The backward reads the input again: where the input takes part in the graph, a change of it before the backward is
+    refused; where it does not (a buffer that is filled anew), the gradients of weight and bias are those of the values that
+    the forward saw, bit for bit; so are all of them where the forward worked on a copy of a strided input."""
+    gen = torch.Generator().manual_seed(11)
+    shape = (2, 16, 9, 10)
+    data, g = torch.randn(shape, generator=gen).cuda(), torch.randn(shape, generator=gen).cuda()
+    m = pl.LayerNormV3(16).cuda()
+    with torch.no_grad():
+        m.weight.add_(0.1 * torch.randn(m.weight.shape, generator=gen).cuda())
+
+    def grads(x, between):
+        m.weight.grad = m.bias.grad = None
+        out = m(x)
+        between(x)
+        out.backward(g)
+        return [t.clone() for t in (m.weight.grad, m.bias.grad)]
+
+    for fill in (lambda x: x.mul_(2).add_(1), lambda x: x.copy_(g), lambda x: x.relu_()):
+        want = grads(data.clone(), lambda x: None)
+        got = grads(data.clone(), fill)                                     # a buffer without gradient
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            grads(data.clone().requires_grad_() * 1, fill)                  # part of the graph
+    x = data.clone().requires_grad_()
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        grads(x, lambda x: x.detach().mul_(2))
+    # a strided input: what the backward reads is a copy of its own
+    wide = torch.randn((2, 32, 9, 10), generator=gen).cuda()
+    leaf = wide.clone().requires_grad_()
+    want = grads((leaf * 1)[:, ::2], lambda x: None) + [leaf.grad]
+    leaf = wide.clone().requires_grad_()
+    got = grads((leaf * 1)[:, ::2], lambda x: x.mul_(2)) + [leaf.grad]
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert torch.equal(got[2], want[2])
+    # an in-place operation on the result, as an activation does, is nobody's loss
+    x = data.clone().requires_grad_()
+    out = m(x).relu_()
+    out.backward(g)
+    y = data.clone().requires_grad_()
+    torch.relu(m(y)).backward(g)
+    assert torch.equal(x.grad, y.grad)
+
+
+@pytest.mark.parametrize("trained", ["neither", "weight", "bias"])
+def test_frozen_input_computes_no_gradient_of_it(pl, trained):
+    """Without a gradient of the input the backward allocates nothing of the input's size (peak: the upstream gradient times
+    the normalised input, where the weight is trained)."""
+    shape = (4, 64, 64, 64)
+    x, g = torch.randn(shape, device="cuda"), torch.randn(shape, device="cuda")
+    m = pl.LayerNormV3(64).cuda()
+    m.weight.requires_grad_(trained == "weight")
+    m.bias.requires_grad_(trained == "bias")
+    out = m(x)
+    assert out.requires_grad == (trained != "neither")
+    if trained == "neither":
+        return
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    out.backward(g)
+    peak = torch.cuda.max_memory_allocated() - before
+    assert peak < (0.5 if trained == "bias" else 1.5) * x.numel() * 4
+    assert x.grad is None
