@@ -16,7 +16,7 @@
 //                     largest positive key per class (per-block table + lov_class_max): keys
 //                     beyond it have dJ = 0 exactly and are left out of the sort (keep_key).
 //   2.-4. for rows of up to kBkMaxRow pixels: by value buckets, see lovasz_buckets.hpp. Otherwise, and in the look-back
-//                     variant, with the same results bit for bit:
+//                     variant, with the same differences bit for bit:
 //   2. 3 x (tile_hist, row_scan, scatter): stable LSD radix passes, 8 bits each, batched over
 //                     classes with blockIdx.y. Ranking inside a tile is done per wavefront with
 //                     ballot-built match masks, tiles are re-ordered in LDS so that the global
@@ -28,8 +28,8 @@
 //                     so J, dJ and the tile's share of the loss follow at once; dJ goes to
 //                     pixel order through region-binned staging (final) and an in-LDS permute
 //                     per region (unbin), which also writes the zeros of the keys left out.
-//   4. loss per class sum of the per-tile partials, whose terms are multiples of 2^-51 and add exactly (loss_term): by the first unbin block of the class, or by
-//                     reduce_loss when the rows are too long for the staging regions.
+//   4. loss per class sum of the per-tile partials in double, in a fixed order (add_loss): by the first unbin block of the
+//                     class, or by reduce_loss when the rows are too long for the staging regions.
 // A 4096-key tile is handled by 512 threads with 8 keys each; neighbouring tiles of a class row run
 // on the same XCD (sort_tile) so that the sectors they share merge in one L2.
 // Equal errors keep pixel order (the sort is stable); the reference leaves tie order open.
@@ -952,7 +952,7 @@ __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, floa
                 const uint32_t pos = out_base[d] + counts[wave][d] + rank[r];            // rank in the descending order
                 const uint32_t cs = hot_base[d] + counts_hot[wave][d] + hrank[r];      // positives before it
                 dj = jaccard_step(npos, pos, cs, hot);
-                part += loss_term(key_error(k), dj);
+                part = add_loss(part, key_error(k), dj);
             }
             if constexpr (Binned) {
                 const uint32_t lp = region_start[val[r] >> region_bits] + slot[r];

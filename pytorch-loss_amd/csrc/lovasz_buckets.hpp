@@ -71,11 +71,11 @@ __device__ __forceinline__ uint32_t bk_limit(const BucketArgs &a, int c) {
     return lowest <= kOne ? lowest : kOne;
 }
 
-// A term of a class's loss, rounded to a multiple of 2^-51: such terms, and their sums below 4 (a loss is at most 1), are
-// exact in double, so that the sum does not depend on the order of its terms.
-__device__ __forceinline__ double loss_term(float e, float dj) {
-    const double t = (double)(e * dj);
-    return (t + 3.0) - 3.0;
+// A class's loss with one term more. The product of two floats is exact in double, and the terms are added in a fixed order:
+// small losses keep their digits, and a loss is the same on every call. Another order of the terms (radix passes, buckets)
+// moves the sum by a few 2^-53 of it, which its rounding to float all but never shows.
+__device__ __forceinline__ double add_loss(double sum, float e, float dj) {
+    return __builtin_fma((double)e, (double)dj, sum);
 }
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll
@@ -832,7 +832,7 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) 
         if (a.count[(int64_t)c * kStride + d] & kBkFlat) {
             const uint32_t pos = out_base[d] + p0 + e;
             const float dj = jaccard_step(npos, pos, hot_start[d] + cs, k >> 31);
-            part += loss_term(key_error(k), dj);
+            part = add_loss(part, key_error(k), dj);
             a.dj[(int64_t)c * a.P + pos] = dj;
         }
         cs += k >> 31;
@@ -943,7 +943,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
             const float j_now = 1.f - inter / (inter + (float)(pos + 1u + e));
             const float dj = j_now - j_prev;                                           // csrc/lovasz_softmax.cu:141-147
             j_prev = j_now;
-            part += loss_term(key_error(bk_key_of(v[e])), dj);
+            part = add_loss(part, key_error(bk_key_of(v[e])), dj);
             result[bk_item_of(v[e])] = dj;
         };
         if (p0 + kBkChunk <= kept) {
@@ -1024,7 +1024,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
                 if ((valid >> r) & 1u) {
                     const uint32_t k = Direct ? key[r] : kin[li];       // read again: not held across the sort
                     dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), k >> 31);
-                    part += loss_term(key_error(k), dj);
+                    part = add_loss(part, key_error(k), dj);
                 }
                 out[li] = dj;
             }
@@ -1137,7 +1137,7 @@ __device__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t
                             if (i < n && bits >= first && bits < end) {
                                 if (single) {
                                     const float dj = jaccard_step(npos, rank0 + at, hot0 + at_hot, k[r] >> 31);
-                                    part += loss_term(key_error(k[r]), dj);
+                                    part = add_loss(part, key_error(k[r]), dj);
                                     out[i] = dj;
                                 } else {
                                     s.key()[at] = what == 0 ? k[r] : (uint32_t)i;
@@ -1172,7 +1172,7 @@ __device__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t
                         for (int r = 0; r < kBkItems; ++r) {
                             if ((valid >> r) & 1u) {
                                 const float dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), key[r] >> 31);
-                                part += loss_term(key_error(key[r]), dj);
+                                part = add_loss(part, key_error(key[r]), dj);
                                 out[place[r]] = dj;
                             }
                         }

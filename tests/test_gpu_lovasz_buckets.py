@@ -1,6 +1,7 @@
 """The Lovasz forward's sort by value buckets against the look-back variant, which sorts the same keys by radix passes: the
-Jaccard differences have to be the same bit for bit (same ranks, equal keys in pixel order), and so do the losses, whose
-terms are added exactly. Rows at the limits of the paths (one block, each number of buckets), values that crowd: ties,
+Jaccard differences have to be the same bit for bit (same ranks, equal keys in pixel order), and so do the losses: their terms
+are exact in double and added in double, in an order of its own per path, so that the sums are some 2^-50 of their value
+apart before they are rounded to float (equal for these inputs; for one in some 2^26 a rounding would fall between). Rows at the limits of the paths (one block, each number of buckets), values that crowd: ties,
 clusters, one value only, rows without positives, and buckets that outgrow a block because the sampled bounds miss them."""
 import numpy as np
 import pytest
@@ -122,3 +123,24 @@ def test_planes_of_odd_length(native, n_cls, dtype, plane):
         out.append((losses, jacc, a.grad))
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
     assert torch.equal(out[0][2], out[1][2][0].transpose(0, 1).reshape(x.shape))
+
+
+@pytest.mark.parametrize("pixels", [5000, 300000, 2560 * 1024, 2700000])
+@pytest.mark.parametrize("gap", [18.5, 30.0])
+def test_small_losses_keep_their_digits(native, pixels, gap):
+    """A network that is all but certain: class losses down to 1e-14, whose terms are far below a loss's usual last bit. The
+    errors follow from the logits (1 + exp(-gap) rounds to 1: the positives have none), the Jaccard differences from the
+    forward, and the loss is the sum of their products. An error is good to some 2 units in its last place (expf), 3e-7."""
+    rng = np.random.default_rng(pixels)
+    y = rng.integers(0, 2, (1, 1, pixels))
+    below = (gap + rng.integers(0, 64, pixels) / 64).astype(np.float32)
+    x = np.zeros((1, 2, 1, pixels), np.float32)
+    np.put_along_axis(x, 1 - y[:, None], -below[None, None, None, :], 1)
+    xt, yt = torch.as_tensor(x).cuda(), torch.as_tensor(y).cuda()
+    error = np.exp(-below.astype(np.float64))
+    for look_back in (False, True):
+        losses, jacc = native.lovasz_forward(xt, yt, 255, look_back=look_back)
+        jacc = jacc.cpu().numpy().astype(np.float64).reshape(2, pixels)
+        for c in range(2):
+            want = (error * jacc[c])[y.reshape(-1) != c].sum()
+            assert abs(losses[c].item() - want) <= 1e-6 * want
