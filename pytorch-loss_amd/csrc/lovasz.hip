@@ -1169,6 +1169,7 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
     if (dimsize >= 512) return PLH_ERR_TOO_MANY_CLASSES;
     const double numel = (double)n_size * (double)dimsize * (double)m_size;
     if (numel >= 2147483648.0) return PLH_ERR_BAD_SIZE;
+    pl = {};                // what a route has no use for is 0
     pl.P = n_size * m_size;
     pl.E = pl.P * dimsize;
     pl.tiles = (int)ceil_div(pl.P, kSortTile);
@@ -1179,8 +1180,6 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
     // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
     // 8 keys of a tile. At 2048 buckets (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
     // and two classes took 0.63 ms against 0.39 of the radix passes.
-    pl.look_back = false;
-    pl.regions = 0;
     pl.buckets = !look_back && pl.P <= kBkMaxRow;
     if (pl.buckets) {
         pl.bk_tiles = (int)ceil_div(pl.P, kBkTile);
@@ -1320,15 +1319,6 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
     hipStream_t st = (hipStream_t)stream;
     char *ws = static_cast<char *>(workspace);
     uint32_t *keys_0 = reinterpret_cast<uint32_t *>(jacc);          // the keys as built, in pixel order; jacc is free until the last pass
-    uint32_t *keys_a = reinterpret_cast<uint32_t *>(ws + pl.off_keys_a);
-    uint32_t *keys_c = reinterpret_cast<uint32_t *>(ws + pl.off_keys_c);
-    uint32_t *vals_a = reinterpret_cast<uint32_t *>(ws + pl.off_vals_a);
-    uint32_t *vals_b = reinterpret_cast<uint32_t *>(ws + pl.off_vals_b);
-    uint32_t *hist = reinterpret_cast<uint32_t *>(ws + pl.off_hist);
-    uint32_t *hot = reinterpret_cast<uint32_t *>(ws + pl.off_hot);
-    uint32_t *digit_total = reinterpret_cast<uint32_t *>(ws + pl.off_digit_total);
-    uint32_t *hot_total = reinterpret_cast<uint32_t *>(ws + pl.off_hot_total);
-    double *tile_loss = reinterpret_cast<double *>(ws + pl.off_tile_loss);
     uint32_t *pos_max = reinterpret_cast<uint32_t *>(ws + pl.off_class);
     uint32_t *kept = pos_max + dimsize;
     uint32_t *all_min = pos_max + 2 * dimsize;
@@ -1366,12 +1356,24 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
                                pl.P, m_size, C, ignore_index);
         }
     });
-    hipLaunchKernelGGL(lov_class_max, dim3((unsigned)C), dim3(1024), 0, st, block_table, (int)key_blocks, C, pos_max,
-                       reinterpret_cast<uint32_t *>(ws + pl.off_cursors), pl.regions);
+    uint32_t *cursors = pl.regions > 0 ? reinterpret_cast<uint32_t *>(ws + pl.off_cursors) : nullptr;
+    hipLaunchKernelGGL(lov_class_max, dim3((unsigned)C), dim3(1024), 0, st, block_table, (int)key_blocks, C, pos_max, cursors,
+                       pl.regions);
     hipLaunchKernelGGL(lov_absent_min, dim3(kAbsentBlocks, (unsigned)C), dim3(256), 0, st, keys_0, pos_max, all_min,
                        (int)pl.P);
 
     if (pl.buckets) return lovasz_buckets(pl, ws, keys_0, pos_max, losses, C, st);
+
+    // what the plan lays out for the radix passes only
+    uint32_t *keys_a = reinterpret_cast<uint32_t *>(ws + pl.off_keys_a);
+    uint32_t *keys_c = reinterpret_cast<uint32_t *>(ws + pl.off_keys_c);
+    uint32_t *vals_a = reinterpret_cast<uint32_t *>(ws + pl.off_vals_a);
+    uint32_t *vals_b = reinterpret_cast<uint32_t *>(ws + pl.off_vals_b);
+    uint32_t *hist = reinterpret_cast<uint32_t *>(ws + pl.off_hist);
+    uint32_t *hot = reinterpret_cast<uint32_t *>(ws + pl.off_hot);
+    uint32_t *digit_total = reinterpret_cast<uint32_t *>(ws + pl.off_digit_total);
+    uint32_t *hot_total = reinterpret_cast<uint32_t *>(ws + pl.off_hot_total);
+    double *tile_loss = reinterpret_cast<double *>(ws + pl.off_tile_loss);
 
     // 2. up to three stable scatter passes: (keys_0, -) -> (keys_a, vals_a) -> (keys_c, vals_b) -> (keys_a, vals_a);
     //    how many a class takes follows from the width of its keys (DigitPlan), the blocks of a pass
@@ -1460,7 +1462,7 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
                            pl.tiles_pad, key_bits, kLastPass, kept, (int)pl.P);
     }
     if (pl.regions > 0) {
-        uint32_t *cursors = reinterpret_cast<uint32_t *>(ws + pl.off_cursors);      // zeroed by lov_class_max
+        // the cursors were zeroed by lov_class_max
         // the value buffer that a class's last pass does not read receives the pixel offsets that go with
         // the staged values
         if (pl.look_back)
