@@ -1164,6 +1164,26 @@ struct LovaszPlan {
 
 static int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
+// Whether rows of P keys in C classes go by value buckets. Steps of radix passes -> buckets, us, captured, of ten kinds of
+// logits (soft, a new network's, all equal, confident by 8 / 14 / 20, trained, bf16, in steps of 1/16): the ordinary one and the
+// one that buckets like least, mostly a network so sure that thousands of keys share a value (multiples of 2^-24 below 1)
+// and have to be sorted apart in LDS, by few blocks if the classes are few.
+//   one block per row: always (two classes of 7680 pixels 88 -> 49, at worst 90 -> 75)
+//   2 classes of 262144 97 -> 104, at worst 102 -> 180; 4 of 263169 116 -> 108, 119 -> 182; 8 of 262144 132 -> 121, 142 -> 186
+//   16 of 65536 112 -> 95, 131 -> 164; of 262144 168 -> 140, 210 -> 210; of 524288 234 -> 189, 328 -> 279
+//   12 of 262144 155 -> 135, 189 -> 211; of 524288 205 -> 171, 242 -> 241
+//   24 of 65536 132 -> 102, 151 -> 163; of 131072 154 -> 118, 195 -> 195
+//   8 of 524288 173 -> 155, 197 -> 213; of 1048576 271 -> 216, 303 -> 289; 6 of 2097152 369 -> 293, 424 -> 432
+//   32 of 8192 113 -> 88, 131 -> 115; of 65536 155 -> 117, 166 -> 167; 64 of 8192 182 -> 140, 166 -> 142
+// P C^2 >= 2^26 and C >= 32 leave out what may lose. (On rows of some 2 M pixels all-equal logits, whose keys mostly
+// take no part, stay up to 7 % slower, a new network's up to 3 %.)
+// Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
+// 8 keys of a tile. With 2048 buckets of 3072 (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
+// and two classes took 0.63 ms against 0.39 of the radix passes.
+static bool bk_pays(int64_t P, int64_t C) {
+    return P <= kBkCap || (P <= kBkMaxRow && (C >= 32 || P * C * C >= ((int64_t)1 << 26)));
+}
+
 static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan &pl, bool look_back = false) {
     if (n_size < 0 || dimsize < 0 || m_size < 0) return PLH_ERR_BAD_SIZE;
     if (dimsize >= 512) return PLH_ERR_TOO_MANY_CLASSES;
@@ -1177,10 +1197,7 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
     int64_t off = 0;
     pl.off_class = off;       off += round_up(4 * dimsize * 4, 256);      // pos_max[C], kept[C], all_min[C], key_bits[C]
     pl.off_block_max = off;   off += round_up(4 * dimsize * ceil_div(pl.P, 256), 256);   // [key blocks][C]
-    // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
-    // 8 keys of a tile. At 2048 buckets (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
-    // and two classes took 0.63 ms against 0.39 of the radix passes.
-    pl.buckets = !look_back && pl.P <= kBkMaxRow;
+    pl.buckets = !look_back && bk_pays(pl.P, dimsize);
     if (pl.buckets) {
         pl.bk_tiles = (int)ceil_div(pl.P, kBkTile);
         const int64_t most = ceil_div(pl.P, kBkTarget);

@@ -35,14 +35,34 @@ def compare(native, x, y):
     return losses
 
 
+def by_buckets(n_cls, pixels):
+    """The route of a row, by its workspace: 10 bytes per key and tables (buckets), 16 and tables (radix passes)."""
+    from pytorch_loss import _native
+    return _native.load().plh_lovasz_workspace_bytes(1, n_cls, pixels) < 16 * n_cls * pixels
+
+
+def test_which_rows_go_by_buckets(native):
+    """Few classes of more pixels than one block holds went by buckets at first, up to three quarters slower than by radix
+    passes where predictions are confident (2 classes of 262144 pixels: 102 -> 180 us)."""
+    many = 2560 * 1024
+    for n_cls, pixels, want in [(2, 7681, False), (2, 65536, False), (2, 262144, False), (2, many, False), (4, 263169, False),
+                                (4, many, False), (8, 262144, False), (16, 65536, False), (19, 90300, False), (31, 65536, False),
+                                (6, many, True), (8, 1048576, True), (16, 262144, True), (19, 4 * 512 * 1024, True),
+                                (32, 65536, True), (150, 65536, True), (19, many + 1, False)]:
+        assert by_buckets(n_cls, pixels) == want, (n_cls, pixels)
+
+
 # pixels: one block's limit, 64 / 256 / 1024 buckets, the longest row that is cut into buckets and the first that is not
+# classes: few (radix passes above one block's limit) and enough for buckets
 @pytest.mark.parametrize("pixels", [1, 63, 512, 513, 7679, 7680, 7681, 8193, 20011, 2560 * 64, 2560 * 64 + 1, 2560 * 256 + 7])
 @pytest.mark.parametrize("boost", [0.0, 10.0])
-def test_row_lengths(native, pixels, boost):
+@pytest.mark.parametrize("n_cls", [3, 33])
+def test_row_lengths(native, pixels, boost, n_cls):
+    assert n_cls == 3 or pixels < 1000 or by_buckets(n_cls, pixels)
     rng = np.random.default_rng(pixels)
-    x = rng.standard_normal((1, 3, 1, pixels), dtype=np.float32) * 2
-    y = labels(rng, (1, 1, pixels), 3)
-    x += np.float32(boost) * (np.arange(3)[None, :, None, None] == y[:, None])
+    x = rng.standard_normal((1, n_cls, 1, pixels), dtype=np.float32) * 2
+    y = labels(rng, (1, 1, pixels), n_cls)
+    x += np.float32(boost) * (np.arange(n_cls)[None, :, None, None] == y[:, None])
     losses = compare(native, x, y)
     if pixels < 10000 and not boost:
         want, _ = oracle.lovasz_forward(x.astype(np.float64), y, 255)
@@ -50,18 +70,22 @@ def test_row_lengths(native, pixels, boost):
 
 
 @pytest.mark.parametrize("pixels", [1024 * 2560, 1024 * 2560 + 1])
-def test_longest_rows(native, pixels):
+@pytest.mark.parametrize("n_cls", [2, 6])
+def test_longest_rows(native, pixels, n_cls):
+    assert by_buckets(n_cls, pixels) == (n_cls == 6 and pixels == 1024 * 2560)
     g = torch.Generator(device="cuda").manual_seed(3)
-    x = torch.randn((1, 2, 1, pixels), device="cuda", generator=g)
-    y = torch.randint(0, 2, (1, 1, pixels), device="cuda", generator=g)
+    x = torch.randn((1, n_cls, 1, pixels), device="cuda", generator=g)
+    y = torch.randint(0, n_cls, (1, 1, pixels), device="cuda", generator=g)
     compare(native, x, y)
 
 
 @pytest.mark.parametrize("pixels", [5000, 40000, 300000])
 @pytest.mark.parametrize("kind", ["constant", "few values", "half steps", "cluster", "two clusters", "certain", "absent"])
-def test_crowded_values(native, pixels, kind):
+@pytest.mark.parametrize("many", [False, True])
+def test_crowded_values(native, pixels, kind, many):
     rng = np.random.default_rng(len(kind) + pixels)
-    n_cls = 2 if kind in ("few values", "half steps") else 4
+    n_cls = 32 if many else (2 if kind in ("few values", "half steps") else 4)
+    assert not many or by_buckets(n_cls, pixels)
     x = rng.standard_normal((1, n_cls, 1, pixels), dtype=np.float32)
     y = labels(rng, (1, 1, pixels), n_cls)
     if kind == "constant":              # every error the same
@@ -91,14 +115,17 @@ def sampled(pixels):
 
 @pytest.mark.parametrize("pixels", [70000, 500000])
 @pytest.mark.parametrize("kind", ["spread", "one value", "both"])
-def test_buckets_that_the_sample_misses(native, pixels, kind):
+@pytest.mark.parametrize("n_cls", [2, 32])
+def test_buckets_that_the_sample_misses(native, pixels, kind, n_cls):
+    assert n_cls == 2 or by_buckets(n_cls, pixels)
     rng = np.random.default_rng(pixels)
     d = rng.random(pixels) * (0.0 if kind == "one value" else 1e-2)
     if kind == "both":
         d[rng.random(pixels) < 0.5] = 5e-3
     at = sampled(pixels).astype(np.int64)
     d[at] = 1 + rng.random(at.size)
-    x = np.stack([d, np.zeros(pixels)])[None, :, None, :].astype(np.float32)
+    # the classes beyond the first two are absent, and hardly predicted
+    x = np.stack([d, np.zeros(pixels)] + [np.full(pixels, -30.0)] * (n_cls - 2))[None, :, None, :].astype(np.float32)
     compare(native, x, labels(rng, (1, 1, pixels), 2))
 
 
@@ -127,20 +154,22 @@ def test_planes_of_odd_length(native, n_cls, dtype, plane):
 
 @pytest.mark.parametrize("pixels", [5000, 300000, 2560 * 1024, 2700000])
 @pytest.mark.parametrize("gap", [18.5, 30.0])
-def test_small_losses_keep_their_digits(native, pixels, gap):
+@pytest.mark.parametrize("n_cls", [2, 32])
+def test_small_losses_keep_their_digits(native, pixels, gap, n_cls):
     """A network that is all but certain: class losses down to 1e-14, whose terms are far below a loss's usual last bit. The
     errors follow from the logits (1 + exp(-gap) rounds to 1: the positives have none), the Jaccard differences from the
     forward, and the loss is the sum of their products. An error is good to some 2 units in its last place (expf), 3e-7."""
     rng = np.random.default_rng(pixels)
     y = rng.integers(0, 2, (1, 1, pixels))
     below = (gap + rng.integers(0, 64, pixels) / 64).astype(np.float32)
-    x = np.zeros((1, 2, 1, pixels), np.float32)
+    x = np.full((1, n_cls, 1, pixels), -200.0, np.float32)          # classes that nothing predicts: exp(-200) is 0
+    x[:, :2] = 0.0
     np.put_along_axis(x, 1 - y[:, None], -below[None, None, None, :], 1)
     xt, yt = torch.as_tensor(x).cuda(), torch.as_tensor(y).cuda()
     error = np.exp(-below.astype(np.float64))
     for look_back in (False, True):
         losses, jacc = native.lovasz_forward(xt, yt, 255, look_back=look_back)
-        jacc = jacc.cpu().numpy().astype(np.float64).reshape(2, pixels)
+        jacc = jacc[:2].cpu().numpy().astype(np.float64).reshape(2, pixels)
         for c in range(2):
             want = (error * jacc[c])[y.reshape(-1) != c].sum()
             assert abs(losses[c].item() - want) <= 1e-6 * want
