@@ -1157,7 +1157,7 @@ struct LovaszPlan {
     bool buckets;
     int bk_tiles, bk_bits;
     int64_t off_sorted, off_dj, off_tile_count, off_count, off_bounds, off_buckets, off_fine, off_loss_part,
-        off_crowded, off_bucket, off_tile_hot, off_bk_tile_loss;
+        off_crowded, off_bucket;
     int hist_blocks;
     int64_t off_lb_clear, lb_clear_bytes, off_lb_totals, off_lb_partial;
 };
@@ -1175,8 +1175,8 @@ static int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 //   24 of 65536 132 -> 102, 151 -> 163; of 131072 154 -> 118, 195 -> 195
 //   8 of 524288 173 -> 155, 197 -> 213; of 1048576 271 -> 216, 303 -> 289; 6 of 2097152 369 -> 293, 424 -> 432
 //   32 of 8192 113 -> 88, 131 -> 115; of 65536 155 -> 117, 166 -> 167; 64 of 8192 182 -> 140, 166 -> 142
-// P C^2 >= 2^26 and C >= 32 leave out what may lose. (On rows of some 2 M pixels all-equal logits, whose keys mostly
-// take no part, stay up to 7 % slower, a new network's up to 3 %.)
+// P C^2 >= 2^26 and C >= 32 leave out what may lose. (On rows of some 2 M pixels a new network's predictions, whose keys mostly
+// take no part, are level: (8,19,512,512) 419 -> 421, (8,21,513,513) 496 -> 510.)
 // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
 // 8 keys of a tile. With 2048 buckets of 3072 (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
 // and two classes took 0.63 ms against 0.39 of the radix passes.
@@ -1209,11 +1209,9 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
         pl.off_dj = off;         off += round_up(4 * pl.E, 256);
         pl.off_bucket = off;     off += round_up(2 * pl.E, 256);
         pl.off_tile_count = off; off += round_up(4 * cells * pl.bk_tiles, 256);
-        pl.off_tile_hot = off;   off += round_up(4 * cells * pl.bk_tiles, 256);
-        pl.off_bk_tile_loss = off; off += round_up(8 * dimsize * pl.bk_tiles, 256);
         pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // count, hot, base, hot_base, runs
         pl.off_bounds = off;     off += round_up(4 * cells, 256);
-        pl.off_buckets = off;    off += round_up(4 * 6 * dimsize, 256);
+        pl.off_buckets = off;    off += round_up(4 * 5 * dimsize, 256);
         pl.off_fine = off;       off += round_up(2 * dimsize * (kBkFine + 2), 256);
         pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
         pl.bytes = off;
@@ -1285,8 +1283,6 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
     a.sorted = reinterpret_cast<uint32_t *>(ws + pl.off_sorted);
     a.dj = reinterpret_cast<float *>(ws + pl.off_dj);
     a.bucket = reinterpret_cast<uint16_t *>(ws + pl.off_bucket);
-    a.tile_hot = reinterpret_cast<uint32_t *>(ws + pl.off_tile_hot);
-    a.tile_loss = reinterpret_cast<double *>(ws + pl.off_bk_tile_loss);
     a.tile_count = reinterpret_cast<uint32_t *>(ws + pl.off_tile_count);
     a.count = reinterpret_cast<uint32_t *>(ws + pl.off_count);
     a.hot = reinterpret_cast<uint32_t *>(ws + pl.off_count + step);

@@ -10,10 +10,10 @@
 //                 left in the place of its keys
 //   bk_rank       a block per run of buckets: sorted in LDS, Jaccard difference of every key at its place
 //   bk_rank_crowded  the same for runs whose values crowd
-//   bk_rank_wide  the same for buckets that outgrew the LDS
+//   bk_rank_wide  the same for buckets that outgrew the LDS, and for single values that fill more than that
 //   bk_gather     Jaccard differences back to pixel order, tile by tile
 // Sampled bounds follow any distribution; a value that fills several buckets by itself gets one of its own, which
-// needs no sort (flat: bk_scatter knows the ranks), and a bucket that outgrew the LDS all the same is taken in value ranges
+// needs no sort (flat: its keys are ranked as they stand), and a bucket that outgrew the LDS all the same is taken in value ranges
 // that fit.
 // Bound by vector instructions (scatter and rank: some 80 and 110 per 64 keys at 16 waves per CU) and short runs, not by
 // the 40 bytes a key moves. Forward and backward, against the radix passes: (8,21,513,513) bf16 trained 1.21 -> 0.82 ms,
@@ -50,17 +50,14 @@ struct BucketArgs {
     uint16_t *bucket;           // [C][P] bucket of every pixel
     uint32_t *tile_count;       // [C][tiles][stride]: keys | positives << 16, exclusive sums over the tiles, start of the
                                 // tile's keys of the bucket in the row less their start in the tile
-    uint32_t *tile_hot;         // [C][tiles][stride] positives in the tiles before, of buckets with more than kBkCap keys
     uint32_t *count, *hot;      // [C][stride] keys (kBkFlat: and a single value), positives per bucket
     uint32_t *base, *hot_base;  // [C][stride + 1] the same before the bucket
     uint32_t *bounds;           // [C][stride] least key of buckets 1, 2, ...
     uint32_t *runs;             // [C][stride + 1] first bucket of every run, and the end
     uint32_t *crowded;          // [C][stride] runs (rows of one block: [C]) whose values crowd
-    uint32_t *numbers;          // [6][C]: buckets, runs, positives, least key of the sample, flat buckets,
-                                // largest key of the sample below the limit
+    uint32_t *numbers;          // [5][C]: buckets, runs, positives, least key of the sample, largest one below the limit
     uint16_t *fine;             // [C][kBkFine + 2]
-    double *loss_part;          // [C][2 * stride]: runs, wide buckets
-    double *tile_loss;          // [C][tiles] of the flat buckets, where there are any
+    double *loss_part;          // [C][2 * stride]: runs, wide and flat buckets
     int P, C, tiles, stride;
 };
 
@@ -460,7 +457,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
             if (sorted[mid] < limit) lo = mid + 1;
             else hi = mid;
         }
-        a.numbers[5 * a.C + c] = lo ? sorted[lo - 1] : 0u;
+        a.numbers[4 * a.C + c] = lo ? sorted[lo - 1] : 0u;
     }
     // the bucket of the least key with each pattern of the top bits
     const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
@@ -572,15 +569,6 @@ __global__ __launch_bounds__(1024) void bk_scan(const BucketArgs a) {
         total += v;
         hot += hots[g][threadIdx.x & 63];
     }
-    if (total > (uint32_t)kBkCap) {
-        uint32_t *hot_at = a.tile_hot + (int64_t)c * a.tiles * a.stride + b;
-        uint32_t hot_before = 0;
-        for (int g = 0; g < group; ++g) hot_before += hots[g][threadIdx.x & 63];
-        for (int t = first; t < last; ++t) {
-            hot_at[(int64_t)t * a.stride] = hot_before;
-            hot_before += at[(int64_t)t * a.stride] >> 16;
-        }
-    }
 #pragma unroll 8
     for (int t = first; t < last; ++t) {
         const uint32_t v = at[(int64_t)t * a.stride];
@@ -633,16 +621,13 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
     const uint32_t least = a.numbers[3 * a.C + c];
     auto width = [&](int b) { return (float)(bound[b] - (b ? bound[b - 1] : min(least, bound[0]))) / (float)(base[b + 1] - base[b] + 1u); };
     bool start[kPer];
-    uint32_t starts = 0, flats = 0;
+    uint32_t starts = 0;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
         const int b = b0 + i;
         start[i] = false;
         if (b >= buckets) continue;
-        if (n[i] > (uint32_t)kBkCap && b && bound[b] - bound[b - 1] == 1u) {
-            a.count[(int64_t)c * a.stride + b] = n[i] | kBkFlat;
-            flats = 1;
-        }
+        if (n[i] > (uint32_t)kBkCap && b && bound[b] - bound[b - 1] == 1u) a.count[(int64_t)c * a.stride + b] = n[i] | kBkFlat;
         const uint32_t slab = base[b] / kBkSlab;
         start[i] = b == 0 || base[b - 1] / kBkSlab != slab;
         if (!start[i]) {
@@ -654,9 +639,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
         }
         starts += start[i] ? 1u : 0u;
     }
-    uint32_t runs, any_flat, unused;
-    uint32_t k;
-    block_excl_scan2(starts, flats, scan_tmp, k, runs, unused, any_flat);
+    uint32_t runs;
+    uint32_t k = block_excl_scan(starts, scan_tmp, runs);
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
         if (start[i]) a.runs[row + k++] = (uint32_t)(b0 + i);
@@ -664,7 +648,6 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
         a.runs[row + runs] = (uint32_t)buckets;
         a.numbers[a.C + c] = runs;
         a.numbers[2 * a.C + c] = n_hot;
-        a.numbers[4 * a.C + c] = any_flat;
     }
 }
 
@@ -800,52 +783,6 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) 
         kout[out_base[d] + (uint32_t)i] = s_key[i];
         places[n + i] = (uint16_t)d;
     }
-    if (a.numbers[4 * a.C + c] == 0) return;                // block-uniform
-    // Buckets of a single value that no block would hold: their keys are in order, so the place is the rank; the positives
-    // before it are those of the buckets before, of the tiles before and of the places before. A thread takes 16 neighbours.
-    __shared__ double wave_loss[kBkWaves];
-    // positives before the bucket's first place, less those of the tile before it
-    uint32_t *hot_start = a.tile_hot + ((int64_t)c * a.tiles + tile) * kStride;
-    const uint32_t p0 = threadIdx.x * kBkTileItems;
-    uint32_t hots = 0, all;
-#pragma unroll
-    for (int e = 0; e < kBkTileItems; ++e) hots += p0 + e < n_here ? s_key[p0 + e] >> 31 : 0u;
-    uint32_t cs = block_excl_scan(hots, scan_tmp, all);
-    {
-        uint32_t before = cs;
-#pragma unroll
-        for (int e = 0; e < kBkTileItems; ++e) {
-            if (p0 + e < n_here) {
-                const uint32_t d = s_bucket[p0 + e];
-                if ((p0 + e == 0 || s_bucket[p0 + e - 1] != d) && (a.count[(int64_t)c * kStride + d] & kBkFlat))
-                    hot_start[d] += a.hot_base[(int64_t)c * (kStride + 1) + d] - before;
-                before += s_key[p0 + e] >> 31;
-            }
-        }
-    }
-    __syncthreads();
-    const float npos = (float)a.numbers[2 * a.C + c];
-    double part = 0.0;
-    for (int e = 0; e < kBkTileItems; ++e) {
-        if (p0 + e >= n_here) break;
-        const uint32_t d = s_bucket[p0 + e], k = s_key[p0 + e];
-        if (a.count[(int64_t)c * kStride + d] & kBkFlat) {
-            const uint32_t pos = out_base[d] + p0 + e;
-            const float dj = jaccard_step(npos, pos, hot_start[d] + cs, k >> 31);
-            part = add_loss(part, key_error(k), dj);
-            a.dj[(int64_t)c * a.P + pos] = dj;
-        }
-        cs += k >> 31;
-    }
-    part = wave_sum_f64(part);
-    if ((threadIdx.x & 63) == 0) wave_loss[wave] = part;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double sum = 0.0;
-#pragma unroll
-        for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
-        a.tile_loss[(int64_t)c * a.tiles + tile] = sum;
-    }
 }
 
 // One run of buckets (or, Direct: a whole row of at most kBkCap pixels, straight from the keys in pixel order, with the
@@ -904,7 +841,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
         if (!flat && (b0 == 0 || b1 + 1u >= buckets)) {
             // beyond the sample lie a few more, far apart: their own bins
             bk_range(s, key, valid, least, most);
-            knee = b0 ? a.numbers[5 * a.C + c] + 1u : a.numbers[3 * a.C + c];
+            knee = b0 ? a.numbers[4 * a.C + c] + 1u : a.numbers[3 * a.C + c];
             share = b0 ? 0.75f : 0.25f;
         }
     }
@@ -1189,21 +1126,88 @@ __device__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t
     return part;
 }
 
-constexpr int kBkWideBlocks = 32;               // per class: one bucket at a time each
+constexpr int kBkWideBlocks = 32;               // per class: one wide bucket at a time each, all of them for a flat one
+
+// Jaccard index of a class's first k keys, cs of its npos positives among them: a multiple of 2^-24, whatever the division
+// gives (a quotient from 1/2 on is one, and its difference from 1 is exact; one below leaves a difference from 1/2 on).
+__device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
+    const float inter = npos - (float)cs;
+    return k == 0 ? 0.f : 1.f - inter / (inter + (float)k);
+}
+
+// This block's part of a bucket of one value, n keys from rank0 on with hot0 positives before them and `hot` among them: in
+// order as they stand. The positives before the part are counted again by every block where the flags are mixed (a value
+// that many share is mostly the positives' or the others' alone). Done by bk_scatter, 16 places per thread, this took that
+// kernel from 94 to 149 us where all logits are equal ((8,19,512,512)); step 459 -> 418 us, radix passes 425.
+__device__ void bk_flat_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n, uint32_t hot) {
+    constexpr uint32_t kPer = 8, kStep = kPer * kBkThreads;
+    const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
+    float *out = a.dj + (int64_t)c * a.P + rank0;
+    const float npos = (float)a.numbers[2 * a.C + c];
+    const uint32_t part = ((n + kBkWideBlocks - 1) / kBkWideBlocks + kStep - 1) / kStep * kStep;
+    const uint32_t from = blockIdx.x * part, end = min(n, from + part);
+    if (from >= n) return;                                  // block-uniform
+    const bool mixed = hot != 0u && hot != n;
+    uint32_t before = hot ? from : 0u;                      // positives of the bucket before the part
+    if (mixed) {
+        uint32_t mine = 0;
+#pragma unroll 8
+        for (uint32_t i = threadIdx.x; i < from; i += kBkThreads) mine += kin[i] >> 31;
+        block_excl_scan(mine, s.scan, before);
+    }
+    for (uint32_t i0 = from; i0 < end; i0 += kStep) {
+        const uint32_t p0 = i0 + threadIdx.x * kPer;
+        uint32_t flags = hot ? 0xFFu : 0u;
+        uint32_t cs = hot0 + (hot ? p0 : 0u);
+        if (mixed) {
+            flags = 0;
+#pragma unroll
+            for (uint32_t e = 0; e < kPer; ++e) flags |= (p0 + e < end ? kin[p0 + e] >> 31 : 0u) << e;
+            uint32_t all;
+            cs = hot0 + before + block_excl_scan((uint32_t)__builtin_popcount(flags), s.scan, all);
+            before += all;
+        }
+        float j_prev = jaccard(npos, rank0 + p0, cs);
+#pragma unroll
+        for (uint32_t e = 0; e < kPer; ++e) {
+            cs += (flags >> e) & 1u;
+            const float j_now = jaccard(npos, rank0 + p0 + e + 1u, cs);
+            if (p0 + e < end) out[p0 + e] = j_now - j_prev;                            // csrc/lovasz_softmax.cu:141-147
+            j_prev = j_now;
+        }
+    }
+}
+
 __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
     __shared__ BkShared s;
     __shared__ double wave_loss[kBkWaves];
     __shared__ int todo[kBkMax / kBkWideBlocks + 1], found;
+    __shared__ int flats[kBkMaxRow / kBkCap + 1], n_flats;
     const int c = blockIdx.y, buckets = (int)a.numbers[c];
     const int64_t cells = (int64_t)c * (a.stride + 1), row = (int64_t)c * a.stride;
-    if (threadIdx.x == 0) found = 0;
+    if (threadIdx.x == 0) found = n_flats = 0;
     __syncthreads();
-    for (int i = (int)blockIdx.x + kBkWideBlocks * (int)threadIdx.x; i < buckets; i += kBkWideBlocks * kBkThreads) {
+    // in any order: each has a sum and differences of its own
+    for (int i = (int)threadIdx.x; i < buckets; i += kBkThreads) {
         const uint32_t n = a.count[row + i];
-        if (n > (uint32_t)kBkCap && !(n & kBkFlat)) todo[atomicAdd(&found, 1)] = i;    // in any order: each has a sum of its own
-        else a.loss_part[2 * row + a.stride + i] = 0.0;
+        const bool mine = i % kBkWideBlocks == (int)blockIdx.x, wide = n > (uint32_t)kBkCap;
+        if (n & kBkFlat) flats[atomicAdd(&n_flats, 1)] = i;
+        else if (mine && wide) todo[atomicAdd(&found, 1)] = i;
+        if (mine && !(n & kBkFlat) && !wide) a.loss_part[2 * row + a.stride + i] = 0.0;
+        if (mine && (n & kBkFlat)) {
+            // one error, and the differences, exact as multiples of 2^-24, add up to that of the ends
+            const uint32_t first = a.base[cells + i], last = first + (n & ~kBkFlat), hots = a.hot_base[cells + i];
+            const float npos = (float)a.numbers[2 * a.C + c];
+            const float rise = jaccard(npos, last, hots + a.hot[row + i]) - jaccard(npos, first, hots);
+            a.loss_part[2 * row + a.stride + i] = add_loss(0.0, key_error(a.sorted[(int64_t)c * a.P + first]), rise);
+        }
     }
     __syncthreads();
+    const int n_flat = n_flats;
+    for (int i = 0; i < n_flat; ++i) {                      // block-uniform
+        const int b = flats[i];
+        bk_flat_keys(s, a, c, a.base[cells + b], a.hot_base[cells + b], a.count[row + b] & ~kBkFlat, a.hot[row + b]);
+    }
     const int n_todo = found;
     for (int i = 0; i < n_todo; ++i) {
         const int b = todo[i];
@@ -1273,8 +1277,6 @@ __global__ __launch_bounds__(kBkThreads) void bk_gather(const BucketArgs a, floa
     double sum = 0.0;
     for (int i = threadIdx.x; i < runs; i += kBkThreads) sum += sums[i];
     for (int i = threadIdx.x; i < buckets; i += kBkThreads) sum += sums[a.stride + i];
-    if (a.numbers[4 * a.C + c])
-        for (int i = threadIdx.x; i < a.tiles; i += kBkThreads) sum += a.tile_loss[(int64_t)c * a.tiles + i];
     sum = wave_sum_f64(sum);
     if (lane == 0) wave_sum[wave] = sum;
     __syncthreads();

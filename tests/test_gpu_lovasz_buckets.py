@@ -80,7 +80,7 @@ def test_longest_rows(native, pixels, n_cls):
 
 
 @pytest.mark.parametrize("pixels", [5000, 40000, 300000])
-@pytest.mark.parametrize("kind", ["constant", "few values", "half steps", "cluster", "two clusters", "certain", "absent"])
+@pytest.mark.parametrize("kind", ["constant", "few values", "half steps", "cluster", "two clusters", "certain", "absent", "halves"])
 @pytest.mark.parametrize("many", [False, True])
 def test_crowded_values(native, pixels, kind, many):
     rng = np.random.default_rng(len(kind) + pixels)
@@ -100,6 +100,10 @@ def test_crowded_values(native, pixels, kind, many):
         x = x * np.float32(1e-6) + np.float32(3) * (rng.random(x.shape) < 0.5)
     elif kind == "certain":             # probabilities of exactly 1, and the steps of 2^-24 below
         x += np.float32(17) * (np.arange(n_cls)[None, :, None, None] == y[:, None])
+    elif kind == "halves":              # one value, 1/2, for the positives and the others of two classes; 0 for the others
+        x[:] = -200
+        x[:, :2] = 0
+        y = np.where(y == 255, 255, y % 2)
     else:                               # classes that no pixel has
         y[:] = np.where(y == 255, 255, 1)
     compare(native, x.astype(np.float32), y)
