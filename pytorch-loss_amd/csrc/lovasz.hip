@@ -1174,7 +1174,7 @@ static int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 //   12 of 262144 155 -> 135, 189 -> 211; of 524288 205 -> 171, 242 -> 241
 //   24 of 65536 132 -> 102, 151 -> 163; of 131072 154 -> 118, 195 -> 195
 //   8 of 524288 173 -> 155, 197 -> 213; of 1048576 271 -> 216, 303 -> 289; 6 of 2097152 369 -> 293, 424 -> 432
-//   32 of 8192 113 -> 88, 131 -> 115; of 65536 155 -> 117, 166 -> 167; 64 of 8192 182 -> 140, 166 -> 142
+//   32 of 8192 113 -> 88, 131 -> 115; of 65536 141 -> 110, 166 -> 165; 64 of 8192 182 -> 140, 166 -> 142
 // P C^2 >= 2^26 and C >= 32 leave out what may lose. (On rows of some 2 M pixels a new network's predictions, whose keys mostly
 // take no part, are level: (8,19,512,512) 419 -> 421, (8,21,513,513) 496 -> 510.)
 // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
