@@ -733,7 +733,8 @@ def test_autocast_gives_fp32_losses_and_input_typed_gradients(pl, op, in_dtype, 
 def test_lovasz_sort_passes_follow_the_key_width(pl, n_cls, scale, boost, passes):
     """The sort looks only at the key bits below a class's limit: near-uniform predictions over many classes
     (best positive's error above 0.996: at most 16 key bits) take two passes, soft ones three, confident ones
-    all four. Every plan against the fp32 restatement bit for bit, and the loss against the fp64 one."""
+    all four. (Rows of 4000 pixels are one block's, which sorts the same keys whole; test_gpu_lovasz_lookback runs every plan
+    on rows that go by passes.) Every plan against the fp32 restatement bit for bit, and the loss against the fp64 one."""
     from pytorch_loss import _native
     shape = (2, n_cls, 40, 50)
     y = synth.seg_labels(53, (2, 40, 50), n_cls, 255, 0.1)
