@@ -983,149 +983,247 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
     }
 }
 
-// n keys from rank `rank0` on, with hot0 positives before them, whatever their number and values: ranges of values
-// [from, end) with at most kBkCap keys, one after the other, collected in order; a single value that more keys share is
-// ranked by position. n is at most a few times kBkCap unless one value makes it up.
-__device__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, int n) {
-    const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
-    float *out = a.dj + (int64_t)c * a.P + rank0;
+// What bk_wide_keys keeps in the block's memory: first, where the pairs are, the bounds of up to kBkIntervals value intervals
+// and their keys; then, per group, in what the crowded path leaves free behind its 256 words of counters and behind its keys
+// and items.
+constexpr int kBkIntervals = 4096, kBkGroups = 1100;
+struct BkIntervals {
+    uint32_t bound[2][kBkIntervals];
+    uint32_t count[kBkIntervals];
+};
+struct BkGroups {
+    uint32_t *least, *first;                    // [groups], [groups + 1]: least key, first rank
+    uint32_t *next, *start;                     // the next place of one of its keys, its start in the tile
+    __device__ explicit BkGroups(BkShared &s)
+        : least(s.bin + kBkWaves * 64 / 2), first(least + kBkGroups), next(reinterpret_cast<uint32_t *>(s.src() + kBkCap)),
+          start(next + kBkGroups) {}
+};
+static_assert(kBkIntervals % kBkThreads == 0 && 3 * (kBkMaxRow / kBkCap + 2) < kBkGroups, "groups, see bk_wide_groups");
+static_assert(sizeof(BkIntervals) <= sizeof(BkPair) * (kBkCap + kBkChunk) && kBkWaves * 32 + 2 * kBkGroups + 1 <= kBkBins &&
+              6 * kBkCap + 8 * kBkGroups <= (int)sizeof(BkPair) * (kBkCap + kBkChunk), "they fit");
+
+// The interval of a key: the last of m ascending bounds that is not above it.
+__device__ __forceinline__ uint32_t bk_interval(const uint32_t *bound, uint32_t m, uint32_t key) {
+    uint32_t lo = 0, hi = m;
+    while (hi - lo > 1u) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (bound[mid] <= key) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Cuts the n keys of the values lo..hi - 1 into groups of at most kBkCap keys, or of one value: intervals that hold more are
+// split, by a third at least, until none is left, and neighbours that come to no more than kBkCap are one again (those in one
+// of the n / kBkCap slabs of the order; those that lie across two stand alone). Every turn reads the keys once; the
+// values are 30 bits wide, so there are 19 at most, and 1 to 6 for what was tried. Returns the number of groups.
+__device__ __forceinline__ uint32_t bk_wide_groups(BkShared &s, const BkGroups &out, const uint32_t *kin, uint32_t n, uint32_t lo, uint32_t hi) {
+    constexpr uint32_t kPer = kBkIntervals / kBkThreads, kCap = kBkCap;
+    BkIntervals &w = *reinterpret_cast<BkIntervals *>(s.pair);
+    uint32_t m = 1, cur = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        w.bound[0][0] = lo;
+        w.count[0] = n;
+    }
+    __syncthreads();
+    for (;;) {
+        const uint32_t *bound = w.bound[cur];
+        uint32_t *next = w.bound[cur ^ 1u];
+        const uint32_t j0 = threadIdx.x * kPer;
+        uint32_t cnt[kPer], sum = 0, all;
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) {
+            cnt[u] = j0 + u < m ? w.count[j0 + u] : 0u;
+            sum += cnt[u];
+        }
+        const uint32_t cnt_before = j0 > 0u && j0 <= m ? w.count[j0 - 1u] : 0u;
+        const uint32_t first = block_excl_scan(sum, s.scan, all);
+        auto alone = [&](uint32_t at, uint32_t c) { return c > 0u && (at + c - 1u) / kCap != at / kCap; };
+        uint32_t at = first, keep = 0, split = 0;
+        bool was_alone = alone(first - cnt_before, cnt_before);
+        uint32_t slab = (first - cnt_before) / kCap;
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) {
+            const uint32_t j = j0 + u;
+            const bool is_alone = alone(at, cnt[u]);
+            if (j < m) {
+                const uint32_t width = (j + 1u < m ? bound[j + 1u] : hi) - bound[j];
+                if (cnt[u] > kCap && width > 1u) split |= 1u << u;
+                else if (j == 0 || is_alone || was_alone || at / kCap != slab) keep |= 1u << u;
+            }
+            was_alone = is_alone;
+            slab = at / kCap;
+            at += cnt[u];
+        }
+        uint32_t k, kept, d, splits;
+        block_excl_scan2((uint32_t)__builtin_popcount(keep), (uint32_t)__builtin_popcount(split), s.scan, k, kept, d, splits);
+        if (splits == 0) {                                  // block-uniform
+            at = first;
+#pragma unroll
+            for (uint32_t u = 0; u < kPer; ++u) {
+                if ((keep >> u) & 1u) {
+                    out.least[k] = bound[j0 + u];
+                    out.first[k++] = at;
+                }
+                at += cnt[u];
+            }
+            if (threadIdx.x == 0) out.first[kept] = n;
+            __syncthreads();
+            return kept;
+        }
+        const uint32_t parts = (kBkIntervals - kept) / splits;          // 3 or more: see the bound on groups
+        auto width_of = [&](uint32_t j) { return (j + 1u < m ? bound[j + 1u] : hi) - bound[j]; };
+        auto step_of = [&](uint32_t width) { return (width + parts - 1u) / parts; };
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) {
+            if ((keep >> u) & 1u) ++mine;
+            if ((split >> u) & 1u) {
+                const uint32_t width = width_of(j0 + u), step = step_of(width);
+                mine += (width + step - 1u) / step;
+            }
+        }
+        uint32_t total;
+        uint32_t to = block_excl_scan(mine, s.scan, total);
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; ++u) {
+            if ((keep >> u) & 1u) next[to++] = bound[j0 + u];
+            if ((split >> u) & 1u) {                        // a list for all threads: the parts of one may be thousands
+                const uint32_t width = width_of(j0 + u), step = step_of(width);
+                out.least[d] = j0 + u;
+                out.first[d++] = to;
+                to += (width + step - 1u) / step;
+            }
+        }
+        __syncthreads();
+        for (uint32_t i = 0; i < splits; ++i) {
+            const uint32_t j = out.least[i], width = width_of(j), step = step_of(width);
+            for (uint32_t q = threadIdx.x; q * step < width; q += kBkThreads) next[out.first[i] + q] = bound[j] + q * step;
+        }
+        m = total;
+        cur ^= 1u;
+        for (uint32_t j = threadIdx.x; j < m; j += kBkThreads) w.count[j] = 0;
+        __syncthreads();
+        for (uint32_t i0 = 0; i0 < n; i0 += kBkCap) {
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r) {
+                const uint32_t i = i0 + (uint32_t)bk_item(kBkItems, r);
+                if (i < n) atomicAdd(&w.count[bk_interval(next, m, kin[i] & 0x7FFFFFFFu)], 1u);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// A bucket of n keys of the values lo..hi - 1, from rank `rank0` on, with hot0 positives before them, many times what a block
+// holds: its keys are moved to their groups (bk_wide_groups), in order inside each, a group at a time is ranked in LDS,
+// and the differences come back through the places left where the keys were. Every key is read and moved a bounded number
+// of times: bounds that the sample misses by far ((1,32,1,500000), all keys in one bucket) cost 6.5 ms, where a sweep over
+// the bucket per 7680 keys cost 56 (radix passes 0.23); twice the keys 14 and 262.
+__device__ __forceinline__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n,
+                               uint32_t lo, uint32_t hi) {
+    uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;   // the keys, then every key's place, then its difference
+    uint32_t *moved = reinterpret_cast<uint32_t *>(a.dj) + (int64_t)c * a.P + rank0;
     const float npos = (float)a.numbers[2 * a.C + c];
+    const BkGroups of(s);
+    const uint32_t groups = bk_wide_groups(s, of, kin, n, lo, hi);
+    uint32_t *next = of.next, *start = of.start;
+    for (uint32_t g = threadIdx.x; g < groups; g += kBkThreads) next[g] = of.first[g];
+    uint32_t key[kBkItems], rank[kBkItems];
+    for (uint32_t i0 = 0; i0 < n; i0 += kBkCap) {           // to their groups
+        const int here = (int)min((uint32_t)kBkCap, n - i0), rounds = (here + kBkThreads - 1) / kBkThreads;
+        uint32_t group[kBkItems], valid = 0;
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            const int li = bk_item(rounds, r);
+            key[r] = group[r] = 0;
+            if (r < rounds && li < here) {
+                key[r] = kin[i0 + li];
+                group[r] = bk_interval(of.least, groups, key[r] & 0x7FFFFFFFu);
+                valid |= 1u << r;
+            }
+        }
+        bk_ranks_crowded(s, group, valid, rounds, 0u, groups - 1u, rank);
+        uint32_t *order = s.key();                          // groups in the tile's order
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r)
+            if ((valid >> r) & 1u) order[rank[r] & 0xFFFFu] = group[r];
+        __syncthreads();
+        for (int p = threadIdx.x; p < here; p += kBkThreads)
+            if (p == 0 || order[p - 1] != order[p]) start[order[p]] = (uint32_t)p;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            if (!((valid >> r) & 1u)) continue;
+            const uint32_t place = next[group[r]] + (rank[r] & 0xFFFFu) - start[group[r]];
+            moved[place] = key[r];
+            kin[i0 + bk_item(rounds, r)] = place;
+        }
+        __syncthreads();
+        for (int p = threadIdx.x; p < here; p += kBkThreads)
+            if (p == here - 1 || order[p + 1] != order[p]) next[order[p]] += (uint32_t)p + 1u - start[order[p]];
+        __syncthreads();
+    }
     double part = 0.0;
-    uint32_t key[kBkItems], rank[kBkItems], valid = 0, least, most;
-    uint32_t lo = 0xFFFFFFFFu, hi = 0;
-            for (int i = threadIdx.x; i < n; i += kBkThreads) {
-                const uint32_t k = kin[i] & 0x7FFFFFFFu;
-                lo = min(lo, k);
-                hi = max(hi, k);
+    for (uint32_t g = 0; g < groups; ++g) {
+        const uint32_t from = of.first[g], end = of.first[g + 1u];
+        // more than fit: one value, in order as it stands, a block's fill at a time
+        const bool single = end - from > (uint32_t)kBkCap;
+        for (uint32_t i0 = from; i0 < end; i0 += kBkCap) {
+            const int here = (int)min((uint32_t)kBkCap, end - i0), rounds = (here + kBkThreads - 1) / kBkThreads;
+            uint32_t valid = 0, hot = 0, least, most;
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r) {
+                const int li = bk_item(rounds, r);
+                key[r] = 0;
+                if (r < rounds && li < here) {
+                    key[r] = moved[i0 + li];
+                    valid |= 1u << r;
+                    hot += key[r] >> 31;
+                }
             }
-            key[0] = lo;
-            bk_range(s, key, 1u, least, most);
-            uint32_t unused;
-            key[0] = hi;
-            bk_range(s, key, 1u, unused, most);
-            uint32_t from = least, done = 0;
-            int shift = 32 - (int)__builtin_clz((most - from) | 1u);
-            shift = shift > 12 ? shift - 12 : 0;
-            while (done < (uint32_t)n) {                        // a turn takes keys or narrows the bins (shift falls)
-                __syncthreads();
-                for (int i = threadIdx.x; i < kBkBins; i += kBkThreads) s.bin[i] = 0;
-                __syncthreads();
-                for (int i = threadIdx.x; i < n; i += kBkThreads) {
-                    const uint32_t k = kin[i] & 0x7FFFFFFFu;
-                    if (k >= from && ((k - from) >> shift) < (uint32_t)kBkBins) atomicAdd(&s.bin[(k - from) >> shift], 1u);
-                }
-                __syncthreads();
-                constexpr int kPer = kBkBins / kBkThreads;
-                uint32_t sum = 0, total;
-                for (int i = 0; i < kPer; ++i) sum += s.bin[threadIdx.x * kPer + i];
-                uint32_t run = block_excl_scan(sum, s.scan, total);
-                uint32_t bins = 0, keys = 0;                    // leading bins that fit together, and their keys
-                for (int i = 0; i < kPer; ++i) {
-                    run += s.bin[threadIdx.x * kPer + i];
-                    if (run <= (uint32_t)kBkCap) {
-                        ++bins;
-                        keys = run;
-                    }
-                }
-                uint32_t take, take_keys, d0, d1;
-                block_excl_scan2(bins, 0u, s.scan, d0, take, d1, unused);
-                {
-                    uint32_t m = keys;
-    #pragma unroll
-                    for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-                    if ((threadIdx.x & 63) == 0) s.crowd[threadIdx.x >> 6] = m;
-                    __syncthreads();
-                    take_keys = 0;
-                    for (int w = 0; w < kBkWaves; ++w) take_keys = max(take_keys, s.crowd[w]);
-                    __syncthreads();
-                }
-                if (take_keys == 0 && take < (uint32_t)kBkBins && shift > 0) {       // the first bin with keys is too full
-                    from += take << shift;
-                    shift = shift > 12 ? shift - 12 : 0;
-                    continue;
-                }
-                const bool single = take_keys == 0;             // ... and holds a single value
-                // 64 bits: the last range may end past 2^32
-                const uint64_t first = (uint64_t)from + (single ? take : 0u);
-                const uint64_t end = single ? first + 1u : first + ((uint64_t)take << shift);
-                const int turns = (n + kBkCap - 1) / kBkCap;
-                uint32_t seen = 0, seen_hot = 0;
-                uint32_t place[kBkItems];
-                // keys of the range in their order: into LDS, or (single) ranked as they come; then their places the same way
-                for (int what = 0; what < (single ? 1 : 2); ++what) {
-                    seen = 0;
-                    for (int t = 0; t < turns; ++t) {
-                        uint32_t k[kBkItems], mine = 0, hot = 0;
-    #pragma unroll
-                        for (int r = 0; r < kBkItems; ++r) {    // a thread's keys are neighbours here
-                            const int i = t * kBkCap + (int)threadIdx.x * kBkItems + r;
-                            k[r] = i < n ? kin[i] : kIgnoredKey;
-                            const uint32_t bits = k[r] & 0x7FFFFFFFu;
-                            if (i < n && bits >= first && bits < end) {
-                                ++mine;
-                                hot += k[r] >> 31;
-                            }
-                        }
-                        uint32_t at, all, at_hot, all_hot;
-                        block_excl_scan2(mine, hot, s.scan, at, all, at_hot, all_hot);
-                        at += seen;
-                        at_hot += seen_hot;
-    #pragma unroll
-                        for (int r = 0; r < kBkItems; ++r) {
-                            const int i = t * kBkCap + (int)threadIdx.x * kBkItems + r;
-                            const uint32_t bits = k[r] & 0x7FFFFFFFu;
-                            if (i < n && bits >= first && bits < end) {
-                                if (single) {
-                                    const float dj = jaccard_step(npos, rank0 + at, hot0 + at_hot, k[r] >> 31);
-                                    part = add_loss(part, key_error(k[r]), dj);
-                                    out[i] = dj;
-                                } else {
-                                    s.key()[at] = what == 0 ? k[r] : (uint32_t)i;
-                                }
-                                ++at;
-                                at_hot += k[r] >> 31;
-                            }
-                        }
-                        seen += all;
-                        seen_hot += what == 0 ? all_hot : 0u;
-                    }
-                    if (single) break;
-                    __syncthreads();
-                    const int rounds = (int)(take_keys + kBkThreads - 1) / kBkThreads;
-                    valid = 0;
-    #pragma unroll
-                    for (int r = 0; r < kBkItems; ++r) {
-                        const int li = bk_item(rounds, r);
-                        if (r < rounds && li < (int)take_keys) {
-                            if (what == 0) key[r] = s.key()[li];
-                            else place[r] = s.key()[li];
-                            valid |= 1u << r;
-                        }
-                    }
-                    __syncthreads();
-                    if (what == 1) {
-                        bk_range(s, key, valid, least, unused);
-                        uint32_t largest;
-                        bk_range(s, key, valid, unused, largest);
-                        bk_ranks_crowded(s, key, valid, rounds, least, largest, rank);
-    #pragma unroll
-                        for (int r = 0; r < kBkItems; ++r) {
-                            if ((valid >> r) & 1u) {
-                                const float dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), key[r] >> 31);
-                                part = add_loss(part, key_error(key[r]), dj);
-                                out[place[r]] = dj;
-                            }
-                        }
-                    }
-                }
-                done += seen;
-                rank0 += seen;
-                hot0 += seen_hot;
-                if (done >= (uint32_t)n || seen == 0) break;        // every turn takes keys
-                from = (uint32_t)end;                           // keys are left, so it is below 2^31
-                shift = 32 - (int)__builtin_clz((most - from) | 1u);
-                shift = shift > 12 ? shift - 12 : 0;
+            uint32_t hots;
+            block_excl_scan(hot, s.scan, hots);
+            bk_range(s, key, valid, least, most);
+            if (single) most = least;
+            bk_ranks_crowded(s, key, valid, rounds, least, most, rank);
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r) {
+                if (!((valid >> r) & 1u)) continue;
+                const float dj = jaccard_step(npos, rank0 + i0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), key[r] >> 31);
+                part = add_loss(part, key_error(key[r]), dj);
+                moved[i0 + bk_item(rounds, r)] = __builtin_bit_cast(uint32_t, dj);
             }
+            hot0 += hots;
+        }
+    }
+    __syncthreads();
+    for (int copy = 0; copy < 2; ++copy) {                  // the reads of a tile before its writes, not one after the other
+        const uint32_t *at = copy ? kin : moved;
+        uint32_t *to = copy ? moved : kin;
+        for (uint32_t i0 = 0; i0 < n; i0 += kBkCap) {
+            if (!copy) {
+#pragma unroll
+                for (int r = 0; r < kBkItems; ++r) {
+                    const uint32_t i = i0 + (uint32_t)bk_item(kBkItems, r);
+                    rank[r] = i < n ? kin[i] : 0u;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r) {
+                const uint32_t i = i0 + (uint32_t)bk_item(kBkItems, r);
+                key[r] = i < n ? at[copy ? i : rank[r]] : 0u;
+            }
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r) {
+                const uint32_t i = i0 + (uint32_t)bk_item(kBkItems, r);
+                if (i < n) to[i] = key[r];
+            }
+        }
+        __syncthreads();
+    }
     return part;
 }
 
@@ -1142,7 +1240,7 @@ __device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
 // order as they stand. The positives before the part are counted again by every block where the flags are mixed (a value
 // that many share is mostly the positives' or the others' alone). Done by bk_scatter, 16 places per thread, this took that
 // kernel from 94 to 149 us where all logits are equal ((8,19,512,512)); step 459 -> 418 us, radix passes 425.
-__device__ void bk_flat_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n, uint32_t hot) {
+__device__ __forceinline__ void bk_flat_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n, uint32_t hot) {
     constexpr uint32_t kPer = 8, kStep = kPer * kBkThreads;
     const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
     float *out = a.dj + (int64_t)c * a.P + rank0;
@@ -1214,7 +1312,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
     const int n_todo = found;
     for (int i = 0; i < n_todo; ++i) {
         const int b = todo[i];
-        double part = bk_wide_keys(s, a, c, a.base[cells + b], a.hot_base[cells + b], (int)a.count[row + b]);
+        const uint32_t lo = b ? a.bounds[row + b - 1] : 0u, hi = b + 1 < buckets ? a.bounds[row + b] : bk_limit(a, c) + 1u;
+        double part = bk_wide_keys(s, a, c, a.base[cells + b], a.hot_base[cells + b], a.count[row + b], lo, hi);
         part = wave_sum_f64(part);
         __syncthreads();
         if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;

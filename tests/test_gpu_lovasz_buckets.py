@@ -118,7 +118,7 @@ def sampled(pixels):
 
 
 @pytest.mark.parametrize("pixels", [70000, 500000])
-@pytest.mark.parametrize("kind", ["spread", "one value", "both"])
+@pytest.mark.parametrize("kind", ["spread", "one value", "both", "nested"])
 @pytest.mark.parametrize("n_cls", [2, 32])
 def test_buckets_that_the_sample_misses(native, pixels, kind, n_cls):
     assert n_cls == 2 or by_buckets(n_cls, pixels)
@@ -126,6 +126,9 @@ def test_buckets_that_the_sample_misses(native, pixels, kind, n_cls):
     d = rng.random(pixels) * (0.0 if kind == "one value" else 1e-2)
     if kind == "both":
         d[rng.random(pixels) < 0.5] = 5e-3
+    if kind == "nested":                # a cluster in a cluster, and values that more keys share than a block holds
+        d = 10.0 ** -rng.integers(0, 6, pixels) * rng.random(pixels)
+        d[rng.random(pixels) < 0.3] = 0.25
     at = sampled(pixels).astype(np.int64)
     d[at] = 1 + rng.random(at.size)
     # the classes beyond the first two are absent, and hardly predicted
