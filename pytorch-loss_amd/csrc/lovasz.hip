@@ -15,7 +15,7 @@
 //                     pattern is monotone), ignored pixel = 0x7FFFFFFF (sorts last). Also the
 //                     largest positive key per class (per-block table + lov_class_max): keys
 //                     beyond it have dJ = 0 exactly and are left out of the sort (keep_key).
-//   2.-4. for rows of up to kBkMaxRow pixels: by value buckets, see lovasz_buckets.hpp. Otherwise, and in the look-back
+//   2.-4. for the rows that bk_pays names: by value buckets, see lovasz_buckets.hpp. Otherwise, and in the look-back
 //                     variant, with the same differences bit for bit:
 //   2. 3 x (tile_hist, row_scan, scatter): stable LSD radix passes, 8 bits each, batched over
 //                     classes with blockIdx.y. Ranking inside a tile is done per wavefront with

@@ -13,12 +13,13 @@
 //   bk_rank_wide  the same for buckets that outgrew the LDS, and for single values that fill more than that
 //   bk_gather     Jaccard differences back to pixel order, tile by tile
 // Sampled bounds follow any distribution; a value that fills several buckets by itself gets one of its own, which
-// needs no sort (flat: its keys are ranked as they stand), and a bucket that outgrew the LDS all the same is taken in value ranges
-// that fit.
-// Bound by vector instructions (scatter and rank: some 80 and 110 per 64 keys at 16 waves per CU) and short runs, not by
-// the 40 bytes a key moves. Forward and backward, against the radix passes: (8,21,513,513) bf16 trained 1.21 -> 0.82 ms,
-// (4,19,512,1024) fp32 0.72 -> 0.56, (1,150,256,256) 0.51 -> 0.37; near-uniform predictions, whose keys need two
-// radix passes only, take the same time as before ((4,19,512,1024) 0.42 both ways).
+// needs no sort (flat: its keys are ranked as they stand), and a bucket that outgrew the LDS all the same is cut into value
+// groups that fit.
+// Bound by vector instructions (nearly all keys taking part: scatter 95 and rank 121 per 64 keys, at 24 and 16 waves per CU,
+// 106 of 154 and 136 of 225 us of issue) and short runs, not by the 40 bytes a key moves. Forward and backward, against
+// the radix passes: (8,21,513,513) bf16 trained 1.21 -> 0.79 ms, (4,19,512,1024) fp32 0.72 -> 0.56, (1,150,256,256)
+// 0.51 -> 0.37; a new network's near-uniform predictions and all-equal ones, whose keys need few radix passes, take the same time
+// as before ((4,19,512,1024) 0.42 both ways). Which rows come here: bk_pays.
 #pragma once
 
 namespace plh {
@@ -699,7 +700,7 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) 
     }
     for (int i = threadIdx.x; i < kBkWaves * kStride / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(s_counts)[i] = 0;
     __syncthreads();
-    // Four rounds at a time: their masks first, then a read of the counter and the leader's addition to it per round. LDS
+    // Two rounds at a time (four spill): their masks first, then a read of the counter and the leader's addition to it per round. LDS
     // takes a wave's operations in their order, so no addition waits for what a read returns.
     constexpr int kGroup = 2;
 #pragma unroll
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) 
 
 // One run of buckets (or, Direct: a whole row of at most kBkCap pixels, straight from the keys in pixel order, with the
 // Jaccard differences left in their place and the loss complete).
-// Time goes into vector instructions, about 110 per 64 keys: a thread's places of the order are neighbours, so that a
+// Time goes into vector instructions, 121 per 64 keys: a thread's places of the order are neighbours, so that a
 // difference is one new quotient less the one before, and the positives before a place are a sum over the block's threads.
 template <bool Direct>
 __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, float *__restrict__ losses) {
