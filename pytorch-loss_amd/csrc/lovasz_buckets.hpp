@@ -14,7 +14,7 @@
 //   bk_gather     Jaccard differences back to pixel order, tile by tile
 // Sampled bounds follow any distribution; a value that fills several buckets by itself gets one of its own, which
 // needs no sort (flat: its keys are ranked as they stand), and a bucket that outgrew the LDS all the same is cut into value
-// groups that fit.
+// ranges that fit.
 // Bound by vector instructions (nearly all keys taking part: scatter 95 and rank 121 per 64 keys, at 24 and 16 waves per CU,
 // 106 of 154 and 136 of 225 us of issue) and short runs, not by the 40 bytes a key moves. Forward and backward, against
 // the radix passes: (8,21,513,513) bf16 trained 1.21 -> 0.79 ms, (4,19,512,1024) fp32 0.72 -> 0.56, (1,150,256,256)
@@ -984,7 +984,153 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
     }
 }
 
-// What bk_wide_keys keeps in the block's memory: first, where the pairs are, the bounds of up to kBkIntervals value intervals
+// n keys, a few times kBkCap at most, from rank `rank0` on, with hot0 positives before them: ranges of values [from, end)
+// with at most kBkCap keys, one after the other, collected in order by sweeps over all n; a single value that more keys share
+// is ranked by position.
+__device__ __forceinline__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, int n) {
+    const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
+    float *out = a.dj + (int64_t)c * a.P + rank0;
+    const float npos = (float)a.numbers[2 * a.C + c];
+    double part = 0.0;
+    uint32_t key[kBkItems], rank[kBkItems], valid = 0, least, most;
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+    for (int i = threadIdx.x; i < n; i += kBkThreads) {
+        const uint32_t k = kin[i] & 0x7FFFFFFFu;
+        lo = min(lo, k);
+        hi = max(hi, k);
+    }
+    key[0] = lo;
+    bk_range(s, key, 1u, least, most);
+    uint32_t unused;
+    key[0] = hi;
+    bk_range(s, key, 1u, unused, most);
+    uint32_t from = least, done = 0;
+    int shift = 32 - (int)__builtin_clz((most - from) | 1u);
+    shift = shift > 12 ? shift - 12 : 0;
+    while (done < (uint32_t)n) {                        // a turn takes keys or narrows the bins (shift falls)
+        __syncthreads();
+        for (int i = threadIdx.x; i < kBkBins; i += kBkThreads) s.bin[i] = 0;
+        __syncthreads();
+        for (int i = threadIdx.x; i < n; i += kBkThreads) {
+            const uint32_t k = kin[i] & 0x7FFFFFFFu;
+            if (k >= from && ((k - from) >> shift) < (uint32_t)kBkBins) atomicAdd(&s.bin[(k - from) >> shift], 1u);
+        }
+        __syncthreads();
+        constexpr int kPer = kBkBins / kBkThreads;
+        uint32_t sum = 0, total;
+        for (int i = 0; i < kPer; ++i) sum += s.bin[threadIdx.x * kPer + i];
+        uint32_t run = block_excl_scan(sum, s.scan, total);
+        uint32_t bins = 0, keys = 0;                    // leading bins that fit together, and their keys
+        for (int i = 0; i < kPer; ++i) {
+            run += s.bin[threadIdx.x * kPer + i];
+            if (run <= (uint32_t)kBkCap) {
+                ++bins;
+                keys = run;
+            }
+        }
+        uint32_t take, take_keys, d0, d1;
+        block_excl_scan2(bins, 0u, s.scan, d0, take, d1, unused);
+        {
+            uint32_t m = keys;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+            if ((threadIdx.x & 63) == 0) s.crowd[threadIdx.x >> 6] = m;
+            __syncthreads();
+            take_keys = 0;
+            for (int w = 0; w < kBkWaves; ++w) take_keys = max(take_keys, s.crowd[w]);
+            __syncthreads();
+        }
+        if (take_keys == 0 && take < (uint32_t)kBkBins && shift > 0) {       // the first bin with keys is too full
+            from += take << shift;
+            shift = shift > 12 ? shift - 12 : 0;
+            continue;
+        }
+        const bool single = take_keys == 0;             // ... and holds a single value
+        // 64 bits: the last range may end past 2^32
+        const uint64_t first = (uint64_t)from + (single ? take : 0u);
+        const uint64_t end = single ? first + 1u : first + ((uint64_t)take << shift);
+        const int turns = (n + kBkCap - 1) / kBkCap;
+        uint32_t seen = 0, seen_hot = 0;
+        uint32_t place[kBkItems];
+        // keys of the range in their order: into LDS, or (single) ranked as they come; then their places the same way
+        for (int what = 0; what < (single ? 1 : 2); ++what) {
+            seen = 0;
+            for (int t = 0; t < turns; ++t) {
+                uint32_t k[kBkItems], mine = 0, hot = 0;
+#pragma unroll
+                for (int r = 0; r < kBkItems; ++r) {    // a thread's keys are neighbours here
+                    const int i = t * kBkCap + (int)threadIdx.x * kBkItems + r;
+                    k[r] = i < n ? kin[i] : kIgnoredKey;
+                    const uint32_t bits = k[r] & 0x7FFFFFFFu;
+                    if (i < n && bits >= first && bits < end) {
+                        ++mine;
+                        hot += k[r] >> 31;
+                    }
+                }
+                uint32_t at, all, at_hot, all_hot;
+                block_excl_scan2(mine, hot, s.scan, at, all, at_hot, all_hot);
+                at += seen;
+                at_hot += seen_hot;
+#pragma unroll
+                for (int r = 0; r < kBkItems; ++r) {
+                    const int i = t * kBkCap + (int)threadIdx.x * kBkItems + r;
+                    const uint32_t bits = k[r] & 0x7FFFFFFFu;
+                    if (i < n && bits >= first && bits < end) {
+                        if (single) {
+                            const float dj = jaccard_step(npos, rank0 + at, hot0 + at_hot, k[r] >> 31);
+                            part = add_loss(part, key_error(k[r]), dj);
+                            out[i] = dj;
+                        } else {
+                            s.key()[at] = what == 0 ? k[r] : (uint32_t)i;
+                        }
+                        ++at;
+                        at_hot += k[r] >> 31;
+                    }
+                }
+                seen += all;
+                seen_hot += what == 0 ? all_hot : 0u;
+            }
+            if (single) break;
+            __syncthreads();
+            const int rounds = (int)(take_keys + kBkThreads - 1) / kBkThreads;
+            valid = 0;
+#pragma unroll
+            for (int r = 0; r < kBkItems; ++r) {
+                const int li = bk_item(rounds, r);
+                if (r < rounds && li < (int)take_keys) {
+                    if (what == 0) key[r] = s.key()[li];
+                    else place[r] = s.key()[li];
+                    valid |= 1u << r;
+                }
+            }
+            __syncthreads();
+            if (what == 1) {
+                bk_range(s, key, valid, least, unused);
+                uint32_t largest;
+                bk_range(s, key, valid, unused, largest);
+                bk_ranks_crowded(s, key, valid, rounds, least, largest, rank);
+#pragma unroll
+                for (int r = 0; r < kBkItems; ++r) {
+                    if ((valid >> r) & 1u) {
+                        const float dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), key[r] >> 31);
+                        part = add_loss(part, key_error(key[r]), dj);
+                        out[place[r]] = dj;
+                    }
+                }
+            }
+        }
+        done += seen;
+        rank0 += seen;
+        hot0 += seen_hot;
+        if (done >= (uint32_t)n || seen == 0) break;        // every turn takes keys
+        from = (uint32_t)end;                           // keys are left, so it is below 2^31
+        shift = 32 - (int)__builtin_clz((most - from) | 1u);
+        shift = shift > 12 ? shift - 12 : 0;
+    }
+    return part;
+}
+
+// What bk_huge_keys keeps in the block's memory: first, where the pairs are, the bounds of up to kBkIntervals value intervals
 // and their keys; then, per group, in what the crowded path leaves free behind its 256 words of counters and behind its keys
 // and items.
 constexpr int kBkIntervals = 4096, kBkGroups = 1100;
@@ -999,7 +1145,7 @@ struct BkGroups {
         : least(s.bin + kBkWaves * 64 / 2), first(least + kBkGroups), next(reinterpret_cast<uint32_t *>(s.src() + kBkCap)),
           start(next + kBkGroups) {}
 };
-static_assert(kBkIntervals % kBkThreads == 0 && 3 * (kBkMaxRow / kBkCap + 2) < kBkGroups, "groups, see bk_wide_groups");
+static_assert(kBkIntervals % kBkThreads == 0 && 3 * (kBkMaxRow / kBkCap + 2) < kBkGroups, "groups, see bk_huge_groups");
 static_assert(sizeof(BkIntervals) <= sizeof(BkPair) * (kBkCap + kBkChunk) && kBkWaves * 32 + 2 * kBkGroups + 1 <= kBkBins &&
               6 * kBkCap + 8 * kBkGroups <= (int)sizeof(BkPair) * (kBkCap + kBkChunk), "they fit");
 
@@ -1022,7 +1168,7 @@ __device__ __forceinline__ void bk_intervals(const uint32_t *bound, uint32_t m, 
 // split, by a third at least, until none is left, and neighbours that come to no more than kBkCap are one again (those in one
 // of the n / kBkCap slabs of the order; those that lie across two stand alone). Every turn reads the keys once; the
 // values are 30 bits wide, so there are 19 at most, and 1 to 6 for what was tried. Returns the number of groups.
-__device__ __forceinline__ uint32_t bk_wide_groups(BkShared &s, const BkGroups &out, const uint32_t *kin, uint32_t n, uint32_t lo, uint32_t hi) {
+__device__ __forceinline__ uint32_t bk_huge_groups(BkShared &s, const BkGroups &out, const uint32_t *kin, uint32_t n, uint32_t lo, uint32_t hi) {
     constexpr uint32_t kPer = kBkIntervals / kBkThreads, kCap = kBkCap;
     BkIntervals &w = *reinterpret_cast<BkIntervals *>(s.pair);
     uint32_t m = 1, cur = 0;
@@ -1127,17 +1273,17 @@ __device__ __forceinline__ uint32_t bk_wide_groups(BkShared &s, const BkGroups &
 }
 
 // A bucket of n keys of the values lo..hi - 1, from rank `rank0` on, with hot0 positives before them, many times what a block
-// holds: its keys are moved to their groups (bk_wide_groups), in order inside each, a group at a time is ranked in LDS,
+// holds: its keys are moved to their groups (bk_huge_groups), in order inside each, a group at a time is ranked in LDS,
 // and the differences come back through the places left where the keys were. Every key is read and moved a bounded number
 // of times: bounds that the sample misses by far ((1,32,1,500000), all keys in one bucket) cost 6.5 ms, where a sweep over
 // the bucket per 7680 keys cost 56 (radix passes 0.23); twice the keys 14 and 262.
-__device__ __forceinline__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n,
+__device__ __forceinline__ double bk_huge_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n,
                                uint32_t lo, uint32_t hi) {
     uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;   // the keys, then every key's place, then its difference
     uint32_t *moved = reinterpret_cast<uint32_t *>(a.dj) + (int64_t)c * a.P + rank0;
     const float npos = (float)a.numbers[2 * a.C + c];
     const BkGroups of(s);
-    const uint32_t groups = bk_wide_groups(s, of, kin, n, lo, hi);
+    const uint32_t groups = bk_huge_groups(s, of, kin, n, lo, hi);
     uint32_t *next = of.next, *start = of.start;
     for (uint32_t g = threadIdx.x; g < groups; g += kBkThreads) next[g] = of.first[g];
     uint32_t key[kBkItems], rank[kBkItems];
@@ -1323,7 +1469,9 @@ __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
     for (int i = 0; i < n_todo; ++i) {
         const int b = todo[i];
         const uint32_t lo = b ? a.bounds[row + b - 1] : 0u, hi = b + 1 < buckets ? a.bounds[row + b] : bk_limit(a, c) + 1u;
-        double part = bk_wide_keys(s, a, c, a.base[cells + b], a.hot_base[cells + b], a.count[row + b], lo, hi);
+        const uint32_t n = a.count[row + b], rank0 = a.base[cells + b], hot0 = a.hot_base[cells + b];
+        // Sampled bounds leave a bucket of 7700 to 9000 keys in every other step or so: by ranges 30 us, by groups 45.
+        double part = n <= 4u * kBkCap ? bk_wide_keys(s, a, c, rank0, hot0, (int)n) : bk_huge_keys(s, a, c, rank0, hot0, n, lo, hi);
         part = wave_sum_f64(part);
         __syncthreads();
         if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
