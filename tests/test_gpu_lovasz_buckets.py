@@ -117,7 +117,8 @@ def sampled(pixels):
     return i * pixels // 7680 + ((h * (pixels // 7680)) >> 32)
 
 
-@pytest.mark.parametrize("pixels", [70000, 500000])
+# most keys in one bucket: up to four times what a block holds, and more
+@pytest.mark.parametrize("pixels", [20000, 70000, 500000])
 @pytest.mark.parametrize("kind", ["spread", "one value", "both", "nested"])
 @pytest.mark.parametrize("n_cls", [2, 32])
 def test_buckets_that_the_sample_misses(native, pixels, kind, n_cls):
