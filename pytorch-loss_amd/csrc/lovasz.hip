@@ -1156,8 +1156,8 @@ struct LovaszPlan {
     // ranks whole)
     bool buckets;
     int bk_tiles, bk_bits;
-    int64_t off_sorted, off_dj, off_tile_count, off_count, off_bounds, off_buckets, off_fine, off_loss_part,
-        off_crowded, off_bucket;
+    int64_t off_sorted, off_dj, off_tile_start, off_start, off_count, off_bounds, off_buckets, off_fine, off_loss_part,
+        off_crowded, off_place;
     int hist_blocks;
     int64_t off_lb_clear, lb_clear_bytes, off_lb_totals, off_lb_partial;
 };
@@ -1207,12 +1207,13 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
         // one layout for every row length, also where one block ranks the row
         pl.off_sorted = off;     off += round_up(4 * pl.E, 256);
         pl.off_dj = off;         off += round_up(4 * pl.E, 256);
-        pl.off_bucket = off;     off += round_up(2 * pl.E, 256);
-        pl.off_tile_count = off; off += round_up(4 * cells * pl.bk_tiles, 256);
-        pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // count, hot, base, hot_base, runs
+        pl.off_place = off;      off += round_up(2 * pl.E, 256);
+        pl.off_tile_start = off; off += round_up(4 * (cells + dimsize) * pl.bk_tiles, 256);
+        pl.off_start = off;      off += round_up(4 * (cells + dimsize) * pl.bk_tiles, 256);
+        pl.off_count = off;      off += 4 * round_up(4 * (cells + dimsize), 256);     // count, base, hot_base, runs
         pl.off_bounds = off;     off += round_up(4 * cells, 256);
-        pl.off_buckets = off;    off += round_up(4 * 5 * dimsize, 256);
-        pl.off_fine = off;       off += round_up(2 * dimsize * (kBkFine + 2), 256);
+        pl.off_buckets = off;    off += round_up(4 * 6 * dimsize, 256);
+        pl.off_fine = off;       off += round_up(2 * dimsize * kBkFine, 256);
         pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
         pl.bytes = off;
         return PLH_OK;
@@ -1281,14 +1282,14 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
     a.stride = 1 << pl.bk_bits;
     const int64_t step = round_up(4 * (((int64_t)C << pl.bk_bits) + C), 256);
     a.sorted = reinterpret_cast<uint32_t *>(ws + pl.off_sorted);
-    a.dj = reinterpret_cast<float *>(ws + pl.off_dj);
-    a.bucket = reinterpret_cast<uint16_t *>(ws + pl.off_bucket);
-    a.tile_count = reinterpret_cast<uint32_t *>(ws + pl.off_tile_count);
+    a.dj = reinterpret_cast<uint32_t *>(ws + pl.off_dj);
+    a.place = reinterpret_cast<uint16_t *>(ws + pl.off_place);
+    a.tile_start = reinterpret_cast<uint32_t *>(ws + pl.off_tile_start);
+    a.start = reinterpret_cast<uint32_t *>(ws + pl.off_start);
     a.count = reinterpret_cast<uint32_t *>(ws + pl.off_count);
-    a.hot = reinterpret_cast<uint32_t *>(ws + pl.off_count + step);
-    a.base = reinterpret_cast<uint32_t *>(ws + pl.off_count + 2 * step);
-    a.hot_base = reinterpret_cast<uint32_t *>(ws + pl.off_count + 3 * step);
-    a.runs = reinterpret_cast<uint32_t *>(ws + pl.off_count + 4 * step);
+    a.base = reinterpret_cast<uint32_t *>(ws + pl.off_count + step);
+    a.hot_base = reinterpret_cast<uint32_t *>(ws + pl.off_count + 2 * step);
+    a.runs = reinterpret_cast<uint32_t *>(ws + pl.off_count + 3 * step);
     a.bounds = reinterpret_cast<uint32_t *>(ws + pl.off_bounds);
     a.numbers = reinterpret_cast<uint32_t *>(ws + pl.off_buckets);
     a.fine = reinterpret_cast<uint16_t *>(ws + pl.off_fine);
@@ -1301,14 +1302,13 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
     switch (pl.bk_bits) {
 #define PLH_BUCKETS(B)                                                                                               \
     case B:                                                                                                          \
-        hipLaunchKernelGGL(bk_hist<1 << B>, tiles, threads, 0, st, a);                                               \
-        hipLaunchKernelGGL(bk_scan, dim3((unsigned)ceil_div(most, 64), (unsigned)C), dim3(1024), 0, st, a);          \
+        hipLaunchKernelGGL(bk_cut<B>, tiles, threads, 0, st, a);                                                     \
+        hipLaunchKernelGGL(bk_sum, dim3((unsigned)ceil_div(most + 1, 64), (unsigned)C), dim3(1024), 0, st, a);       \
         hipLaunchKernelGGL(bk_group, dim3((unsigned)C), threads, 0, st, a);                                          \
-        hipLaunchKernelGGL(bk_scatter<B>, tiles, threads, 0, st, a);                                                 \
         hipLaunchKernelGGL(bk_rank<false>, dim3(most, (unsigned)C), threads, 0, st, a, losses);                      \
         hipLaunchKernelGGL(bk_rank_crowded<false>, dim3(crowded_blocks, (unsigned)C), threads, 0, st, a, losses);    \
         hipLaunchKernelGGL(bk_rank_wide, dim3(kBkWideBlocks, (unsigned)C), threads, 0, st, a);                       \
-        hipLaunchKernelGGL(bk_gather<B>, tiles, threads, 0, st, a, losses);                                          \
+        hipLaunchKernelGGL(bk_restore, tiles, threads, 0, st, a, losses);                                            \
         break;
         PLH_BUCKETS(6) PLH_BUCKETS(8) PLH_BUCKETS(10)
 #undef PLH_BUCKETS

@@ -1,25 +1,24 @@
 // The sort of the Lovasz forward by value buckets (included by lovasz.hip, after the keys and the rank primitives).
 //
-// A radix sort moves every (key, pixel) pair three times before its rank is known. Here a key moves once: the class row
-// is cut into buckets of neighbouring key values, and what fits a block's LDS is sorted there.
+// A radix sort moves every (key, pixel) pair three times before its rank is known. Here a key moves inside its tile only: the
+// class row is cut into buckets of neighbouring key values, every tile is put in the order of the buckets, and what lies in a
+// few neighbouring buckets, a segment of every tile, is sorted in a block's LDS.
 //   bk_split      a block per class sorts a sample of the row's keys; every n-th of them starts a bucket
-//   bk_hist       keys (and positives) per tile and bucket
-//   bk_scan       the tiles' counts to exclusive sums per bucket
-//   bk_group      where every bucket starts in the row, and runs of buckets that a block can sort at once
-//   bk_scatter    keys to their buckets, in pixel order inside a bucket (stable ranks from match masks); the tile's order is
-//                 left in the place of its keys
-//   bk_rank       a block per run of buckets: sorted in LDS, Jaccard difference of every key at its place
+//   bk_cut        every tile's keys in the order of their buckets, in pixel order inside one (stable ranks), in the keys' place
+//   bk_sum        the tiles' counts by bucket: where every bucket starts in the row
+//   bk_group      runs of buckets that a block can sort at once
+//   bk_rank       a block per run of buckets: its segments sorted in LDS, Jaccard difference of every key in its place
 //   bk_rank_crowded  the same for runs whose values crowd
 //   bk_rank_wide  the same for buckets that outgrew the LDS, and for single values that fill more than that
-//   bk_gather     Jaccard differences back to pixel order, tile by tile
+//   bk_restore    Jaccard differences back to pixel order, tile by tile
 // Sampled bounds follow any distribution; a value that fills several buckets by itself gets one of its own, which
 // needs no sort (flat: its keys are ranked as they stand), and a bucket that outgrew the LDS all the same is cut into value
 // ranges that fit.
-// Bound by vector instructions (nearly all keys taking part: scatter 95 and rank 121 per 64 keys, at 24 and 16 waves per CU,
-// 106 of 154 and 136 of 225 us of issue) and short runs, not by the 40 bytes a key moves. Forward and backward, against
-// the radix passes: (8,21,513,513) bf16 trained 1.21 -> 0.79 ms, (4,19,512,1024) fp32 0.72 -> 0.56, (1,150,256,256)
-// 0.51 -> 0.37; a new network's near-uniform predictions and all-equal ones, whose keys need few radix passes, take the same time
-// as before ((4,19,512,1024) 0.42 both ways). Which rows come here: bk_pays.
+// A key moves 28 bytes: read and written by bk_cut, bk_rank and bk_restore, and a place of 2 bytes. The form before this one
+// wrote the buckets out one after the other: that takes a histogram first (6 bytes a key more, buckets kept for the second
+// pass) and writes of some 10 keys, where a segment of a run has 24 here. (4,19,512,1024) fp32: histogram and scatter
+// 67 + 117 us against 102 now, rank 119 against 134, gather 72 against 57, step 585 -> 518 us; (8,21,513,513) bf16 trained
+// 77 + 154 against 137, 217 against 270, 116 against 68, step 794 -> 700. Which rows come here: bk_pays.
 #pragma once
 
 namespace plh {
@@ -44,20 +43,21 @@ constexpr uint32_t kBkFlat = 0x80000000u;
 constexpr uint16_t kBkNowhere = 0xFFFFu;            // place of a pixel that takes no part
 
 struct BucketArgs {
-    uint32_t *keys;             // [C][P] in pixel order; bk_scatter leaves the tile's order there (jacc's memory)
+    uint32_t *keys;             // [C][P] in pixel order; bk_cut leaves every tile's keys by bucket, the rank kernels a key's Jaccard
+                                // difference in its place, bk_restore those in pixel order (jacc's memory)
     const uint32_t *pos_max;    // pos_max[C], kept[C], all_min[C], key_bits[C] (see keep_key, lov_class_max)
-    uint32_t *sorted;           // [C][P] keys by bucket
-    float *dj;                  // [C][P] Jaccard differences by bucket
-    uint16_t *bucket;           // [C][P] bucket of every pixel
-    uint32_t *tile_count;       // [C][tiles][stride]: keys | positives << 16, exclusive sums over the tiles, start of the
-                                // tile's keys of the bucket in the row less their start in the tile
-    uint32_t *count, *hot;      // [C][stride] keys (kBkFlat: and a single value), positives per bucket
-    uint32_t *base, *hot_base;  // [C][stride + 1] the same before the bucket
+    uint16_t *place;            // [C][P] every pixel's place in its tile's order
+    uint32_t *sorted, *dj;      // [C][P] keys and differences of the buckets that bk_rank_wide ranks
+    uint32_t *tile_start;       // [C][tiles][stride + 1] in the tile's order: keys | positives << 16 before the bucket
+    uint32_t *start;            // [C][stride + 1][tiles] the same
+    uint32_t *count;            // [C][stride] keys per bucket (kBkFlat: and a single value)
+    uint32_t *base, *hot_base;  // [C][stride + 1] keys and positives before the bucket
     uint32_t *bounds;           // [C][stride] least key of buckets 1, 2, ...
     uint32_t *runs;             // [C][stride + 1] first bucket of every run, and the end
     uint32_t *crowded;          // [C][stride] runs (rows of one block: [C]) whose values crowd
-    uint32_t *numbers;          // [5][C]: buckets, runs, positives, least key of the sample, largest one below the limit
-    uint16_t *fine;             // [C][kBkFine + 2]
+    uint32_t *numbers;          // [6][C]: buckets, runs, positives, least key of the sample, largest one below the limit,
+                                // first step of the search in `bounds`
+    uint16_t *fine;             // [C][kBkFine] bucket of the least key with these top bits
     double *loss_part;          // [C][2 * stride]: runs, wide and flat buckets
     int P, C, tiles, stride;
 };
@@ -128,6 +128,42 @@ __device__ __forceinline__ void bk_merge(BkPair (&v)[kBkChunk]) {
                 if (pair) bk_order(v[i], v[i + k]);
             }
 }
+
+// Where the keys of a few neighbouring buckets stand: in every tile a segment of its order. The segments one after the other are
+// the keys in the order that the sort keeps among equals; places from..from + kBkCap - 1 of it are covered.
+constexpr int kBkWords = kBkCap / kWave;
+struct BkSegments {
+    uint64_t starts[kBkWords];                  // bit i of word k: a segment starts at place 64 k + i + 1
+    uint32_t segment[kBkWords];                 // of place 64 k
+    uint32_t shift[kBkMaxRow / kBkTile + 1];    // where the segment starts in the row less its first place
+    // Every thread of the block calls it; ends with a barrier. The memory is free before, with a barrier in between.
+    __device__ void collect(const BucketArgs &a, int c, uint32_t b0, uint32_t b1, uint32_t from, uint32_t *scan) {
+        uint32_t *words = reinterpret_cast<uint32_t *>(starts);
+        if (threadIdx.x < 2 * kBkWords) words[threadIdx.x] = 0;
+        const int64_t cell = (int64_t)c * (a.stride + 1);
+        const uint32_t t = threadIdx.x;
+        uint32_t at = 0, n = 0;
+        if (t < (uint32_t)a.tiles) {
+            at = a.start[(cell + b0) * a.tiles + t] & 0xFFFFu;
+            n = (a.start[(cell + b1) * a.tiles + t] & 0xFFFFu) - at;
+        }
+        uint32_t place, all, index, segments;
+        block_excl_scan2(n, n ? 1u : 0u, scan, place, all, index, segments);
+        if (n && place + n > from && place < from + kBkCap) {
+            shift[index] = t * kBkTile + at - place;
+            const uint32_t first = place > from ? place - from : 0u, end = min(place + n - from, (uint32_t)kBkCap);
+            if (first & 63u) atomicOr(&words[(first - 1u) >> 5], 1u << ((first - 1u) & 31u));
+            for (uint32_t k = (first + 63u) / 64u; k * 64u < end; ++k) segment[k] = index;
+        }
+        __syncthreads();
+    }
+    // Where the key at place from + p stands in the row; p / 64 is the same for the whole wave.
+    __device__ __forceinline__ uint32_t where(uint32_t p, uint32_t from = 0) const {
+        const uint32_t k = p >> 6;
+        return shift[segment[k] + peers_below(starts[k])] + from + p;
+    }
+};
+static_assert(kBkMaxRow / kBkTile < kBkThreads && 2 * kBkWords <= kBkThreads, "a thread per tile and per word");
 
 struct BkShared {
     // the pairs, 16 neighbours in the order of thread t in row t; the crowded path's keys and items; the results by item
@@ -460,126 +496,290 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
         }
         a.numbers[4 * a.C + c] = lo ? sorted[lo - 1] : 0u;
     }
-    // the bucket of the least key with each pattern of the top bits
+    // the bucket of the least key with each pattern of the top bits, and the most bounds that one pattern's keys can lie between
     const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
-    for (int f = threadIdx.x; f <= kBkFine; f += kBkThreads) {
-        const uint32_t k = (uint32_t)f << shift;
+    constexpr int kPerFine = kBkFine / kBkThreads;
+    uint32_t at_fine[kPerFine + 1], width = 0;
+#pragma unroll
+    for (int u = 0; u <= kPerFine; ++u) {
+        const uint32_t k = (threadIdx.x * kPerFine + u) << shift;
         uint32_t lo = 0, hi = bounds;
         while (lo < hi) {
             const uint32_t mid = (lo + hi) >> 1;
             if (s.bin[mid] <= k) lo = mid + 1;
             else hi = mid;
         }
-        a.fine[(int64_t)c * (kBkFine + 2) + f] = (uint16_t)lo;
+        at_fine[u] = lo;
+    }
+#pragma unroll
+    for (int u = 0; u < kPerFine; ++u) {
+        a.fine[(int64_t)c * kBkFine + threadIdx.x * kPerFine + u] = (uint16_t)at_fine[u];
+        width = max(width, at_fine[u + 1] - at_fine[u]);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) width = max(width, (uint32_t)__shfl_xor((int)width, off, 64));
+    if ((threadIdx.x & 63) == 0) s.crowd[threadIdx.x >> 6] = width;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 0; w < kBkWaves; ++w) width = max(width, s.crowd[w]);
+        a.numbers[5 * a.C + c] = width ? 0x80000000u >> __builtin_clz(width) : 0u;
     }
 }
 
 // The bounds and the table in LDS.
 template <int kStride>
 struct BkLookup {
-    uint32_t bounds[kStride];
-    uint32_t fine2[kBkFine / 2 + 1];
-    __device__ void fetch(const BucketArgs &a, int c, uint32_t buckets) {
+    uint32_t bounds[2 * kStride];
+    uint16_t fine[kBkFine];
+    // first_step: 2^k of which 2^(k+1) - 1 is no less than the bounds in any cell of `fine`
+    __device__ void fetch(const BucketArgs &a, int c, uint32_t buckets, uint32_t first_step) {
         for (uint32_t i = threadIdx.x; i + 1 < buckets; i += kBkThreads) bounds[i] = a.bounds[(int64_t)c * kStride + i];
-        const uint32_t *f = reinterpret_cast<const uint32_t *>(a.fine + (int64_t)c * (kBkFine + 2));
-        for (int i = threadIdx.x; i <= kBkFine / 2; i += kBkThreads) fine2[i] = f[i];
+        for (uint32_t i = threadIdx.x; i < 2 * first_step; i += kBkThreads)
+            if (buckets - 1 + i < 2 * kStride) bounds[buckets - 1 + i] = 0xFFFFFFFFu;
+        const uint32_t *from = reinterpret_cast<const uint32_t *>(a.fine + (int64_t)c * kBkFine);
+        uint32_t *to = reinterpret_cast<uint32_t *>(fine);
+#pragma unroll
+        for (int i = 0; i < kBkFine / 2 / kBkThreads; ++i) to[i * kBkThreads + threadIdx.x] = from[i * kBkThreads + threadIdx.x];
     }
-    // bucket of a key that takes part (key bits below 2^bits)
-    __device__ __forceinline__ uint32_t find(uint32_t key, int shift) const {
-        const uint16_t *fine = reinterpret_cast<const uint16_t *>(fine2);
-        const uint32_t f = key >> shift;
-        uint32_t lo = fine[f], hi = fine[f + 1];
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (bounds[mid] <= key) lo = mid + 1;
-            else hi = mid;
+    // buckets of N keys (kStride for one that takes no part): a step of all their searches at a time. Bounds behind a cell's
+    // are above its keys, so the search needs no end.
+    template <int N>
+    __device__ __forceinline__ void find(const uint32_t *key, uint32_t limit, int shift, uint32_t first_step, uint32_t *bucket) const {
+        uint32_t at[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) at[i] = fine[min(key[i] & 0x7FFFFFFFu, limit) >> shift];
+        for (uint32_t step = first_step; step; step >>= 1) {        // block-uniform
+#pragma unroll
+            for (int i = 0; i < N; ++i) at[i] += bounds[at[i] + step - 1u] <= (key[i] & 0x7FFFFFFFu) ? step : 0u;
         }
-        return lo;
+#pragma unroll
+        for (int i = 0; i < N; ++i) bucket[i] = keep_key(key[i], limit) ? at[i] : (uint32_t)kStride;
     }
 };
 
-template <int kStride>
-__global__ __launch_bounds__(kBkThreads) void bk_hist(const BucketArgs a) {
-    __shared__ BkLookup<kStride> look;
-    __shared__ uint32_t counts[kStride];
-    const int c = blockIdx.y, tile = blockIdx.x;
-    const int lane = threadIdx.x & 63;
-    const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
-    const uint32_t *kin = a.keys + (int64_t)c * a.P + begin;
-    uint32_t key[kBkTileItems];
+template <int kBits>
+__device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
+    uint32_t diff_lo = 0, diff_hi = 0;
 #pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) {
-        const int li = bk_item(kBkTileItems, r);
-        key[r] = li < n ? kin[li] : kIgnoredKey;
+    for (int b = 0; b < kBits; ++b) {
+        uint32_t splat = (uint32_t)((int32_t)(digit << (31 - b)) >> 31);
+        asm("" : "+v"(splat));
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(splat != 0u);
+        diff_lo |= (uint32_t)vote ^ splat;
+        diff_hi |= (uint32_t)(vote >> 32) ^ splat;
     }
-    const uint32_t buckets = a.numbers[c], limit = bk_limit(a, c);
-    const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
-    look.fetch(a, c, buckets);
-    for (uint32_t i = threadIdx.x; i < buckets; i += kBkThreads) counts[i] = 0;
-    __syncthreads();
-    uint16_t *bucket = a.bucket + (int64_t)c * a.P + begin;
-#pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) {
-        const int li = bk_item(kBkTileItems, r);
-        const bool valid = keep_key(key[r], limit);
-        const uint64_t vmask = __builtin_amdgcn_ballot_w64(valid);
-        uint32_t b = kBkNowhere;
-        if (valid) b = look.find(key[r] & 0x7FFFFFFFu, shift);
-        if (li < n) bucket[li] = (uint16_t)b;
-        if (vmask == 0) continue;                           // wave-uniform
-        const uint32_t one = (uint32_t)__builtin_amdgcn_readlane((int)b, __builtin_ctzll(vmask));
-        if (__builtin_amdgcn_ballot_w64(valid && b == one) == vmask) {          // one bucket for the whole round
-            const uint64_t hot = __builtin_amdgcn_ballot_w64(valid && (key[r] >> 31));
-            if (lane == 0)
-                atomicAdd(&counts[one], (uint32_t)__builtin_popcountll(vmask) | (uint32_t)__builtin_popcountll(hot) << 16);
-        } else if (valid) {
-            atomicAdd(&counts[b], 1u | (key[r] >> 31) << 16);
-        }
-    }
-    __syncthreads();
-    uint32_t *out = a.tile_count + ((int64_t)c * a.tiles + tile) * kStride;
-    for (uint32_t i = threadIdx.x; i < buckets; i += kBkThreads) out[i] = counts[i];
+    const uint64_t diff = ((uint64_t)diff_hi << 32) | diff_lo;
+    return __builtin_amdgcn_ballot_w64(valid) & ~diff;
 }
 
-// 64 buckets x 16 groups of tiles per block: the group's sums first, then the exclusive sums in place.
-__global__ __launch_bounds__(1024) void bk_scan(const BucketArgs a) {
-    __shared__ uint32_t sums[16][64], hots[16][64];
-    const int c = blockIdx.y, b = blockIdx.x * 64 + (threadIdx.x & 63), group = threadIdx.x >> 6;
-    const int buckets = (int)a.numbers[c];
-    if ((int)blockIdx.x * 64 >= buckets) return;            // block-uniform
-    const int per = (a.tiles + 15) / 16, first = group * per, last = min(a.tiles, first + per);
-    uint32_t *at = a.tile_count + (int64_t)c * a.tiles * a.stride + b;
-    uint32_t n = 0, h = 0;
-    if (b < buckets) {
-#pragma unroll 8
-        for (int t = first; t < last; ++t) {
-            const uint32_t v = at[(int64_t)t * a.stride];
-            n += v & 0xFFFFu;
-            h += v >> 16;
+// The tile's keys in the order of their buckets (in pixel order inside one), in the place of its keys, and every pixel's place
+// in that order.
+// Bound by vector and LDS instructions, 70 and 15 per 64 keys (nearly all taking part: 78 of 137 us of vector issue), at 24 waves
+// per CU. Match masks of 10 votes for every key were 126 per 64 keys (149 -> 102 us at (4,19,512,1024) fp32, 177 -> 137 at
+// (8,21,513,513) bf16 trained); a wave's 64 keys lie in up to 1024 buckets, so that some 5 of them meet another.
+template <int kBits>
+__global__ __launch_bounds__(kBkThreads, 6) void bk_cut(const BucketArgs a) {
+    constexpr int kStride = 1 << kBits, kPer = (kStride + kBkThreads - 1) / kBkThreads, kChunks = kBkTile / kWave;
+    // 49 KiB, three blocks per CU: the look-up's tables are done with when the tile is put in order
+    union Tile {
+        BkLookup<kStride> look;
+        uint32_t key[kBkTile];
+    };
+    __shared__ Tile s;
+    __shared__ __align__(16) uint16_t counts[kBkWaves][kStride + 2];        // a wave's keys so far; the last of those that take no part
+    __shared__ uint64_t hot_mask[kChunks + 1];
+    __shared__ uint32_t hot_before[kChunks + 1];
+    __shared__ uint32_t scan_tmp[kSortWaves];
+    const int c = blockIdx.y, tile = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
+    uint32_t *row = a.keys + (int64_t)c * a.P + begin;
+    uint32_t key[kBkTileItems], b[kBkTileItems], rank[kBkTileItems];
+    if (n == kBkTile) {
+#pragma unroll
+        for (int r = 0; r < kBkTileItems; ++r) key[r] = row[bk_item(kBkTileItems, r)];
+    } else {
+#pragma unroll
+        for (int r = 0; r < kBkTileItems; ++r) {
+            const int li = bk_item(kBkTileItems, r);
+            key[r] = li < n ? row[li] : kIgnoredKey;
         }
     }
-    sums[group][threadIdx.x & 63] = n;
-    hots[group][threadIdx.x & 63] = h;
+    const uint32_t buckets = a.numbers[c], first_step = a.numbers[5 * a.C + c], limit = bk_limit(a, c);
+    const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
+    s.look.fetch(a, c, buckets, first_step);
+    for (int i = threadIdx.x; i < kBkWaves * (kStride + 2) / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(counts)[i] = 0;
     __syncthreads();
-    if (b >= buckets) return;
-    uint32_t before = 0, total = 0, hot = 0;
+    constexpr int kFind = 8;
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; r += kFind) s.look.template find<kFind>(key + r, limit, shift, first_step, b + r);
+    // A key's rank among the wave's keys of its bucket: the counter, moved on by every key, tells what came in earlier rounds
+    // and how many come in this one. LDS takes a wave's operations in their order, so the rounds of a group wait for nothing.
+    // The few that meet others of their round find their place by a vote per bucket met twice; many, by a vote per bit.
+    constexpr int kGroup = 2;
+    constexpr uint32_t kFew = 16;
+    uint16_t *mine_of = counts[wave];
+#pragma unroll
+    for (int r0 = 0; r0 < kBkTileItems; r0 += kGroup) {
+        uint32_t after[kGroup];
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) {
+            const uint32_t d = b[r0 + h];
+            rank[r0 + h] = mine_of[d];
+            asm volatile("" ::: "memory");
+            if (d != (uint32_t)kStride)         // additions to one address take their turns
+                atomicAdd(reinterpret_cast<uint32_t *>(mine_of) + (d >> 1), 1u << (16u * (d & 1u)));
+            asm volatile("" ::: "memory");
+            after[h] = mine_of[d];
+            asm volatile("" ::: "memory");
+        }
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) {
+            const uint32_t d = b[r0 + h], seen = rank[r0 + h];
+            uint64_t met = __builtin_amdgcn_ballot_w64(after[h] - seen > 1u && d != (uint32_t)kStride);
+            bool first = true;
+            while (met && (first || __builtin_popcountll(met) <= kFew)) {   // wave-uniform
+                const uint32_t one = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(met));
+                const uint64_t peers = __builtin_amdgcn_ballot_w64(d == one);
+                if (d == one) rank[r0 + h] = seen + peers_below(peers);
+                met &= ~peers;
+                first = false;
+            }
+            if (met) {
+                const uint64_t peers = bk_peers<kBits>(d, d != (uint32_t)kStride);
+                rank[r0 + h] = seen + peers_below(peers);
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t mine[kPer], n_mine = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = threadIdx.x * kPer + i;
+        mine[i] = 0;
+        if (d < buckets) {
+#pragma unroll
+            for (int w = 0; w < kBkWaves; ++w) {
+                const uint32_t t = counts[w][d];
+                counts[w][d] = (uint16_t)mine[i];
+                mine[i] += t;
+            }
+        }
+        n_mine += mine[i];
+    }
+    uint32_t n_here;
+    const uint32_t first = block_excl_scan(n_mine, scan_tmp, n_here);
+    uint32_t at = first;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = threadIdx.x * kPer + i;
+        if (d < buckets) {
+#pragma unroll
+            for (int w = 0; w < kBkWaves; ++w) counts[w][d] = (uint16_t)(counts[w][d] + at);
+        }
+        at += mine[i];
+    }
+    __syncthreads();
+    uint16_t *place = a.place + (int64_t)c * a.P + begin;
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        asm volatile("" : "+v"(b[r]));                      // the counter's address again, not held in a register each
+        const bool valid = b[r] != (uint32_t)kStride;       // not past the end: those keys take no part
+        rank[r] = valid ? mine_of[b[r]] + rank[r] : (uint32_t)kBkNowhere;
+        if (valid) s.key[rank[r]] = key[r];
+    }
+    if (n == kBkTile) {
+#pragma unroll
+        for (int r = 0; r < kBkTileItems; ++r) place[bk_item(kBkTileItems, r)] = (uint16_t)rank[r];
+    } else {
+#pragma unroll
+        for (int r = 0; r < kBkTileItems; ++r) {
+            const int li = bk_item(kBkTileItems, r);
+            if (li < n) place[li] = (uint16_t)rank[r];
+        }
+    }
+    __syncthreads();
+    // out in order; the positives before a place from masks of 64 places each
+#pragma unroll
+    for (int r = 0; r < kBkTileItems; ++r) {
+        const uint32_t i = (uint32_t)r * kBkThreads + threadIdx.x;
+        const uint32_t k = i < n_here ? s.key[i] : 0u;
+        const uint64_t hot = __builtin_amdgcn_ballot_w64(k >> 31);
+        if (i < n_here) row[i] = k;
+        if (lane == 0) hot_mask[i >> 6] = hot;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        static_assert(kChunks == 2 * kWave, "two masks a lane");
+        const uint32_t h0 = (uint32_t)__builtin_popcountll(hot_mask[2 * lane]), h1 = (uint32_t)__builtin_popcountll(hot_mask[2 * lane + 1]);
+        const uint32_t incl = wave_incl_scan(h0 + h1);
+        hot_before[2 * lane] = incl - h0 - h1;
+        hot_before[2 * lane + 1] = incl - h1;
+        if (lane == kWave - 1) {
+            hot_before[kChunks] = incl;
+            hot_mask[kChunks] = 0;
+        }
+    }
+    __syncthreads();
+    uint32_t *out = a.tile_start + ((int64_t)c * a.tiles + tile) * (kStride + 1);
+    at = first;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t d = threadIdx.x * kPer + i;
+        const uint32_t hot = hot_before[at >> 6] + (uint32_t)__builtin_popcountll(hot_mask[at >> 6] & ((1ull << (at & 63u)) - 1ull));
+        if (d < buckets) out[d] = at | hot << 16;
+        at += mine[i];
+    }
+    if (threadIdx.x == 0) out[buckets] = n_here | hot_before[kChunks] << 16;
+}
+
+// Keys and positives before each bucket in the row: the sums of the tiles', which are left by bucket for the rank kernels.
+// 64 buckets x 64 tiles at a time.
+__global__ __launch_bounds__(1024) void bk_sum(const BucketArgs a) {
+    __shared__ uint32_t part[64][65];
+    __shared__ uint32_t sums[16][64], hots[16][64];
+    const int c = blockIdx.y, first = blockIdx.x * 64, lane = threadIdx.x & 63, group = threadIdx.x >> 6;
+    const int entries = (int)a.numbers[c] + 1;
+    if (first >= entries) return;                           // block-uniform
+    const int pitch = a.stride + 1;
+    const uint32_t *in = a.tile_start + (int64_t)c * a.tiles * pitch;
+    uint32_t *out = a.start + (int64_t)c * pitch * a.tiles;
+    uint32_t n = 0, h = 0, v[4];
+    auto fetch = [&](int t0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t0 + i * 16 + group;
+            v[i] = t < a.tiles && first + lane < entries ? in[(int64_t)t * pitch + first + lane] : 0u;
+        }
+    };
+    fetch(0);
+    for (int t0 = 0; t0 < a.tiles; t0 += 64) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            n += v[i] & 0xFFFFu;
+            h += v[i] >> 16;
+            part[i * 16 + group][lane] = v[i];
+        }
+        if (t0 + 64 < a.tiles) fetch(t0 + 64);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int b = first + i * 16 + group;
+            if (b < entries && t0 + lane < a.tiles) out[(int64_t)b * a.tiles + t0 + lane] = part[lane][i * 16 + group];
+        }
+        __syncthreads();
+    }
+    sums[group][lane] = n;
+    hots[group][lane] = h;
+    __syncthreads();
+    if (group != 0 || first + lane >= entries) return;
+    uint32_t total = 0, hot = 0;
 #pragma unroll
     for (int g = 0; g < 16; ++g) {
-        const uint32_t v = sums[g][threadIdx.x & 63];
-        before += g < group ? v : 0u;
-        total += v;
-        hot += hots[g][threadIdx.x & 63];
+        total += sums[g][lane];
+        hot += hots[g][lane];
     }
-#pragma unroll 8
-    for (int t = first; t < last; ++t) {
-        const uint32_t v = at[(int64_t)t * a.stride];
-        at[(int64_t)t * a.stride] = before;
-        before += v & 0xFFFFu;
-    }
-    if (group == 0) {
-        a.count[(int64_t)c * a.stride + b] = total;
-        a.hot[(int64_t)c * a.stride + b] = hot;
-    }
+    a.base[(int64_t)c * pitch + first + lane] = total;
+    a.hot_base[(int64_t)c * pitch + first + lane] = hot;
 }
 
 // Where the buckets start, and the runs of them that one block sorts: neighbours that start in the same kBkSlab keys of the
@@ -588,35 +788,10 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
     __shared__ uint32_t base[kBkMax + 1], bound[kBkMax + 1], scan_tmp[2 * kSortWaves];
     constexpr int kPer = kBkMax / kBkThreads;
     const int c = blockIdx.x, buckets = (int)a.numbers[c], b0 = threadIdx.x * kPer;
-    uint32_t n[kPer], h[kPer], n_sum = 0, h_sum = 0;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const bool is = b0 + i < buckets;
-        n[i] = is ? a.count[(int64_t)c * a.stride + b0 + i] : 0u;
-        h[i] = is ? a.hot[(int64_t)c * a.stride + b0 + i] : 0u;
-        bound[b0 + i] = b0 + i + 1 < buckets ? a.bounds[(int64_t)c * a.stride + b0 + i] : bk_limit(a, c) + 1u;  // of the next bucket
-        n_sum += n[i];
-        h_sum += h[i];
-    }
-    uint32_t at, n_all, at_hot, n_hot;
-    block_excl_scan2(n_sum, h_sum, scan_tmp, at, n_all, at_hot, n_hot);
     const int64_t row = (int64_t)c * (a.stride + 1);
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        base[b0 + i] = at;
-        if (b0 + i <= buckets) {
-            a.base[row + b0 + i] = at;
-            a.hot_base[row + b0 + i] = at_hot;
-        }
-        at += n[i];
-        at_hot += h[i];
-    }
-    if (threadIdx.x == kBkThreads - 1) {
-        base[kBkMax] = at;
-        if (buckets == kBkMax) {
-            a.base[row + kBkMax] = at;
-            a.hot_base[row + kBkMax] = at_hot;
-        }
+    for (int b = threadIdx.x; b <= buckets; b += kBkThreads) {
+        base[b] = a.base[row + b];
+        bound[b] = b + 1 < buckets ? a.bounds[(int64_t)c * a.stride + b] : bk_limit(a, c) + 1u;     // of the next bucket
     }
     __syncthreads();
     const uint32_t least = a.numbers[3 * a.C + c];
@@ -628,7 +803,8 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
         const int b = b0 + i;
         start[i] = false;
         if (b >= buckets) continue;
-        if (n[i] > (uint32_t)kBkCap && b && bound[b] - bound[b - 1] == 1u) a.count[(int64_t)c * a.stride + b] = n[i] | kBkFlat;
+        const uint32_t n = base[b + 1] - base[b];
+        a.count[(int64_t)c * a.stride + b] = n > (uint32_t)kBkCap && b && bound[b] - bound[b - 1] == 1u ? n | kBkFlat : n;
         const uint32_t slab = base[b] / kBkSlab;
         start[i] = b == 0 || base[b - 1] / kBkSlab != slab;
         if (!start[i]) {
@@ -648,141 +824,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
     if (threadIdx.x == 0) {
         a.runs[row + runs] = (uint32_t)buckets;
         a.numbers[a.C + c] = runs;
-        a.numbers[2 * a.C + c] = n_hot;
-    }
-}
-
-template <int kBits>
-__device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
-    uint32_t diff_lo = 0, diff_hi = 0;
-#pragma unroll
-    for (int b = 0; b < kBits; ++b) {
-        uint32_t splat = (uint32_t)((int32_t)(digit << (31 - b)) >> 31);
-        asm("" : "+v"(splat));
-        const uint64_t vote = __builtin_amdgcn_ballot_w64(splat != 0u);
-        diff_lo |= (uint32_t)vote ^ splat;
-        diff_hi |= (uint32_t)(vote >> 32) ^ splat;
-    }
-    const uint64_t diff = ((uint64_t)diff_hi << 32) | diff_lo;
-    return __builtin_amdgcn_ballot_w64(valid) & ~diff;
-}
-
-// The tile's keys by bucket, written out in runs. In the place of the tile's keys it leaves, in 16 bits each, every pixel's
-// place in the tile's order, then the bucket of every place.
-template <int kBits>
-__global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) {
-    constexpr int kStride = 1 << kBits, kPer = (kStride + kBkThreads - 1) / kBkThreads;
-    // 52 KiB, three blocks per CU: the buckets by place take the counters' memory
-    __shared__ uint32_t s_key[kBkTile];                     // the tile by bucket
-    __shared__ __align__(4) uint16_t s_counts[kBkTile > kBkWaves * kStride ? kBkTile : kBkWaves * kStride];
-    __shared__ uint32_t out_base[kStride];
-    __shared__ uint32_t scan_tmp[kSortWaves];
-    uint16_t *s_bucket = s_counts;
-    uint16_t(*counts)[kStride] = reinterpret_cast<uint16_t(*)[kStride]>(s_counts);
-    const int c = blockIdx.y, wave = threadIdx.x >> 6;
-    const int tile = sort_tile(a.P, kBkTile);
-    const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
-    uint32_t *kin = a.keys + (int64_t)c * a.P + begin;
-    uint32_t key[kBkTileItems], b[kBkTileItems], rank[kBkTileItems];
-#pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) {
-        const int li = bk_item(kBkTileItems, r);
-        key[r] = li < n ? kin[li] : 0u;
-        b[r] = li < n ? a.bucket[(int64_t)c * a.P + begin + li] : kBkNowhere;
-    }
-    const uint32_t buckets = a.numbers[c];
-    uint32_t first[kPer];
-    uint32_t *table = a.tile_count + ((int64_t)c * a.tiles + tile) * kStride;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const uint32_t d = threadIdx.x * kPer + i;
-        first[i] = d < buckets ? table[d] + a.base[(int64_t)c * (kStride + 1) + d] : 0u;
-    }
-    for (int i = threadIdx.x; i < kBkWaves * kStride / 2; i += kBkThreads) reinterpret_cast<uint32_t *>(s_counts)[i] = 0;
-    __syncthreads();
-    // Two rounds at a time (four spill): their masks first, then a read of the counter and the leader's addition to it per round. LDS
-    // takes a wave's operations in their order, so no addition waits for what a read returns.
-    constexpr int kGroup = 2;
-#pragma unroll
-    for (int r0 = 0; r0 < kBkTileItems; r0 += kGroup) {
-        uint64_t peers[kGroup];
-        uint32_t seen[kGroup];
-        bool any = false;
-#pragma unroll
-        for (int h = 0; h < kGroup; ++h) {
-            rank[r0 + h] = 0;
-            any = any || b[r0 + h] != kBkNowhere;
-        }
-        if (__builtin_amdgcn_ballot_w64(any) == 0) continue;        // wave-uniform
-#pragma unroll
-        for (int h = 0; h < kGroup; ++h) peers[h] = bk_peers<kBits>(b[r0 + h], b[r0 + h] != kBkNowhere);
-#pragma unroll
-        for (int h = 0; h < kGroup; ++h) {
-            const uint32_t d = b[r0 + h], before = peers_below(peers[h]);
-            const bool valid = d != kBkNowhere;
-            seen[h] = 0;
-            if (valid) seen[h] = counts[wave][d];
-            asm volatile("" ::: "memory");
-            if (valid && before == 0u)
-                atomicAdd(reinterpret_cast<uint32_t *>(counts[wave]) + (d >> 1),
-                          (uint32_t)__builtin_popcountll(peers[h]) << (16u * (d & 1u)));
-            asm volatile("" ::: "memory");
-            rank[r0 + h] = before;
-        }
-#pragma unroll
-        for (int h = 0; h < kGroup; ++h) rank[r0 + h] += seen[h];
-    }
-    __syncthreads();
-    uint32_t mine[kPer], n_mine = 0;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const uint32_t d = threadIdx.x * kPer + i;
-        mine[i] = 0;
-        if (d < buckets) {
-#pragma unroll
-            for (int w = 0; w < kBkWaves; ++w) {
-                const uint32_t t = counts[w][d];
-                counts[w][d] = (uint16_t)mine[i];
-                mine[i] += t;
-            }
-        }
-        n_mine += mine[i];
-    }
-    uint32_t n_here;
-    uint32_t at = block_excl_scan(n_mine, scan_tmp, n_here);
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-        const uint32_t d = threadIdx.x * kPer + i;
-        if (d < buckets) {
-#pragma unroll
-            for (int w = 0; w < kBkWaves; ++w) counts[w][d] = (uint16_t)(counts[w][d] + at);
-            out_base[d] = first[i] - at;
-            table[d] = first[i] - at;
-        }
-        at += mine[i];
-    }
-    __syncthreads();
-    uint16_t *places = reinterpret_cast<uint16_t *>(kin);
-#pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r)
-        rank[r] = b[r] != kBkNowhere ? counts[wave][b[r]] + rank[r] : kBkNowhere;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) {
-        const int li = bk_item(kBkTileItems, r);
-        if (li >= n) continue;
-        if (b[r] != kBkNowhere) {
-            s_key[rank[r]] = key[r];
-            s_bucket[rank[r]] = (uint16_t)b[r];
-        }
-        places[li] = (uint16_t)rank[r];
-    }
-    __syncthreads();
-    uint32_t *kout = a.sorted + (int64_t)c * a.P;
-    for (int i = threadIdx.x; i < (int)n_here; i += kBkThreads) {
-        const uint32_t d = s_bucket[i];
-        kout[out_base[d] + (uint32_t)i] = s_key[i];
-        places[n + i] = (uint16_t)d;
+        a.numbers[2 * a.C + c] = a.hot_base[row + buckets];
     }
 }
 
@@ -793,10 +835,14 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_scatter(const BucketArgs a) 
 template <bool Direct>
 __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, float *__restrict__ losses) {
     __shared__ BkShared s;
+    __shared__ BkSegments at;                               // not for a whole row
     __shared__ double wave_loss[kBkWaves];
-    const int c = Direct ? blockIdx.x : blockIdx.y, g = Direct ? 0 : blockIdx.x;
+    const int c = Direct ? blockIdx.x : blockIdx.y;
     const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
-    if (!Direct && g >= (int)a.numbers[a.C + c]) return;    // block-uniform
+    const int runs = Direct ? 1 : (int)a.numbers[a.C + c];
+    if (!Direct && (int)blockIdx.x >= runs) return;         // block-uniform
+    // neighbouring runs on one XCD: a tile's segments of theirs share cache lines
+    const int g = Direct ? 0 : sort_tile(runs, 1);
     const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
     const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
     const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
@@ -807,10 +853,11 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
         }
         return;
     }
-    const uint32_t *kin = Direct ? a.keys + row : a.sorted + row + rank0;
-    float *out = Direct ? reinterpret_cast<float *>(a.keys) + row : a.dj + row + rank0;
+    uint32_t *kin = a.keys + row;                           // the differences take the keys' places
     const uint32_t limit = bk_limit(a, c);
     float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
+    if constexpr (!Direct) at.collect(a, c, b0, b1, 0u, s.scan);
+    auto where = [&](int li) { return Direct ? (uint32_t)li : at.where((uint32_t)li); };
 
     uint32_t key[kBkItems], valid = 0, least, most, knee = 0;
     float share = 0.25f;
@@ -821,7 +868,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
         const int li = bk_item(rounds, r);
         key[r] = 0;
         if (r < rounds && li < n) {
-            key[r] = kin[li];
+            key[r] = kin[where(li)];
             if (!Direct || keep_key(key[r], limit)) valid |= 1u << r;
         }
     }
@@ -904,8 +951,9 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kBkItems; ++r) {
-        const int li = bk_item(rounds, r);
-        if (r < rounds && li < n) out[li] = (!Direct || ((valid >> r) & 1u)) ? result[li] : 0.f;
+        int li = bk_item(rounds, r);
+        asm volatile("" : "+v"(li));                        // looked up again, not held across the sort
+        if (r < rounds && li < n) kin[where(li)] = __builtin_bit_cast(uint32_t, (!Direct || ((valid >> r) & 1u)) ? result[li] : 0.f);
     }
     if (threadIdx.x == 0) {
         double sum = 0.0;
@@ -921,6 +969,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
 template <bool Direct>
 __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArgs a, float *__restrict__ losses) {
     __shared__ BkShared s;
+    __shared__ BkSegments at;
     __shared__ double wave_loss[kBkWaves];
     const int c = Direct ? blockIdx.x : blockIdx.y;
     const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
@@ -933,16 +982,17 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
         const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
         const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
         const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
-        const uint32_t *kin = Direct ? a.keys + row : a.sorted + row + rank0;
-        float *out = Direct ? reinterpret_cast<float *>(a.keys) + row : a.dj + row + rank0;
+        uint32_t *kin = a.keys + row;
         const uint32_t limit = bk_limit(a, c);
         const int rounds = (n + kBkThreads - 1) / kBkThreads;
         uint32_t key[kBkItems], rank[kBkItems], valid = 0, hot = 0, least, most;
         __syncthreads();
+        if constexpr (!Direct) at.collect(a, c, b0, b1, 0u, s.scan);
+        auto where = [&](int li) { return Direct ? (uint32_t)li : at.where((uint32_t)li); };
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r) {
             const int li = bk_item(rounds, r);
-            key[r] = r < rounds && li < n ? kin[li] : kIgnoredKey;
+            key[r] = r < rounds && li < n ? kin[where(li)] : kIgnoredKey;
             if (keep_key(key[r], limit)) {
                 valid |= 1u << r;
                 hot += key[r] >> 31;
@@ -963,11 +1013,11 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
             if (r < rounds && li < n) {
                 float dj = 0.f;
                 if ((valid >> r) & 1u) {
-                    const uint32_t k = Direct ? key[r] : kin[li];       // read again: not held across the sort
+                    const uint32_t k = Direct ? key[r] : kin[where(li)];       // read again: not held across the sort
                     dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), k >> 31);
                     part = add_loss(part, key_error(k), dj);
                 }
-                out[li] = dj;
+                kin[where(li)] = __builtin_bit_cast(uint32_t, dj);
             }
         }
         part = wave_sum_f64(part);
@@ -989,7 +1039,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
 // is ranked by position.
 __device__ __forceinline__ double bk_wide_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, int n) {
     const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
-    float *out = a.dj + (int64_t)c * a.P + rank0;
+    float *out = reinterpret_cast<float *>(a.dj) + (int64_t)c * a.P + rank0;
     const float npos = (float)a.numbers[2 * a.C + c];
     double part = 0.0;
     uint32_t key[kBkItems], rank[kBkItems], valid = 0, least, most;
@@ -1280,7 +1330,7 @@ __device__ __forceinline__ uint32_t bk_huge_groups(BkShared &s, const BkGroups &
 __device__ __forceinline__ double bk_huge_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n,
                                uint32_t lo, uint32_t hi) {
     uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;   // the keys, then every key's place, then its difference
-    uint32_t *moved = reinterpret_cast<uint32_t *>(a.dj) + (int64_t)c * a.P + rank0;
+    uint32_t *moved = a.dj + (int64_t)c * a.P + rank0;
     const float npos = (float)a.numbers[2 * a.C + c];
     const BkGroups of(s);
     const uint32_t groups = bk_huge_groups(s, of, kin, n, lo, hi);
@@ -1392,51 +1442,86 @@ __device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
     return k == 0 ? 0.f : 1.f - inter / (inter + (float)k);
 }
 
-// This block's part of a bucket of one value, n keys from rank0 on with hot0 positives before them and `hot` among them: in
-// order as they stand. The positives before the part are counted again by every block where the flags are mixed (a value
-// that many share is mostly the positives' or the others' alone). Done by bk_scatter, 16 places per thread, this took that
-// kernel from 94 to 149 us where all logits are equal ((8,19,512,512)); step 459 -> 418 us, radix passes 425.
-__device__ __forceinline__ void bk_flat_keys(BkShared &s, const BucketArgs &a, int c, uint32_t rank0, uint32_t hot0, uint32_t n, uint32_t hot) {
+// This block's part, every kBkWideBlocks-th tile, of bucket b with one value and n keys, from rank0 on with hot0 positives
+// before them and `hot` among them: in order as they stand. (A value that many share is mostly the positives' or the others'
+// alone.)
+__device__ __forceinline__ void bk_flat_keys(BkShared &s, const BucketArgs &a, int c, int b, uint32_t rank0, uint32_t hot0) {
     constexpr uint32_t kPer = 8, kStep = kPer * kBkThreads;
-    const uint32_t *kin = a.sorted + (int64_t)c * a.P + rank0;
-    float *out = a.dj + (int64_t)c * a.P + rank0;
+    // per tile: its first key of the bucket and their number; keys and positives of the bucket in the tiles before, positives here
+    uint32_t *first = s.key(), *count = first + kBkThreads, *before = count + kBkThreads, *hot_before = before + kBkThreads,
+             *hot = hot_before + kBkThreads;
     const float npos = (float)a.numbers[2 * a.C + c];
-    const uint32_t part = ((n + kBkWideBlocks - 1) / kBkWideBlocks + kStep - 1) / kStep * kStep;
-    const uint32_t from = blockIdx.x * part, end = min(n, from + part);
-    if (from >= n) return;                                  // block-uniform
-    const bool mixed = hot != 0u && hot != n;
-    uint32_t before = hot ? from : 0u;                      // positives of the bucket before the part
-    if (mixed) {
-        uint32_t mine = 0;
-#pragma unroll 8
-        for (uint32_t i = threadIdx.x; i < from; i += kBkThreads) mine += kin[i] >> 31;
-        block_excl_scan(mine, s.scan, before);
+    const int64_t cell = ((int64_t)c * (a.stride + 1) + b) * a.tiles;
+    uint32_t start = 0, end = 0, unused;
+    if ((int)threadIdx.x < a.tiles) {
+        start = a.start[cell + threadIdx.x];
+        end = a.start[cell + a.tiles + threadIdx.x];
     }
-    for (uint32_t i0 = from; i0 < end; i0 += kStep) {
-        const uint32_t p0 = i0 + threadIdx.x * kPer;
-        uint32_t flags = hot ? 0xFFu : 0u;
-        uint32_t cs = hot0 + (hot ? p0 : 0u);
-        if (mixed) {
-            flags = 0;
+    const uint32_t keys = (end & 0xFFFFu) - (start & 0xFFFFu), hots = (end >> 16) - (start >> 16);
+    __syncthreads();
+    first[threadIdx.x] = start & 0xFFFFu;
+    count[threadIdx.x] = keys;
+    hot[threadIdx.x] = hots;
+    block_excl_scan2(keys, hots, s.scan, before[threadIdx.x], unused, hot_before[threadIdx.x], unused);
+    __syncthreads();
+    for (int t = blockIdx.x; t < a.tiles; t += kBkWideBlocks) {
+        const uint32_t n = count[t], rank_t = rank0 + before[t];
+        uint32_t hot_t = hot0 + hot_before[t];
+        const bool mixed = hot[t] != 0u && hot[t] != n;     // block-uniform
+        uint32_t *at = a.keys + (int64_t)c * a.P + (uint32_t)t * kBkTile + first[t];
+        for (uint32_t i0 = 0; i0 < n; i0 += kStep) {
+            const uint32_t p0 = i0 + threadIdx.x * kPer;
+            uint32_t flags = hot[t] ? 0xFFu : 0u;
+            uint32_t cs = hot_t + (hot[t] ? p0 : 0u);
+            if (mixed) {
+                flags = 0;
 #pragma unroll
-            for (uint32_t e = 0; e < kPer; ++e) flags |= (p0 + e < end ? kin[p0 + e] >> 31 : 0u) << e;
-            uint32_t all;
-            cs = hot0 + before + block_excl_scan((uint32_t)__builtin_popcount(flags), s.scan, all);
-            before += all;
-        }
-        float j_prev = jaccard(npos, rank0 + p0, cs);
+                for (uint32_t e = 0; e < kPer; ++e) flags |= (p0 + e < n ? at[p0 + e] >> 31 : 0u) << e;
+                uint32_t all;
+                cs = hot_t + block_excl_scan((uint32_t)__builtin_popcount(flags), s.scan, all);
+                hot_t += all;
+            }
+            float j_prev = jaccard(npos, rank_t + p0, cs);
 #pragma unroll
-        for (uint32_t e = 0; e < kPer; ++e) {
-            cs += (flags >> e) & 1u;
-            const float j_now = jaccard(npos, rank0 + p0 + e + 1u, cs);
-            if (p0 + e < end) out[p0 + e] = j_now - j_prev;                            // csrc/lovasz_softmax.cu:141-147
-            j_prev = j_now;
+            for (uint32_t e = 0; e < kPer; ++e) {
+                cs += (flags >> e) & 1u;
+                const float j_now = jaccard(npos, rank_t + p0 + e + 1u, cs);
+                if (p0 + e < n) at[p0 + e] = __builtin_bit_cast(uint32_t, j_now - j_prev);     // csrc/lovasz_softmax.cu:141-147
+                j_prev = j_now;
+            }
         }
     }
+    __syncthreads();
+}
+
+// The n keys of bucket b to a row of their own from rank0 on, or the differences found there back to their places.
+__device__ __forceinline__ void bk_wide_copy(BkShared &s, BkSegments &segments, const BucketArgs &a, int c, int b, uint32_t rank0, uint32_t n, bool back) {
+    const int64_t row = (int64_t)c * a.P;
+    for (uint32_t from = 0; from < n; from += kBkCap) {
+        uint32_t v[kBkItems], at[kBkItems];
+        __syncthreads();
+        segments.collect(a, c, (uint32_t)b, (uint32_t)b + 1u, from, s.scan);
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            const uint32_t li = (uint32_t)bk_item(kBkItems, r);
+            at[r] = v[r] = 0;
+            if (from + li < n) {
+                at[r] = segments.where(li, from);
+                v[r] = back ? a.dj[row + rank0 + from + li] : a.keys[row + at[r]];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            const uint32_t li = (uint32_t)bk_item(kBkItems, r);
+            if (from + li < n) (back ? a.keys[row + at[r]] : a.sorted[row + rank0 + from + li]) = v[r];
+        }
+    }
+    __syncthreads();
 }
 
 __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
     __shared__ BkShared s;
+    __shared__ BkSegments at;
     __shared__ double wave_loss[kBkWaves];
     __shared__ int todo[kBkMax / kBkWideBlocks + 1], found;
     __shared__ int flats[kBkMaxRow / kBkCap + 1], n_flats;
@@ -1452,18 +1537,18 @@ __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
         else if (mine && wide) todo[atomicAdd(&found, 1)] = i;
         if (mine && !(n & kBkFlat) && !wide) a.loss_part[2 * row + a.stride + i] = 0.0;
         if (mine && (n & kBkFlat)) {
-            // one error, and the differences, exact as multiples of 2^-24, add up to that of the ends
-            const uint32_t first = a.base[cells + i], last = first + (n & ~kBkFlat), hots = a.hot_base[cells + i];
+            // one error, its bound, and the differences, exact as multiples of 2^-24, add up to that of the ends
             const float npos = (float)a.numbers[2 * a.C + c];
-            const float rise = jaccard(npos, last, hots + a.hot[row + i]) - jaccard(npos, first, hots);
-            a.loss_part[2 * row + a.stride + i] = add_loss(0.0, key_error(a.sorted[(int64_t)c * a.P + first]), rise);
+            const float rise = jaccard(npos, a.base[cells + i + 1], a.hot_base[cells + i + 1]) -
+                               jaccard(npos, a.base[cells + i], a.hot_base[cells + i]);
+            a.loss_part[2 * row + a.stride + i] = add_loss(0.0, key_error(a.bounds[row + i - 1]), rise);
         }
     }
     __syncthreads();
     const int n_flat = n_flats;
     for (int i = 0; i < n_flat; ++i) {                      // block-uniform
         const int b = flats[i];
-        bk_flat_keys(s, a, c, a.base[cells + b], a.hot_base[cells + b], a.count[row + b] & ~kBkFlat, a.hot[row + b]);
+        bk_flat_keys(s, a, c, b, a.base[cells + b], a.hot_base[cells + b]);
     }
     const int n_todo = found;
     for (int i = 0; i < n_todo; ++i) {
@@ -1471,6 +1556,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
         const uint32_t lo = b ? a.bounds[row + b - 1] : 0u, hi = b + 1 < buckets ? a.bounds[row + b] : bk_limit(a, c) + 1u;
         const uint32_t n = a.count[row + b], rank0 = a.base[cells + b], hot0 = a.hot_base[cells + b];
         // Sampled bounds leave a bucket of 7700 to 9000 keys in every other step or so: by ranges 30 us, by groups 45.
+        bk_wide_copy(s, at, a, c, b, rank0, n, false);
         double part = n <= 4u * kBkCap ? bk_wide_keys(s, a, c, rank0, hot0, (int)n) : bk_huge_keys(s, a, c, rank0, hot0, n, lo, hi);
         part = wave_sum_f64(part);
         __syncthreads();
@@ -1482,45 +1568,23 @@ __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
             for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
             a.loss_part[2 * row + a.stride + b] = sum;
         }
+        bk_wide_copy(s, at, a, c, b, rank0, n, true);
     }
 }
 
-// The tile's Jaccard differences in pixel order in the place of what bk_scatter left there: read in the runs that it wrote, put
-// in order in LDS. The first block of a class adds up its loss.
-template <int kBits>
-__global__ __launch_bounds__(kBkThreads) void bk_gather(const BucketArgs a, float *__restrict__ losses) {
-    constexpr int kStride = 1 << kBits;
-    __shared__ float dj[kBkTile];
-    __shared__ uint32_t from[kStride];
-    __shared__ uint32_t here[kBkWaves];
-    const int c = blockIdx.y, tile = sort_tile(a.P, kBkTile), lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// The tile's Jaccard differences in pixel order. The first block of a class adds up its loss.
+__global__ __launch_bounds__(kBkThreads) void bk_restore(const BucketArgs a, float *__restrict__ losses) {
+    __shared__ uint32_t dj[kBkTile];
+    const int c = blockIdx.y, tile = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
     uint32_t *row = a.keys + (int64_t)c * a.P + begin;
-    const uint16_t *places = reinterpret_cast<const uint16_t *>(row);
-    const uint32_t *table = a.tile_count + ((int64_t)c * a.tiles + tile) * kStride;
-    uint32_t place[kBkTileItems], bucket[kBkTileItems], kept = 0;
+    const uint16_t *places = a.place + (int64_t)c * a.P + begin;
+    uint32_t place[kBkTileItems], v[kBkTileItems];
 #pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) {
         const int li = bk_item(kBkTileItems, r);
+        v[r] = li < n ? row[li] : 0u;                       // past the keys that take part: not used
         place[r] = li < n ? places[li] : kBkNowhere;
-        bucket[r] = li < n ? places[n + li] : 0u;           // past the kept ones: keys that were never overwritten, unused
-    }
-    const int buckets = (int)a.numbers[c];
-    for (int i = threadIdx.x; i < buckets; i += kBkThreads) from[i] = table[i];
-#pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) kept += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(place[r] != kBkNowhere));
-    if (lane == 0) here[wave] = kept;
-    __syncthreads();
-    int n_here = 0;
-#pragma unroll
-    for (int w = 0; w < kBkWaves; ++w) n_here += (int)here[w];
-    const float *src = a.dj + (int64_t)c * a.P;
-    float v[kBkTileItems];
-#pragma unroll
-    for (int r = 0; r < kBkTileItems; ++r) {
-        const int i = bk_item(kBkTileItems, r);
-        v[r] = 0.f;
-        if (i < n_here) v[r] = src[from[bucket[r]] + (uint32_t)i];
     }
 #pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) dj[bk_item(kBkTileItems, r)] = v[r];
@@ -1528,11 +1592,11 @@ __global__ __launch_bounds__(kBkThreads) void bk_gather(const BucketArgs a, floa
 #pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) {
         const int li = bk_item(kBkTileItems, r);
-        if (li < n) row[li] = place[r] != kBkNowhere ? __builtin_bit_cast(uint32_t, dj[place[r]]) : 0u;
+        if (li < n) row[li] = place[r] != kBkNowhere ? dj[place[r]] : 0u;
     }
     if (tile != 0) return;
     __shared__ double wave_sum[kBkWaves];
-    const int runs = (int)a.numbers[a.C + c];
+    const int runs = (int)a.numbers[a.C + c], buckets = (int)a.numbers[c];
     const double *sums = a.loss_part + 2 * (int64_t)c * a.stride;
     double sum = 0.0;
     for (int i = threadIdx.x; i < runs; i += kBkThreads) sum += sums[i];

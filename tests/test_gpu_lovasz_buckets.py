@@ -137,6 +137,21 @@ def test_buckets_that_the_sample_misses(native, pixels, kind, n_cls):
     compare(native, x, labels(rng, (1, 1, pixels), 2))
 
 
+# how many buckets the 64 neighbouring keys of a wave lie in: one (no vote), a few that all are met, many that few are met
+@pytest.mark.parametrize("ways", [1, 2, 7, 16, 33, 64])
+@pytest.mark.parametrize("pixels", [8192, 70001, 2560 * 256 + 4095])
+def test_neighbours_in_few_buckets(native, ways, pixels):
+    assert by_buckets(32, pixels)
+    rng = np.random.default_rng(ways)
+    per = -(-pixels // ways)
+    order = np.sort(rng.standard_normal(per * ways).astype(np.float32) * 2)
+    i = np.arange(pixels)
+    x = rng.standard_normal((1, 32, 1, pixels), dtype=np.float32)
+    x[0, 0, 0] = order[i % ways * per + i // ways]
+    x[0, 1, 0] = np.where(rng.random(pixels) < 0.9, x[0, 0, 0], x[0, 1, 0])
+    compare(native, x, labels(rng, (1, 1, pixels), 32))
+
+
 @pytest.mark.parametrize("n_cls", [2, 19, 24, 32])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("plane", [(65, 67), (64, 65), (85, 121)])
