@@ -17,8 +17,8 @@
 // A key moves 28 bytes: read and written by bk_cut, bk_rank and bk_restore, and a place of 2 bytes. The form before this one
 // wrote the buckets out one after the other: that takes a histogram first (6 bytes a key more, buckets kept for the second
 // pass) and writes of some 10 keys, where a segment of a run has 24 here. (4,19,512,1024) fp32: histogram and scatter
-// 67 + 117 us against 102 now, rank 119 against 134, gather 72 against 57, step 585 -> 518 us; (8,21,513,513) bf16 trained
-// 77 + 154 against 137, 217 against 270, 116 against 68, step 794 -> 700. Which rows come here: bk_pays.
+// 67 + 117 us against 102 now, rank 119 against 111, gather 72 against 57, step 585 -> 487 us; (8,21,513,513) bf16 trained
+// 77 + 154 against 137, 217 against 227, 116 against 68, step 794 -> 642. Which rows come here: bk_pays.
 #pragma once
 
 namespace plh {
@@ -81,12 +81,24 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     return v;
 }
 
+// a / b as the division operator rounds it, for whole numbers 0 <= a <= b <= kBkMaxRow, b > 0: Newton's step on the reciprocal
+// leaves it 2^-24 of its value off, the product 2 units in its last place, the residual's correction 2^-23 of a unit. No
+// quotient of such numbers is nearer than 1 / 2b > 2^-23 of a unit to where the rounding changes (2a / unit and b times an odd
+// number are whole and differ). The operator's second residual and its scaling are for other operands.
+__device__ __forceinline__ float whole_ratio(float a, float b) {
+    float y = __builtin_amdgcn_rcpf(b);
+    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+    const float q = a * y;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+static_assert(kBkMaxRow < 1 << 22, "2b < 2^23");
+
 // Jaccard difference of the key at rank `pos`, with `cs` of the class's npos positives before it.
 __device__ __forceinline__ float jaccard_step(float npos, uint32_t pos, uint32_t cs, uint32_t hot) {
     const float inter_prev = npos - (float)cs;                             // csrc/lovasz_softmax.cu:124-127
     const float inter = npos - (float)(cs + hot);
-    const float j_now = 1.f - inter / (inter + (float)(pos + 1));
-    const float j_prev = (pos == 0) ? 0.f : 1.f - inter_prev / (inter_prev + (float)pos);
+    const float j_now = 1.f - whole_ratio(inter, inter + (float)(pos + 1));
+    const float j_prev = (pos == 0) ? 0.f : 1.f - whole_ratio(inter_prev, inter_prev + (float)pos);
     return j_now - j_prev;                                                 // csrc/lovasz_softmax.cu:141-147
 }
 
@@ -94,16 +106,16 @@ __device__ __forceinline__ float jaccard_step(float npos, uint32_t pos, uint32_t
 // [1, 2): the smaller and the larger of two are one instruction each.
 typedef double BkPair;
 __device__ __forceinline__ BkPair bk_pair(uint32_t key, uint32_t item) {
-    const uint32_t k = key & 0x7FFFFFFFu;
-    const uint64_t bits = (uint64_t)(0x3FF00000u | (k >> 18)) << 32 | (k << 14 | item << 1 | key >> 31);
-    return __builtin_bit_cast(double, bits);
+    const uint32_t hi = __builtin_amdgcn_alignbit(0x3FF00000u >> 14, key & 0x7FFFFFFFu, 18);       // exponent | key >> 18
+    const uint32_t lo = key << 14 | __builtin_amdgcn_alignbit(item, key, 31);                      // item << 1 | key >> 31
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 __device__ __forceinline__ uint32_t bk_item_of(BkPair p) { return ((uint32_t)__builtin_bit_cast(uint64_t, p) >> 1) & 0x1FFFu; }
 __device__ __forceinline__ uint32_t bk_hot_of(BkPair p) { return (uint32_t)__builtin_bit_cast(uint64_t, p) & 1u; }
 __device__ __forceinline__ uint32_t bk_key_of(BkPair p) {              // below 2^30: the exponent's bits fall out
     return (uint32_t)(__builtin_bit_cast(uint64_t, p) >> 14);
 }
-__device__ __forceinline__ BkPair bk_last() { return __builtin_bit_cast(double, (uint64_t)0x3FFFFFFFFFFFFFFFull); }
+__device__ __forceinline__ BkPair bk_last() { return __builtin_bit_cast(double, (uint64_t)0x3FFFFFFFFFFFFFFEull); }   // no positive
 static_assert(kBkCap <= 1 << 13 && kOne < 1u << 30, "13 bits of a pair name the item, 30 hold the key");
 
 __device__ __forceinline__ void bk_order(BkPair &a, BkPair &b) {
@@ -132,38 +144,59 @@ __device__ __forceinline__ void bk_merge(BkPair (&v)[kBkChunk]) {
 // Where the keys of a few neighbouring buckets stand: in every tile a segment of its order. The segments one after the other are
 // the keys in the order that the sort keeps among equals; places from..from + kBkCap - 1 of it are covered.
 constexpr int kBkWords = kBkCap / kWave;
+constexpr int kBkGroup = 3;                     // rounds whose LDS accesses are waited for together
+static_assert(kBkItems % kBkGroup == 0, "groups of rounds");
 struct BkSegments {
-    uint64_t starts[kBkWords];                  // bit i of word k: a segment starts at place 64 k + i + 1
-    uint32_t segment[kBkWords];                 // of place 64 k
+    struct alignas(16) Word {
+        uint64_t starts;                        // bit i: a segment starts at place 64 k + i + 1
+        uint32_t segment, unused;               // that of place 64 k
+    };
+    Word word[kBkWords + kBkGroup - 1];         // the last ones are looked at, and not used
     uint32_t shift[kBkMaxRow / kBkTile + 1];    // where the segment starts in the row less its first place
-    // Every thread of the block calls it; ends with a barrier. The memory is free before, with a barrier in between.
-    __device__ void collect(const BucketArgs &a, int c, uint32_t b0, uint32_t b1, uint32_t from, uint32_t *scan) {
-        uint32_t *words = reinterpret_cast<uint32_t *>(starts);
-        if (threadIdx.x < 2 * kBkWords) words[threadIdx.x] = 0;
-        const int64_t cell = (int64_t)c * (a.stride + 1);
-        const uint32_t t = threadIdx.x;
-        uint32_t at = 0, n = 0;
-        if (t < (uint32_t)a.tiles) {
-            at = a.start[(cell + b0) * a.tiles + t] & 0xFFFFu;
-            n = (a.start[(cell + b1) * a.tiles + t] & 0xFFFFu) - at;
+    // The thread's tile: first key of the buckets from b0 to before b1 in its order, and their number.
+    struct Tile {
+        uint32_t first, keys;
+        __device__ __forceinline__ Tile() : first(0), keys(0) {}
+        __device__ __forceinline__ Tile(const BucketArgs &a, int c, uint32_t b0, uint32_t b1) : first(0), keys(0) {
+            const int64_t cell = (int64_t)c * (a.stride + 1);
+            if ((int)threadIdx.x < a.tiles) {
+                first = a.start[(cell + b0) * a.tiles + threadIdx.x] & 0xFFFFu;
+                keys = (a.start[(cell + b1) * a.tiles + threadIdx.x] & 0xFFFFu) - first;
+            }
         }
+    };
+    // Every thread of the block calls it; ends with a barrier. The memory is free before, with a barrier in between.
+    __device__ __forceinline__ void collect(const Tile tile, uint32_t from, uint32_t *scan) {
+        uint32_t *words = reinterpret_cast<uint32_t *>(word);
+        if (threadIdx.x < 4 * (kBkWords + kBkGroup - 1)) words[threadIdx.x] = 0;
+        const uint32_t n = tile.keys;
         uint32_t place, all, index, segments;
         block_excl_scan2(n, n ? 1u : 0u, scan, place, all, index, segments);
         if (n && place + n > from && place < from + kBkCap) {
-            shift[index] = t * kBkTile + at - place;
+            shift[index] = threadIdx.x * kBkTile + tile.first - place;
             const uint32_t first = place > from ? place - from : 0u, end = min(place + n - from, (uint32_t)kBkCap);
-            if (first & 63u) atomicOr(&words[(first - 1u) >> 5], 1u << ((first - 1u) & 31u));
-            for (uint32_t k = (first + 63u) / 64u; k * 64u < end; ++k) segment[k] = index;
+            if (first & 63u) atomicOr(&words[((first - 1u) >> 6) * 4u + (((first - 1u) >> 5) & 1u)], 1u << ((first - 1u) & 31u));
+            for (uint32_t k = (first + 63u) / 64u; k * 64u < end; ++k) word[k].segment = index;
         }
         __syncthreads();
     }
-    // Where the key at place from + p stands in the row; p / 64 is the same for the whole wave.
-    __device__ __forceinline__ uint32_t where(uint32_t p, uint32_t from = 0) const {
-        const uint32_t k = p >> 6;
-        return shift[segment[k] + peers_below(starts[k])] + from + p;
+    // Where the keys at places from + p, from + p + 64, ... stand in the row (lane i of a wave: a place p = 64 k + i), and any
+    // place up to `most` for a key that is not there. The words of all, then their segments, so that LDS is waited for twice.
+    template <int N>
+    __device__ __forceinline__ void where(uint32_t p, uint32_t most, uint32_t (&at)[N], uint32_t from = 0) const {
+        const Word *words = word + (p >> 6);
+        Word w[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) w[i] = words[i];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            at[i] = shift[__builtin_amdgcn_mbcnt_hi((uint32_t)(w[i].starts >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((uint32_t)w[i].starts, w[i].segment))];
+#pragma unroll
+        for (int i = 0; i < N; ++i) at[i] = min(at[i] + (from + p + (uint32_t)i * kWave), most);
     }
 };
-static_assert(kBkMaxRow / kBkTile < kBkThreads && 2 * kBkWords <= kBkThreads, "a thread per tile and per word");
+static_assert(kBkMaxRow / kBkTile < kBkThreads && 4 * (kBkWords + kBkGroup - 1) <= kBkThreads, "a thread per tile and per word");
 
 struct BkShared {
     // the pairs, 16 neighbours in the order of thread t in row t; the crowded path's keys and items; the results by item
@@ -215,7 +248,7 @@ __device__ __forceinline__ int bk_item(int rounds, int r) {
 }
 
 // The bins of the values from..to: one width for all, or another below `knee`, which then gets the first `share` of them.
-// Monotone in the key, and below kBkBins (or rounded to kBkBins itself).
+// Monotone in the key, and below kBkBins.
 struct BkBinning {
     uint32_t from, knee;
     float below, above, start;
@@ -227,9 +260,10 @@ struct BkBinning {
         above = ((float)(kBkBins - 1) - start) / (float)(to - (bent ? knee : from) + 1u);
     }
     __device__ __forceinline__ uint32_t of(uint32_t key) const {
-        const uint32_t k = max(key & 0x7FFFFFFFu, from);
-        if (!bent) return (uint32_t)((float)(k - from) * above);
-        return k < knee ? (uint32_t)((float)(k - from) * below) : (uint32_t)__builtin_fmaf((float)(k - knee), above, start);
+        const uint32_t k = key & 0x7FFFFFFFu;               // not below `from`, or not looked at
+        const float last = (float)(kBkBins - 1);
+        if (!bent) return (uint32_t)fminf((float)(k - from) * above, last);
+        return (uint32_t)fminf(k < knee ? (float)(k - from) * below : __builtin_fmaf((float)(k - knee), above, start), last);
     }
 };
 
@@ -239,7 +273,16 @@ struct BkBinning {
 // Counting the keys into 4096 bins of their range puts them in order but for the one or two per bin; those are sorted by
 // the threads, 16 places each, then across the chunks' borders (8 places of either side) and within the chunks in turn:
 // odd-even transposition of halves of 8, of which a bin of L keys touches at most 2 + (L - 2) / 8.
-__device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds,
+struct BkMask {                                 // which of a thread's items are keys: any
+    uint32_t bits;
+    __device__ __forceinline__ bool operator()(int r) const { return (bits >> r) & 1u; }
+};
+struct BkFirst {                                // or the first ones
+    int count;
+    __device__ __forceinline__ bool operator()(int r) const { return r < count; }
+};
+template <class Valid>
+__device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkItems], Valid valid, int rounds,
                                         const BkBinning bins, uint32_t &n, BkPair (&v)[kBkChunk]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     {
@@ -250,12 +293,18 @@ __device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkIt
     __syncthreads();
     uint32_t slot[kBkItems];                    // bin << 16 | arrival
 #pragma unroll
-    for (int r = 0; r < kBkItems; ++r) {
-        slot[r] = 0;
-        if (r < rounds && ((valid >> r) & 1u)) {
-            const uint32_t b = min(bins.of(key[r]), (uint32_t)kBkBins - 1u);
-            slot[r] = b << 16 | atomicAdd(&s.bin[b], 1u);
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                // block-uniform
+        uint32_t arrival[kBkGroup];
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) {
+            const int r = r0 + i;
+            slot[r] = bins.of(key[r]);
+            arrival[i] = 0;
+            if (valid(r)) arrival[i] = atomicAdd(&s.bin[slot[r]], 1u);
         }
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) slot[r0 + i] = slot[r0 + i] << 16 | arrival[i];
     }
     __syncthreads();
     constexpr int kPer = kBkBins / kBkThreads;
@@ -280,15 +329,24 @@ __device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkIt
     __syncthreads();
     if (crowd > kBkCrowd) return false;
 #pragma unroll
-    for (int r = 0; r < kBkItems; ++r)
-        if (r < rounds && ((valid >> r) & 1u))
-            s.at(s.bin[slot[r] >> 16] + (slot[r] & 0xFFFFu)) = bk_pair(key[r], (uint32_t)bk_item(rounds, r));
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                // block-uniform
+        uint32_t to[kBkGroup];
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) to[i] = s.bin[slot[r0 + i] >> 16] + (slot[r0 + i] & 0xFFFFu);
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) {
+            const int r = r0 + i;
+            if (valid(r)) s.at(to[i]) = bk_pair(key[r], (uint32_t)bk_item(rounds, r));
+        }
+    }
+    if (threadIdx.x < kBkChunk) s.at(n + threadIdx.x) = bk_last();
     __syncthreads();
     const uint32_t p0 = threadIdx.x * kBkChunk;
     const bool busy = p0 < n;
     if (busy) {
 #pragma unroll
-        for (int e = 0; e < kBkChunk; ++e) v[e] = p0 + e < n ? s.at(p0 + e) : bk_last();
+        for (int e = 0; e < kBkChunk; ++e) v[e] = s.at(p0 + e);
         bk_merge<1>(v);
     }
     const bool next = p0 + kBkChunk < n;        // the thread above holds places too
@@ -438,7 +496,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
         BkPair v[kBkChunk];
         uint32_t m;
         // errors near 1 crowd in classes that the network misses: a quarter of the bins for the first 64th of the range
-        if (bk_sort(s, key, valid, kBkItems, BkBinning(least, least + (most - least) / 64u, most, 0.25f), m, v)) {
+        if (bk_sort(s, key, BkMask{valid}, kBkItems, BkBinning(least, least + (most - least) / 64u, most, 0.25f), m, v)) {
 #pragma unroll
             for (int e = 0; e < kBkChunk; ++e)
                 if (threadIdx.x * kBkChunk + e < n) sorted[threadIdx.x * kBkChunk + e] = bk_key_of(v[e]);
@@ -830,8 +888,11 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
 
 // One run of buckets (or, Direct: a whole row of at most kBkCap pixels, straight from the keys in pixel order, with the
 // Jaccard differences left in their place and the loss complete).
-// Time goes into vector instructions, 121 per 64 keys: a thread's places of the order are neighbours, so that a
-// difference is one new quotient less the one before, and the positives before a place are a sum over the block's threads.
+// Time goes into vector instructions, 118 per 64 keys (69 % of it at 16 waves per CU): a thread's places of the order are
+// neighbours, so that a difference is one new quotient less the one before, and the positives before a place are a sum over
+// the block's threads. The rounds of a group of three wait for LDS once where each waited by itself, and what tells a key's place
+// lies at constant offsets: with the quotients' fewer steps and scans by DPP 149 -> 118 instructions, (8,21,513,513) bf16 trained 270 -> 227 us,
+// (4,19,512,1024) fp32 134 -> 111.
 template <bool Direct>
 __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, float *__restrict__ losses) {
     __shared__ BkShared s;
@@ -846,6 +907,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
     const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
     const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
     const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
+    const BkSegments::Tile tile = Direct ? BkSegments::Tile() : BkSegments::Tile(a, c, b0, b1);
     if (!Direct && (n > kBkCap || n == 0)) {                // block-uniform; too many are bk_rank_wide's
         if (threadIdx.x == 0) {
             a.loss_part[2 * (int64_t)c * a.stride + g] = 0.0;
@@ -856,21 +918,36 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
     uint32_t *kin = a.keys + row;                           // the differences take the keys' places
     const uint32_t limit = bk_limit(a, c);
     float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
-    if constexpr (!Direct) at.collect(a, c, b0, b1, 0u, s.scan);
-    auto where = [&](int li) { return Direct ? (uint32_t)li : at.where((uint32_t)li); };
+    if constexpr (!Direct) at.collect(tile, 0u, s.scan);
 
     uint32_t key[kBkItems], valid = 0, least, most, knee = 0;
     float share = 0.25f;
     bool flat = false;                                      // block-uniform: one value, in order as it stands
     const int rounds = (n + kBkThreads - 1) / kBkThreads;
+    int first = bk_item(rounds, 0);
+    // the thread's items: first, first + 64, ... inside the wave's part
+    const int count = max(0, (min(n, first - (int)(threadIdx.x & 63) + rounds * kWave) - first + kWave - 1) / kWave);
 #pragma unroll
-    for (int r = 0; r < kBkItems; ++r) {
-        const int li = bk_item(rounds, r);
-        key[r] = 0;
-        if (r < rounds && li < n) {
-            key[r] = kin[where(li)];
-            if (!Direct || keep_key(key[r], limit)) valid |= 1u << r;
+    for (int r = 0; r < kBkItems; ++r) key[r] = 0;
+#pragma unroll
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                            // block-uniform
+        uint32_t from[kBkGroup];
+        if constexpr (!Direct) {
+            at.where((uint32_t)(first + r0 * kWave), (uint32_t)a.P - 1u, from);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kBkGroup; ++i) from[i] = (uint32_t)min(first + (r0 + i) * kWave, n - 1);
         }
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) key[r0 + i] = kin[from[i]];
+    }
+    if constexpr (Direct) {
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r)
+            if (r < count && keep_key(key[r], limit)) valid |= 1u << r;
+    } else {
+        valid = (1u << count) - 1u;
     }
     if constexpr (Direct) {
         bk_range(s, key, valid, least, most);
@@ -910,25 +987,31 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
 #pragma unroll
         for (int e = 0; e < kBkChunk; ++e) {
             const uint32_t p = threadIdx.x * kBkChunk + e;
-            if (p < kept) v[e] = s.at(p);
+            v[e] = p < kept ? s.at(p) : bk_last();
         }
         __syncthreads();
     } else {
-        in_order = bk_sort(s, key, valid, rounds, BkBinning(least, knee, most, share), kept, v);
+        const BkBinning bins(least, knee, most, share);
+        if constexpr (Direct) in_order = bk_sort(s, key, BkMask{valid}, rounds, bins, kept, v);
+        else in_order = bk_sort(s, key, BkFirst{count}, rounds, bins, kept, v);
     }
     if (in_order) {                                         // block-uniform
         const uint32_t p0 = threadIdx.x * kBkChunk;
         uint32_t hot = 0, all;
+        if (p0 < kept) {
 #pragma unroll
-        for (int e = 0; e < kBkChunk; ++e) hot += p0 + e < kept ? bk_hot_of(v[e]) : 0u;
-        uint32_t cs = hot0 + block_excl_scan(hot, s.scan, all);
+            for (int e = 0; e < kBkChunk; ++e) hot += bk_hot_of(v[e]);
+        }
+        const uint32_t cs = hot0 + block_excl_scan(hot, s.scan, all);
         const uint32_t pos = rank0 + p0;
-        float inter = npos - (float)cs;                                                // csrc/lovasz_softmax.cu:124-127
-        float j_prev = pos == 0 ? 0.f : 1.f - inter / (inter + (float)pos);
+        // whole numbers: the positives that are left, and those and the keys so far
+        float inter = npos - (float)cs, both = inter + (float)pos;                     // csrc/lovasz_softmax.cu:124-127
+        float j_prev = pos == 0 ? 0.f : 1.f - whole_ratio(inter, both);
         auto step = [&](int e) {
-            cs += bk_hot_of(v[e]);
-            inter = npos - (float)cs;
-            const float j_now = 1.f - inter / (inter + (float)(pos + 1u + e));
+            const float now = (float)bk_hot_of(v[e]);
+            inter -= now;
+            both = (both + 1.f) - now;
+            const float j_now = 1.f - whole_ratio(inter, both);
             const float dj = j_now - j_prev;                                           // csrc/lovasz_softmax.cu:141-147
             j_prev = j_now;
             part = add_loss(part, key_error(bk_key_of(v[e])), dj);
@@ -949,11 +1032,24 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
     part = wave_sum_f64(part);
     if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
     __syncthreads();
+    asm volatile("" : "+v"(first));                         // looked up again, not held across the sort
 #pragma unroll
-    for (int r = 0; r < kBkItems; ++r) {
-        int li = bk_item(rounds, r);
-        asm volatile("" : "+v"(li));                        // looked up again, not held across the sort
-        if (r < rounds && li < n) kin[where(li)] = __builtin_bit_cast(uint32_t, (!Direct || ((valid >> r) & 1u)) ? result[li] : 0.f);
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                            // block-uniform
+        uint32_t to[kBkGroup];
+        float dj[kBkGroup];
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) dj[i] = result[first + (r0 + i) * kWave];   // past the last: inside the pairs
+        if constexpr (!Direct) {
+            at.where((uint32_t)(first + r0 * kWave), (uint32_t)a.P - 1u, to);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kBkGroup; ++i) to[i] = (uint32_t)(first + (r0 + i) * kWave);
+        }
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i)
+            if (r0 + i < count)
+                kin[to[i]] = __builtin_bit_cast(uint32_t, (!Direct || ((valid >> (r0 + i)) & 1u)) ? dj[i] : 0.f);
     }
     if (threadIdx.x == 0) {
         double sum = 0.0;
@@ -987,8 +1083,12 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArg
         const int rounds = (n + kBkThreads - 1) / kBkThreads;
         uint32_t key[kBkItems], rank[kBkItems], valid = 0, hot = 0, least, most;
         __syncthreads();
-        if constexpr (!Direct) at.collect(a, c, b0, b1, 0u, s.scan);
-        auto where = [&](int li) { return Direct ? (uint32_t)li : at.where((uint32_t)li); };
+        if constexpr (!Direct) at.collect(BkSegments::Tile(a, c, b0, b1), 0u, s.scan);
+        auto where = [&](int li) {
+            uint32_t to[1] = {(uint32_t)li};
+            if constexpr (!Direct) at.where((uint32_t)li, (uint32_t)a.P - 1u, to);
+            return to[0];
+        };
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r) {
             const int li = bk_item(rounds, r);
@@ -1439,7 +1539,7 @@ constexpr int kBkWideBlocks = 32;               // per class: one wide bucket at
 // gives (a quotient from 1/2 on is one, and its difference from 1 is exact; one below leaves a difference from 1/2 on).
 __device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
     const float inter = npos - (float)cs;
-    return k == 0 ? 0.f : 1.f - inter / (inter + (float)k);
+    return k == 0 ? 0.f : 1.f - whole_ratio(inter, inter + (float)k);
 }
 
 // This block's part, every kBkWideBlocks-th tile, of bucket b with one value and n keys, from rank0 on with hot0 positives
@@ -1497,18 +1597,22 @@ __device__ __forceinline__ void bk_flat_keys(BkShared &s, const BucketArgs &a, i
 // The n keys of bucket b to a row of their own from rank0 on, or the differences found there back to their places.
 __device__ __forceinline__ void bk_wide_copy(BkShared &s, BkSegments &segments, const BucketArgs &a, int c, int b, uint32_t rank0, uint32_t n, bool back) {
     const int64_t row = (int64_t)c * a.P;
+    const BkSegments::Tile tile(a, c, (uint32_t)b, (uint32_t)b + 1u);
     for (uint32_t from = 0; from < n; from += kBkCap) {
         uint32_t v[kBkItems], at[kBkItems];
         __syncthreads();
-        segments.collect(a, c, (uint32_t)b, (uint32_t)b + 1u, from, s.scan);
+        segments.collect(tile, from, s.scan);
+#pragma unroll
+        for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+            uint32_t to[kBkGroup];
+            segments.where((uint32_t)bk_item(kBkItems, r0), (uint32_t)a.P - 1u, to, from);
+#pragma unroll
+            for (int i = 0; i < kBkGroup; ++i) at[r0 + i] = to[i];
+        }
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r) {
-            const uint32_t li = (uint32_t)bk_item(kBkItems, r);
-            at[r] = v[r] = 0;
-            if (from + li < n) {
-                at[r] = segments.where(li, from);
-                v[r] = back ? a.dj[row + rank0 + from + li] : a.keys[row + at[r]];
-            }
+            const uint32_t li = min((uint32_t)bk_item(kBkItems, r), n - from - 1u);
+            v[r] = back ? a.dj[row + rank0 + from + li] : a.keys[row + at[r]];
         }
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r) {
