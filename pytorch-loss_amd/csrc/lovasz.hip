@@ -63,25 +63,23 @@ __device__ __forceinline__ float key_error(uint32_t key) {
 // ------------------------------------------------------ 1. build keys ----
 
 // Besides the keys, both kernels leave per block and class the largest key among the block's
-// positives of that class, plus 1 (0 = none), in block_table[block][C]; lov_class_max folds the
+// positives of that class, plus 1 (0 = none), in block_table[C][block]; lov_class_max folds the
 // table into pos_max[c], the error of the class's lowest-ranked positive. Everything sorted after
 // that one has a Jaccard difference of exactly 0 (see keep_key), so the sort never sees it.
 __device__ __forceinline__ void publish_block_max(const uint32_t *block_max, uint32_t *block_table, int C) {
-    uint32_t *row = block_table + (int64_t)blockIdx.x * C;
-    for (int j = threadIdx.x; j < C; j += blockDim.x) row[j] = block_max[j];
+    for (int j = threadIdx.x; j < C; j += blockDim.x) block_table[(int64_t)j * gridDim.x + blockIdx.x] = block_max[j];
 }
 
 // It also leaves, per class, the number of key bits the sort has to look at: keys that take part are
 // not above the limit, so the bits above the limit's highest set bit are zero in every one of them.
-__global__ __launch_bounds__(1024) void lov_class_max(const uint32_t *__restrict__ block_table, int blocks, int C,
-                                                     uint32_t *__restrict__ pos_max, uint32_t *__restrict__ cursors,
-                                                     int regions) {
-    __shared__ uint32_t wave_max[16];
-    const int c = blockIdx.x;
-    // the class's staging cursors start at zero (they are first used by the last pass)
-    for (int i = threadIdx.x; i < regions; i += 1024) cursors[(int64_t)c * regions + i] = 0;
+// The body for the block of class c: kThreads threads, each with kThreads / 64 words of `wave_max`.
+template <int kThreads>
+__device__ __forceinline__ void class_max(const uint32_t *__restrict__ block_table, int blocks, int C, int c, uint32_t *__restrict__ pos_max,
+                                          uint32_t *wave_max) {
+    const uint32_t *row = block_table + (int64_t)c * blocks;
     uint32_t m = 0;
-    for (int b = threadIdx.x; b < blocks; b += 1024) m = max(m, block_table[(int64_t)b * C + c]);
+#pragma unroll 8
+    for (int b = threadIdx.x; b < blocks; b += kThreads) m = max(m, row[b]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
     if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
@@ -89,31 +87,50 @@ __global__ __launch_bounds__(1024) void lov_class_max(const uint32_t *__restrict
     if (threadIdx.x == 0) {
         uint32_t top = 0;
 #pragma unroll
-        for (int w = 0; w < 16; ++w) top = max(top, wave_max[w]);
+        for (int w = 0; w < kThreads / 64; ++w) top = max(top, wave_max[w]);
         pos_max[c] = top;
-        pos_max[2 * C + c] = 0xFFFFFFFFu;       // all_min[c], for lov_absent_min
+        pos_max[2 * C + c] = 0xFFFFFFFFu;       // all_min[c], for absent_min
         // key_bits[c]: a class without positives keeps a single key value, wherever it lies
         pos_max[3 * C + c] = (top > 1u) ? (uint32_t)(32 - __builtin_clz(top - 1u)) : (top ? 1u : 30u);
     }
 }
 
+__global__ __launch_bounds__(1024) void lov_class_max(const uint32_t *__restrict__ block_table, int blocks, int C,
+                                                     uint32_t *__restrict__ pos_max, uint32_t *__restrict__ cursors,
+                                                     int regions) {
+    __shared__ uint32_t wave_max[16];
+    const int c = blockIdx.x;
+    // the class's staging cursors start at zero (they are first used by the last pass)
+    for (int i = threadIdx.x; i < regions; i += 1024) cursors[(int64_t)c * regions + i] = 0;
+    class_max<1024>(block_table, blocks, C, c, pos_max, wave_max);
+}
+
 // A class without positives has J = 1 from the first sorted key on: only its largest error (smallest
 // key) has a non-zero Jaccard difference. For such classes (blocks of the others return at once)
-// this finds the smallest key of the row, which then serves as the class's limit.
+// this finds the smallest key of the row, which then serves as the class's limit. Block `block` of kAbsentBlocks.
 constexpr int kAbsentBlocks = 64;
-__global__ __launch_bounds__(256) void lov_absent_min(const uint32_t *__restrict__ keys, const uint32_t *pos_max,
-                                                      uint32_t *all_min, int P) {
-    __shared__ uint32_t wave_min[4];
-    const int c = blockIdx.y;
+template <int kThreads>
+__device__ __forceinline__ void absent_min(const uint32_t *__restrict__ keys, const uint32_t *pos_max, uint32_t *all_min, int P,
+                                           int c, int block, uint32_t *wave_min) {
     if (pos_max[c] != 0) return;                // block-uniform
     const uint32_t *row = keys + (int64_t)c * P;
     uint32_t m = 0xFFFFFFFFu;
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < P; i += kAbsentBlocks * 256) m = min(m, row[i] & 0x7FFFFFFFu);
+#pragma unroll 8
+    for (int i = block * kThreads + threadIdx.x; i < P; i += kAbsentBlocks * kThreads) m = min(m, row[i] & 0x7FFFFFFFu);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = min(m, (uint32_t)__shfl_xor((int)m, off, 64));
     if ((threadIdx.x & 63) == 0) wave_min[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) atomicMin(all_min + c, min(min(wave_min[0], wave_min[1]), min(wave_min[2], wave_min[3])));
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < kThreads / 64; ++w) m = min(m, wave_min[w]);
+        atomicMin(all_min + c, m);
+    }
+}
+__global__ __launch_bounds__(256) void lov_absent_min(const uint32_t *__restrict__ keys, const uint32_t *pos_max,
+                                                      uint32_t *all_min, int P) {
+    __shared__ uint32_t wave_min[4];
+    absent_min<256>(keys, pos_max, all_min, P, (int)blockIdx.y, (int)blockIdx.x, wave_min);
 }
 
 template <class T, int CP, int V>
@@ -279,9 +296,12 @@ __device__ __forceinline__ int row_items(const SortArgs &a, int c) { return a.ke
 // one sector) and the sectors in which one tile's run of a digit ends and the next tile's begins.
 // Only the tiles that hold keys are permuted (the rest of a pruned row exits at once, and would
 // leave the XCDs of the last chunks idle).
-__device__ __forceinline__ int sort_tile(int items, int tile_keys = kSortTile) {
-    const int x = blockIdx.x, q = ((items + tile_keys - 1) / tile_keys) >> 3;
+__device__ __forceinline__ int xcd_chunk(int x, int n) {
+    const int q = n >> 3;
     return x < 8 * q ? (x & 7) * q + (x >> 3) : x;
+}
+__device__ __forceinline__ int sort_tile(int items, int tile_keys = kSortTile) {
+    return xcd_chunk((int)blockIdx.x, (items + tile_keys - 1) / tile_keys);
 }
 
 // Inclusive scan over the 64 lanes of a wave, all of them active: inside the rows of 16 lanes, then the last lane of a row to the
@@ -1162,7 +1182,7 @@ struct LovaszPlan {
     bool buckets;
     int bk_tiles, bk_bits;
     int64_t off_sorted, off_dj, off_tile_start, off_start, off_count, off_bounds, off_buckets, off_fine, off_loss_part,
-        off_crowded, off_place;
+        off_place;
     int hist_blocks;
     int64_t off_lb_clear, lb_clear_bytes, off_lb_totals, off_lb_partial;
 };
@@ -1208,16 +1228,15 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
         const int64_t most = ceil_div(pl.P, kBkTarget);
         pl.bk_bits = pl.P <= kBkCap ? 0 : (most <= 64 ? 6 : (most <= 256 ? 8 : 10));
         const int64_t cells = dimsize << pl.bk_bits;
-        pl.off_crowded = off;        off += round_up(4 * cells, 256);
         // one layout for every row length, also where one block ranks the row
         pl.off_sorted = off;     off += round_up(4 * pl.E, 256);
         pl.off_dj = off;         off += round_up(4 * pl.E, 256);
         pl.off_place = off;      off += round_up(2 * pl.E, 256);
         pl.off_tile_start = off; off += round_up(4 * (cells + dimsize) * pl.bk_tiles, 256);
         pl.off_start = off;      off += round_up(4 * (cells + dimsize) * pl.bk_tiles, 256);
-        pl.off_count = off;      off += 4 * round_up(4 * (cells + dimsize), 256);     // count, base, hot_base, runs
+        pl.off_count = off;      off += 5 * round_up(4 * (cells + dimsize), 256);     // large, base, hot_base, runs, crowded
         pl.off_bounds = off;     off += round_up(4 * cells, 256);
-        pl.off_buckets = off;    off += round_up(4 * 6 * dimsize, 256);
+        pl.off_buckets = off;    off += round_up(4 * 9 * dimsize, 256);
         pl.off_fine = off;       off += round_up(2 * dimsize * kBkFine, 256);
         pl.off_loss_part = off;  off += round_up(2 * 8 * cells, 256);
         pl.bytes = off;
@@ -1269,20 +1288,25 @@ extern "C" int64_t plh_lovasz_lookback_workspace_bytes(int64_t n_size, int64_t d
     return rc == PLH_OK ? pl.bytes : (int64_t)rc;
 }
 
-// 2. and 3. by value buckets: ranks of the keys in keys_0 (jacc's memory), which becomes the Jaccard differences.
-static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, const uint32_t *pos_max, float *losses, int C,
-                          hipStream_t st) {
+// 2. and 3. for rows that one block ranks whole: the keys in keys_0 (jacc's memory) become the Jaccard differences.
+static int lovasz_blocks(const LovaszPlan &pl, uint32_t *keys_0, uint32_t *pos_max, float *losses, int C, hipStream_t st) {
     BucketArgs a = {};
     a.keys = keys_0;
     a.pos_max = pos_max;
     a.P = (int)pl.P;
     a.C = C;
-    a.crowded = reinterpret_cast<uint32_t *>(ws + pl.off_crowded);
-    if (pl.bk_bits == 0) {
-        hipLaunchKernelGGL(bk_rank<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);
-        hipLaunchKernelGGL(bk_rank_crowded<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);
-        return check_launch();
-    }
+    hipLaunchKernelGGL(bk_rank<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);
+    return check_launch();
+}
+
+// The same by value buckets, and the classes' limits (pos_max) before them.
+static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, uint32_t *pos_max, const uint32_t *block_table,
+                          int key_blocks, float *losses, int C, hipStream_t st) {
+    BucketArgs a = {};
+    a.keys = keys_0;
+    a.pos_max = pos_max;
+    a.P = (int)pl.P;
+    a.C = C;
     a.tiles = pl.bk_tiles;
     a.stride = 1 << pl.bk_bits;
     const int64_t step = round_up(4 * (((int64_t)C << pl.bk_bits) + C), 256);
@@ -1291,7 +1315,8 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
     a.place = reinterpret_cast<uint16_t *>(ws + pl.off_place);
     a.tile_start = reinterpret_cast<uint32_t *>(ws + pl.off_tile_start);
     a.start = reinterpret_cast<uint32_t *>(ws + pl.off_start);
-    a.count = reinterpret_cast<uint32_t *>(ws + pl.off_count);
+    a.large = reinterpret_cast<uint32_t *>(ws + pl.off_count);
+    a.crowded = reinterpret_cast<uint32_t *>(ws + pl.off_count + 4 * step);
     a.base = reinterpret_cast<uint32_t *>(ws + pl.off_count + step);
     a.hot_base = reinterpret_cast<uint32_t *>(ws + pl.off_count + 2 * step);
     a.runs = reinterpret_cast<uint32_t *>(ws + pl.off_count + 3 * step);
@@ -1301,9 +1326,10 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
     a.loss_part = reinterpret_cast<double *>(ws + pl.off_loss_part);
     const dim3 tiles((unsigned)pl.bk_tiles, (unsigned)C), threads(kBkThreads);
     const unsigned most = (unsigned)ceil_div(pl.P, kBkTarget) + 1;  // buckets a class can have
-    // two blocks fit a CU; each looks at every so many of the class's runs
-    const unsigned crowded_blocks = (unsigned)(ceil_div(2048, C) < most ? ceil_div(2048, C) : most);
-    hipLaunchKernelGGL(bk_split, dim3((unsigned)C), threads, 0, st, a);
+    // two blocks fit a CU; each takes every so many of the class's crowded runs
+    const unsigned crowded_blocks = (unsigned)(ceil_div(1024, C) < most ? ceil_div(1024, C) : most);
+    hipLaunchKernelGGL(bk_sample, dim3(1 + kBkItems, (unsigned)C), threads, 0, st, a, block_table, key_blocks);
+    hipLaunchKernelGGL(bk_split, dim3((1 + kAbsentBlocks) * (unsigned)C), threads, 0, st, a);
     switch (pl.bk_bits) {
 #define PLH_BUCKETS(B)                                                                                               \
     case B:                                                                                                          \
@@ -1311,8 +1337,7 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, cons
         hipLaunchKernelGGL(bk_sum, dim3((unsigned)ceil_div(most + 1, 64), (unsigned)C), dim3(1024), 0, st, a);       \
         hipLaunchKernelGGL(bk_group, dim3((unsigned)C), threads, 0, st, a);                                          \
         hipLaunchKernelGGL(bk_rank<false>, dim3(most, (unsigned)C), threads, 0, st, a, losses);                      \
-        hipLaunchKernelGGL(bk_rank_crowded<false>, dim3(crowded_blocks, (unsigned)C), threads, 0, st, a, losses);    \
-        hipLaunchKernelGGL(bk_rank_wide, dim3(kBkWideBlocks, (unsigned)C), threads, 0, st, a);                       \
+        hipLaunchKernelGGL(bk_rank_rest, dim3(kBkWideBlocks + crowded_blocks, (unsigned)C), threads, 0, st, a);      \
         hipLaunchKernelGGL(bk_restore, tiles, threads, 0, st, a, losses);                                            \
         break;
         PLH_BUCKETS(6) PLH_BUCKETS(8) PLH_BUCKETS(10)
@@ -1374,13 +1399,14 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
                                pl.P, m_size, C, ignore_index);
         }
     });
+    if (pl.buckets && pl.bk_bits) return lovasz_buckets(pl, ws, keys_0, pos_max, block_table, (int)key_blocks, losses, C, st);
     uint32_t *cursors = pl.regions > 0 ? reinterpret_cast<uint32_t *>(ws + pl.off_cursors) : nullptr;
     hipLaunchKernelGGL(lov_class_max, dim3((unsigned)C), dim3(1024), 0, st, block_table, (int)key_blocks, C, pos_max, cursors,
                        pl.regions);
     hipLaunchKernelGGL(lov_absent_min, dim3(kAbsentBlocks, (unsigned)C), dim3(256), 0, st, keys_0, pos_max, all_min,
                        (int)pl.P);
 
-    if (pl.buckets) return lovasz_buckets(pl, ws, keys_0, pos_max, losses, C, st);
+    if (pl.buckets) return lovasz_blocks(pl, keys_0, pos_max, losses, C, st);
 
     // what the plan lays out for the radix passes only
     uint32_t *keys_a = reinterpret_cast<uint32_t *>(ws + pl.off_keys_a);

@@ -3,22 +3,22 @@
 // A radix sort moves every (key, pixel) pair three times before its rank is known. Here a key moves inside its tile only: the
 // class row is cut into buckets of neighbouring key values, every tile is put in the order of the buckets, and what lies in a
 // few neighbouring buckets, a segment of every tile, is sorted in a block's LDS.
-//   bk_split      a block per class sorts a sample of the row's keys; every n-th of them starts a bucket
+//   bk_sample     the classes' limits, and a sample of their keys
+//   bk_split      a block per class sorts the sample; every n-th key of it starts a bucket
 //   bk_cut        every tile's keys in the order of their buckets, in pixel order inside one (stable ranks), in the keys' place
 //   bk_sum        the tiles' counts by bucket: where every bucket starts in the row
 //   bk_group      runs of buckets that a block can sort at once
 //   bk_rank       a block per run of buckets: its segments sorted in LDS, Jaccard difference of every key in its place
-//   bk_rank_crowded  the same for runs whose values crowd
-//   bk_rank_wide  the same for buckets that outgrew the LDS, and for single values that fill more than that
-//   bk_restore    Jaccard differences back to pixel order, tile by tile
+//   bk_rank_rest  the same for runs whose values crowd, and for buckets that outgrew the LDS (wide)
+//   bk_restore    Jaccard differences back to pixel order, tile by tile, with those of single values that fill more than a block
 // Sampled bounds follow any distribution; a value that fills several buckets by itself gets one of its own, which
 // needs no sort (flat: its keys are ranked as they stand), and a bucket that outgrew the LDS all the same is cut into value
 // ranges that fit.
 // A key moves 28 bytes: read and written by bk_cut, bk_rank and bk_restore, and a place of 2 bytes. The form before this one
 // wrote the buckets out one after the other: that takes a histogram first (6 bytes a key more, buckets kept for the second
 // pass) and writes of some 10 keys, where a segment of a run has 24 here. (4,19,512,1024) fp32: histogram and scatter
-// 67 + 117 us against 102 now, rank 119 against 111, gather 72 against 57, step 585 -> 487 us; (8,21,513,513) bf16 trained
-// 77 + 154 against 137, 217 against 227, 116 against 68, step 794 -> 642. Which rows come here: bk_pays.
+// 67 + 117 us against 102 now, rank 119 against 111, gather 72 against 57, step 557 -> 436 us; (8,21,513,513) bf16 trained
+// 77 + 154 against 137, 217 against 227, 116 against 68, step 795 -> 614. Which rows come here: bk_pays.
 #pragma once
 
 namespace plh {
@@ -38,27 +38,27 @@ constexpr int kBkSlab = 6144;                       // buckets that start in one
 constexpr int kBkMax = 1024;                        // buckets per class
 constexpr int64_t kBkMaxRow = (int64_t)kBkTarget * kBkMax;
 constexpr uint32_t kBkCrowd = 257;                  // keys in one bin up to which merges between chunks put them in order: 97 left
-                                                    // lumps of bf16 logits to bk_rank_crowded (227 + 37 -> 231 + 9 us)
-constexpr uint32_t kBkFlat = 0x80000000u;
+                                                    // lumps of bf16 logits to the crowded path (227 + 37 -> 231 + 9 us)
 constexpr uint16_t kBkNowhere = 0xFFFFu;            // place of a pixel that takes no part
 
 struct BucketArgs {
     uint32_t *keys;             // [C][P] in pixel order; bk_cut leaves every tile's keys by bucket, the rank kernels a key's Jaccard
                                 // difference in its place, bk_restore those in pixel order (jacc's memory)
-    const uint32_t *pos_max;    // pos_max[C], kept[C], all_min[C], key_bits[C] (see keep_key, lov_class_max)
+    uint32_t *pos_max;          // pos_max[C], kept[C], all_min[C], key_bits[C] (see keep_key, lov_class_max)
     uint16_t *place;            // [C][P] every pixel's place in its tile's order
-    uint32_t *sorted, *dj;      // [C][P] keys and differences of the buckets that bk_rank_wide ranks
+    uint32_t *sorted, *dj;      // [C][P] keys and differences of the wide buckets; in dj's memory first the
+                                // sample, [C][kBkCap]
     uint32_t *tile_start;       // [C][tiles][stride + 1] in the tile's order: keys | positives << 16 before the bucket
     uint32_t *start;            // [C][stride + 1][tiles] the same
-    uint32_t *count;            // [C][stride] keys per bucket (kBkFlat: and a single value)
     uint32_t *base, *hot_base;  // [C][stride + 1] keys and positives before the bucket
     uint32_t *bounds;           // [C][stride] least key of buckets 1, 2, ...
     uint32_t *runs;             // [C][stride + 1] first bucket of every run, and the end
-    uint32_t *crowded;          // [C][stride] runs (rows of one block: [C]) whose values crowd
-    uint32_t *numbers;          // [6][C]: buckets, runs, positives, least key of the sample, largest one below the limit,
-                                // first step of the search in `bounds`
+    uint32_t *large;            // [C][stride] buckets of more keys than kBkCap: the wide ones, then the flat ones
+    uint32_t *crowded;          // [C][stride] runs whose values crowd, in any order
+    uint32_t *numbers;          // [9][C]: buckets, runs, positives, least key of the sample, largest one below the limit,
+                                // first step of the search in `bounds`, wide buckets, flat buckets, crowded runs
     uint16_t *fine;             // [C][kBkFine] bucket of the least key with these top bits
-    double *loss_part;          // [C][2 * stride]: runs, wide and flat buckets
+    double *loss_part;          // [C][2 * stride]: runs, from `stride` on large buckets
     int P, C, tiles, stride;
 };
 
@@ -92,6 +92,13 @@ __device__ __forceinline__ float whole_ratio(float a, float b) {
     return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
 }
 static_assert(kBkMaxRow < 1 << 22, "2b < 2^23");
+
+// Jaccard index of a class's first k keys, cs of its npos positives among them: a multiple of 2^-24, whatever the division
+// gives (a quotient from 1/2 on is one, and its difference from 1 is exact; one below leaves a difference from 1/2 on).
+__device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
+    const float inter = npos - (float)cs;
+    return k == 0 ? 0.f : 1.f - whole_ratio(inter, inter + (float)k);
+}
 
 // Jaccard difference of the key at rank `pos`, with `cs` of the class's npos positives before it.
 __device__ __forceinline__ float jaccard_step(float npos, uint32_t pos, uint32_t cs, uint32_t hot) {
@@ -465,25 +472,40 @@ __device__ __forceinline__ void bk_ranks_crowded(BkShared &s, const uint32_t (&k
     __syncthreads();
 }
 
-// Bounds of a class's buckets from kBkCap sampled keys, one from each of as many equal parts of the row: every
-// (sample / buckets)-th key in their order. A value that would bound two buckets gets one to itself: (v, v + 1).
+// A class's limit, and kBkCap sampled keys, one from each of as many equal parts of the row. The sample lies anywhere in memory:
+// by 15 blocks beside the one for the limit 3 us, by the one that sorts it 10.
+__global__ __launch_bounds__(kBkThreads) void bk_sample(const BucketArgs a, const uint32_t *__restrict__ block_table, int key_blocks) {
+    __shared__ uint32_t wave_max[kBkWaves];
+    const int c = blockIdx.y;
+    if (blockIdx.x == 0) {                                  // block-uniform
+        class_max<kBkThreads>(block_table, key_blocks, a.C, c, a.pos_max, wave_max);
+        return;
+    }
+    const uint32_t part = (uint32_t)a.P / kBkCap;           // >= 1: shorter rows are not cut
+    const uint32_t i = (blockIdx.x - 1u) * kBkThreads + threadIdx.x;
+    uint32_t h = i * 0x9E3779B1u;                           // somewhere in the part, so that no stride meets the image's
+    h = (h ^ (h >> 15)) * 0x85EBCA6Bu;
+    a.dj[(int64_t)c * kBkCap + i] = a.keys[(int64_t)c * a.P + (uint32_t)((uint64_t)i * (uint32_t)a.P / kBkCap) + __umulhi(h, part)];
+}
+
+// Bounds of a class's buckets from the sample: every (sample / buckets)-th key in its order. A value that would bound two
+// buckets gets one to itself: (v, v + 1). A class without positives, whose keys that take part are equal, has one bucket; the
+// blocks behind the first C look for their value.
 __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
     __shared__ BkShared s;
-    const int c = blockIdx.x;
-    const uint32_t limit = bk_limit(a, c);
-    const uint32_t *row = a.keys + (int64_t)c * a.P;
-    uint32_t key[kBkItems], valid = 0, mine = 0;
-    const uint32_t part = (uint32_t)a.P / kBkCap;           // >= 1: shorter rows are not cut
-#pragma unroll
-    for (int r = 0; r < kBkItems; ++r) {
-        const uint32_t i = (uint32_t)bk_item(kBkItems, r);
-        uint32_t h = i * 0x9E3779B1u;                       // somewhere in the part, so that no stride meets the image's
-        h = (h ^ (h >> 15)) * 0x85EBCA6Bu;
-        key[r] = row[(uint32_t)((uint64_t)i * (uint32_t)a.P / kBkCap) + __umulhi(h, part)];
+    const int c = (int)blockIdx.x % a.C, turn = (int)blockIdx.x / a.C;
+    if (turn > 0) {                                         // block-uniform
+        absent_min<kBkThreads>(a.keys, a.pos_max, a.pos_max + 2 * a.C, a.P, c, turn - 1, s.least);
+        return;
     }
+    const bool absent = a.pos_max[c] == 0u;
+    const uint32_t limit = a.pos_max[c] - 1u;               // not for an absent class
+    uint32_t key[kBkItems], valid = 0, mine = 0;
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) key[r] = a.dj[(int64_t)c * kBkCap + bk_item(kBkItems, r)];
 #pragma unroll
     for (int r = 0; r < kBkItems; ++r)
-        if (keep_key(key[r], limit)) {
+        if (!absent && keep_key(key[r], limit)) {
             valid |= 1u << r;
             ++mine;
         }
@@ -543,36 +565,35 @@ __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
         __syncthreads();
     }
     for (uint32_t i = threadIdx.x; i < bounds; i += kBkThreads) a.bounds[(int64_t)c * a.stride + i] = s.bin[i];
+    for (uint32_t i = threadIdx.x; i < n; i += kBkThreads)  // the last one below the limit
+        if (sorted[i] < limit && (i + 1u == n || sorted[i + 1u] >= limit)) a.numbers[4 * a.C + c] = sorted[i];
     if (threadIdx.x == 0) {
         a.numbers[c] = bounds + 1u;
         a.numbers[3 * a.C + c] = n ? least : 0u;
-        uint32_t lo = 0, hi = n;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (sorted[mid] < limit) lo = mid + 1;
-            else hi = mid;
-        }
-        a.numbers[4 * a.C + c] = lo ? sorted[lo - 1] : 0u;
+        if (n == 0u || sorted[0] >= limit) a.numbers[4 * a.C + c] = 0u;
     }
+    __syncthreads();                                        // the sample is done with: the cells of the top bits take its place
     // the bucket of the least key with each pattern of the top bits, and the most bounds that one pattern's keys can lie between
     const int bits = (int)a.pos_max[3 * a.C + c], shift = bits > kBkFineBits ? bits - kBkFineBits : 0;
     constexpr int kPerFine = kBkFine / kBkThreads;
-    uint32_t at_fine[kPerFine + 1], width = 0;
-#pragma unroll
-    for (int u = 0; u <= kPerFine; ++u) {
-        const uint32_t k = (threadIdx.x * kPerFine + u) << shift;
-        uint32_t lo = 0, hi = bounds;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s.bin[mid] <= k) lo = mid + 1;
-            else hi = mid;
-        }
-        at_fine[u] = lo;
-    }
+    uint32_t *above = s.key();                              // [kBkFine + 1] bounds above the least key of the pattern before
+    for (int f = threadIdx.x; f <= kBkFine; f += kBkThreads) above[f] = 0;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < bounds; i += kBkThreads)
+        atomicAdd(&above[min((s.bin[i] + (1u << shift) - 1u) >> shift, (uint32_t)kBkFine)], 1u);
+    __syncthreads();
+    uint32_t here[kPerFine], sum = 0, width = 0, all;
 #pragma unroll
     for (int u = 0; u < kPerFine; ++u) {
-        a.fine[(int64_t)c * kBkFine + threadIdx.x * kPerFine + u] = (uint16_t)at_fine[u];
-        width = max(width, at_fine[u + 1] - at_fine[u]);
+        here[u] = above[threadIdx.x * kPerFine + u];
+        sum += here[u];
+        width = max(width, above[threadIdx.x * kPerFine + u + 1]);
+    }
+    uint32_t bucket = block_excl_scan(sum, s.scan, all);
+#pragma unroll
+    for (int u = 0; u < kPerFine; ++u) {
+        bucket += here[u];
+        a.fine[(int64_t)c * kBkFine + threadIdx.x * kPerFine + u] = (uint16_t)bucket;
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) width = max(width, (uint32_t)__shfl_xor((int)width, off, 64));
@@ -791,7 +812,8 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_cut(const BucketArgs a) {
 }
 
 // Keys and positives before each bucket in the row: the sums of the tiles', which are left by bucket for the rank kernels.
-// 64 buckets x 64 tiles at a time.
+// 64 buckets x 64 tiles at a time, the next ones' loads under way. (With the work of bk_group done by the last block of a class,
+// which has to see what the others wrote, 37 us instead of 7 + 5: every block's fence writes its L2 back.)
 __global__ __launch_bounds__(1024) void bk_sum(const BucketArgs a) {
     __shared__ uint32_t part[64][65];
     __shared__ uint32_t sums[16][64], hots[16][64];
@@ -801,23 +823,25 @@ __global__ __launch_bounds__(1024) void bk_sum(const BucketArgs a) {
     const int pitch = a.stride + 1;
     const uint32_t *in = a.tile_start + (int64_t)c * a.tiles * pitch;
     uint32_t *out = a.start + (int64_t)c * pitch * a.tiles;
-    uint32_t n = 0, h = 0, v[4];
-    auto fetch = [&](int t0) {
+    uint32_t n = 0, h = 0, v[2][4];
+    auto fetch = [&](uint32_t (&to)[4], int t0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int t = t0 + i * 16 + group;
-            v[i] = t < a.tiles && first + lane < entries ? in[(int64_t)t * pitch + first + lane] : 0u;
+            to[i] = t < a.tiles && first + lane < entries ? in[(int64_t)t * pitch + first + lane] : 0u;
         }
     };
-    fetch(0);
+    fetch(v[0], 0);
+    fetch(v[1], 64);
     for (int t0 = 0; t0 < a.tiles; t0 += 64) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            n += v[i] & 0xFFFFu;
-            h += v[i] >> 16;
-            part[i * 16 + group][lane] = v[i];
+            n += v[0][i] & 0xFFFFu;
+            h += v[0][i] >> 16;
+            part[i * 16 + group][lane] = v[0][i];
+            v[0][i] = v[1][i];
         }
-        if (t0 + 64 < a.tiles) fetch(t0 + 64);
+        fetch(v[1], t0 + 128);
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -840,12 +864,13 @@ __global__ __launch_bounds__(1024) void bk_sum(const BucketArgs a) {
     a.hot_base[(int64_t)c * pitch + first + lane] = hot;
 }
 
-// Where the buckets start, and the runs of them that one block sorts: neighbours that start in the same kBkSlab keys of the
-// row, unless they come to more than kBkCap, or lie so differently dense that bins of one width would not do.
+// The runs of buckets that one block sorts: neighbours that start in the same kBkSlab keys of the row, unless they come to
+// more than kBkCap, or lie so differently dense that bins of one width would not do.
 __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
     __shared__ uint32_t base[kBkMax + 1], bound[kBkMax + 1], scan_tmp[2 * kSortWaves];
     constexpr int kPer = kBkMax / kBkThreads;
     const int c = blockIdx.x, buckets = (int)a.numbers[c], b0 = threadIdx.x * kPer;
+    const bool absent = a.pos_max[c] == 0u;                 // one bucket of one value
     const int64_t row = (int64_t)c * (a.stride + 1);
     for (int b = threadIdx.x; b <= buckets; b += kBkThreads) {
         base[b] = a.base[row + b];
@@ -855,14 +880,13 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
     const uint32_t least = a.numbers[3 * a.C + c];
     auto width = [&](int b) { return (float)(bound[b] - (b ? bound[b - 1] : min(least, bound[0]))) / (float)(base[b + 1] - base[b] + 1u); };
     bool start[kPer];
-    uint32_t starts = 0;
+    uint32_t starts = 0, wide = 0, flat = 0;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
         const int b = b0 + i;
         start[i] = false;
         if (b >= buckets) continue;
-        const uint32_t n = base[b + 1] - base[b];
-        a.count[(int64_t)c * a.stride + b] = n > (uint32_t)kBkCap && b && bound[b] - bound[b - 1] == 1u ? n | kBkFlat : n;
+        if (base[b + 1] - base[b] > (uint32_t)kBkCap) ((absent || (b && bound[b] - bound[b - 1] == 1u)) ? flat : wide) |= 1u << i;
         const uint32_t slab = base[b] / kBkSlab;
         start[i] = b == 0 || base[b - 1] / kBkSlab != slab;
         if (!start[i]) {
@@ -879,258 +903,26 @@ __global__ __launch_bounds__(kBkThreads) void bk_group(const BucketArgs a) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
         if (start[i]) a.runs[row + k++] = (uint32_t)(b0 + i);
+    uint32_t w, f, wides, flats;
+    block_excl_scan2((uint32_t)__builtin_popcount(wide), (uint32_t)__builtin_popcount(flat), scan_tmp, w, wides, f, flats);
+    const float npos = (float)a.hot_base[row + buckets];
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int b = b0 + i;
+        if ((wide >> i) & 1u) a.large[(int64_t)c * a.stride + w++] = (uint32_t)b;
+        if (!((flat >> i) & 1u)) continue;
+        // one error, and the differences, exact as multiples of 2^-24, add up to that of the ends
+        const float rise = jaccard(npos, base[b + 1], a.hot_base[row + b + 1]) - jaccard(npos, base[b], a.hot_base[row + b]);
+        a.large[(int64_t)c * a.stride + wides + f] = (uint32_t)b;
+        a.loss_part[(2 * (int64_t)c + 1) * a.stride + wides + f++] = add_loss(0.0, key_error(bound[b] - 1u), rise);
+    }
     if (threadIdx.x == 0) {
+        a.numbers[6 * a.C + c] = wides;
+        a.numbers[7 * a.C + c] = flats;
+        a.numbers[8 * a.C + c] = 0;
         a.runs[row + runs] = (uint32_t)buckets;
         a.numbers[a.C + c] = runs;
         a.numbers[2 * a.C + c] = a.hot_base[row + buckets];
-    }
-}
-
-// One run of buckets (or, Direct: a whole row of at most kBkCap pixels, straight from the keys in pixel order, with the
-// Jaccard differences left in their place and the loss complete).
-// Time goes into vector instructions, 118 per 64 keys (69 % of it at 16 waves per CU): a thread's places of the order are
-// neighbours, so that a difference is one new quotient less the one before, and the positives before a place are a sum over
-// the block's threads. The rounds of a group of three wait for LDS once where each waited by itself, and what tells a key's place
-// lies at constant offsets: with the quotients' fewer steps and scans by DPP 149 -> 118 instructions, (8,21,513,513) bf16 trained 270 -> 227 us,
-// (4,19,512,1024) fp32 134 -> 111.
-template <bool Direct>
-__global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, float *__restrict__ losses) {
-    __shared__ BkShared s;
-    __shared__ BkSegments at;                               // not for a whole row
-    __shared__ double wave_loss[kBkWaves];
-    const int c = Direct ? blockIdx.x : blockIdx.y;
-    const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
-    const int runs = Direct ? 1 : (int)a.numbers[a.C + c];
-    if (!Direct && (int)blockIdx.x >= runs) return;         // block-uniform
-    // neighbouring runs on one XCD: a tile's segments of theirs share cache lines
-    const int g = Direct ? 0 : sort_tile(runs, 1);
-    const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
-    const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
-    const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
-    const BkSegments::Tile tile = Direct ? BkSegments::Tile() : BkSegments::Tile(a, c, b0, b1);
-    if (!Direct && (n > kBkCap || n == 0)) {                // block-uniform; too many are bk_rank_wide's
-        if (threadIdx.x == 0) {
-            a.loss_part[2 * (int64_t)c * a.stride + g] = 0.0;
-            a.crowded[(int64_t)c * a.stride + g] = 0u;
-        }
-        return;
-    }
-    uint32_t *kin = a.keys + row;                           // the differences take the keys' places
-    const uint32_t limit = bk_limit(a, c);
-    float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
-    if constexpr (!Direct) at.collect(tile, 0u, s.scan);
-
-    uint32_t key[kBkItems], valid = 0, least, most, knee = 0;
-    float share = 0.25f;
-    bool flat = false;                                      // block-uniform: one value, in order as it stands
-    const int rounds = (n + kBkThreads - 1) / kBkThreads;
-    int first = bk_item(rounds, 0);
-    // the thread's items: first, first + 64, ... inside the wave's part
-    const int count = max(0, (min(n, first - (int)(threadIdx.x & 63) + rounds * kWave) - first + kWave - 1) / kWave);
-#pragma unroll
-    for (int r = 0; r < kBkItems; ++r) key[r] = 0;
-#pragma unroll
-    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
-        if (r0 >= rounds) break;                            // block-uniform
-        uint32_t from[kBkGroup];
-        if constexpr (!Direct) {
-            at.where((uint32_t)(first + r0 * kWave), (uint32_t)a.P - 1u, from);
-        } else {
-#pragma unroll
-            for (int i = 0; i < kBkGroup; ++i) from[i] = (uint32_t)min(first + (r0 + i) * kWave, n - 1);
-        }
-#pragma unroll
-        for (int i = 0; i < kBkGroup; ++i) key[r0 + i] = kin[from[i]];
-    }
-    if constexpr (Direct) {
-#pragma unroll
-        for (int r = 0; r < kBkItems; ++r)
-            if (r < count && keep_key(key[r], limit)) valid |= 1u << r;
-    } else {
-        valid = (1u << count) - 1u;
-    }
-    if constexpr (Direct) {
-        bk_range(s, key, valid, least, most);
-        uint32_t hot = 0, all;
-#pragma unroll
-        for (int r = 0; r < kBkItems; ++r) hot += ((valid >> r) & 1u) ? key[r] >> 31 : 0u;
-        block_excl_scan(hot, s.scan, all);
-        npos = (float)all;
-        most = max(least, most);                            // no valid key: nothing below looks at the range
-    } else {
-        const uint32_t *bound = a.bounds + (int64_t)c * a.stride;
-        const uint32_t buckets = a.numbers[c];
-        most = b1 < buckets ? bound[b1 - 1] - 1u : limit;
-        least = b0 ? bound[b0 - 1] : 0u;
-        flat = least == most;
-        if (!flat && (b0 == 0 || b1 + 1u >= buckets)) {
-            // beyond the sample lie a few more, far apart: their own bins
-            bk_range(s, key, valid, least, most);
-            knee = b0 ? a.numbers[4 * a.C + c] + 1u : a.numbers[3 * a.C + c];
-            // Nor do the first keys lie evenly: errors near 1 crowd in classes that the network misses, as in bk_split. A
-            // knee right at the first key left 260 keys in one bin ((1,32,256,256), soft: bk_rank and bk_rank_crowded 34 + 36 -> 19 + 4 us).
-            if (!b0) knee = max(knee, least + (most - least) / 64u);
-            share = b0 ? 0.75f : 0.25f;
-        }
-    }
-    double part = 0.0;
-    BkPair v[kBkChunk];
-    uint32_t kept;
-    float *result = reinterpret_cast<float *>(s.pair);      // by item
-    bool in_order = flat;
-    if (flat) {
-        kept = (uint32_t)n;
-#pragma unroll
-        for (int r = 0; r < kBkItems; ++r)
-            if ((valid >> r) & 1u) s.at((uint32_t)bk_item(rounds, r)) = bk_pair(key[r], (uint32_t)bk_item(rounds, r));
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < kBkChunk; ++e) {
-            const uint32_t p = threadIdx.x * kBkChunk + e;
-            v[e] = p < kept ? s.at(p) : bk_last();
-        }
-        __syncthreads();
-    } else {
-        const BkBinning bins(least, knee, most, share);
-        if constexpr (Direct) in_order = bk_sort(s, key, BkMask{valid}, rounds, bins, kept, v);
-        else in_order = bk_sort(s, key, BkFirst{count}, rounds, bins, kept, v);
-    }
-    if (in_order) {                                         // block-uniform
-        const uint32_t p0 = threadIdx.x * kBkChunk;
-        uint32_t hot = 0, all;
-        if (p0 < kept) {
-#pragma unroll
-            for (int e = 0; e < kBkChunk; ++e) hot += bk_hot_of(v[e]);
-        }
-        const uint32_t cs = hot0 + block_excl_scan(hot, s.scan, all);
-        const uint32_t pos = rank0 + p0;
-        // whole numbers: the positives that are left, and those and the keys so far
-        float inter = npos - (float)cs, both = inter + (float)pos;                     // csrc/lovasz_softmax.cu:124-127
-        float j_prev = pos == 0 ? 0.f : 1.f - whole_ratio(inter, both);
-        auto step = [&](int e) {
-            const float now = (float)bk_hot_of(v[e]);
-            inter -= now;
-            both = (both + 1.f) - now;
-            const float j_now = 1.f - whole_ratio(inter, both);
-            const float dj = j_now - j_prev;                                           // csrc/lovasz_softmax.cu:141-147
-            j_prev = j_now;
-            part = add_loss(part, key_error(bk_key_of(v[e])), dj);
-            result[bk_item_of(v[e])] = dj;
-        };
-        if (p0 + kBkChunk <= kept) {
-#pragma unroll
-            for (int e = 0; e < kBkChunk; ++e) step(e);
-        } else {
-#pragma unroll
-            for (int e = 0; e < kBkChunk; ++e)
-                if (p0 + e < kept) step(e);
-        }
-    } else {                                                // bk_rank_crowded's
-        if (threadIdx.x == 0) a.crowded[Direct ? c : (int64_t)c * a.stride + g] = 1u;
-        return;
-    }
-    part = wave_sum_f64(part);
-    if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
-    __syncthreads();
-    asm volatile("" : "+v"(first));                         // looked up again, not held across the sort
-#pragma unroll
-    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
-        if (r0 >= rounds) break;                            // block-uniform
-        uint32_t to[kBkGroup];
-        float dj[kBkGroup];
-#pragma unroll
-        for (int i = 0; i < kBkGroup; ++i) dj[i] = result[first + (r0 + i) * kWave];   // past the last: inside the pairs
-        if constexpr (!Direct) {
-            at.where((uint32_t)(first + r0 * kWave), (uint32_t)a.P - 1u, to);
-        } else {
-#pragma unroll
-            for (int i = 0; i < kBkGroup; ++i) to[i] = (uint32_t)(first + (r0 + i) * kWave);
-        }
-#pragma unroll
-        for (int i = 0; i < kBkGroup; ++i)
-            if (r0 + i < count)
-                kin[to[i]] = __builtin_bit_cast(uint32_t, (!Direct || ((valid >> (r0 + i)) & 1u)) ? dj[i] : 0.f);
-    }
-    if (threadIdx.x == 0) {
-        double sum = 0.0;
-#pragma unroll
-        for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
-        if constexpr (Direct) losses[c] = (float)sum;
-        else a.loss_part[2 * (int64_t)c * a.stride + g] = sum;
-        a.crowded[Direct ? c : (int64_t)c * a.stride + g] = 0u;
-    }
-}
-
-// The runs (Direct: rows of one block) whose values crowd.
-template <bool Direct>
-__global__ __launch_bounds__(kBkThreads, 4) void bk_rank_crowded(const BucketArgs a, float *__restrict__ losses) {
-    __shared__ BkShared s;
-    __shared__ BkSegments at;
-    __shared__ double wave_loss[kBkWaves];
-    const int c = Direct ? blockIdx.x : blockIdx.y;
-    const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
-    const int runs = Direct ? 1 : (int)a.numbers[a.C + c];
-    for (int g = Direct ? 0 : blockIdx.x; g < runs; g += gridDim.x) {       // block-uniform
-        if (!a.crowded[Direct ? c : (int64_t)c * a.stride + g]) {
-            if (Direct) return;
-            continue;
-        }
-        const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
-        const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
-        const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
-        uint32_t *kin = a.keys + row;
-        const uint32_t limit = bk_limit(a, c);
-        const int rounds = (n + kBkThreads - 1) / kBkThreads;
-        uint32_t key[kBkItems], rank[kBkItems], valid = 0, hot = 0, least, most;
-        __syncthreads();
-        if constexpr (!Direct) at.collect(BkSegments::Tile(a, c, b0, b1), 0u, s.scan);
-        auto where = [&](int li) {
-            uint32_t to[1] = {(uint32_t)li};
-            if constexpr (!Direct) at.where((uint32_t)li, (uint32_t)a.P - 1u, to);
-            return to[0];
-        };
-#pragma unroll
-        for (int r = 0; r < kBkItems; ++r) {
-            const int li = bk_item(rounds, r);
-            key[r] = r < rounds && li < n ? kin[where(li)] : kIgnoredKey;
-            if (keep_key(key[r], limit)) {
-                valid |= 1u << r;
-                hot += key[r] >> 31;
-            }
-        }
-        float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
-        if constexpr (Direct) {
-            uint32_t all;
-            block_excl_scan(hot, s.scan, all);
-            npos = (float)all;
-        }
-        bk_range(s, key, valid, least, most);
-        bk_ranks_crowded(s, key, valid, rounds, least, most, rank);    // keys crowd, so there are some
-        double part = 0.0;
-#pragma unroll
-        for (int r = 0; r < kBkItems; ++r) {
-            const int li = bk_item(rounds, r);
-            if (r < rounds && li < n) {
-                float dj = 0.f;
-                if ((valid >> r) & 1u) {
-                    const uint32_t k = Direct ? key[r] : kin[where(li)];       // read again: not held across the sort
-                    dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), k >> 31);
-                    part = add_loss(part, key_error(k), dj);
-                }
-                kin[where(li)] = __builtin_bit_cast(uint32_t, dj);
-            }
-        }
-        part = wave_sum_f64(part);
-        if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double sum = 0.0;
-#pragma unroll
-            for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
-            if constexpr (Direct) losses[c] = (float)sum;
-            else a.loss_part[2 * (int64_t)c * a.stride + g] = sum;
-        }
-        if (Direct) return;
     }
 }
 
@@ -1533,67 +1325,6 @@ __device__ __forceinline__ double bk_huge_keys(BkShared &s, const BucketArgs &a,
     return part;
 }
 
-constexpr int kBkWideBlocks = 32;               // per class: one wide bucket at a time each, all of them for a flat one
-
-// Jaccard index of a class's first k keys, cs of its npos positives among them: a multiple of 2^-24, whatever the division
-// gives (a quotient from 1/2 on is one, and its difference from 1 is exact; one below leaves a difference from 1/2 on).
-__device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
-    const float inter = npos - (float)cs;
-    return k == 0 ? 0.f : 1.f - whole_ratio(inter, inter + (float)k);
-}
-
-// This block's part, every kBkWideBlocks-th tile, of bucket b with one value and n keys, from rank0 on with hot0 positives
-// before them and `hot` among them: in order as they stand. (A value that many share is mostly the positives' or the others'
-// alone.)
-__device__ __forceinline__ void bk_flat_keys(BkShared &s, const BucketArgs &a, int c, int b, uint32_t rank0, uint32_t hot0) {
-    constexpr uint32_t kPer = 8, kStep = kPer * kBkThreads;
-    // per tile: its first key of the bucket and their number; keys and positives of the bucket in the tiles before, positives here
-    uint32_t *first = s.key(), *count = first + kBkThreads, *before = count + kBkThreads, *hot_before = before + kBkThreads,
-             *hot = hot_before + kBkThreads;
-    const float npos = (float)a.numbers[2 * a.C + c];
-    const int64_t cell = ((int64_t)c * (a.stride + 1) + b) * a.tiles;
-    uint32_t start = 0, end = 0, unused;
-    if ((int)threadIdx.x < a.tiles) {
-        start = a.start[cell + threadIdx.x];
-        end = a.start[cell + a.tiles + threadIdx.x];
-    }
-    const uint32_t keys = (end & 0xFFFFu) - (start & 0xFFFFu), hots = (end >> 16) - (start >> 16);
-    __syncthreads();
-    first[threadIdx.x] = start & 0xFFFFu;
-    count[threadIdx.x] = keys;
-    hot[threadIdx.x] = hots;
-    block_excl_scan2(keys, hots, s.scan, before[threadIdx.x], unused, hot_before[threadIdx.x], unused);
-    __syncthreads();
-    for (int t = blockIdx.x; t < a.tiles; t += kBkWideBlocks) {
-        const uint32_t n = count[t], rank_t = rank0 + before[t];
-        uint32_t hot_t = hot0 + hot_before[t];
-        const bool mixed = hot[t] != 0u && hot[t] != n;     // block-uniform
-        uint32_t *at = a.keys + (int64_t)c * a.P + (uint32_t)t * kBkTile + first[t];
-        for (uint32_t i0 = 0; i0 < n; i0 += kStep) {
-            const uint32_t p0 = i0 + threadIdx.x * kPer;
-            uint32_t flags = hot[t] ? 0xFFu : 0u;
-            uint32_t cs = hot_t + (hot[t] ? p0 : 0u);
-            if (mixed) {
-                flags = 0;
-#pragma unroll
-                for (uint32_t e = 0; e < kPer; ++e) flags |= (p0 + e < n ? at[p0 + e] >> 31 : 0u) << e;
-                uint32_t all;
-                cs = hot_t + block_excl_scan((uint32_t)__builtin_popcount(flags), s.scan, all);
-                hot_t += all;
-            }
-            float j_prev = jaccard(npos, rank_t + p0, cs);
-#pragma unroll
-            for (uint32_t e = 0; e < kPer; ++e) {
-                cs += (flags >> e) & 1u;
-                const float j_now = jaccard(npos, rank_t + p0 + e + 1u, cs);
-                if (p0 + e < n) at[p0 + e] = __builtin_bit_cast(uint32_t, j_now - j_prev);     // csrc/lovasz_softmax.cu:141-147
-                j_prev = j_now;
-            }
-        }
-    }
-    __syncthreads();
-}
-
 // The n keys of bucket b to a row of their own from rank0 on, or the differences found there back to their places.
 __device__ __forceinline__ void bk_wide_copy(BkShared &s, BkSegments &segments, const BucketArgs &a, int c, int b, uint32_t rank0, uint32_t n, bool back) {
     const int64_t row = (int64_t)c * a.P;
@@ -1623,45 +1354,256 @@ __device__ __forceinline__ void bk_wide_copy(BkShared &s, BkSegments &segments, 
     __syncthreads();
 }
 
-__global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
+// One run of buckets (or, Direct: a whole row of at most kBkCap pixels, straight from the keys in pixel order, with the
+// Jaccard differences left in their place and the loss complete).
+// Time goes into vector instructions, 118 per 64 keys (69 % of it at 16 waves per CU): a thread's places of the order are
+// neighbours, so that a difference is one new quotient less the one before, and the positives before a place are a sum over
+// the block's threads. The rounds of a group of three wait for LDS once where each waited by itself, and what tells a key's place
+// lies at constant offsets: with the quotients' fewer steps and scans by DPP 149 -> 118 instructions, (8,21,513,513) bf16 trained 270 -> 227 us,
+// (4,19,512,1024) fp32 134 -> 111.
+template <bool Direct>
+__global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, float *__restrict__ losses) {
+    __shared__ BkShared s;
+    __shared__ BkSegments at;                               // not for a whole row
+    __shared__ double wave_loss[kBkWaves];
+    const int c = Direct ? blockIdx.x : blockIdx.y;
+    const int64_t row = (int64_t)c * a.P, cells = (int64_t)c * (a.stride + 1);
+    const int runs = Direct ? 1 : (int)a.numbers[a.C + c];
+    if (!Direct && (int)blockIdx.x >= runs) return;                    // block-uniform
+    // neighbouring runs on one XCD: a tile's segments of theirs share cache lines
+    const int g = Direct ? 0 : xcd_chunk((int)blockIdx.x, runs);
+    const uint32_t b0 = Direct ? 0u : a.runs[cells + g], b1 = Direct ? 0u : a.runs[cells + g + 1];
+    const uint32_t rank0 = Direct ? 0u : a.base[cells + b0], hot0 = Direct ? 0u : a.hot_base[cells + b0];
+    const int n = Direct ? a.P : (int)(a.base[cells + b1] - rank0);
+    const BkSegments::Tile tile = Direct ? BkSegments::Tile() : BkSegments::Tile(a, c, b0, b1);
+    if (!Direct && (n > kBkCap || n == 0)) {                // block-uniform; too many: a large bucket
+        if (threadIdx.x == 0) a.loss_part[2 * (int64_t)c * a.stride + g] = 0.0;
+        return;
+    }
+    uint32_t *kin = a.keys + row;                           // the differences take the keys' places
+    const uint32_t limit = bk_limit(a, c);
+    float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
+    if constexpr (!Direct) at.collect(tile, 0u, s.scan);
+
+    uint32_t key[kBkItems], valid = 0, least, most, knee = 0;
+    float share = 0.25f;
+    bool flat = false;                                      // block-uniform: one value, in order as it stands
+    const int rounds = (n + kBkThreads - 1) / kBkThreads;
+    int first = bk_item(rounds, 0);
+    // the thread's items: first, first + 64, ... inside the wave's part
+    const int count = max(0, (min(n, first - (int)(threadIdx.x & 63) + rounds * kWave) - first + kWave - 1) / kWave);
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) key[r] = 0;
+#pragma unroll
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                            // block-uniform
+        uint32_t from[kBkGroup];
+        if constexpr (!Direct) {
+            at.where((uint32_t)(first + r0 * kWave), (uint32_t)a.P - 1u, from);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kBkGroup; ++i) from[i] = (uint32_t)min(first + (r0 + i) * kWave, n - 1);
+        }
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) key[r0 + i] = kin[from[i]];
+    }
+    if constexpr (Direct) {
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r)
+            if (r < count && keep_key(key[r], limit)) valid |= 1u << r;
+    } else {
+        valid = (1u << count) - 1u;
+    }
+    if constexpr (Direct) {
+        bk_range(s, key, valid, least, most);
+        uint32_t hot = 0, all;
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) hot += ((valid >> r) & 1u) ? key[r] >> 31 : 0u;
+        block_excl_scan(hot, s.scan, all);
+        npos = (float)all;
+        most = max(least, most);                            // no valid key: nothing below looks at the range
+    } else {
+        const uint32_t *bound = a.bounds + (int64_t)c * a.stride;
+        const uint32_t buckets = a.numbers[c];
+        most = b1 < buckets ? bound[b1 - 1] - 1u : limit;
+        least = b0 ? bound[b0 - 1] : 0u;
+        flat = least == most || npos == 0.f;                // a class without positives: the one value of its limit
+        if (!flat && (b0 == 0 || b1 + 1u >= buckets)) {
+            // beyond the sample lie a few more, far apart: their own bins
+            bk_range(s, key, valid, least, most);
+            knee = b0 ? a.numbers[4 * a.C + c] + 1u : a.numbers[3 * a.C + c];
+            // Nor do the first keys lie evenly: errors near 1 crowd in classes that the network misses, as in bk_split. A
+            // knee right at the first key left 260 keys in one bin ((1,32,256,256), soft: bk_rank and the crowded path 34 + 36 -> 19 + 4 us).
+            if (!b0) knee = max(knee, least + (most - least) / 64u);
+            share = b0 ? 0.75f : 0.25f;
+        }
+    }
+    double part = 0.0;
+    BkPair v[kBkChunk];
+    uint32_t kept;
+    float *result = reinterpret_cast<float *>(s.pair);      // by item
+    bool in_order = flat;
+    if (flat) {
+        kept = (uint32_t)n;
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r)
+            if ((valid >> r) & 1u) s.at((uint32_t)bk_item(rounds, r)) = bk_pair(key[r], (uint32_t)bk_item(rounds, r));
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < kBkChunk; ++e) {
+            const uint32_t p = threadIdx.x * kBkChunk + e;
+            v[e] = p < kept ? s.at(p) : bk_last();
+        }
+        __syncthreads();
+    } else {
+        const BkBinning bins(least, knee, most, share);
+        if constexpr (Direct) in_order = bk_sort(s, key, BkMask{valid}, rounds, bins, kept, v);
+        else in_order = bk_sort(s, key, BkFirst{count}, rounds, bins, kept, v);
+    }
+    if (in_order) {                                         // block-uniform
+        const uint32_t p0 = threadIdx.x * kBkChunk;
+        uint32_t hot = 0, all;
+        if (p0 < kept) {
+#pragma unroll
+            for (int e = 0; e < kBkChunk; ++e) hot += bk_hot_of(v[e]);
+        }
+        const uint32_t cs = hot0 + block_excl_scan(hot, s.scan, all);
+        const uint32_t pos = rank0 + p0;
+        // whole numbers: the positives that are left, and those and the keys so far
+        float inter = npos - (float)cs, both = inter + (float)pos;                     // csrc/lovasz_softmax.cu:124-127
+        float j_prev = pos == 0 ? 0.f : 1.f - whole_ratio(inter, both);
+        auto step = [&](int e) {
+            const float now = (float)bk_hot_of(v[e]);
+            inter -= now;
+            both = (both + 1.f) - now;
+            const float j_now = 1.f - whole_ratio(inter, both);
+            const float dj = j_now - j_prev;                                           // csrc/lovasz_softmax.cu:141-147
+            j_prev = j_now;
+            part = add_loss(part, key_error(bk_key_of(v[e])), dj);
+            result[bk_item_of(v[e])] = dj;
+        };
+        if (p0 + kBkChunk <= kept) {
+#pragma unroll
+            for (int e = 0; e < kBkChunk; ++e) step(e);
+        } else {
+#pragma unroll
+            for (int e = 0; e < kBkChunk; ++e)
+                if (p0 + e < kept) step(e);
+        }
+    } else if constexpr (!Direct) {                         // values crowd: bk_rank_rest's
+        if (threadIdx.x == 0) a.crowded[(int64_t)c * a.stride + atomicAdd(&a.numbers[8 * a.C + c], 1u)] = (uint32_t)g;
+        return;
+    } else {
+        bk_range(s, key, valid, least, most);
+        uint32_t rank[kBkItems];
+        bk_ranks_crowded(s, key, valid, rounds, least, most, rank);
+#pragma unroll
+        for (int r = 0; r < kBkItems; ++r) {
+            if (!((valid >> r) & 1u)) continue;
+            const float dj = jaccard_step(npos, rank[r] & 0xFFFFu, rank[r] >> 16, key[r] >> 31);
+            part = add_loss(part, key_error(key[r]), dj);
+            result[bk_item(rounds, r)] = dj;
+        }
+    }
+    part = wave_sum_f64(part);
+    if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
+    __syncthreads();
+    asm volatile("" : "+v"(first));                         // looked up again, not held across the sort
+#pragma unroll
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                            // block-uniform
+        uint32_t to[kBkGroup];
+        float dj[kBkGroup];
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) dj[i] = result[first + (r0 + i) * kWave];   // past the last: inside the pairs
+        if constexpr (!Direct) {
+            at.where((uint32_t)(first + r0 * kWave), (uint32_t)a.P - 1u, to);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kBkGroup; ++i) to[i] = (uint32_t)(first + (r0 + i) * kWave);
+        }
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i)
+            if (r0 + i < count)
+                kin[to[i]] = __builtin_bit_cast(uint32_t, (!Direct || ((valid >> (r0 + i)) & 1u)) ? dj[i] : 0.f);
+    }
+    if (threadIdx.x == 0) {
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
+        if constexpr (Direct) losses[c] = (float)sum;
+        else a.loss_part[2 * (int64_t)c * a.stride + g] = sum;
+    }
+}
+
+// A run whose values crowd.
+__device__ __forceinline__ double bk_crowded_keys(BkShared &s, BkSegments &at, const BucketArgs &a, int c, int g) {
+    const int64_t cells = (int64_t)c * (a.stride + 1);
+    const uint32_t b0 = a.runs[cells + g], b1 = a.runs[cells + g + 1];
+    const uint32_t rank0 = a.base[cells + b0], hot0 = a.hot_base[cells + b0];
+    const int n = (int)(a.base[cells + b1] - rank0), rounds = (n + kBkThreads - 1) / kBkThreads;
+    uint32_t *kin = a.keys + (int64_t)c * a.P;
+    uint32_t key[kBkItems], rank[kBkItems], valid = 0, least, most;
+    __syncthreads();
+    at.collect(BkSegments::Tile(a, c, b0, b1), 0u, s.scan);
+    auto where = [&](int li) {
+        uint32_t to[1];
+        at.where((uint32_t)li, (uint32_t)a.P - 1u, to);
+        return to[0];
+    };
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        const int li = bk_item(rounds, r);
+        key[r] = 0;
+        if (r < rounds && li < n) {
+            key[r] = kin[where(li)];
+            valid |= 1u << r;
+        }
+    }
+    bk_range(s, key, valid, least, most);
+    bk_ranks_crowded(s, key, valid, rounds, least, most, rank);
+    const float npos = (float)a.numbers[2 * a.C + c];
+    double part = 0.0;
+#pragma unroll
+    for (int r = 0; r < kBkItems; ++r) {
+        if (!((valid >> r) & 1u)) continue;
+        const uint32_t to = where(bk_item(rounds, r)), k = kin[to];         // read again: not held across the sort
+        const float dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), k >> 31);
+        part = add_loss(part, key_error(k), dj);
+        kin[to] = __builtin_bit_cast(uint32_t, dj);
+    }
+    return part;
+}
+
+// A bucket that outgrew the LDS.
+__device__ __forceinline__ double bk_wide_bucket(BkShared &s, BkSegments &at, const BucketArgs &a, int c, int b) {
+    const int buckets = (int)a.numbers[c];
+    const int64_t cells = (int64_t)c * (a.stride + 1), row = (int64_t)c * a.stride;
+    const uint32_t lo = b ? a.bounds[row + b - 1] : 0u, hi = b + 1 < buckets ? a.bounds[row + b] : bk_limit(a, c) + 1u;
+    const uint32_t rank0 = a.base[cells + b], n = a.base[cells + b + 1] - rank0, hot0 = a.hot_base[cells + b];
+    bk_wide_copy(s, at, a, c, b, rank0, n, false);
+    // Sampled bounds leave a bucket of 7700 to 9000 keys in every other step or so: by ranges 30 us, by groups 45.
+    const double part = n <= 4u * kBkCap ? bk_wide_keys(s, a, c, rank0, hot0, (int)n) : bk_huge_keys(s, a, c, rank0, hot0, n, lo, hi);
+    bk_wide_copy(s, at, a, c, b, rank0, n, true);
+    return part;
+}
+
+constexpr int kBkWideBlocks = 8;                // per class: a wide bucket at a time each; then as many as there are for crowded runs
+
+// What bk_rank leaves: the wide buckets and the crowded runs. 256 registers, one block per CU: with two, a wide bucket's code
+// spills (a bucket of (8,8,512,512) bf16 logits 94 -> 235 us, against the crowded runs of a sure network 107 -> 98).
+__global__ __launch_bounds__(kBkThreads) void bk_rank_rest(const BucketArgs a) {
     __shared__ BkShared s;
     __shared__ BkSegments at;
     __shared__ double wave_loss[kBkWaves];
-    __shared__ int todo[kBkMax / kBkWideBlocks + 1], found;
-    __shared__ int flats[kBkMaxRow / kBkCap + 1], n_flats;
-    const int c = blockIdx.y, buckets = (int)a.numbers[c];
-    const int64_t cells = (int64_t)c * (a.stride + 1), row = (int64_t)c * a.stride;
-    if (threadIdx.x == 0) found = n_flats = 0;
-    __syncthreads();
-    // in any order: each has a sum and differences of its own
-    for (int i = (int)threadIdx.x; i < buckets; i += kBkThreads) {
-        const uint32_t n = a.count[row + i];
-        const bool mine = i % kBkWideBlocks == (int)blockIdx.x, wide = n > (uint32_t)kBkCap;
-        if (n & kBkFlat) flats[atomicAdd(&n_flats, 1)] = i;
-        else if (mine && wide) todo[atomicAdd(&found, 1)] = i;
-        if (mine && !(n & kBkFlat) && !wide) a.loss_part[2 * row + a.stride + i] = 0.0;
-        if (mine && (n & kBkFlat)) {
-            // one error, its bound, and the differences, exact as multiples of 2^-24, add up to that of the ends
-            const float npos = (float)a.numbers[2 * a.C + c];
-            const float rise = jaccard(npos, a.base[cells + i + 1], a.hot_base[cells + i + 1]) -
-                               jaccard(npos, a.base[cells + i], a.hot_base[cells + i]);
-            a.loss_part[2 * row + a.stride + i] = add_loss(0.0, key_error(a.bounds[row + i - 1]), rise);
-        }
-    }
-    __syncthreads();
-    const int n_flat = n_flats;
-    for (int i = 0; i < n_flat; ++i) {                      // block-uniform
-        const int b = flats[i];
-        bk_flat_keys(s, a, c, b, a.base[cells + b], a.hot_base[cells + b]);
-    }
-    const int n_todo = found;
-    for (int i = 0; i < n_todo; ++i) {
-        const int b = todo[i];
-        const uint32_t lo = b ? a.bounds[row + b - 1] : 0u, hi = b + 1 < buckets ? a.bounds[row + b] : bk_limit(a, c) + 1u;
-        const uint32_t n = a.count[row + b], rank0 = a.base[cells + b], hot0 = a.hot_base[cells + b];
-        // Sampled bounds leave a bucket of 7700 to 9000 keys in every other step or so: by ranges 30 us, by groups 45.
-        bk_wide_copy(s, at, a, c, b, rank0, n, false);
-        double part = n <= 4u * kBkCap ? bk_wide_keys(s, a, c, rank0, hot0, (int)n) : bk_huge_keys(s, a, c, rank0, hot0, n, lo, hi);
+    const int c = blockIdx.y;
+    const bool wide = blockIdx.x < kBkWideBlocks;           // block-uniform
+    const int todo = (int)a.numbers[(wide ? 6 : 8) * a.C + c];
+    const uint32_t *list = (wide ? a.large : a.crowded) + (int64_t)c * a.stride;
+    double *loss_part = a.loss_part + 2 * (int64_t)c * a.stride;
+    for (int i = wide ? blockIdx.x : blockIdx.x - kBkWideBlocks; i < todo; i += wide ? kBkWideBlocks : gridDim.x - kBkWideBlocks) {
+        const int what = (int)list[i];
+        double part = wide ? bk_wide_bucket(s, at, a, c, what) : bk_crowded_keys(s, at, a, c, what);
         part = wave_sum_f64(part);
         __syncthreads();
         if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = part;
@@ -1670,15 +1612,57 @@ __global__ __launch_bounds__(kBkThreads) void bk_rank_wide(const BucketArgs a) {
             double sum = 0.0;
 #pragma unroll
             for (int w = 0; w < kBkWaves; ++w) sum += wave_loss[w];
-            a.loss_part[2 * row + a.stride + b] = sum;
+            loss_part[wide ? a.stride + i : what] = sum;
         }
-        bk_wide_copy(s, at, a, c, b, rank0, n, true);
+    }
+}
+
+// The tile's part of a class's flat bucket b, in `tile` (LDS) in order: the keys become their Jaccard differences. (A value that
+// many share is mostly the positives' or the others' alone.)
+__device__ __forceinline__ void bk_flat_keys(uint32_t *keys, uint32_t *scan, const BucketArgs &a, int c, int tile, int b) {
+    constexpr uint32_t kPer = 8, kStep = kPer * kBkThreads;
+    const int64_t cells = (int64_t)c * (a.stride + 1) + b, cell = cells * a.tiles;
+    const uint32_t start = a.start[cell + tile], end = a.start[cell + a.tiles + tile];
+    const uint32_t first = start & 0xFFFFu, n = (end & 0xFFFFu) - first, hots = (end >> 16) - (start >> 16);
+    const float npos = (float)a.numbers[2 * a.C + c];
+    if (n == 0) return;                                     // block-uniform
+    uint32_t before = 0, hot_before = 0, rank0, hot0, unused;
+    if ((int)threadIdx.x < tile) {
+        const uint32_t from = a.start[cell + threadIdx.x], to = a.start[cell + a.tiles + threadIdx.x];
+        before = (to & 0xFFFFu) - (from & 0xFFFFu);
+        hot_before = (to >> 16) - (from >> 16);
+    }
+    block_excl_scan2(before, hot_before, scan, unused, rank0, unused, hot0);
+    rank0 += a.base[cells];
+    hot0 += a.hot_base[cells];
+    const bool mixed = hots != 0u && hots != n;
+    for (uint32_t i0 = 0; i0 < n; i0 += kStep) {
+        const uint32_t p0 = i0 + threadIdx.x * kPer;
+        uint32_t flags = hots ? 0xFFu : 0u;
+        uint32_t cs = hot0 + (hots ? p0 : 0u);
+        if (mixed) {
+            flags = 0;
+#pragma unroll
+            for (uint32_t e = 0; e < kPer; ++e) flags |= (p0 + e < n ? keys[first + p0 + e] >> 31 : 0u) << e;
+            uint32_t all;
+            cs = hot0 + block_excl_scan((uint32_t)__builtin_popcount(flags), scan, all);
+            hot0 += all;
+        }
+        float j_prev = jaccard(npos, rank0 + p0, cs);
+#pragma unroll
+        for (uint32_t e = 0; e < kPer; ++e) {
+            cs += (flags >> e) & 1u;
+            const float j_now = jaccard(npos, rank0 + p0 + e + 1u, cs);
+            if (p0 + e < n) keys[first + p0 + e] = __builtin_bit_cast(uint32_t, j_now - j_prev);       // csrc/lovasz_softmax.cu:141-147
+            j_prev = j_now;
+        }
     }
 }
 
 // The tile's Jaccard differences in pixel order. The first block of a class adds up its loss.
 __global__ __launch_bounds__(kBkThreads) void bk_restore(const BucketArgs a, float *__restrict__ losses) {
     __shared__ uint32_t dj[kBkTile];
+    __shared__ uint32_t scan_tmp[2 * kSortWaves];
     const int c = blockIdx.y, tile = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int begin = tile * kBkTile, n = min(kBkTile, a.P - begin);
     uint32_t *row = a.keys + (int64_t)c * a.P + begin;
@@ -1692,7 +1676,13 @@ __global__ __launch_bounds__(kBkThreads) void bk_restore(const BucketArgs a, flo
     }
 #pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) dj[bk_item(kBkTileItems, r)] = v[r];
+    const int wides = (int)a.numbers[6 * a.C + c], flats = (int)a.numbers[7 * a.C + c];
     __syncthreads();
+    if (flats > 0) {                                        // block-uniform
+        for (int i = 0; i < flats; ++i)
+            bk_flat_keys(dj, scan_tmp, a, c, tile, (int)a.large[(int64_t)c * a.stride + wides + i]);
+        __syncthreads();
+    }
 #pragma unroll
     for (int r = 0; r < kBkTileItems; ++r) {
         const int li = bk_item(kBkTileItems, r);
@@ -1700,11 +1690,11 @@ __global__ __launch_bounds__(kBkThreads) void bk_restore(const BucketArgs a, flo
     }
     if (tile != 0) return;
     __shared__ double wave_sum[kBkWaves];
-    const int runs = (int)a.numbers[a.C + c], buckets = (int)a.numbers[c];
+    const int runs = (int)a.numbers[a.C + c];
     const double *sums = a.loss_part + 2 * (int64_t)c * a.stride;
     double sum = 0.0;
     for (int i = threadIdx.x; i < runs; i += kBkThreads) sum += sums[i];
-    for (int i = threadIdx.x; i < buckets; i += kBkThreads) sum += sums[a.stride + i];
+    for (int i = threadIdx.x; i < wides + flats; i += kBkThreads) sum += sums[a.stride + i];
     sum = wave_sum_f64(sum);
     if (lane == 0) wave_sum[wave] = sum;
     __syncthreads();
