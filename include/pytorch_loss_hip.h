@@ -143,6 +143,22 @@ int plh_lsr_backward_scaled_lse(const void *logits, int32_t dtype, const int64_t
                                 int64_t n_size, int64_t dimsize, int64_t m_size,
                                 int64_t ignore_index, float smooth, void *stream);
 
+/* The same for 16-bit logits on channel planes of at least 4096 pixels that do not start on 128-byte lines, with 16..256
+ * channels. */
+int plh_lsr_saves_lse_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);
+
+int plh_lsr_forward_reduced_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *lse_out,
+                                         float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                         void *workspace, int64_t workspace_bytes,
+                                         int64_t n_size, int64_t dimsize, int64_t m_size,
+                                         int64_t ignore_index, float smooth, void *stream);
+
+int plh_lsr_backward_scaled_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, const float *lse,
+                                         const float *grad_scalar, float scale, const int64_t *divide_by,
+                                         void *grad_logits,
+                                         int64_t n_size, int64_t dimsize, int64_t m_size,
+                                         int64_t ignore_index, float smooth, void *stream);
+
 /* plh_lsr_forward_reduced for callers that cannot allocate device memory or bring a workspace
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). It has no
  * counterpart in the reference. Same arguments and results as plh_lsr_forward_reduced, without the
@@ -486,6 +502,20 @@ int plh_taylor_ce_backward_scaled_sums(const void *logits, int32_t dtype, const 
                                        const int64_t *divide_by, void *grad_logits,
                                        int64_t n_size, int64_t dimsize, int64_t m_size,
                                        int64_t order, int64_t ignore_index, void *stream);
+
+/* The same for 16-bit logits on channel planes of at least 4096 pixels that do not start on 128-byte lines, with 16..256
+ * channels (orders 2 and 4; other orders leave sums_out unwritten and recompute). */
+int plh_taylor_ce_saves_sums_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);
+int plh_taylor_ce_forward_reduced_sums_planes16(const void *logits, int32_t dtype, const int64_t *labels,
+                                                float *sums_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                                void *workspace, int64_t workspace_bytes,
+                                                int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                int64_t order, int64_t ignore_index, void *stream);
+int plh_taylor_ce_backward_scaled_sums_planes16(const void *logits, int32_t dtype, const int64_t *labels,
+                                                const float *sums, const float *grad_scalar, float scale,
+                                                const int64_t *divide_by, void *grad_logits,
+                                                int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                int64_t order, int64_t ignore_index, void *stream);
 
 /* ---- soft dice loss ---------------------------------------------------------------------
  * Replaces soft_dice_cpp.soft_dice_forward / soft_dice_backward (csrc/soft_dice_kernel_v2.cu:258-436).

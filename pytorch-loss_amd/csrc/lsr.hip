@@ -39,15 +39,19 @@ PLH_LSR_EXTERN(float)
 PLH_LSR_EXTERN(f16)
 PLH_LSR_EXTERN(bf16)
 
+static bool lse_applies(int32_t dtype, int64_t dimsize, int64_t m_size, bool planes16) {
+    return (planes16 ? planes16_apply : lsr_lse_applies)(dtype_size(dtype), dimsize, m_size);
+}
+
 static int backward(const void *logits, int32_t dtype, const int64_t *labels, const Upstream &up, void *grad_logits,
                     int64_t n_size, int64_t dimsize, int64_t m_size, int64_t ignore_index, float smooth,
-                    void *stream, const float *lse = nullptr) {
+                    void *stream, const float *lse = nullptr, bool planes16 = false) {
     if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
     const int rc = check_slice_args(logits, labels, grad_logits, n_size, dimsize, m_size, dtype_size(dtype),
                                     dtype_size(dtype));
     if (rc != PLH_OK) return rc;
     if (n_size * dimsize * m_size == 0) return PLH_OK;
-    if (lse && (misaligned(lse, 4) || !lsr_lse_applies(dtype_size(dtype), dimsize, m_size))) return PLH_ERR_BAD_SIZE;
+    if (lse && (misaligned(lse, 4) || !lse_applies(dtype, dimsize, m_size, planes16))) return PLH_ERR_BAD_SIZE;
     LsrParams p = make_params(n_size, dimsize, m_size, ignore_index, smooth, dtype_size(dtype));
     p.lse = const_cast<float *>(lse);           // read only in the backward
     dispatch_dtype(dtype, [&](auto tag) {
@@ -81,9 +85,9 @@ extern "C" int plh_lsr_forward(const void *logits, int32_t dtype, const int64_t 
 static int forward_reduced(const void *logits, int32_t dtype, const int64_t *labels, float *losses, float *lse_out,
                            float *loss_out, int64_t *n_valid_out, int32_t mean, void *workspace, int64_t workspace_bytes,
                            int64_t n_size, int64_t dimsize, int64_t m_size, int64_t ignore_index, float smooth,
-                           void *stream) {
+                           void *stream, bool planes16 = false) {
     if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
-    if (lse_out && (misaligned(lse_out, 4) || !lsr_lse_applies(dtype_size(dtype), dimsize, m_size))) return PLH_ERR_BAD_SIZE;
+    if (lse_out && (misaligned(lse_out, 4) || !lse_applies(dtype, dimsize, m_size, planes16))) return PLH_ERR_BAD_SIZE;
     int rc = check_slice_args(logits, labels, loss_out, n_size, dimsize, m_size, dtype_size(dtype), 4);
     if (rc != PLH_OK) return rc;
     Partials part;
@@ -179,6 +183,31 @@ extern "C" int plh_lsr_forward_reduced_lse(const void *logits, int32_t dtype, co
     if (!lse_out && n_size * dimsize * m_size != 0) return PLH_ERR_NULL_POINTER;
     return forward_reduced(logits, dtype, labels, nullptr, lse_out, loss_out, n_valid_out, mean, workspace, workspace_bytes,
                            n_size, dimsize, m_size, ignore_index, smooth, stream);
+}
+
+extern "C" int plh_lsr_saves_lse_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size) {
+    return dtype_ok(dtype) && n_size > 0 && dimsize > 0 && m_size > 0 && lse_applies(dtype, dimsize, m_size, true) ? 1 : 0;
+}
+
+extern "C" int plh_lsr_forward_reduced_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *lse_out,
+                                                    float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                                    void *workspace, int64_t workspace_bytes,
+                                                    int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                    int64_t ignore_index, float smooth, void *stream) {
+    if (!lse_out && n_size * dimsize * m_size != 0) return PLH_ERR_NULL_POINTER;
+    return forward_reduced(logits, dtype, labels, nullptr, lse_out, loss_out, n_valid_out, mean, workspace, workspace_bytes,
+                           n_size, dimsize, m_size, ignore_index, smooth, stream, true);
+}
+
+extern "C" int plh_lsr_backward_scaled_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, const float *lse,
+                                                    const float *grad_scalar, float scale, const int64_t *divide_by,
+                                                    void *grad_logits,
+                                                    int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                    int64_t ignore_index, float smooth, void *stream) {
+    if (n_size * dimsize * m_size != 0 && (!grad_scalar || !lse)) return PLH_ERR_NULL_POINTER;
+    if (misaligned(grad_scalar, 4) || misaligned(divide_by, 8)) return PLH_ERR_MISALIGNED;
+    const Upstream up{grad_scalar, 0, divide_by, scale, nullptr};
+    return backward(logits, dtype, labels, up, grad_logits, n_size, dimsize, m_size, ignore_index, smooth, stream, lse, true);
 }
 
 extern "C" int plh_lsr_forward_reduced_static(const void *logits, int32_t dtype, const int64_t *labels, float *losses,

@@ -14,6 +14,7 @@
 // module-level reduction costs no further pass over the pixels.
 #pragma once
 #include "plh_common.hpp"
+#include "planes16.hpp"
 
 namespace plh {
 
@@ -24,10 +25,10 @@ struct LsrParams {
     int64_t ignore;
     float w_pos, w_neg, sumw;
     unsigned xcd_run;   // tile permutation run length (xcd_run_for)
-    // Per-pixel log-sum-exp of the logits, fp32 [P]. Forward, fp32 logits in NCHW: written when set, by the per-image
-    // form of the register-resident kernel, the split kernels and the lane-per-pixel kernel (the shapes that
-    // lsr_lse_applies sends here).
-    // Backward: when set, lsr_bwd_planes forms the gradient from it plane by plane (see there).
+    // Per-pixel log-sum-exp of the logits, fp32 [P]. Forward, logits in NCHW: written when set, by the per-image
+    // form of the register-resident kernel, the split kernels and (fp32) the lane-per-pixel kernel (the shapes that
+    // lsr_lse_applies and planes16_apply send here).
+    // Backward: when set, lsr_bwd_planes and planes16_bwd form the gradient from it plane by plane (see there).
     float *lse = nullptr;
 };
 
@@ -59,8 +60,8 @@ __global__ __launch_bounds__(kRegsBlock) void lsr_fwd_regs(const T *__restrict__
     float mine = 0.f;
     int cnt = 0;
     const float fc = (float)p.C;
-    // the per-image form on fp32 logits also leaves each pixel's log-sum-exp where it is given a place (LsrParams::lse)
-    constexpr bool kMayLse = Form == kPerImage && sizeof(T) == 4;
+    // the per-image form also leaves each pixel's log-sum-exp where it is given a place (LsrParams::lse)
+    constexpr bool kMayLse = Form == kPerImage;
     float lse_abs[kMayLse ? V : 1];
 #pragma unroll
     for (int k = 0; k < V; ++k) {
@@ -300,6 +301,23 @@ __global__ __launch_bounds__(256) void lsr_bwd_planes(const T *__restrict__ x, c
     }
 }
 
+// The same for 16-bit logits (planes16_bwd).
+struct LsrPlaneOp {
+    float sumw, w_pos, w_neg, scale, n_pos, n_neg;
+    __device__ __forceinline__ void begin(float gk) {
+        scale = sumw * gk;
+        n_pos = -w_pos * gk;
+        n_neg = -w_neg * gk;
+    }
+    __device__ __forceinline__ float value(float lse) const { return lse; }
+    __device__ __forceinline__ int label(int64_t lb, int64_t ignore, int C) const {
+        return lb == ignore ? -1 : ((lb < 0 || lb >= C) ? C : (int)lb);
+    }
+    __device__ __forceinline__ float grad(float x, float lse, bool hot) const {
+        return __builtin_fmaf(__builtin_amdgcn_exp2f((x - lse) * kLog2e), scale, hot ? n_pos : n_neg);
+    }
+};
+
 // Whether the forward leaves the log-sum-exp for these sizes and the backward runs plane by plane: fp32 logits on
 // planes of 4096 pixels or more that do not start on 128-byte lines - up to 24 channels (the register-resident
 // forward's per-image form) or 33 and more (channels shared among wavefronts in tiles per image: fwd+bwd at
@@ -308,9 +326,7 @@ __global__ __launch_bounds__(256) void lsr_bwd_planes(const T *__restrict__ x, c
 // (4,512,256,256) 0.343 -> 0.301 ms) or have a lane walk its pixel's channels ((4,600,256,256) 0.761 -> 0.523 ms).
 // On aligned planes with up to 256 channels the recomputing backward is as fast or faster (40 channels: 0.179 against
 // 0.196 ms for the pair, 150: 0.629 / 0.634).
-// fp32 logits only: with 16-bit logits (8 elements per lane, 64 per line) the pair measured no gain - bf16
-// (16,19,769,769): forward 0.0815 -> 0.0963 ms with the extra output, backward 0.180 -> 0.160 ms, bound by its
-// conversions.
+// fp32 logits only; 16-bit ones: planes16_apply.
 // (N, C) rows of more than 32 classes, any element type: the forward leaves one value per row (lsr_fwd_wrow, lsr_fwd_row)
 // and the backward from it (lsr_bwd_flat_lse) needs no reduction and no row in registers; which rows take it:
 // row_backward_is_elementwise.
@@ -401,9 +417,7 @@ __global__ __launch_bounds__(kSplitBlock) void lsr_fwd_split(const T *__restrict
     const bool valid = here && !ign;
     const float out = valid ? acc : 0.f;
     if (here && loss) loss[at.pix + wave] = out;
-    if constexpr (sizeof(T) == 4) {
-        if (here && p.lse) __builtin_nontemporal_store(M + lse, p.lse + at.pix + wave);      // LsrParams::lse
-    }
+    if (here && p.lse) __builtin_nontemporal_store(M + lse, p.lse + at.pix + wave);          // LsrParams::lse
     if (Reduce) split_block_partials<V>(out, valid, wave, lane, part);
 }
 
@@ -1441,6 +1455,11 @@ void lsr_backward_typed(const T *logits, const int64_t *labels, const Upstream &
                                dim3(256), 0, st, logits, labels, up, grad_logits, p, (int)tiles, per);
             return;
         }
+    }
+    if constexpr (sizeof(T) == 2) {
+        if (p.lse && p.m_size > 1 && !go_vec && !up.keep && planes16_apply(sizeof(T), p.C, p.m_size) &&
+            planes16_launch(logits, labels, p.lse, up, grad_logits, LsrPlaneOp{p.sumw, p.w_pos, p.w_neg}, p.P, p.m_size, p.C, p.ignore, st))
+            return;
     }
     switch (pick_shape(p.C, p.m_size, V, sizeof(T), logits, grad_logits, labels, go_vec, nullptr, true, true, true,
                        kImageFormMaxChannels<T>)) {

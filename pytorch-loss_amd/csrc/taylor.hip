@@ -146,16 +146,16 @@ extern "C" int plh_taylor_ce_saves_sums(int32_t dtype, int64_t n_size, int64_t d
                    taylor_sums_apply(dtype_size(dtype), dimsize, m_size) ? 1 : 0;
 }
 
-extern "C" int plh_taylor_ce_forward_reduced_sums(const void *logits, int32_t dtype, const int64_t *labels,
-                                                  float *sums_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
-                                                  void *workspace, int64_t workspace_bytes,
-                                                  int64_t n_size, int64_t dimsize, int64_t m_size,
-                                                  int64_t order, int64_t ignore_index, void *stream) {
+static int forward_reduced_sums(const void *logits, int32_t dtype, const int64_t *labels,
+                                float *sums_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                void *workspace, int64_t workspace_bytes,
+                                int64_t n_size, int64_t dimsize, int64_t m_size,
+                                int64_t order, int64_t ignore_index, void *stream, bool planes16) {
     if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
     int rc = check_order(order);
     if (rc != PLH_OK) return rc;
     if (n_size < 0 || m_size < 0 || n_size > kMaxNumel || m_size > kMaxNumel) return PLH_ERR_BAD_SIZE;
-    if (!taylor_sums_apply(dtype_size(dtype), dimsize, m_size)) return PLH_ERR_BAD_SIZE;
+    if (!(planes16 ? planes16_apply : taylor_sums_apply)(dtype_size(dtype), dimsize, m_size)) return PLH_ERR_BAD_SIZE;
     if (!loss_out) return PLH_ERR_NULL_POINTER;
     if (!sums_out && n_size * dimsize * m_size != 0) return PLH_ERR_NULL_POINTER;
     if (misaligned(sums_out, 4)) return PLH_ERR_MISALIGNED;
@@ -178,15 +178,15 @@ extern "C" int plh_taylor_ce_forward_reduced_sums(const void *logits, int32_t dt
     return check_launch();
 }
 
-extern "C" int plh_taylor_ce_backward_scaled_sums(const void *logits, int32_t dtype, const int64_t *labels,
-                                                  const float *sums, const float *grad_scalar, float scale,
-                                                  const int64_t *divide_by, void *grad_logits,
-                                                  int64_t n_size, int64_t dimsize, int64_t m_size,
-                                                  int64_t order, int64_t ignore_index, void *stream) {
+static int backward_scaled_sums(const void *logits, int32_t dtype, const int64_t *labels,
+                                const float *sums, const float *grad_scalar, float scale,
+                                const int64_t *divide_by, void *grad_logits,
+                                int64_t n_size, int64_t dimsize, int64_t m_size,
+                                int64_t order, int64_t ignore_index, void *stream, bool planes16) {
     if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
     int rc = check_order(order);
     if (rc != PLH_OK) return rc;
-    if (!taylor_sums_apply(dtype_size(dtype), dimsize, m_size)) return PLH_ERR_BAD_SIZE;
+    if (!(planes16 ? planes16_apply : taylor_sums_apply)(dtype_size(dtype), dimsize, m_size)) return PLH_ERR_BAD_SIZE;
     if (n_size * dimsize * m_size != 0 && (!grad_scalar || !sums)) return PLH_ERR_NULL_POINTER;
     if (misaligned(grad_scalar, 4) || misaligned(divide_by, 8) || misaligned(sums, 4)) return PLH_ERR_MISALIGNED;
     const size_t es = dtype_size(dtype);
@@ -198,4 +198,45 @@ extern "C" int plh_taylor_ce_backward_scaled_sums(const void *logits, int32_t dt
     p.sums = (m_size > 1 && order > 4) ? nullptr : const_cast<float *>(sums);
     run(kTaylorCeBwd, dtype, logits, nullptr, labels, up, grad_logits, nullptr, kNone, p, (hipStream_t)stream);
     return check_launch();
+}
+
+extern "C" int plh_taylor_ce_forward_reduced_sums(const void *logits, int32_t dtype, const int64_t *labels,
+                                                  float *sums_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                                  void *workspace, int64_t workspace_bytes,
+                                                  int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                  int64_t order, int64_t ignore_index, void *stream) {
+    return forward_reduced_sums(logits, dtype, labels, sums_out, loss_out, n_valid_out, mean, workspace,
+                                workspace_bytes, n_size, dimsize, m_size, order, ignore_index, stream, false);
+}
+
+extern "C" int plh_taylor_ce_backward_scaled_sums(const void *logits, int32_t dtype, const int64_t *labels,
+                                                  const float *sums, const float *grad_scalar, float scale,
+                                                  const int64_t *divide_by, void *grad_logits,
+                                                  int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                  int64_t order, int64_t ignore_index, void *stream) {
+    return backward_scaled_sums(logits, dtype, labels, sums, grad_scalar, scale, divide_by, grad_logits, n_size,
+                                dimsize, m_size, order, ignore_index, stream, false);
+}
+
+extern "C" int plh_taylor_ce_saves_sums_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size) {
+    return dtype_ok(dtype) && n_size > 0 && dimsize > 0 && m_size > 0 &&
+                   planes16_apply(dtype_size(dtype), dimsize, m_size) ? 1 : 0;
+}
+
+extern "C" int plh_taylor_ce_forward_reduced_sums_planes16(const void *logits, int32_t dtype, const int64_t *labels,
+                                                           float *sums_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                                           void *workspace, int64_t workspace_bytes,
+                                                           int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                           int64_t order, int64_t ignore_index, void *stream) {
+    return forward_reduced_sums(logits, dtype, labels, sums_out, loss_out, n_valid_out, mean, workspace,
+                                workspace_bytes, n_size, dimsize, m_size, order, ignore_index, stream, true);
+}
+
+extern "C" int plh_taylor_ce_backward_scaled_sums_planes16(const void *logits, int32_t dtype, const int64_t *labels,
+                                                           const float *sums, const float *grad_scalar, float scale,
+                                                           const int64_t *divide_by, void *grad_logits,
+                                                           int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                           int64_t order, int64_t ignore_index, void *stream) {
+    return backward_scaled_sums(logits, dtype, labels, sums, grad_scalar, scale, divide_by, grad_logits, n_size,
+                                dimsize, m_size, order, ignore_index, stream, true);
 }

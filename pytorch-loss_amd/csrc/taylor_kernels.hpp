@@ -12,6 +12,7 @@
 //   loss_i = log S - log f(x_y),   grad_k = gout_i * (f'(x_k) / S - [k == y] f'(x_k) / f(x_k)).
 #pragma once
 #include "plh_common.hpp"
+#include "planes16.hpp"
 
 namespace plh {
 
@@ -41,6 +42,11 @@ inline bool taylor_sums_apply(size_t elem_bytes, int64_t dimsize, int64_t m_size
     if (dimsize > kMaxSplitChannels && dimsize <= kMaxDeepChannels) return true;
     if ((m_size * 4) % 128 == 0) return false;
     return image_form_pays<float>((int)dimsize, m_size) || (dimsize > kMaxRegsChannels && dimsize <= kMaxSplitChannels);
+}
+
+// Whether the forward leaves S: there, and for 16-bit channel planes (planes16_apply).
+inline bool taylor_keeps_sums(size_t elem_bytes, int64_t dimsize, int64_t m_size) {
+    return taylor_sums_apply(elem_bytes, dimsize, m_size) || planes16_apply(elem_bytes, dimsize, m_size);
 }
 
 // 1 / i! for i = 0..33; 34! does not fit fp32 (the reference's running factorial becomes inf there and
@@ -1121,6 +1127,23 @@ __global__ __launch_bounds__(256) void taylor_ce_bwd_planes(const T *__restrict_
     }
 }
 
+// The same for 16-bit logits (planes16_bwd).
+template <int ORD>
+struct TaylorPlaneOp {
+    float gk;
+    __device__ __forceinline__ void begin(float g) { gk = g; }
+    __device__ __forceinline__ float value(float sum) const { return gk / sum; }
+    __device__ __forceinline__ int label(int64_t lb, int64_t ignore, int C) const {
+        return lb != ignore && lb >= 0 && lb < C ? (int)lb : -1;    // pixels without a target: exact zeros (taylor_ce_bwd_regs)
+    }
+    __device__ __forceinline__ float grad(float x, float k, bool hot) const {
+        float f, df;
+        taylor_pair24<ORD>(x, f, df);
+        if (hot) k -= gk / f;
+        return df * k;
+    }
+};
+
 // ------------------------------------------------------------ dispatch ----
 
 template <class T, int Kind>
@@ -1154,6 +1177,14 @@ unsigned taylor_launch(const T *x, const T *g, const int64_t *lab, const Upstrea
             else
                 hipLaunchKernelGGL((taylor_ce_bwd_planes<T, 4>), grid, dim3(256), 0, st, x, lab, up, out, p, (int)tiles, per);
             return (unsigned)tiles_all;
+        }
+    }
+    if constexpr (Kind == kTaylorCeBwd && sizeof(T) == 2) {
+        if (p.sums && !go_vec && p.m_size > 1 && !walk && planes16_apply(sizeof(T), p.C, p.m_size)) {
+            const bool done = p.order == 2
+                ? planes16_launch(x, lab, p.sums, up, out, TaylorPlaneOp<2>{}, p.P, p.m_size, p.C, p.ignore, st)
+                : planes16_launch(x, lab, p.sums, up, out, TaylorPlaneOp<4>{}, p.P, p.m_size, p.C, p.ignore, st);
+            if (done) return 1;
         }
     }
     if constexpr (Kind == kTaylorCeBwd) {
@@ -1207,7 +1238,7 @@ unsigned taylor_launch(const T *x, const T *g, const int64_t *lab, const Upstrea
         const unsigned grid = image ? split_image_grid<VT>(p.P / p.m_size, p.m_size) : split_grid<VT>(p.P);
         // (the tiles-per-image forward that leaves the pixels' S has no per-pixel losses to write, so their slot serves)
         float *const loss_sp = (Kind == kTaylorCeFwd && shape == Shape::SplitImage && p.sums != nullptr && loss == nullptr &&
-                                taylor_sums_apply(sizeof(T), p.C, p.m_size)) ? p.sums : loss;
+                                taylor_keeps_sums(sizeof(T), p.C, p.m_size)) ? p.sums : loss;
 #define PLH_GO(KW, IMG)                                                                                               \
     do {                                                                                                              \
         if constexpr (Kind == kTaylorFwd)                                                                             \
@@ -1243,7 +1274,7 @@ unsigned taylor_launch(const T *x, const T *g, const int64_t *lab, const Upstrea
         const unsigned grid = vec ? regs_grid<VT>(p.P) : (image ? image_grid<4>(p.P / p.m_size, p.m_size) : regs_grid<1>(p.P));
         // (the per-image forward that leaves the pixels' S has no per-pixel losses to write, so their slot serves)
         float *const loss_px = (Kind == kTaylorCeFwd && image && p.sums != nullptr && loss == nullptr && p.m_size > 1 &&
-                                taylor_sums_apply(sizeof(T), p.C, p.m_size)) ? p.sums : loss;
+                                taylor_keeps_sums(sizeof(T), p.C, p.m_size)) ? p.sums : loss;
 #define PLH_GO(CPV, VV, UU)                                                                                          \
     do {                                                                                                             \
         if constexpr (Kind == kTaylorFwd)                                                                            \

@@ -58,6 +58,9 @@ _SIGNATURES = {
     "plh_lsr_saves_lse": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
     "plh_lsr_forward_reduced_lse": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_backward_scaled_lse": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
+    "plh_lsr_saves_lse_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
+    "plh_lsr_forward_reduced_lse_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
+    "plh_lsr_backward_scaled_lse_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lovasz_lookback_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "plh_lovasz_forward_lookback": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_lovasz_backward": (ctypes.c_int, [_p, _p, _i32, _p, _p, _p, _i64, _i64, _i64, _i64, _p]),
@@ -83,6 +86,9 @@ _SIGNATURES = {
     "plh_taylor_ce_saves_sums": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
     "plh_taylor_ce_forward_reduced_sums": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_taylor_ce_backward_scaled_sums": (ctypes.c_int, [_p, _i32, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
+    "plh_taylor_ce_saves_sums_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
+    "plh_taylor_ce_forward_reduced_sums_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p]),
+    "plh_taylor_ce_backward_scaled_sums_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_soft_dice_workspace_bytes": (_i64, [_i64, _i64]),
     "plh_soft_dice_forward": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i64, _i64, _i64, _f32, _f32, _p]),
     "plh_soft_dice_backward": (ctypes.c_int, [_p, _p, _i32, _p, _p, _p, _i64, _i64, _f32, _p]),
@@ -347,18 +353,25 @@ def lsr_backward_scaled(logits, labels, ignore_index, smooth, grad_scalar, divid
                                   grad_scalar, divide_by)
 
 
+def _planes16(a):
+    """What the entry points for 16-bit channel planes are called beside those for fp32 planes and rows."""
+    return "_planes16" if a.tag != 0 and a.m > 1 else ""
+
+
 def lsr_forward_reduced_lse(logits, labels, ignore_index, smooth, mean, args=None):
-    """lsr_forward_reduced that also keeps every pixel's log-sum-exp where the library's backward can use it (fp32
-    logits on channel planes of odd length, see plh_lsr_saves_lse). -> (loss, n_valid, lse or None)."""
+    """lsr_forward_reduced that also keeps every pixel's log-sum-exp where the library's backward can use it (channel
+    planes, long rows: see plh_lsr_saves_lse, and for 16-bit logits plh_lsr_saves_lse_planes16).
+    -> (loss, n_valid, lse or None)."""
     a = args or lsr_args(logits, labels)
-    if a.x.numel() == 0 or not load().plh_lsr_saves_lse(a.tag, a.n, a.c, a.m):
+    planes = _planes16(a)
+    if a.x.numel() == 0 or not getattr(load(), "plh_lsr_saves_lse" + planes)(a.tag, a.n, a.c, a.m):
         return _pixel_forward_reduced("plh_lsr_forward_reduced", a, ignore_index, smooth, mean) + (None,)
     dev = a.x.device
     loss = torch.empty((), dtype=torch.float32, device=dev)
     n_valid = torch.empty((), dtype=torch.int64, device=dev)
     lse = torch.empty((a.n * a.m,), dtype=torch.float32, device=dev)
     ws, ws_bytes = _reduce_workspace(a.n * a.m, dev)
-    _call(a.x, "plh_lsr_forward_reduced_lse", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(loss), _ptr(n_valid),
+    _call(a.x, "plh_lsr_forward_reduced_lse" + planes, _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(loss), _ptr(n_valid),
           1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m, int(ignore_index), float(smooth))
     return _back_to(loss, _loss_dtype(a.dtype)), n_valid, lse
 
@@ -368,6 +381,10 @@ def lsr_backward_scaled_lse(lse, ignore_index, smooth, grad_scalar, divide_by, a
     a = args
     grad = torch.empty_like(a.x)
     go = _scalar_f32(grad_scalar)
+    if _planes16(a):                    # (no mask there: `kept` comes from losses that do not keep the log-sum-exp)
+        _call(a.x, "plh_lsr_backward_scaled_lse_planes16", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(go), 1.0, _ptr(divide_by),
+              _ptr(grad), a.n, a.c, a.m, int(ignore_index), float(smooth))
+        return _back_to(grad, a.dtype)
     _call(a.x, "plh_lsr_backward_scaled_lse", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(kept) if kept is not None else None,
           _ptr(go), 1.0, _ptr(divide_by), _ptr(grad), a.n, a.c, a.m, int(ignore_index), float(smooth))
     return _back_to(grad, a.dtype)
@@ -770,11 +787,13 @@ def taylor_ce_forward(logits, labels, n, ignore_index, reduction, args=None):
 
 
 def taylor_ce_forward_reduced_sums(logits, labels, n, ignore_index, mean, args=None):
-    """The reduced forward that also leaves each row's sum of f for the backward, where the shape has a backward that
-    uses it (long (N, C) rows, see plh_taylor_ce_saves_sums). -> (loss, n_valid, sums or None)."""
+    """The reduced forward that also leaves each row's (pixel's) sum of f for the backward, where the shape has a backward
+    that uses it (see plh_taylor_ce_saves_sums, and for 16-bit planes plh_taylor_ce_saves_sums_planes16).
+    -> (loss, n_valid, sums or None)."""
     _check_order(n)
     a = args or taylor_args(logits, labels)
-    if a.x.numel() == 0 or not load().plh_taylor_ce_saves_sums(a.tag, a.n, a.c, a.m):
+    planes = _planes16(a)
+    if a.x.numel() == 0 or not getattr(load(), "plh_taylor_ce_saves_sums" + planes)(a.tag, a.n, a.c, a.m):
         loss, n_valid = taylor_ce_forward(logits, labels, n, ignore_index, "mean" if mean else "sum", args=a)
         return loss, n_valid, None
     dev = a.x.device
@@ -782,7 +801,7 @@ def taylor_ce_forward_reduced_sums(logits, labels, n, ignore_index, mean, args=N
     n_valid = torch.empty((), dtype=torch.int64, device=dev)
     sums = torch.empty((a.n * a.m,), dtype=torch.float32, device=dev)
     ws, ws_bytes = _reduce_workspace(a.n * a.m, dev)
-    _call(a.x, "plh_taylor_ce_forward_reduced_sums", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(loss), _ptr(n_valid),
+    _call(a.x, "plh_taylor_ce_forward_reduced_sums" + planes, _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(loss), _ptr(n_valid),
           1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m, int(n), int(ignore_index))
     return _back_to(loss, _loss_dtype(a.dtype)), n_valid, sums
 
@@ -792,7 +811,7 @@ def taylor_ce_backward_scaled_sums(sums, n, ignore_index, grad_scalar, divide_by
     a = args
     grad = torch.empty_like(a.x)
     go = _scalar_f32(grad_scalar)
-    _call(a.x, "plh_taylor_ce_backward_scaled_sums", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(go), 1.0,
+    _call(a.x, "plh_taylor_ce_backward_scaled_sums" + _planes16(a), _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(go), 1.0,
           _ptr(divide_by), _ptr(grad), a.n, a.c, a.m, int(n), int(ignore_index))
     return _back_to(grad, a.dtype)
 
