@@ -60,6 +60,20 @@ __device__ __forceinline__ float key_error(uint32_t key) {
     return __builtin_bit_cast(float, kOne - (key & 0x7FFFFFFFu));
 }
 
+// e / s for the exponentials e in [0, 1] of a pixel and their sum s in [1, 512): the division operator's own steps (Newton's on
+// the reciprocal, once per pixel, and two residuals) less its scaling, which operands from 2^-100 on pass through unchanged.
+struct BySum {
+    float s, y;
+    __device__ __forceinline__ explicit BySum(float sum) : s(sum), y(__builtin_amdgcn_rcpf(sum)) {
+        y = __builtin_fmaf(__builtin_fmaf(-s, y, 1.f), y, y);
+    }
+    __device__ __forceinline__ float operator()(float e) const {
+        float q = e * y;
+        q = __builtin_fmaf(__builtin_fmaf(-s, q, e), y, q);
+        return __builtin_fmaf(__builtin_fmaf(-s, q, e), y, q);
+    }
+};
+
 // ------------------------------------------------------ 1. build keys ----
 
 // Besides the keys, both kernels leave per block and class the largest key among the block's
@@ -166,13 +180,14 @@ __global__ __launch_bounds__(kRegsBlock) void lov_keys_regs(const T *__restrict_
                 s += v[j][k];
             }
         const bool ign = (lb[k] == ignore);
+        const BySum share(s);
         uint32_t key_y = 0;                     // the positive's key, if the pixel has one
         bool has_y = false;
 #pragma unroll
         for (int j = 0; j < CP; ++j)
             if (chan_ok<CP>(j, C)) {
                 const bool hot = (lb[k] == j);
-                const uint32_t key = make_key(v[j][k] / s, hot, ign);
+                const uint32_t key = make_key(share(v[j][k]), hot, ign);
                 key_y = hot ? key : key_y;
                 has_y = has_y || hot;
                 v[j][k] = __builtin_bit_cast(float, key);
@@ -1114,11 +1129,12 @@ __global__ __launch_bounds__(kRegsBlock) void lov_bwd_regs(const float *__restri
                 v[j][k] = expf(v[j][k] - mx);
                 s += v[j][k];
             }
+        const BySum share(s);
         float dot = 0.f;
 #pragma unroll
         for (int j = 0; j < CP; ++j)
             if (chan_ok<CP>(j, C)) {
-                v[j][k] = v[j][k] / s;
+                v[j][k] = share(v[j][k]);
                 const float dj = d[j][k] * gout[j];
                 d[j][k] = (lb[k] == j) ? -dj : dj;
                 dot += v[j][k] * d[j][k];

@@ -17,8 +17,8 @@
 // A key moves 28 bytes: read and written by bk_cut, bk_rank and bk_restore, and a place of 2 bytes. The form before this one
 // wrote the buckets out one after the other: that takes a histogram first (6 bytes a key more, buckets kept for the second
 // pass) and writes of some 10 keys, where a segment of a run has 24 here. (4,19,512,1024) fp32: histogram and scatter
-// 67 + 117 us against 102 now, rank 119 against 111, gather 72 against 57, step 557 -> 436 us; (8,21,513,513) bf16 trained
-// 77 + 154 against 137, 217 against 227, 116 against 68, step 795 -> 614. Which rows come here: bk_pays.
+// 67 + 117 us against 96 now, rank 119 against 111, gather 72 against 57, step 557 -> 436 us; (8,21,513,513) bf16 trained
+// 77 + 154 against 127, 217 against 224, 116 against 68, step 792 -> 608. Which rows come here: bk_pays.
 #pragma once
 
 namespace plh {
@@ -31,7 +31,7 @@ constexpr int kBkTile = kBkThreads * kBkTileItems;  // keys of a tile
 constexpr int kBkWaves = kBkThreads / kWave;
 constexpr int kBkChunk = 16;                        // neighbours in the order that one thread sorts
 constexpr int kBkBins = 4096;                       // bins of a run's value range
-constexpr int kBkFineBits = 11;                     // table from a key's top bits to the first bucket it can be in
+constexpr int kBkFineBits = 13;                     // table from a key's top bits to the first bucket it can be in
 constexpr int kBkFine = 1 << kBkFineBits;
 constexpr int kBkTarget = 2560;                     // mean keys per bucket: sampled bounds leave few above kBkCap
 constexpr int kBkSlab = 6144;                       // buckets that start in one such part of the row are sorted together
@@ -653,9 +653,10 @@ __device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
 
 // The tile's keys in the order of their buckets (in pixel order inside one), in the place of its keys, and every pixel's place
 // in that order.
-// Bound by vector and LDS instructions, 70 and 15 per 64 keys (nearly all taking part: 78 of 137 us of vector issue), at 24 waves
-// per CU. Match masks of 10 votes for every key were 126 per 64 keys (149 -> 102 us at (4,19,512,1024) fp32, 177 -> 137 at
-// (8,21,513,513) bf16 trained); a wave's 64 keys lie in up to 1024 buckets, so that some 5 of them meet another.
+// Bound by vector and LDS instructions, 68 and 13 per 64 keys (two thirds of the time at 24 waves per CU). Match masks of 10
+// votes for every key were 126 (149 -> 102 us at (4,19,512,1024) fp32, 177 -> 137 at (8,21,513,513) bf16 trained); a wave's 64 keys
+// lie in up to 1024 buckets, so that some 5 of them meet another. A look-up table of 13 bits instead of 11 leaves two steps
+// less to the search (100 -> 96, 133 -> 127).
 template <int kBits>
 __global__ __launch_bounds__(kBkThreads, 6) void bk_cut(const BucketArgs a) {
     constexpr int kStride = 1 << kBits, kPer = (kStride + kBkThreads - 1) / kBkThreads, kChunks = kBkTile / kWave;
@@ -691,30 +692,30 @@ __global__ __launch_bounds__(kBkThreads, 6) void bk_cut(const BucketArgs a) {
     constexpr int kFind = 8;
 #pragma unroll
     for (int r = 0; r < kBkTileItems; r += kFind) s.look.template find<kFind>(key + r, limit, shift, first_step, b + r);
-    // A key's rank among the wave's keys of its bucket: the counter, moved on by every key, tells what came in earlier rounds
-    // and how many come in this one. LDS takes a wave's operations in their order, so the rounds of a group wait for nothing.
-    // The few that meet others of their round find their place by a vote per bucket met twice; many, by a vote per bit.
+    // A key's rank among the wave's keys of its bucket: the counter tells what came in earlier rounds, and whether every key of
+    // this one moved it on from there. LDS takes a wave's operations in their order, so the rounds of a group wait for nothing.
+    // The few that meet others of their round (whichever of them LDS took first) find their place by a vote per bucket met
+    // twice; many, by a vote per bit.
     constexpr int kGroup = 2;
     constexpr uint32_t kFew = 16;
     uint16_t *mine_of = counts[wave];
 #pragma unroll
     for (int r0 = 0; r0 < kBkTileItems; r0 += kGroup) {
-        uint32_t after[kGroup];
+        uint32_t moved[kGroup];
 #pragma unroll
         for (int h = 0; h < kGroup; ++h) {
             const uint32_t d = b[r0 + h];
             rank[r0 + h] = mine_of[d];
             asm volatile("" ::: "memory");
+            moved[h] = 0;
             if (d != (uint32_t)kStride)         // additions to one address take their turns
-                atomicAdd(reinterpret_cast<uint32_t *>(mine_of) + (d >> 1), 1u << (16u * (d & 1u)));
-            asm volatile("" ::: "memory");
-            after[h] = mine_of[d];
+                moved[h] = atomicAdd(reinterpret_cast<uint32_t *>(mine_of) + (d >> 1), 1u << (16u * (d & 1u)));
             asm volatile("" ::: "memory");
         }
 #pragma unroll
         for (int h = 0; h < kGroup; ++h) {
             const uint32_t d = b[r0 + h], seen = rank[r0 + h];
-            uint64_t met = __builtin_amdgcn_ballot_w64(after[h] - seen > 1u && d != (uint32_t)kStride);
+            uint64_t met = __builtin_amdgcn_ballot_w64(d != (uint32_t)kStride && ((moved[h] >> (16u * (d & 1u))) & 0xFFFFu) != seen);
             bool first = true;
             while (met && (first || __builtin_popcountll(met) <= kFew)) {   // wave-uniform
                 const uint32_t one = (uint32_t)__builtin_amdgcn_readlane((int)d, __builtin_ctzll(met));
