@@ -13,7 +13,7 @@
 //                     (class, pixel):  bit 31 = positive flag, bits 0..30 = 0x3F800000 - bits(e)
 //                     (ascending key order = descending error; e lies in [0,1] so its bit
 //                     pattern is monotone), ignored pixel = 0x7FFFFFFF (sorts last). Also the
-//                     largest positive key per class (per-block table + lov_class_max): keys
+//                     largest positive key per class (per-block table + class_top): keys
 //                     beyond it have dJ = 0 exactly and are left out of the sort (keep_key).
 //   2.-4. for the rows that bk_pays names: by value buckets, see lovasz_buckets.hpp. Otherwise, and in the look-back
 //                     variant, with the same differences bit for bit:
@@ -77,56 +77,47 @@ struct BySum {
 // ------------------------------------------------------ 1. build keys ----
 
 // Besides the keys, both kernels leave per block and class the largest key among the block's
-// positives of that class, plus 1 (0 = none), in block_table[C][block]; lov_class_max folds the
+// positives of that class, plus 1 (0 = none), in block_table[C][block]; class_top folds the
 // table into pos_max[c], the error of the class's lowest-ranked positive. Everything sorted after
 // that one has a Jaccard difference of exactly 0 (see keep_key), so the sort never sees it.
-__device__ __forceinline__ void publish_block_max(const uint32_t *block_max, uint32_t *block_table, int C) {
+__device__ __forceinline__ void publish_block_max(const uint32_t *block_max, uint32_t *block_table, uint32_t *all_min, int C) {
+    if (blockIdx.x == 0)
+        for (int j = threadIdx.x; j < C; j += blockDim.x) all_min[j] = 0xFFFFFFFFu;     // see absent_min
     for (int j = threadIdx.x; j < C; j += blockDim.x) block_table[(int64_t)j * gridDim.x + blockIdx.x] = block_max[j];
 }
 
-// It also leaves, per class, the number of key bits the sort has to look at: keys that take part are
-// not above the limit, so the bits above the limit's highest set bit are zero in every one of them.
-// The body for the block of class c: kThreads threads, each with kThreads / 64 words of `wave_max`.
+// The largest entry of class c's row of the table, for the whole block of kThreads threads; kThreads / 64 words of `waves`.
 template <int kThreads>
-__device__ __forceinline__ void class_max(const uint32_t *__restrict__ block_table, int blocks, int C, int c, uint32_t *__restrict__ pos_max,
-                                          uint32_t *wave_max) {
+__device__ __forceinline__ uint32_t class_top(const uint32_t *__restrict__ block_table, int blocks, int c, uint32_t *waves) {
     const uint32_t *row = block_table + (int64_t)c * blocks;
     uint32_t m = 0;
 #pragma unroll 8
     for (int b = threadIdx.x; b < blocks; b += kThreads) m = max(m, row[b]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-    if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t top = 0;
 #pragma unroll
-        for (int w = 0; w < kThreads / 64; ++w) top = max(top, wave_max[w]);
-        pos_max[c] = top;
-        pos_max[2 * C + c] = 0xFFFFFFFFu;       // all_min[c], for absent_min
-        // key_bits[c]: a class without positives keeps a single key value, wherever it lies
-        pos_max[3 * C + c] = (top > 1u) ? (uint32_t)(32 - __builtin_clz(top - 1u)) : (top ? 1u : 30u);
-    }
+    for (int w = 0; w < kThreads / 64; ++w) m = max(m, waves[w]);
+    __syncthreads();
+    return m;
 }
 
-__global__ __launch_bounds__(1024) void lov_class_max(const uint32_t *__restrict__ block_table, int blocks, int C,
-                                                     uint32_t *__restrict__ pos_max, uint32_t *__restrict__ cursors,
-                                                     int regions) {
-    __shared__ uint32_t wave_max[16];
-    const int c = blockIdx.x;
-    // the class's staging cursors start at zero (they are first used by the last pass)
-    for (int i = threadIdx.x; i < regions; i += 1024) cursors[(int64_t)c * regions + i] = 0;
-    class_max<1024>(block_table, blocks, C, c, pos_max, wave_max);
+// It also leaves, per class, the number of key bits the sort has to look at: keys that take part are
+// not above the limit, so the bits above the limit's highest set bit are zero in every one of them.
+__device__ __forceinline__ void publish_class(uint32_t *__restrict__ pos_max, int C, int c, uint32_t top) {
+    pos_max[c] = top;
+    // key_bits[c]: a class without positives keeps a single key value, wherever it lies
+    pos_max[3 * C + c] = (top > 1u) ? (uint32_t)(32 - __builtin_clz(top - 1u)) : (top ? 1u : 30u);
 }
 
 // A class without positives has J = 1 from the first sorted key on: only its largest error (smallest
-// key) has a non-zero Jaccard difference. For such classes (blocks of the others return at once)
-// this finds the smallest key of the row, which then serves as the class's limit. Block `block` of kAbsentBlocks.
+// key) has a non-zero Jaccard difference. For such classes this finds the smallest key of the row, which then serves as
+// the class's limit; all_min starts at the largest word (lov_keys_*). Block `block` of kAbsentBlocks.
 constexpr int kAbsentBlocks = 64;
 template <int kThreads>
-__device__ __forceinline__ void absent_min(const uint32_t *__restrict__ keys, const uint32_t *pos_max, uint32_t *all_min, int P,
-                                           int c, int block, uint32_t *wave_min) {
-    if (pos_max[c] != 0) return;                // block-uniform
+__device__ __forceinline__ void absent_min(const uint32_t *__restrict__ keys, uint32_t *all_min, int P, int c, int block,
+                                           uint32_t *wave_min) {
     const uint32_t *row = keys + (int64_t)c * P;
     uint32_t m = 0xFFFFFFFFu;
 #pragma unroll 8
@@ -141,16 +132,23 @@ __device__ __forceinline__ void absent_min(const uint32_t *__restrict__ keys, co
         atomicMin(all_min + c, m);
     }
 }
-__global__ __launch_bounds__(256) void lov_absent_min(const uint32_t *__restrict__ keys, const uint32_t *pos_max,
-                                                      uint32_t *all_min, int P) {
-    __shared__ uint32_t wave_min[4];
-    absent_min<256>(keys, pos_max, all_min, P, (int)blockIdx.y, (int)blockIdx.x, wave_min);
+
+// Both for the radix passes, every block finding its class's largest entry for itself (a launch of its own for that took
+// 5 us), and the class's staging cursors at zero (they are first used by the last pass).
+__global__ __launch_bounds__(256) void lov_limits(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ block_table, int blocks,
+                                                  int C, uint32_t *__restrict__ pos_max, int P, uint32_t *__restrict__ cursors, int regions) {
+    __shared__ uint32_t waves[4];
+    const int c = blockIdx.y;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < regions; i += kAbsentBlocks * 256) cursors[(int64_t)c * regions + i] = 0;
+    const uint32_t top = class_top<256>(block_table, blocks, c, waves);
+    if (blockIdx.x == 0 && threadIdx.x == 0) publish_class(pos_max, C, c, top);
+    if (top == 0) absent_min<256>(keys, pos_max + 2 * C, P, c, (int)blockIdx.x, waves);        // block-uniform
 }
 
 template <class T, int CP, int V>
 __global__ __launch_bounds__(kRegsBlock) void lov_keys_regs(const T *__restrict__ x, const int64_t *__restrict__ lab,
                                                            uint32_t *__restrict__ keys, uint32_t *__restrict__ block_table,
-                                                           int64_t P, int64_t m_size, int C,
+                                                           uint32_t *__restrict__ all_min, int64_t P, int64_t m_size, int C,
                                                            int64_t ignore, unsigned xcd_run) {
     __shared__ uint32_t block_max[kMaxRegsChannels];
     if (threadIdx.x < kMaxRegsChannels) block_max[threadIdx.x] = 0;
@@ -201,14 +199,14 @@ __global__ __launch_bounds__(kRegsBlock) void lov_keys_regs(const T *__restrict_
             if (chan_ok<CP>(j, C)) store_vec_cached<V>(reinterpret_cast<float *>(keys) + (int64_t)j * P + pix, v[j]);
     }
     __syncthreads();
-    publish_block_max(block_max, block_table, C);
+    publish_block_max(block_max, block_table, all_min, C);
 }
 
 // Any channel count: a lane per pixel, three sweeps over the slice (the later ones hit cache).
 template <class T>
 __global__ __launch_bounds__(256) void lov_keys_lane(const T *__restrict__ x, const int64_t *__restrict__ lab,
                                                      uint32_t *__restrict__ keys, uint32_t *__restrict__ block_table,
-                                                     int64_t P, int64_t m_size, int C, int64_t ignore) {
+                                                     uint32_t *__restrict__ all_min, int64_t P, int64_t m_size, int C, int64_t ignore) {
     __shared__ uint32_t block_max[512];              // C < 512
     for (int j = threadIdx.x; j < C; j += 256) block_max[j] = 0;
     __syncthreads();
@@ -230,7 +228,7 @@ __global__ __launch_bounds__(256) void lov_keys_lane(const T *__restrict__ x, co
         }
     }
     __syncthreads();
-    publish_block_max(block_max, block_table, C);
+    publish_block_max(block_max, block_table, all_min, C);
 }
 
 // --------------------------------------------------- 2. radix sort pass ----
@@ -264,7 +262,7 @@ struct SortArgs {
 };
 
 // The digits of a class. Keys that take part in a class's sort are below 2^bits (bits from the
-// class's limit, lov_class_max), so the sort runs over `bits` bits only: in 2, 3 or 4 stable passes
+// class's limit, publish_class), so the sort runs over `bits` bits only: in 2, 3 or 4 stable passes
 // of at most kRadixBits bits each, the first passes - 1 of them scatter passes and the last one
 // fused with the Jaccard step (16 bits or fewer, i.e. a best positive's error above 0.99: two
 // passes; up to 24 bits, error above 0.008: three). The bits are shared out evenly: 27 bits (best
@@ -1304,25 +1302,8 @@ extern "C" int64_t plh_lovasz_lookback_workspace_bytes(int64_t n_size, int64_t d
     return rc == PLH_OK ? pl.bytes : (int64_t)rc;
 }
 
-// 2. and 3. for rows that one block ranks whole: the keys in keys_0 (jacc's memory) become the Jaccard differences.
-static int lovasz_blocks(const LovaszPlan &pl, uint32_t *keys_0, uint32_t *pos_max, float *losses, int C, hipStream_t st) {
-    BucketArgs a = {};
-    a.keys = keys_0;
-    a.pos_max = pos_max;
-    a.P = (int)pl.P;
-    a.C = C;
-    hipLaunchKernelGGL(bk_rank<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);
-    return check_launch();
-}
-
-// The same by value buckets, and the classes' limits (pos_max) before them.
-static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, uint32_t *pos_max, const uint32_t *block_table,
-                          int key_blocks, float *losses, int C, hipStream_t st) {
-    BucketArgs a = {};
-    a.keys = keys_0;
-    a.pos_max = pos_max;
-    a.P = (int)pl.P;
-    a.C = C;
+// 2. and 3. by value buckets: the keys in a.keys (jacc's memory) become the Jaccard differences; the classes' limits before that.
+static int lovasz_buckets(const LovaszPlan &pl, char *ws, BucketArgs a, float *losses, int C, hipStream_t st) {
     a.tiles = pl.bk_tiles;
     a.stride = 1 << pl.bk_bits;
     const int64_t step = round_up(4 * (((int64_t)C << pl.bk_bits) + C), 256);
@@ -1344,7 +1325,7 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, uint32_t *keys_0, uint
     const unsigned most = (unsigned)ceil_div(pl.P, kBkTarget) + 1;  // buckets a class can have
     // two blocks fit a CU; each takes every so many of the class's crowded runs
     const unsigned crowded_blocks = (unsigned)(ceil_div(1024, C) < most ? ceil_div(1024, C) : most);
-    hipLaunchKernelGGL(bk_sample, dim3(1 + kBkItems, (unsigned)C), threads, 0, st, a, block_table, key_blocks);
+    hipLaunchKernelGGL(bk_sample, dim3(1 + kBkItems, (unsigned)C), threads, 0, st, a);
     hipLaunchKernelGGL(bk_split, dim3((1 + kAbsentBlocks) * (unsigned)C), threads, 0, st, a);
     switch (pl.bk_bits) {
 #define PLH_BUCKETS(B)                                                                                               \
@@ -1402,9 +1383,9 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
 #define PLH_CASE(K)                                                                                                 \
     case K:                                                                                                         \
         if (vec) hipLaunchKernelGGL((lov_keys_regs<T, 4 * K, VT>), dim3(grid), dim3(kRegsBlock), 0, st, x, labels,  \
-                                    keys_0, block_table, pl.P, m_size, C, ignore_index, run);                       \
+                                    keys_0, block_table, all_min, pl.P, m_size, C, ignore_index, run);                       \
         else hipLaunchKernelGGL((lov_keys_regs<T, 4 * K, 1>), dim3(grid), dim3(kRegsBlock), 0, st, x, labels,       \
-                                keys_0, block_table, pl.P, m_size, C, ignore_index, run);                           \
+                                keys_0, block_table, all_min, pl.P, m_size, C, ignore_index, run);                           \
         break;
                 PLH_CASE(1) PLH_CASE(2) PLH_CASE(3) PLH_CASE(4) PLH_CASE(5) PLH_CASE(6) PLH_CASE(7) PLH_CASE(8)
 #undef PLH_CASE
@@ -1412,17 +1393,24 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
         } else {
             key_blocks = group_grid(pl.P, 256);
             hipLaunchKernelGGL(lov_keys_lane<T>, dim3(key_blocks), dim3(256), 0, st, x, labels, keys_0, block_table,
-                               pl.P, m_size, C, ignore_index);
+                               all_min, pl.P, m_size, C, ignore_index);
         }
     });
-    if (pl.buckets && pl.bk_bits) return lovasz_buckets(pl, ws, keys_0, pos_max, block_table, (int)key_blocks, losses, C, st);
+    if (pl.buckets) {
+        BucketArgs a = {};
+        a.keys = keys_0;
+        a.pos_max = pos_max;
+        a.block_table = block_table;
+        a.key_blocks = (int)key_blocks;
+        a.P = (int)pl.P;
+        a.C = C;
+        if (pl.bk_bits) return lovasz_buckets(pl, ws, a, losses, C, st);
+        hipLaunchKernelGGL(bk_rank<true>, dim3((unsigned)C), dim3(kBkThreads), 0, st, a, losses);      // rows that one block ranks whole
+        return check_launch();
+    }
     uint32_t *cursors = pl.regions > 0 ? reinterpret_cast<uint32_t *>(ws + pl.off_cursors) : nullptr;
-    hipLaunchKernelGGL(lov_class_max, dim3((unsigned)C), dim3(1024), 0, st, block_table, (int)key_blocks, C, pos_max, cursors,
-                       pl.regions);
-    hipLaunchKernelGGL(lov_absent_min, dim3(kAbsentBlocks, (unsigned)C), dim3(256), 0, st, keys_0, pos_max, all_min,
-                       (int)pl.P);
-
-    if (pl.buckets) return lovasz_blocks(pl, keys_0, pos_max, losses, C, st);
+    hipLaunchKernelGGL(lov_limits, dim3(kAbsentBlocks, (unsigned)C), dim3(256), 0, st, keys_0, block_table, (int)key_blocks, C, pos_max,
+                       (int)pl.P, cursors, pl.regions);
 
     // what the plan lays out for the radix passes only
     uint32_t *keys_a = reinterpret_cast<uint32_t *>(ws + pl.off_keys_a);
@@ -1522,7 +1510,7 @@ static int lovasz_forward(const void *logits, int32_t dtype, const int64_t *labe
                            pl.tiles_pad, key_bits, kLastPass, kept, (int)pl.P);
     }
     if (pl.regions > 0) {
-        // the cursors were zeroed by lov_class_max
+        // the cursors were zeroed by lov_limits
         // the value buffer that a class's last pass does not read receives the pixel offsets that go with
         // the staged values
         if (pl.look_back)

@@ -44,7 +44,8 @@ constexpr uint16_t kBkNowhere = 0xFFFFu;            // place of a pixel that tak
 struct BucketArgs {
     uint32_t *keys;             // [C][P] in pixel order; bk_cut leaves every tile's keys by bucket, the rank kernels a key's Jaccard
                                 // difference in its place, bk_restore those in pixel order (jacc's memory)
-    uint32_t *pos_max;          // pos_max[C], kept[C], all_min[C], key_bits[C] (see keep_key, lov_class_max)
+    uint32_t *pos_max;          // pos_max[C], kept[C], all_min[C], key_bits[C] (see keep_key, publish_class); not for a row of one block
+    const uint32_t *block_table;        // [C][key_blocks] largest positive key plus 1 that a block of lov_keys_* met
     uint16_t *place;            // [C][P] every pixel's place in its tile's order
     uint32_t *sorted, *dj;      // [C][P] keys and differences of the wide buckets; in dj's memory first the
                                 // sample, [C][kBkCap]
@@ -59,7 +60,7 @@ struct BucketArgs {
                                 // first step of the search in `bounds`, wide buckets, flat buckets, crowded runs
     uint16_t *fine;             // [C][kBkFine] bucket of the least key with these top bits
     double *loss_part;          // [C][2 * stride]: runs, from `stride` on large buckets
-    int P, C, tiles, stride;
+    int P, C, tiles, stride, key_blocks;
 };
 
 __device__ __forceinline__ uint32_t bk_limit(const BucketArgs &a, int c) {
@@ -474,11 +475,12 @@ __device__ __forceinline__ void bk_ranks_crowded(BkShared &s, const uint32_t (&k
 
 // A class's limit, and kBkCap sampled keys, one from each of as many equal parts of the row. The sample lies anywhere in memory:
 // by 15 blocks beside the one for the limit 3 us, by the one that sorts it 10.
-__global__ __launch_bounds__(kBkThreads) void bk_sample(const BucketArgs a, const uint32_t *__restrict__ block_table, int key_blocks) {
+__global__ __launch_bounds__(kBkThreads) void bk_sample(const BucketArgs a) {
     __shared__ uint32_t wave_max[kBkWaves];
     const int c = blockIdx.y;
     if (blockIdx.x == 0) {                                  // block-uniform
-        class_max<kBkThreads>(block_table, key_blocks, a.C, c, a.pos_max, wave_max);
+        const uint32_t top = class_top<kBkThreads>(a.block_table, a.key_blocks, c, wave_max);
+        if (threadIdx.x == 0) publish_class(a.pos_max, a.C, c, top);
         return;
     }
     const uint32_t part = (uint32_t)a.P / kBkCap;           // >= 1: shorter rows are not cut
@@ -494,11 +496,11 @@ __global__ __launch_bounds__(kBkThreads) void bk_sample(const BucketArgs a, cons
 __global__ __launch_bounds__(kBkThreads) void bk_split(const BucketArgs a) {
     __shared__ BkShared s;
     const int c = (int)blockIdx.x % a.C, turn = (int)blockIdx.x / a.C;
+    const bool absent = a.pos_max[c] == 0u;
     if (turn > 0) {                                         // block-uniform
-        absent_min<kBkThreads>(a.keys, a.pos_max, a.pos_max + 2 * a.C, a.P, c, turn - 1, s.least);
+        if (absent) absent_min<kBkThreads>(a.keys, a.pos_max + 2 * a.C, a.P, c, turn - 1, s.least);
         return;
     }
-    const bool absent = a.pos_max[c] == 0u;
     const uint32_t limit = a.pos_max[c] - 1u;               // not for an absent class
     uint32_t key[kBkItems], valid = 0, mine = 0;
 #pragma unroll
@@ -1382,7 +1384,7 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
         return;
     }
     uint32_t *kin = a.keys + row;                           // the differences take the keys' places
-    const uint32_t limit = bk_limit(a, c);
+    uint32_t limit = Direct ? 0u : bk_limit(a, c);
     float npos = Direct ? 0.f : (float)a.numbers[2 * a.C + c];
     if constexpr (!Direct) at.collect(tile, 0u, s.scan);
 
@@ -1409,6 +1411,12 @@ __global__ __launch_bounds__(kBkThreads, 4) void bk_rank(const BucketArgs a, flo
         for (int i = 0; i < kBkGroup; ++i) key[r0 + i] = kin[from[i]];
     }
     if constexpr (Direct) {
+        const uint32_t top = class_top<kBkThreads>(a.block_table, a.key_blocks, c, s.crowd);
+        limit = top - 1u;
+        if (top == 0u) {                                    // block-uniform: a class without positives, see absent_min
+            bk_range(s, key, (1u << count) - 1u, least, most);
+            limit = min(least, kOne);
+        }
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r)
             if (r < count && keep_key(key[r], limit)) valid |= 1u << r;
