@@ -1207,20 +1207,25 @@ static int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 // logits (soft, a new network's, all equal, confident by 8 / 14 / 20, trained, bf16, in steps of 1/16): the ordinary one and the
 // one that buckets like least, mostly a network so sure that thousands of keys share a value (multiples of 2^-24 below 1)
 // and have to be sorted apart in LDS, by few blocks if the classes are few.
-//   one block per row: always (two classes of 7680 pixels 88 -> 49, at worst 90 -> 75)
-//   2 classes of 262144 97 -> 104, at worst 102 -> 180; 4 of 263169 116 -> 108, 119 -> 182; 8 of 262144 132 -> 121, 142 -> 186
-//   16 of 65536 112 -> 95, 131 -> 164; of 262144 168 -> 140, 210 -> 210; of 524288 234 -> 189, 328 -> 279
-//   12 of 262144 155 -> 135, 189 -> 211; of 524288 205 -> 171, 242 -> 241
-//   24 of 65536 132 -> 102, 151 -> 163; of 131072 154 -> 118, 195 -> 195
-//   8 of 524288 173 -> 155, 197 -> 213; of 1048576 271 -> 216, 303 -> 289; 6 of 2097152 369 -> 293, 424 -> 432
-//   32 of 8192 113 -> 88, 131 -> 115; of 65536 141 -> 110, 166 -> 165; 64 of 8192 182 -> 140, 166 -> 142
-// P C^2 >= 2^26 and C >= 32 leave out what may lose. (On rows of some 2 M pixels a new network's predictions, whose keys mostly
-// take no part, are level: (8,19,512,512) 419 -> 421, (8,21,513,513) 496 -> 510.)
+//   one block per row: always (two classes of 7680 pixels 86 -> 39, at worst 87 -> 60)
+//   P C^2 >= 2^26, or C >= 32:
+//   16 of 262144 164 -> 124, at worst 203 -> 199; of 524288 226 -> 162, 320 -> 245; 12 of 524288 202 -> 147, 239 -> 219
+//   24 of 131072 147 -> 106, 187 -> 183; 8 of 1048576 262 -> 183, 295 -> 269; 6 of 2097152 356 -> 231, 405 -> 365
+//   32 of 8192 108 -> 70, 127 -> 103; of 65536 135 -> 98, 157 -> 151; 64 of 8192 179 -> 125, 165 -> 127
+//   19 of 2097152 751 -> 443, 415 -> 322
+//   below that, 12 classes and more of 131072 pixels and more where P C^2 >= 5 2^23:
+//   13 of 262144 158 -> 121, 192 -> 195; 14 of 342000 182 -> 142, 231 -> 217; 12 of 448000 192 -> 147, 225 -> 196
+//   16 of 200704 148 -> 119, 183 -> 184; 18 of 147456 145 -> 117, 174 -> 179; 19 of 131072 144 -> 108, 178 -> 169
+//   left out, for what they lose at worst: 2 of 262144 94 -> 89, 100 -> 159; 4 of 263169 115 -> 95, 115 -> 155; 8 of 262144
+//   128 -> 106, 136 -> 169; 8 of 524288 168 -> 133, 184 -> 212; 10 of 524288 195 -> 143, 221 -> 232; 12 of 262144 151 -> 118,
+//   184 -> 193; 14 of 200000 147 -> 121, 172 -> 188; 16 of 65536 108 -> 87, 127 -> 150; of 131072 125 -> 102, 149 -> 155
 // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
 // 8 keys of a tile. With 2048 buckets of 3072 (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
 // and two classes took 0.63 ms against 0.39 of the radix passes.
 static bool bk_pays(int64_t P, int64_t C) {
-    return P <= kBkCap || (P <= kBkMaxRow && (C >= 32 || P * C * C >= ((int64_t)1 << 26)));
+    if (P <= kBkCap) return true;
+    const int64_t work = P * C * C;
+    return P <= kBkMaxRow && (C >= 32 || work >= (int64_t)8 << 23 || (C >= 12 && P >= 131072 && work >= (int64_t)5 << 23));
 }
 
 static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan &pl, bool look_back = false) {

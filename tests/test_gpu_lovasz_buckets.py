@@ -52,6 +52,19 @@ def test_which_rows_go_by_buckets(native):
         assert by_buckets(n_cls, pixels) == want, (n_cls, pixels)
 
 
+@pytest.mark.parametrize("boost", [0.0, 20.0])
+@pytest.mark.parametrize("n_cls, pixels, want", [(12, 291272, True), (12, 291271, False), (22, 131072, True), (22, 131071, False),
+                                                 (11, 350000, False)])
+def test_rows_of_a_single_image(native, n_cls, pixels, want, boost):
+    """Where 12 classes and more begin to go by buckets: the same differences on both sides of the line."""
+    assert by_buckets(n_cls, pixels) == want
+    rng = np.random.default_rng(pixels + n_cls)
+    x = rng.standard_normal((1, n_cls, 1, pixels), dtype=np.float32) * 2
+    y = labels(rng, (1, 1, pixels), n_cls)
+    x += np.float32(boost) * (np.arange(n_cls)[None, :, None, None] == y[:, None])
+    compare(native, x, y)
+
+
 # pixels: one block's limit, 64 / 256 / 1024 buckets, the longest row that is cut into buckets and the first that is not
 # classes: few (radix passes above one block's limit) and enough for buckets
 @pytest.mark.parametrize("pixels", [1, 63, 512, 513, 7679, 7680, 7681, 8193, 20011, 2560 * 64, 2560 * 64 + 1, 2560 * 256 + 7])
