@@ -1219,6 +1219,7 @@ static int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 //   left out, for what they lose at worst: 2 of 262144 94 -> 89, 100 -> 159; 4 of 263169 115 -> 95, 115 -> 155; 8 of 262144
 //   128 -> 106, 136 -> 169; 8 of 524288 168 -> 133, 184 -> 212; 10 of 524288 195 -> 143, 221 -> 232; 12 of 262144 151 -> 118,
 //   184 -> 193; 14 of 200000 147 -> 121, 172 -> 188; 16 of 65536 108 -> 87, 127 -> 150; of 131072 125 -> 102, 149 -> 155
+// (The worst cases by buckets are those of bk_ranks_crowded, which has become some 8 us faster since.)
 // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
 // 8 keys of a tile. With 2048 buckets of 3072 (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
 // and two classes took 0.63 ms against 0.39 of the radix passes.

@@ -394,8 +394,30 @@ __device__ __forceinline__ bool bk_sort(BkShared &s, const uint32_t (&key)[kBkIt
     return true;
 }
 
+// Lanes of the wave with the same digit.
+template <int kBits>
+__device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
+    uint32_t diff_lo = 0, diff_hi = 0;
+#pragma unroll
+    for (int b = 0; b < kBits; ++b) {
+        uint32_t splat = (uint32_t)((int32_t)(digit << (31 - b)) >> 31);
+        asm("" : "+v"(splat));
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(splat != 0u);
+        diff_lo |= (uint32_t)vote ^ splat;
+        diff_hi |= (uint32_t)(vote >> 32) ^ splat;
+    }
+    const uint64_t diff = ((uint64_t)diff_hi << 32) | diff_lo;
+    return __builtin_amdgcn_ballot_w64(valid) & ~diff;
+}
+
+constexpr int kBkDigitBits = 7;                   // of a pass of the crowded path
+constexpr int kBkDigitWords = (kBkWaves << kBkDigitBits) / 2;     // its counters, at the start of the bins' memory
+
 // rank[r] = valid keys of the block that sort before key[r] (equal keys in item order) | positives among them << 16, for
-// values that crowd (ties, clusters): a stable radix sort in LDS, 6 bits a pass over the bits of the range least..most.
+// values that crowd (ties, clusters): a stable radix sort in LDS, 7 bits a pass over the bits of the range least..most.
+// Few blocks run it, so that it is latency that counts: 7 bits in place of 6 are a pass less, votes over a fixed number of bits let
+// rounds overlap, and a crowded run's keys are fetched three rounds at a time. Steps, logits of the right class 20 above the others:
+// (1,18,384,384) 177 -> 167 us, (1,14,512,512) 197 -> 187; 14 above: (8,8,512,512) 381 -> 360, (4,19,512,1024) 698 -> 669.
 __device__ __forceinline__ void bk_ranks_crowded(BkShared &s, const uint32_t (&key)[kBkItems], uint32_t valid, int rounds, uint32_t least,
                                  uint32_t most, uint32_t (&rank)[kBkItems]) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -409,33 +431,41 @@ __device__ __forceinline__ void bk_ranks_crowded(BkShared &s, const uint32_t (&k
         k2[r] = v ? (key[r] & 0x80000000u) | ((key[r] & 0x7FFFFFFFu) - least) : span;
         it[r] = (uint32_t)bk_item(rounds, r);
     }
-    uint16_t *counts = reinterpret_cast<uint16_t *>(s.bin);        // [kBkWaves][64], then their exclusive sums
+    constexpr int kDigits = 1 << kBkDigitBits;
+    constexpr int kThreadsPerDigit = kBkThreads / kDigits, kWavesPerThread = kBkWaves / kThreadsPerDigit;
+    uint16_t *counts = reinterpret_cast<uint16_t *>(s.bin);        // [kBkWaves][kDigits], then their exclusive sums
     const int bits = 32 - __builtin_clz(span);
-    for (int shift = 0; shift < bits; shift += 6) {
+    auto digit_of = [&](uint32_t k, int shift) { return ((k & 0x7FFFFFFFu) >> shift) & (uint32_t)(kDigits - 1); };
+    for (int shift = 0; shift < bits; shift += kBkDigitBits) {
         __syncthreads();
-        for (int i = threadIdx.x; i < kBkWaves * 64 / 2; i += kBkThreads) s.bin[i] = 0;
+        for (int i = threadIdx.x; i < kBkDigitWords; i += kBkThreads) s.bin[i] = 0;
         __syncthreads();
-        const int width = min(6, bits - shift);
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r) {
             slot[r] = 0;
             if (r < rounds) {
-                const uint32_t digit = ((k2[r] & 0x7FFFFFFFu) >> shift) & 63u;
+                const uint32_t digit = digit_of(k2[r], shift);
                 uint32_t unused;
-                wave_rank_of<false>(wave_peers_n(digit, true, width), digit, true, false, counts + wave * 64, nullptr, slot[r], unused);
+                wave_rank_of<false>(bk_peers<kBkDigitBits>(digit, true), digit, true, false, counts + wave * kDigits, nullptr, slot[r], unused);
+                if (r % kBkGroup == kBkGroup - 1) __builtin_amdgcn_sched_barrier(0);        // more rounds at once spill
             }
         }
         __syncthreads();
-        const int d = threadIdx.x >> 3, w = threadIdx.x & 7;       // order: digit, then wave
-        const uint32_t n = counts[w * 64 + d];
-        uint32_t all;
-        const uint32_t start = block_excl_scan(n, s.scan, all);
-        counts[w * 64 + d] = (uint16_t)start;
+        const int d = (int)threadIdx.x / kThreadsPerDigit, w = (int)threadIdx.x % kThreadsPerDigit * kWavesPerThread;   // order: digit, then wave
+        uint32_t n[kWavesPerThread], mine = 0, all;
+#pragma unroll
+        for (int i = 0; i < kWavesPerThread; ++i) mine += n[i] = counts[(w + i) * kDigits + d];
+        uint32_t start = block_excl_scan(mine, s.scan, all);
+#pragma unroll
+        for (int i = 0; i < kWavesPerThread; ++i) {
+            counts[(w + i) * kDigits + d] = (uint16_t)start;
+            start += n[i];
+        }
         __syncthreads();
 #pragma unroll
         for (int r = 0; r < kBkItems; ++r) {
             if (r < rounds) {
-                const uint32_t at = counts[wave * 64 + (((k2[r] & 0x7FFFFFFFu) >> shift) & 63u)] + slot[r];
+                const uint32_t at = counts[wave * kDigits + digit_of(k2[r], shift)] + slot[r];
                 s.key()[at] = k2[r];
                 s.src()[at] = (uint16_t)it[r];
             }
@@ -637,21 +667,6 @@ struct BkLookup {
         for (int i = 0; i < N; ++i) bucket[i] = keep_key(key[i], limit) ? at[i] : (uint32_t)kStride;
     }
 };
-
-template <int kBits>
-__device__ __forceinline__ uint64_t bk_peers(uint32_t digit, bool valid) {
-    uint32_t diff_lo = 0, diff_hi = 0;
-#pragma unroll
-    for (int b = 0; b < kBits; ++b) {
-        uint32_t splat = (uint32_t)((int32_t)(digit << (31 - b)) >> 31);
-        asm("" : "+v"(splat));
-        const uint64_t vote = __builtin_amdgcn_ballot_w64(splat != 0u);
-        diff_lo |= (uint32_t)vote ^ splat;
-        diff_hi |= (uint32_t)(vote >> 32) ^ splat;
-    }
-    const uint64_t diff = ((uint64_t)diff_hi << 32) | diff_lo;
-    return __builtin_amdgcn_ballot_w64(valid) & ~diff;
-}
 
 // The tile's keys in the order of their buckets (in pixel order inside one), in the place of its keys, and every pixel's place
 // in that order.
@@ -1076,7 +1091,7 @@ __device__ __forceinline__ double bk_wide_keys(BkShared &s, const BucketArgs &a,
 }
 
 // What bk_huge_keys keeps in the block's memory: first, where the pairs are, the bounds of up to kBkIntervals value intervals
-// and their keys; then, per group, in what the crowded path leaves free behind its 256 words of counters and behind its keys
+// and their keys; then, per group, in what the crowded path leaves free behind its counters and behind its keys
 // and items.
 constexpr int kBkIntervals = 4096, kBkGroups = 1100;
 struct BkIntervals {
@@ -1087,11 +1102,11 @@ struct BkGroups {
     uint32_t *least, *first;                    // [groups], [groups + 1]: least key, first rank
     uint32_t *next, *start;                     // the next place of one of its keys, its start in the tile
     __device__ explicit BkGroups(BkShared &s)
-        : least(s.bin + kBkWaves * 64 / 2), first(least + kBkGroups), next(reinterpret_cast<uint32_t *>(s.src() + kBkCap)),
+        : least(s.bin + kBkDigitWords), first(least + kBkGroups), next(reinterpret_cast<uint32_t *>(s.src() + kBkCap)),
           start(next + kBkGroups) {}
 };
 static_assert(kBkIntervals % kBkThreads == 0 && 3 * (kBkMaxRow / kBkCap + 2) < kBkGroups, "groups, see bk_huge_groups");
-static_assert(sizeof(BkIntervals) <= sizeof(BkPair) * (kBkCap + kBkChunk) && kBkWaves * 32 + 2 * kBkGroups + 1 <= kBkBins &&
+static_assert(sizeof(BkIntervals) <= sizeof(BkPair) * (kBkCap + kBkChunk) && kBkDigitWords + 2 * kBkGroups + 1 <= kBkBins &&
               6 * kBkCap + 8 * kBkGroups <= (int)sizeof(BkPair) * (kBkCap + kBkChunk), "they fit");
 
 // The intervals of the thread's keys: the last of m ascending bounds that is not above a key. All keys a step at a time: one
@@ -1555,18 +1570,23 @@ __device__ __forceinline__ double bk_crowded_keys(BkShared &s, BkSegments &at, c
     uint32_t key[kBkItems], rank[kBkItems], valid = 0, least, most;
     __syncthreads();
     at.collect(BkSegments::Tile(a, c, b0, b1), 0u, s.scan);
-    auto where = [&](int li) {
-        uint32_t to[1];
-        at.where((uint32_t)li, (uint32_t)a.P - 1u, to);
-        return to[0];
+    // three rounds at a time, waited for together, and a key somewhere in the row for what is past the last
+    auto fetch = [&](int r0, uint32_t (&to)[kBkGroup], uint32_t (&k)[kBkGroup]) {
+        at.where((uint32_t)bk_item(rounds, r0), (uint32_t)a.P - 1u, to);
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) k[i] = kin[to[i]];
     };
 #pragma unroll
-    for (int r = 0; r < kBkItems; ++r) {
-        const int li = bk_item(rounds, r);
-        key[r] = 0;
-        if (r < rounds && li < n) {
-            key[r] = kin[where(li)];
-            valid |= 1u << r;
+    for (int r = 0; r < kBkItems; ++r) key[r] = 0;
+#pragma unroll
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                            // block-uniform
+        uint32_t to[kBkGroup], k[kBkGroup];
+        fetch(r0, to, k);
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) {
+            key[r0 + i] = k[i];
+            if (r0 + i < rounds && bk_item(rounds, r0 + i) < n) valid |= 1u << (r0 + i);
         }
     }
     bk_range(s, key, valid, least, most);
@@ -1574,12 +1594,18 @@ __device__ __forceinline__ double bk_crowded_keys(BkShared &s, BkSegments &at, c
     const float npos = (float)a.numbers[2 * a.C + c];
     double part = 0.0;
 #pragma unroll
-    for (int r = 0; r < kBkItems; ++r) {
-        if (!((valid >> r) & 1u)) continue;
-        const uint32_t to = where(bk_item(rounds, r)), k = kin[to];         // read again: not held across the sort
-        const float dj = jaccard_step(npos, rank0 + (rank[r] & 0xFFFFu), hot0 + (rank[r] >> 16), k >> 31);
-        part = add_loss(part, key_error(k), dj);
-        kin[to] = __builtin_bit_cast(uint32_t, dj);
+    for (int r0 = 0; r0 < kBkItems; r0 += kBkGroup) {
+        if (r0 >= rounds) break;                            // block-uniform
+        uint32_t to[kBkGroup], k[kBkGroup];
+        fetch(r0, to, k);                                   // read again: not held across the sort
+#pragma unroll
+        for (int i = 0; i < kBkGroup; ++i) {
+            const uint32_t place = rank[r0 + i];
+            if (!((valid >> (r0 + i)) & 1u)) continue;
+            const float dj = jaccard_step(npos, rank0 + (place & 0xFFFFu), hot0 + (place >> 16), k[i] >> 31);
+            part = add_loss(part, key_error(k[i]), dj);
+            kin[to[i]] = __builtin_bit_cast(uint32_t, dj);
+        }
     }
     return part;
 }
