@@ -377,11 +377,14 @@ def lsr_forward_reduced_lse(logits, labels, ignore_index, smooth, mean, args=Non
 
 
 def lsr_backward_scaled_lse(lse, ignore_index, smooth, grad_scalar, divide_by, args, kept=None):
-    """The gradient from the forward's log-sum-exp (lsr_forward_reduced_lse); `kept`: optional byte mask."""
+    """The gradient from the forward's log-sum-exp (lsr_forward_reduced_lse); `kept`: optional byte mask (not for 16-bit
+    channel planes, whose entry point takes none)."""
     a = args
+    if kept is not None and _planes16(a):
+        raise RuntimeError("pytorch_loss: a mask of kept pixels cannot be given for 16-bit logits on channel planes")
     grad = torch.empty_like(a.x)
     go = _scalar_f32(grad_scalar)
-    if _planes16(a):                    # (no mask there: `kept` comes from losses that do not keep the log-sum-exp)
+    if _planes16(a):
         _call(a.x, "plh_lsr_backward_scaled_lse_planes16", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(go), 1.0, _ptr(divide_by),
               _ptr(grad), a.n, a.c, a.m, int(ignore_index), float(smooth))
         return _back_to(grad, a.dtype)

@@ -88,6 +88,19 @@ def test_views_and_labels_without_a_channel(shape, offset, kind):
     assert ((a.grad.float() - b.grad.float()).abs() <= 2 * HALF_ULP[torch.bfloat16] * b.grad.float().abs() * 1.01 + 1e-6).all()
 
 
+def test_a_mask_is_refused():
+    """The byte mask of a selection has no place in this backward: the call raises, and never returns an unmasked gradient."""
+    from pytorch_loss import _native
+    x, y = inputs((2, 19, 65, 67), torch.bfloat16, 5)
+    args = _native.lsr_args(x, y)
+    _, n_valid, lse = _native.lsr_forward_reduced_lse(x, y, IGN, 0.1, True, args=args)
+    kept = (y != IGN).to(torch.uint8)
+    up = torch.ones((), device="cuda")
+    with pytest.raises(RuntimeError, match="mask"):
+        _native.lsr_backward_scaled_lse(lse, IGN, 0.1, up, n_valid, args, kept=kept)
+    assert _native.lsr_backward_scaled_lse(lse, IGN, 0.1, up, n_valid, args).shape == x.shape
+
+
 def test_where_it_applies():
     from pytorch_loss import _native
     lib = _native.load()
