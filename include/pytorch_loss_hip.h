@@ -144,9 +144,24 @@ int plh_lsr_backward_scaled_lse(const void *logits, int32_t dtype, const int64_t
                                 int64_t ignore_index, float smooth, void *stream);
 
 /* The same for 16-bit logits on channel planes of at least 4096 pixels that do not start on 128-byte lines, with 16..256
- * channels. */
+ * channels, in two parts: max_out[P], a pixel's largest logit (in the logits' type), and sum_out[P], the sum of
+ * 2^(x log2e - fl(max log2e)) over its logits. The gradient is the one of plh_lsr_backward_scaled bit for bit. */
 int plh_lsr_saves_lse_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);
 
+int plh_lsr_forward_reduced_parts_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *sum_out,
+                                           void *max_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                           void *workspace, int64_t workspace_bytes,
+                                           int64_t n_size, int64_t dimsize, int64_t m_size,
+                                           int64_t ignore_index, float smooth, void *stream);
+
+int plh_lsr_backward_scaled_parts_planes16(const void *logits, int32_t dtype, const int64_t *labels, const float *sum,
+                                           const void *max, const float *grad_scalar, float scale,
+                                           const int64_t *divide_by, void *grad_logits,
+                                           int64_t n_size, int64_t dimsize, int64_t m_size,
+                                           int64_t ignore_index, float smooth, void *stream);
+
+/* For callers of the first form, which kept one float per pixel and with it fewer digits (fp16 logits around 16000: a
+ * gradient off by 5e-4 of its value): lse_out is not written, lse is not read, the backward recomputes. */
 int plh_lsr_forward_reduced_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *lse_out,
                                          float *loss_out, int64_t *n_valid_out, int32_t mean,
                                          void *workspace, int64_t workspace_bytes,

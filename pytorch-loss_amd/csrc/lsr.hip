@@ -39,21 +39,34 @@ PLH_LSR_EXTERN(float)
 PLH_LSR_EXTERN(f16)
 PLH_LSR_EXTERN(bf16)
 
-static bool lse_applies(int32_t dtype, int64_t dimsize, int64_t m_size, bool planes16) {
-    return (planes16 ? planes16_apply : lsr_lse_applies)(dtype_size(dtype), dimsize, m_size);
-}
+// A pixel's log-sum-exp as the forward leaves it: one float, or (16-bit planes) the sum and the largest logit.
+struct SavedLse {
+    float *lse = nullptr, *sum = nullptr;
+    void *top = nullptr;
+    int check(int32_t dtype, int64_t dimsize, int64_t m_size) const {
+        if (lse && (misaligned(lse, 4) || !lsr_lse_applies(dtype_size(dtype), dimsize, m_size))) return PLH_ERR_BAD_SIZE;
+        if (sum && (misaligned(sum, 4) || misaligned(top, 2) || !planes16_apply(dtype_size(dtype), dimsize, m_size))) return PLH_ERR_BAD_SIZE;
+        return PLH_OK;
+    }
+    void give(LsrParams &p) const {
+        p.lse = lse;
+        p.sum = sum;
+        p.top = top;
+    }
+};
 
 static int backward(const void *logits, int32_t dtype, const int64_t *labels, const Upstream &up, void *grad_logits,
                     int64_t n_size, int64_t dimsize, int64_t m_size, int64_t ignore_index, float smooth,
-                    void *stream, const float *lse = nullptr, bool planes16 = false) {
+                    void *stream, const SavedLse &saved = SavedLse()) {
     if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
-    const int rc = check_slice_args(logits, labels, grad_logits, n_size, dimsize, m_size, dtype_size(dtype),
-                                    dtype_size(dtype));
+    int rc = check_slice_args(logits, labels, grad_logits, n_size, dimsize, m_size, dtype_size(dtype),
+                              dtype_size(dtype));
     if (rc != PLH_OK) return rc;
     if (n_size * dimsize * m_size == 0) return PLH_OK;
-    if (lse && (misaligned(lse, 4) || !lse_applies(dtype, dimsize, m_size, planes16))) return PLH_ERR_BAD_SIZE;
+    rc = saved.check(dtype, dimsize, m_size);
+    if (rc != PLH_OK) return rc;
     LsrParams p = make_params(n_size, dimsize, m_size, ignore_index, smooth, dtype_size(dtype));
-    p.lse = const_cast<float *>(lse);           // read only in the backward
+    saved.give(p);                              // read only in the backward
     dispatch_dtype(dtype, [&](auto tag) {
         using T = decltype(tag);
         lsr_backward_typed<T>(static_cast<const T *>(logits), labels, up, static_cast<T *>(grad_logits), p,
@@ -82,13 +95,14 @@ extern "C" int plh_lsr_forward(const void *logits, int32_t dtype, const int64_t 
     return check_launch();
 }
 
-static int forward_reduced(const void *logits, int32_t dtype, const int64_t *labels, float *losses, float *lse_out,
+static int forward_reduced(const void *logits, int32_t dtype, const int64_t *labels, float *losses, const SavedLse &saved,
                            float *loss_out, int64_t *n_valid_out, int32_t mean, void *workspace, int64_t workspace_bytes,
                            int64_t n_size, int64_t dimsize, int64_t m_size, int64_t ignore_index, float smooth,
-                           void *stream, bool planes16 = false) {
+                           void *stream) {
     if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
-    if (lse_out && (misaligned(lse_out, 4) || !lse_applies(dtype, dimsize, m_size, planes16))) return PLH_ERR_BAD_SIZE;
-    int rc = check_slice_args(logits, labels, loss_out, n_size, dimsize, m_size, dtype_size(dtype), 4);
+    int rc = saved.check(dtype, dimsize, m_size);
+    if (rc != PLH_OK) return rc;
+    rc = check_slice_args(logits, labels, loss_out, n_size, dimsize, m_size, dtype_size(dtype), 4);
     if (rc != PLH_OK) return rc;
     Partials part;
     rc = carve_partials(workspace, workspace_bytes, n_size * m_size, loss_out, n_valid_out, part);
@@ -98,7 +112,7 @@ static int forward_reduced(const void *logits, int32_t dtype, const int64_t *lab
     unsigned blocks = 0;
     if (n_size * dimsize * m_size != 0) {
         LsrParams p = make_params(n_size, dimsize, m_size, ignore_index, smooth, dtype_size(dtype));
-        p.lse = lse_out;
+        saved.give(p);
         dispatch_dtype(dtype, [&](auto tag) {
             using T = decltype(tag);
             blocks = lsr_forward_typed<T>(static_cast<const T *>(logits), labels, losses, part, true, p, st);
@@ -113,7 +127,7 @@ extern "C" int plh_lsr_forward_reduced(const void *logits, int32_t dtype, const 
                                        void *workspace, int64_t workspace_bytes,
                                        int64_t n_size, int64_t dimsize, int64_t m_size,
                                        int64_t ignore_index, float smooth, void *stream) {
-    return forward_reduced(logits, dtype, labels, losses, nullptr, loss_out, n_valid_out, mean, workspace, workspace_bytes,
+    return forward_reduced(logits, dtype, labels, losses, SavedLse(), loss_out, n_valid_out, mean, workspace, workspace_bytes,
                            n_size, dimsize, m_size, ignore_index, smooth, stream);
 }
 
@@ -181,12 +195,34 @@ extern "C" int plh_lsr_forward_reduced_lse(const void *logits, int32_t dtype, co
                                            int64_t n_size, int64_t dimsize, int64_t m_size,
                                            int64_t ignore_index, float smooth, void *stream) {
     if (!lse_out && n_size * dimsize * m_size != 0) return PLH_ERR_NULL_POINTER;
-    return forward_reduced(logits, dtype, labels, nullptr, lse_out, loss_out, n_valid_out, mean, workspace, workspace_bytes,
-                           n_size, dimsize, m_size, ignore_index, smooth, stream);
+    return forward_reduced(logits, dtype, labels, nullptr, SavedLse{lse_out}, loss_out, n_valid_out, mean, workspace,
+                           workspace_bytes, n_size, dimsize, m_size, ignore_index, smooth, stream);
 }
 
 extern "C" int plh_lsr_saves_lse_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size) {
-    return dtype_ok(dtype) && n_size > 0 && dimsize > 0 && m_size > 0 && lse_applies(dtype, dimsize, m_size, true) ? 1 : 0;
+    return dtype_ok(dtype) && n_size > 0 && dimsize > 0 && m_size > 0 && planes16_apply(dtype_size(dtype), dimsize, m_size) ? 1 : 0;
+}
+
+extern "C" int plh_lsr_forward_reduced_parts_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *sum_out,
+                                                      void *max_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
+                                                      void *workspace, int64_t workspace_bytes,
+                                                      int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                      int64_t ignore_index, float smooth, void *stream) {
+    if ((!sum_out || !max_out) && n_size * dimsize * m_size != 0) return PLH_ERR_NULL_POINTER;
+    return forward_reduced(logits, dtype, labels, nullptr, SavedLse{nullptr, sum_out, max_out}, loss_out, n_valid_out, mean,
+                           workspace, workspace_bytes, n_size, dimsize, m_size, ignore_index, smooth, stream);
+}
+
+extern "C" int plh_lsr_backward_scaled_parts_planes16(const void *logits, int32_t dtype, const int64_t *labels, const float *sum,
+                                                      const void *max, const float *grad_scalar, float scale,
+                                                      const int64_t *divide_by, void *grad_logits,
+                                                      int64_t n_size, int64_t dimsize, int64_t m_size,
+                                                      int64_t ignore_index, float smooth, void *stream) {
+    if (n_size * dimsize * m_size != 0 && (!grad_scalar || !sum || !max)) return PLH_ERR_NULL_POINTER;
+    if (misaligned(grad_scalar, 4) || misaligned(divide_by, 8)) return PLH_ERR_MISALIGNED;
+    const Upstream up{grad_scalar, 0, divide_by, scale, nullptr};
+    return backward(logits, dtype, labels, up, grad_logits, n_size, dimsize, m_size, ignore_index, smooth, stream,
+                    SavedLse{nullptr, const_cast<float *>(sum), const_cast<void *>(max)});
 }
 
 extern "C" int plh_lsr_forward_reduced_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *lse_out,
@@ -194,9 +230,11 @@ extern "C" int plh_lsr_forward_reduced_lse_planes16(const void *logits, int32_t 
                                                     void *workspace, int64_t workspace_bytes,
                                                     int64_t n_size, int64_t dimsize, int64_t m_size,
                                                     int64_t ignore_index, float smooth, void *stream) {
+    if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
     if (!lse_out && n_size * dimsize * m_size != 0) return PLH_ERR_NULL_POINTER;
-    return forward_reduced(logits, dtype, labels, nullptr, lse_out, loss_out, n_valid_out, mean, workspace, workspace_bytes,
-                           n_size, dimsize, m_size, ignore_index, smooth, stream, true);
+    if (!planes16_apply(dtype_size(dtype), dimsize, m_size)) return PLH_ERR_BAD_SIZE;
+    return forward_reduced(logits, dtype, labels, nullptr, SavedLse(), loss_out, n_valid_out, mean, workspace, workspace_bytes,
+                           n_size, dimsize, m_size, ignore_index, smooth, stream);
 }
 
 extern "C" int plh_lsr_backward_scaled_lse_planes16(const void *logits, int32_t dtype, const int64_t *labels, const float *lse,
@@ -204,10 +242,12 @@ extern "C" int plh_lsr_backward_scaled_lse_planes16(const void *logits, int32_t 
                                                     void *grad_logits,
                                                     int64_t n_size, int64_t dimsize, int64_t m_size,
                                                     int64_t ignore_index, float smooth, void *stream) {
+    if (!dtype_ok(dtype)) return PLH_ERR_BAD_DTYPE;
     if (n_size * dimsize * m_size != 0 && (!grad_scalar || !lse)) return PLH_ERR_NULL_POINTER;
     if (misaligned(grad_scalar, 4) || misaligned(divide_by, 8)) return PLH_ERR_MISALIGNED;
+    if (!planes16_apply(dtype_size(dtype), dimsize, m_size)) return PLH_ERR_BAD_SIZE;
     const Upstream up{grad_scalar, 0, divide_by, scale, nullptr};
-    return backward(logits, dtype, labels, up, grad_logits, n_size, dimsize, m_size, ignore_index, smooth, stream, lse, true);
+    return backward(logits, dtype, labels, up, grad_logits, n_size, dimsize, m_size, ignore_index, smooth, stream);
 }
 
 extern "C" int plh_lsr_forward_reduced_static(const void *logits, int32_t dtype, const int64_t *labels, float *losses,
@@ -269,5 +309,6 @@ extern "C" int plh_lsr_backward_scaled_lse(const void *logits, int32_t dtype, co
     if (n_size * dimsize * m_size != 0 && (!grad_scalar || !lse)) return PLH_ERR_NULL_POINTER;
     if (misaligned(grad_scalar, 4) || misaligned(divide_by, 8)) return PLH_ERR_MISALIGNED;
     const Upstream up{grad_scalar, 0, divide_by, scale, kept};
-    return backward(logits, dtype, labels, up, grad_logits, n_size, dimsize, m_size, ignore_index, smooth, stream, lse);
+    return backward(logits, dtype, labels, up, grad_logits, n_size, dimsize, m_size, ignore_index, smooth, stream,
+                    SavedLse{const_cast<float *>(lse)});
 }

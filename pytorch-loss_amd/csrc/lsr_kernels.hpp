@@ -25,11 +25,16 @@ struct LsrParams {
     int64_t ignore;
     float w_pos, w_neg, sumw;
     unsigned xcd_run;   // tile permutation run length (xcd_run_for)
-    // Per-pixel log-sum-exp of the logits, fp32 [P]. Forward, logits in NCHW: written when set, by the per-image
-    // form of the register-resident kernel, the split kernels and (fp32) the lane-per-pixel kernel (the shapes that
-    // lsr_lse_applies and planes16_apply send here).
-    // Backward: when set, lsr_bwd_planes and planes16_bwd form the gradient from it plane by plane (see there).
+    // Per-pixel log-sum-exp of the logits, fp32 [P]. Forward, fp32 logits in NCHW: written when set, by the per-image
+    // form of the register-resident kernel, the split kernels and the lane-per-pixel kernel (the shapes that
+    // lsr_lse_applies sends here).
+    // Backward: when set, lsr_bwd_planes forms the gradient from it plane by plane (see there).
     float *lse = nullptr;
+    // The same of 16-bit logits (planes16_apply), in the two parts that the backward which recomputes forms: a pixel's
+    // largest logit, in the logits' type [P], and S = sum_j 2^(x_j log2e - fl(max log2e)) [P]. One rounded fp32 lost
+    // the digits of max that lie above those of log S: fp16 logits around 1000 were off by up to 3e-5 of a probability.
+    float *sum = nullptr;
+    void *top = nullptr;
 };
 
 // ---------------------------------------------------------------- regs ----
@@ -60,9 +65,9 @@ __global__ __launch_bounds__(kRegsBlock) void lsr_fwd_regs(const T *__restrict__
     float mine = 0.f;
     int cnt = 0;
     const float fc = (float)p.C;
-    // the per-image form also leaves each pixel's log-sum-exp where it is given a place (LsrParams::lse)
-    constexpr bool kMayLse = Form == kPerImage;
-    float lse_abs[kMayLse ? V : 1];
+    // the per-image form also leaves each pixel's log-sum-exp where it is given a place (LsrParams::lse, sum, top)
+    constexpr bool kMayLse = Form == kPerImage && sizeof(T) == 4, kMayParts = Form == kPerImage && sizeof(T) == 2;
+    float lse_abs[kMayLse ? V : 1], sums[kMayParts ? V : 1], tops[kMayParts ? V : 1];
 #pragma unroll
     for (int k = 0; k < V; ++k) {
         bool ign;
@@ -81,6 +86,10 @@ __global__ __launch_bounds__(kRegsBlock) void lsr_fwd_regs(const T *__restrict__
             }
         const float lse = (__builtin_amdgcn_logf(s) - r) * kLn2;
         if constexpr (kMayLse) lse_abs[k] = mx + lse;
+        if constexpr (kMayParts) {
+            sums[k] = s;
+            tops[k] = mx;
+        }
         const float all = (sx - fc * mx) - fc * lse;
         // no target channel (label outside [0, C)): every weight is w_neg
         const float hot = (tgt >= 0) ? (p.w_pos - p.w_neg) * ((x_y - mx) - lse) : 0.f;
@@ -93,6 +102,12 @@ __global__ __launch_bounds__(kRegsBlock) void lsr_fwd_regs(const T *__restrict__
     if (at.live && loss) at.store_f32(loss, out);
     if constexpr (kMayLse) {
         if (p.lse && at.live) at.store_f32(p.lse, lse_abs);     // past the caches: 0.1466 -> 0.1428 ms at (16,19,769,769)
+    }
+    if constexpr (kMayParts) {
+        if (p.sum && at.live) {
+            at.store_f32(p.sum, sums);
+            at.store_typed(static_cast<T *>(p.top), tops);
+        }
     }
     if (Reduce) {
         const float bs = block_sum_256(mine, red);
@@ -301,20 +316,31 @@ __global__ __launch_bounds__(256) void lsr_bwd_planes(const T *__restrict__ x, c
     }
 }
 
-// The same for 16-bit logits (planes16_bwd).
+// The same for 16-bit logits (planes16_bwd), in the expressions of the kernels that recompute: the same gradient bit for bit.
+template <class T>
 struct LsrPlaneOp {
+    const float *sum;
+    const T *top;
     float sumw, w_pos, w_neg, scale, n_pos, n_neg;
+    struct Pixel {
+        float scale;        // sumw gk / S
+        unsigned word;      // the largest logit's bits | the label (C without a target channel, 0xFFFF for an ignored pixel)
+        __device__ __forceinline__ bool dropped() const { return (word & 0xFFFFu) == 0xFFFFu; }
+        __device__ __forceinline__ bool hot(int c) const { return (word & 0xFFFFu) == (unsigned)c; }
+    };
+    static __device__ __forceinline__ Pixel nothing() { return Pixel{0.f, 0xFFFFu}; }
     __device__ __forceinline__ void begin(float gk) {
         scale = sumw * gk;
         n_pos = -w_pos * gk;
         n_neg = -w_neg * gk;
     }
-    __device__ __forceinline__ float value(float lse) const { return lse; }
-    __device__ __forceinline__ int label(int64_t lb, int64_t ignore, int C) const {
-        return lb == ignore ? -1 : ((lb < 0 || lb >= C) ? C : (int)lb);
+    __device__ __forceinline__ Pixel pixel(int64_t at, int64_t lb, int64_t ignore, int C) const {
+        const unsigned label = lb == ignore ? 0xFFFFu : ((lb < 0 || lb >= C) ? (unsigned)C : (unsigned)lb);
+        return Pixel{scale * __builtin_amdgcn_rcpf(sum[at]), (unsigned)top[at].bits << 16 | label};
     }
-    __device__ __forceinline__ float grad(float x, float lse, bool hot) const {
-        return __builtin_fmaf(__builtin_amdgcn_exp2f((x - lse) * kLog2e), scale, hot ? n_pos : n_neg);
+    __device__ __forceinline__ float grad(float x, const Pixel &px, int c) const {
+        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(x, kLog2e, -(widen_hi(px.word, T{}) * kLog2e)));
+        return __builtin_fmaf(e, px.scale, px.hot(c) ? n_pos : n_neg);
     }
 };
 
@@ -357,6 +383,8 @@ __global__ __launch_bounds__(kSplitBlock) void lsr_fwd_split(const T *__restrict
                                                             float *__restrict__ loss, Partials part,
                                                             const LsrParams p) {
     const bool Reduce = part.sum != nullptr;
+    // sums as they are, for LsrParams::sum, instead of less what the rounding of c left in them
+    constexpr bool kMayParts = PerImage && sizeof(T) == 2;
     __shared__ float parts[4][kSplitWaves][kWave * V];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const SplitSlice<T, V, KW, PerImage> at(p.P, p.m_size, p.C, p.xcd_run);
@@ -387,7 +415,7 @@ __global__ __launch_bounds__(kSplitBlock) void lsr_fwd_split(const T *__restrict
             }
             const int q = lane * V + k;
             parts[0][wave][q] = mx;
-            parts[1][wave][q] = s * __builtin_amdgcn_exp2f(-r);      // 2^r is what the rounding of c left in every term
+            parts[1][wave][q] = kMayParts ? s : s * __builtin_amdgcn_exp2f(-r);      // 2^r is what the rounding of c left in every term
             parts[2][wave][q] = d;
             parts[3][wave][q] = x_y;
         }
@@ -395,6 +423,29 @@ __global__ __launch_bounds__(kSplitBlock) void lsr_fwd_split(const T *__restrict
     __syncthreads();
     const int used = (p.C + KW - 1) / KW;               // wavefronts that hold channels
     const float fc = (float)p.C;
+    if constexpr (kMayParts) {
+        // LsrParams::sum and top, with the backward's expressions, by the wavefronts that do not finish pixels: 64 neighbours
+        // each ((6,200,513,513) bf16: forward 226 us without them, 249 so, 261 by one wavefront, four pixels per lane)
+        static_assert(kSplitWaves == 2 * V, "as many as finish");
+        if (wave >= V && p.sum) {                       // wave-uniform
+            const int q = (wave - V) * kWave + lane;
+            const bool here = q % V < __shfl(at.nv, q / V);
+            const int64_t pix = __shfl(at.pix, 0) + q;
+            float top = parts[0][0][q];
+            for (int w = 1; w < used; ++w) top = fmaxf(top, parts[0][w][q]);
+            const float c = top * kLog2e;
+            float sum = 0.f;
+            for (int w = 0; w < used; ++w) {
+#pragma clang fp contract(off)
+                const float less = parts[0][w][q] * kLog2e - c;
+                sum = __builtin_fmaf(parts[1][w][q], __builtin_amdgcn_exp2f(less), sum);
+            }
+            if (here) {
+                __builtin_nontemporal_store(sum, p.sum + pix);
+                store_one(static_cast<T *>(p.top) + pix, top);
+            }
+        }
+    }
     if (wave >= V) return;                              // wavefront k finishes pixel k of every lane
     bool ign;
     PLH_SPLIT_MY_LABEL(my_lb, lb, wave, V)
@@ -405,7 +456,12 @@ __global__ __launch_bounds__(kSplitBlock) void lsr_fwd_split(const T *__restrict
     float S = 0.f, D = 0.f, x_y = 0.f;
     for (int w = 0; w < used; ++w) {
         const float shift = parts[0][w][q] - M;
-        S = __builtin_fmaf(parts[1][w][q], fast_exp(shift), S);
+        float s = parts[1][w][q];
+        if constexpr (kMayParts) {
+            const float c = parts[0][w][q] * kLog2e;
+            s *= __builtin_amdgcn_exp2f(-__builtin_fmaf(parts[0][w][q], kLog2e, -c));
+        }
+        S = __builtin_fmaf(s, fast_exp(shift), S);
         D += __builtin_fmaf((float)split_count(w, KW, p.C), shift, parts[2][w][q]);
         x_y += parts[3][w][q];
     }
@@ -417,7 +473,9 @@ __global__ __launch_bounds__(kSplitBlock) void lsr_fwd_split(const T *__restrict
     const bool valid = here && !ign;
     const float out = valid ? acc : 0.f;
     if (here && loss) loss[at.pix + wave] = out;
-    if (here && p.lse) __builtin_nontemporal_store(M + lse, p.lse + at.pix + wave);          // LsrParams::lse
+    if constexpr (sizeof(T) == 4) {
+        if (here && p.lse) __builtin_nontemporal_store(M + lse, p.lse + at.pix + wave);      // LsrParams::lse
+    }
     if (Reduce) split_block_partials<V>(out, valid, wave, lane, part);
 }
 
@@ -1457,9 +1515,10 @@ void lsr_backward_typed(const T *logits, const int64_t *labels, const Upstream &
         }
     }
     if constexpr (sizeof(T) == 2) {
-        if (p.lse && p.m_size > 1 && !go_vec && !up.keep && planes16_apply(sizeof(T), p.C, p.m_size) &&
-            planes16_launch(logits, labels, p.lse, up, grad_logits, LsrPlaneOp{p.sumw, p.w_pos, p.w_neg}, p.P, p.m_size, p.C, p.ignore, st))
-            return;
+        if (p.sum && !go_vec && !up.keep && planes16_apply(sizeof(T), p.C, p.m_size)) {
+            const LsrPlaneOp<T> op{p.sum, static_cast<const T *>(p.top), p.sumw, p.w_pos, p.w_neg};
+            if (planes16_launch(logits, labels, up, grad_logits, op, p.P, p.m_size, p.C, p.ignore, st)) return;
+        }
     }
     switch (pick_shape(p.C, p.m_size, V, sizeof(T), logits, grad_logits, labels, go_vec, nullptr, true, true, true,
                        kImageFormMaxChannels<T>)) {

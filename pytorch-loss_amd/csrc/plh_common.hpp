@@ -821,6 +821,18 @@ struct PixelRef {
             store_vec<V>(out + pix, v);
         }
     }
+    // one value of the logits' type per pixel (per-image form)
+    template <class T>
+    __device__ __forceinline__ void store_typed(T *out, const float (&v)[V]) const {
+        static_assert(Form == kPerImage, "element boundaries");
+        if (nv == V) {
+            Pack<T, V>::store_unaligned(out + pix, Pack<T, V>::put(v));
+        } else {
+#pragma unroll
+            for (int k = 0; k < V; ++k)
+                if (k < nv) store_one(out + pix + k, v[k]);
+        }
+    }
     // the same through the cache (an output that a later kernel of the same call reads)
     __device__ __forceinline__ void store_f32_cached(float *out, const float (&v)[V]) const {
         if constexpr (Form == kPerImage) {

@@ -1130,16 +1130,22 @@ __global__ __launch_bounds__(256) void taylor_ce_bwd_planes(const T *__restrict_
 // The same for 16-bit logits (planes16_bwd).
 template <int ORD>
 struct TaylorPlaneOp {
+    const float *sums;
     float gk;
+    struct Pixel {
+        float k;            // gk / S
+        int lab;            // -1 without a target: exact zeros (taylor_ce_bwd_regs)
+        __device__ __forceinline__ bool dropped() const { return lab < 0; }
+    };
+    static __device__ __forceinline__ Pixel nothing() { return Pixel{0.f, -1}; }
     __device__ __forceinline__ void begin(float g) { gk = g; }
-    __device__ __forceinline__ float value(float sum) const { return gk / sum; }
-    __device__ __forceinline__ int label(int64_t lb, int64_t ignore, int C) const {
-        return lb != ignore && lb >= 0 && lb < C ? (int)lb : -1;    // pixels without a target: exact zeros (taylor_ce_bwd_regs)
+    __device__ __forceinline__ Pixel pixel(int64_t at, int64_t lb, int64_t ignore, int C) const {
+        return Pixel{gk / sums[at], lb != ignore && lb >= 0 && lb < C ? (int)lb : -1};
     }
-    __device__ __forceinline__ float grad(float x, float k, bool hot) const {
-        float f, df;
+    __device__ __forceinline__ float grad(float x, const Pixel &px, int c) const {
+        float f, df, k = px.k;
         taylor_pair24<ORD>(x, f, df);
-        if (hot) k -= gk / f;
+        if (px.lab == c) k -= gk / f;
         return df * k;
     }
 };
@@ -1182,8 +1188,8 @@ unsigned taylor_launch(const T *x, const T *g, const int64_t *lab, const Upstrea
     if constexpr (Kind == kTaylorCeBwd && sizeof(T) == 2) {
         if (p.sums && !go_vec && p.m_size > 1 && !walk && planes16_apply(sizeof(T), p.C, p.m_size)) {
             const bool done = p.order == 2
-                ? planes16_launch(x, lab, p.sums, up, out, TaylorPlaneOp<2>{}, p.P, p.m_size, p.C, p.ignore, st)
-                : planes16_launch(x, lab, p.sums, up, out, TaylorPlaneOp<4>{}, p.P, p.m_size, p.C, p.ignore, st);
+                ? planes16_launch(x, lab, up, out, TaylorPlaneOp<2>{p.sums}, p.P, p.m_size, p.C, p.ignore, st)
+                : planes16_launch(x, lab, up, out, TaylorPlaneOp<4>{p.sums}, p.P, p.m_size, p.C, p.ignore, st);
             if (done) return 1;
         }
     }

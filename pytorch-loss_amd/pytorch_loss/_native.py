@@ -59,6 +59,8 @@ _SIGNATURES = {
     "plh_lsr_forward_reduced_lse": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_backward_scaled_lse": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_saves_lse_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
+    "plh_lsr_forward_reduced_parts_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
+    "plh_lsr_backward_scaled_parts_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_forward_reduced_lse_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_backward_scaled_lse_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lovasz_lookback_workspace_bytes": (_i64, [_i64, _i64, _i64]),
@@ -361,18 +363,26 @@ def _planes16(a):
 def lsr_forward_reduced_lse(logits, labels, ignore_index, smooth, mean, args=None):
     """lsr_forward_reduced that also keeps every pixel's log-sum-exp where the library's backward can use it (channel
     planes, long rows: see plh_lsr_saves_lse, and for 16-bit logits plh_lsr_saves_lse_planes16).
-    -> (loss, n_valid, lse or None)."""
+    -> (loss, n_valid, lse or None); on 16-bit planes lse holds the two parts, the sums and behind them the largest
+    logits."""
     a = args or lsr_args(logits, labels)
-    planes = _planes16(a)
-    if a.x.numel() == 0 or not getattr(load(), "plh_lsr_saves_lse" + planes)(a.tag, a.n, a.c, a.m):
+    pixels = a.n * a.m
+    planes16 = a.tag != 0 and a.m > 1
+    saves = load().plh_lsr_saves_lse_planes16 if planes16 else load().plh_lsr_saves_lse
+    if pixels * a.c == 0 or not saves(a.tag, a.n, a.c, a.m):
         return _pixel_forward_reduced("plh_lsr_forward_reduced", a, ignore_index, smooth, mean) + (None,)
     dev = a.x.device
     loss = torch.empty((), dtype=torch.float32, device=dev)
     n_valid = torch.empty((), dtype=torch.int64, device=dev)
-    lse = torch.empty((a.n * a.m,), dtype=torch.float32, device=dev)
-    ws, ws_bytes = _reduce_workspace(a.n * a.m, dev)
-    _call(a.x, "plh_lsr_forward_reduced_lse" + planes, _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(loss), _ptr(n_valid),
-          1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m, int(ignore_index), float(smooth))
+    lse = torch.empty((pixels + (pixels + 1) // 2 if planes16 else pixels,), dtype=torch.float32, device=dev)
+    ws, ws_bytes = _reduce_workspace(pixels, dev)
+    if planes16:
+        _call(a.x, "plh_lsr_forward_reduced_parts_planes16", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse),
+              _p(lse.data_ptr() + 4 * pixels), _ptr(loss), _ptr(n_valid), 1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m,
+              int(ignore_index), float(smooth))
+    else:
+        _call(a.x, "plh_lsr_forward_reduced_lse", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(loss), _ptr(n_valid),
+              1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m, int(ignore_index), float(smooth))
     return _back_to(loss, _loss_dtype(a.dtype)), n_valid, lse
 
 
@@ -380,13 +390,15 @@ def lsr_backward_scaled_lse(lse, ignore_index, smooth, grad_scalar, divide_by, a
     """The gradient from the forward's log-sum-exp (lsr_forward_reduced_lse); `kept`: optional byte mask (not for 16-bit
     channel planes, whose entry point takes none)."""
     a = args
-    if kept is not None and _planes16(a):
+    planes16 = a.tag != 0 and a.m > 1
+    if kept is not None and planes16:
         raise RuntimeError("pytorch_loss: a mask of kept pixels cannot be given for 16-bit logits on channel planes")
     grad = torch.empty_like(a.x)
     go = _scalar_f32(grad_scalar)
-    if _planes16(a):
-        _call(a.x, "plh_lsr_backward_scaled_lse_planes16", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(go), 1.0, _ptr(divide_by),
-              _ptr(grad), a.n, a.c, a.m, int(ignore_index), float(smooth))
+    if planes16:
+        _call(a.x, "plh_lsr_backward_scaled_parts_planes16", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse),
+              _p(lse.data_ptr() + 4 * a.n * a.m), _ptr(go), 1.0, _ptr(divide_by), _ptr(grad), a.n, a.c, a.m, int(ignore_index),
+              float(smooth))
         return _back_to(grad, a.dtype)
     _call(a.x, "plh_lsr_backward_scaled_lse", _ptr(a.x), a.tag, _ptr(a.lb), _ptr(lse), _ptr(kept) if kept is not None else None,
           _ptr(go), 1.0, _ptr(divide_by), _ptr(grad), a.n, a.c, a.m, int(ignore_index), float(smooth))

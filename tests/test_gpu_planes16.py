@@ -88,6 +88,31 @@ def test_views_and_labels_without_a_channel(shape, offset, kind):
     assert ((a.grad.float() - b.grad.float()).abs() <= 2 * HALF_ULP[torch.bfloat16] * b.grad.float().abs() * 1.01 + 1e-6).all()
 
 
+# logits with a common offset, whose largest takes digits from anything added to it; planes of a multiple of 8 pixels off the
+# lines; 12 planes per block and a last share of 6 (beyond 4096 blocks)
+@pytest.mark.parametrize("offset", [0.0, 1000.0, -300.0, 16000.0])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", [(2, 19, 57, 72), (1, 32, 65, 67), (2, 17, 1, 4097), (2, 40, 63, 66), (1, 200, 57, 72), (8, 150, 513, 513)],
+                         ids=str)
+def test_lsr_is_the_recomputed_gradient(shape, dtype, offset):
+    """Bit for bit, at ignored pixels and labels without a channel too."""
+    from pytorch_loss import _native
+    x, y = inputs(shape, dtype, 13)
+    x.scatter_add_(1, y.clamp(max=shape[1] - 1).unsqueeze(1), (torch.rand(y.shape, device="cuda") * 12).to(dtype).unsqueeze(1))
+    x += offset
+    y[0, 0, :5] = shape[1] + 3
+    y[0, 0, 5:9] = -7
+    x[:, :, -1, -1] = float("-inf")
+    args = _native.lsr_args(x, y)
+    loss, n_valid, lse = _native.lsr_forward_reduced_lse(x, y, IGN, 0.1, True, args=args)
+    assert lse is not None
+    up = torch.tensor(3.0 if dtype == torch.bfloat16 else 700.0, device="cuda")
+    got = _native.lsr_backward_scaled_lse(lse, IGN, 0.1, up, n_valid, args)
+    want = _native.lsr_backward_scaled(x, y, IGN, 0.1, up, n_valid, args=args)
+    a, b = got.view(torch.int16), want.view(torch.int16)
+    assert torch.equal(a, b) or (torch.equal(a[~torch.isnan(want)], b[~torch.isnan(want)]) and torch.equal(torch.isnan(got), torch.isnan(want)))
+
+
 def test_a_mask_is_refused():
     """The byte mask of a selection has no place in this backward: the call raises, and never returns an unmasked gradient."""
     from pytorch_loss import _native
