@@ -79,7 +79,8 @@ __global__ __launch_bounds__(256) void planes16_bwd(const T *__restrict__ x, con
                 for (int d = 0; d < kPer; ++d)
                     if (q + d >= 0 && q + d < M) {
                         const Pixel a = px(d);
-                        const float g = op.grad(load_one(x + at + q + d), a, c);
+                        float g = op.grad(load_one(x + at + q + d), a, c);
+                        asm("" : "+v"(g));          // rounded to fp32 first, as above: not one v_fma_mixlo_f16
                         store_one(grad + at + q + d, a.dropped() ? 0.f : g);
                     }
             }

@@ -88,29 +88,68 @@ def test_views_and_labels_without_a_channel(shape, offset, kind):
     assert ((a.grad.float() - b.grad.float()).abs() <= 2 * HALF_ULP[torch.bfloat16] * b.grad.float().abs() * 1.01 + 1e-6).all()
 
 
-# logits with a common offset, whose largest takes digits from anything added to it; planes of a multiple of 8 pixels off the
-# lines; 12 planes per block and a last share of 6 (beyond 4096 blocks)
+# planes of a multiple of 8 pixels off the lines; 12 planes per block and a last share of 6 (beyond 4096 blocks)
+DIRECT = SHAPES + [(2, 19, 57, 72), (1, 200, 57, 72), (8, 150, 513, 513)]
+
+
+# logits with a common offset, whose largest takes digits from anything added to it
 @pytest.mark.parametrize("offset", [0.0, 1000.0, -300.0, 16000.0])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("shape", [(2, 19, 57, 72), (1, 32, 65, 67), (2, 17, 1, 4097), (2, 40, 63, 66), (1, 200, 57, 72), (8, 150, 513, 513)],
-                         ids=str)
+@pytest.mark.parametrize("shape", DIRECT, ids=str)
 def test_lsr_is_the_recomputed_gradient(shape, dtype, offset):
-    """Bit for bit, at ignored pixels and labels without a channel too."""
+    """Bit for bit, at ignored pixels and labels without a channel too, and at the ends of the planes."""
     from pytorch_loss import _native
     x, y = inputs(shape, dtype, 13)
-    x.scatter_add_(1, y.clamp(max=shape[1] - 1).unsqueeze(1), (torch.rand(y.shape, device="cuda") * 12).to(dtype).unsqueeze(1))
+    boost = torch.rand(y.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(59)) * 12
+    x.scatter_add_(1, y.clamp(max=shape[1] - 1).unsqueeze(1), boost.to(dtype).unsqueeze(1))
     x += offset
     y[0, 0, :5] = shape[1] + 3
     y[0, 0, 5:9] = -7
     x[:, :, -1, -1] = float("-inf")
+    x[(y == IGN).unsqueeze(1).expand_as(x)] = float("nan")
     args = _native.lsr_args(x, y)
     loss, n_valid, lse = _native.lsr_forward_reduced_lse(x, y, IGN, 0.1, True, args=args)
     assert lse is not None
     up = torch.tensor(3.0 if dtype == torch.bfloat16 else 700.0, device="cuda")
     got = _native.lsr_backward_scaled_lse(lse, IGN, 0.1, up, n_valid, args)
     want = _native.lsr_backward_scaled(x, y, IGN, 0.1, up, n_valid, args=args)
-    a, b = got.view(torch.int16), want.view(torch.int16)
-    assert torch.equal(a, b) or (torch.equal(a[~torch.isnan(want)], b[~torch.isnan(want)]) and torch.equal(torch.isnan(got), torch.isnan(want)))
+    number = ~torch.isnan(want)
+    assert torch.equal(torch.isnan(got), ~number) and torch.equal(got.view(torch.int16)[number], want.view(torch.int16)[number])
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", DIRECT, ids=str)
+def test_taylor_from_its_sums(shape, dtype, order):
+    """As test_gradient, whose sizes the module may have recomputed."""
+    from pytorch_loss import _native
+    x, y = inputs(shape, dtype, 7)
+    args = _native.taylor_args(x, y)
+    _, n_valid, sums = _native.taylor_ce_forward_reduced_sums(x, y, order, IGN, True, args=args)
+    assert sums is not None
+    scale = 512.0 if dtype == torch.float16 else 1.0
+    got = _native.taylor_ce_backward_scaled_sums(sums, order, IGN, torch.tensor(scale, device="cuda"), n_valid, args)
+    want = exact("taylor%d" % order, x, y) * scale
+    assert ((got.double() - want).abs() <= HALF_ULP[dtype] * want.abs() * 1.01 + 2e-6 * want.abs().max() + 2.0 ** -24).all()
+    assert not got[(y == IGN).unsqueeze(1).expand_as(x)].any()
+
+
+@pytest.mark.parametrize("offset", [1, 8, 64])
+@pytest.mark.parametrize("shape", [(2, 19, 65, 67), (2, 40, 66, 65)], ids=str)
+def test_views_from_what_was_kept(shape, offset):
+    """Views at other offsets into their lines, where the gradient may sit elsewhere in its own."""
+    from pytorch_loss import _native
+    x, y = inputs(shape, torch.bfloat16, 17, offset)
+    up = torch.ones((), device="cuda")
+    args = _native.lsr_args(x, y)
+    _, n_valid, lse = _native.lsr_forward_reduced_lse(x, y, IGN, 0.1, True, args=args)
+    got = _native.lsr_backward_scaled_lse(lse, IGN, 0.1, up, n_valid, args)
+    assert torch.equal(got, _native.lsr_backward_scaled(x, y, IGN, 0.1, up, n_valid, args=args))
+    args = _native.taylor_args(x, y)
+    _, n_valid, sums = _native.taylor_ce_forward_reduced_sums(x, y, 4, IGN, True, args=args)
+    got = _native.taylor_ce_backward_scaled_sums(sums, 4, IGN, up, n_valid, args).float()
+    want = _native.taylor_ce_backward(x, y, 4, IGN, up, n_valid, args=args).float()
+    assert ((got - want).abs() <= 2 * HALF_ULP[torch.bfloat16] * want.abs() * 1.01 + 1e-9).all()
 
 
 def test_a_mask_is_refused():
