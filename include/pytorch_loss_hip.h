@@ -145,8 +145,11 @@ int plh_lsr_backward_scaled_lse(const void *logits, int32_t dtype, const int64_t
 
 /* The same for 16-bit logits on channel planes of at least 4096 pixels that do not start on 128-byte lines, with 16..256
  * channels, in two parts: max_out[P], a pixel's largest logit (in the logits' type), and sum_out[P], the sum of
- * 2^(x log2e - fl(max log2e)) over its logits. The gradient is the one of plh_lsr_backward_scaled bit for bit. */
+ * 2^(x log2e - fl(max log2e)) over its logits. The gradient is the one of plh_lsr_backward_scaled bit for bit.
+ * plh_lsr_saves_lse_planes16 says (1 / 0) whether the sizes qualify, plh_lsr_pays_planes16 whether the pair is also the faster
+ * one there (many channels, or more logits than the caches hold). */
 int plh_lsr_saves_lse_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);
+int plh_lsr_pays_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);
 
 int plh_lsr_forward_reduced_parts_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *sum_out,
                                            void *max_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
@@ -521,6 +524,7 @@ int plh_taylor_ce_backward_scaled_sums(const void *logits, int32_t dtype, const 
 /* The same for 16-bit logits on channel planes of at least 4096 pixels that do not start on 128-byte lines, with 16..256
  * channels (orders 2 and 4; other orders leave sums_out unwritten and recompute). */
 int plh_taylor_ce_saves_sums_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);
+int plh_taylor_ce_pays_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size);    /* as plh_lsr_pays_planes16 */
 int plh_taylor_ce_forward_reduced_sums_planes16(const void *logits, int32_t dtype, const int64_t *labels,
                                                 float *sums_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
                                                 void *workspace, int64_t workspace_bytes,

@@ -203,6 +203,11 @@ extern "C" int plh_lsr_saves_lse_planes16(int32_t dtype, int64_t n_size, int64_t
     return dtype_ok(dtype) && n_size > 0 && dimsize > 0 && m_size > 0 && planes16_apply(dtype_size(dtype), dimsize, m_size) ? 1 : 0;
 }
 
+extern "C" int plh_lsr_pays_planes16(int32_t dtype, int64_t n_size, int64_t dimsize, int64_t m_size) {
+    return dtype_ok(dtype) && n_size > 0 && dimsize > 0 && m_size > 0 &&
+                   planes16_pays(true, dtype_size(dtype), n_size, dimsize, m_size) ? 1 : 0;
+}
+
 extern "C" int plh_lsr_forward_reduced_parts_planes16(const void *logits, int32_t dtype, const int64_t *labels, float *sum_out,
                                                       void *max_out, float *loss_out, int64_t *n_valid_out, int32_t mean,
                                                       void *workspace, int64_t workspace_bytes,

@@ -13,14 +13,33 @@
 
 namespace plh {
 
-// Where the pair runs. Steps with the kernels that recompute -> with it, bf16, us: LSR, which keeps 6 bytes per pixel,
-// (16,19,769,769) 269 -> 260, (9,32,770,766) 251 -> 229, (8,150,513,513) 509 -> 440, (6,200,513,513) 684 -> 510; Taylor, 4,
-// (30,40,513,513) 483 -> 459, (8,150,513,513) 483 -> 396.
-// Below 16 channels the forward's float weighs more than the backward gains (2 channels of 769 x 769: 452 -> 576), and on
-// planes of whole lines the kernels that recompute are the faster ones (LSR (8,150,512,512) 398 -> 414, Taylor 356 -> 373).
+// Where the pair can run: from 16 channels on (2 channels of 769 x 769: 452 -> 576 us), and not on planes of whole lines (LSR
+// (8,150,512,512) 398 -> 414, Taylor 356 -> 373).
 inline bool planes16_apply(size_t elem_bytes, int64_t dimsize, int64_t m_size) {
     if (elem_bytes != 2 || dimsize < 16 || m_size < 4096 || m_size * 2 % 128 == 0) return false;
     return dimsize <= kMaxRegsChannels ? image_form_pays<bf16>((int)dimsize, m_size) : dimsize <= kMaxSplitChannels;
+}
+
+// Where a step with the pair is no slower than one with the kernels that recompute. What it gains are the lines that planes
+// share, which come from HBM twice; what it costs are 4 (Taylor) or 6 bytes per pixel and a block that waits for its stage. Under
+// the 256 MiB of the cache in front of HBM there is little to gain: graph-timed steps recomputed -> with the pair, bf16, us
+//   (2,16,257,257) LSR 25 -> 45, (8,20,513,513) 81 -> 92, (8,32,513,513) 113 -> 130, (4,40,129,129) 29 -> 35; Taylor (28,16,129,129) 30 -> 54
+// and above it the gain grows with the planes:
+//   16..32 channels: (16,19,769,769) 360 MB LSR 262 -> 258, Taylor 275 -> 252; of 340..640 MB on 769 x 769 LSR +2..-10 %,
+//     Taylor -1..-11, on 1021 x 1021 +3..-5, -1..-10, on 1281 x 1281 -1..-8, -3..-13; of 500 MB on 513 x 513 +4..-2, -3..-5, on
+//     129 x 129 +3..+8, +4..-3
+//   33..128: of 315..500 MB on 513 x 513 LSR -2..-11 %, Taylor -7..-25; on 129 x 129 +4..-9, 0..-18; on 65 x 67 Taylor up to +4
+// The kernels that recompute hold 33 and more channels in slots of 8 wavefronts (split_slots), and lose by what they hold: with
+// more slots than channels by a whole wavefront, or a few wavefronts per CU, the pair gains from some 32 MB on:
+//   LSR 97..104 channels +3..-24 %, 129..256 +2..-36 (two sizes of 160 +5 and +7); 105..128: +7..-20
+//   Taylor 97..128 +1..-26 %, 161..256 +4..-34; 129..160: +10..-19
+// and with fewer bytes (129..256 channels of 129 x 129, 4 MB) +8, Taylor +19.
+inline bool planes16_pays(bool lsr, size_t elem_bytes, int64_t n_size, int64_t dimsize, int64_t m_size) {
+    if (!planes16_apply(elem_bytes, dimsize, m_size)) return false;
+    const int64_t bytes = n_size * dimsize * m_size * (int64_t)elem_bytes;
+    if (dimsize > 96 && (lsr ? dimsize <= 104 || dimsize > 128 : dimsize <= 128 || dimsize > 160)) return bytes >= (int64_t)1 << 25;
+    const int64_t plane = dimsize <= kMaxRegsChannels ? 768 * 768 : (lsr ? 1 << 18 : 1 << 14);
+    return m_size >= plane && bytes >= (int64_t)5 << 26;
 }
 
 template <class T, class Op>

@@ -59,6 +59,7 @@ _SIGNATURES = {
     "plh_lsr_forward_reduced_lse": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_backward_scaled_lse": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_saves_lse_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
+    "plh_lsr_pays_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
     "plh_lsr_forward_reduced_parts_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_backward_scaled_parts_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _f32, _p]),
     "plh_lsr_forward_reduced_lse_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _f32, _p]),
@@ -89,6 +90,7 @@ _SIGNATURES = {
     "plh_taylor_ce_forward_reduced_sums": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_taylor_ce_backward_scaled_sums": (ctypes.c_int, [_p, _i32, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_taylor_ce_saves_sums_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
+    "plh_taylor_ce_pays_planes16": (ctypes.c_int, [_i32, _i64, _i64, _i64]),
     "plh_taylor_ce_forward_reduced_sums_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _p, _i32, _p, _i64, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_taylor_ce_backward_scaled_sums_planes16": (ctypes.c_int, [_p, _i32, _p, _p, _p, _f32, _p, _p, _i64, _i64, _i64, _i64, _i64, _p]),
     "plh_soft_dice_workspace_bytes": (_i64, [_i64, _i64]),
@@ -358,6 +360,11 @@ def lsr_backward_scaled(logits, labels, ignore_index, smooth, grad_scalar, divid
 def _planes16(a):
     """What the entry points for 16-bit channel planes are called beside those for fp32 planes and rows."""
     return "_planes16" if a.tag != 0 and a.m > 1 else ""
+
+
+def lsr_lse_pays(a):
+    """Whether a step that keeps the log-sum-exp (lsr_forward_reduced_lse) is no slower than one that recomputes."""
+    return a.tag == 0 or a.m == 1 or load().plh_lsr_pays_planes16(a.tag, a.n, a.c, a.m) != 0
 
 
 def lsr_forward_reduced_lse(logits, labels, ignore_index, smooth, mean, args=None):
@@ -799,6 +806,11 @@ def taylor_ce_forward(logits, labels, n, ignore_index, reduction, args=None):
     else:
         losses.zero_()
     return _back_to(losses, _loss_dtype(a.dtype)), None
+
+
+def taylor_ce_sums_pay(a):
+    """Whether a step that keeps the sums (taylor_ce_forward_reduced_sums) is no slower than one that recomputes."""
+    return a.tag == 0 or a.m == 1 or load().plh_taylor_ce_pays_planes16(a.tag, a.n, a.c, a.m) != 0
 
 
 def taylor_ce_forward_reduced_sums(logits, labels, n, ignore_index, mean, args=None):

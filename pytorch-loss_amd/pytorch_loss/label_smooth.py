@@ -32,16 +32,16 @@ class _LSRReducedFunction(torch.autograd.Function):
     """'sum' / 'mean' of the per-pixel losses produced inside the forward kernel (per-block
     partials, then a fixed-order finishing kernel), so the module needs no ATen pass over the
     pixels for `losses.sum()` and `(labels != ignore).sum()`; backward folds the scalar
-    upstream gradient and the 1/n_valid of a mean into the gradient kernel. On fp32 logits whose channel
-    planes have an odd length (513 x 513, 769 x 769 crops) the forward also keeps every pixel's log-sum-exp
-    (4 bytes per pixel, only when a gradient will be asked for) and the backward forms the gradient from it
-    plane by plane instead of recomputing the softmax (see plh_lsr_backward_scaled_lse)."""
+    upstream gradient and the 1/n_valid of a mean into the gradient kernel. Where the backward is faster from
+    every pixel's log-sum-exp than recomputing the softmax (channel planes that do not start on 128-byte lines,
+    as those of 513 x 513 crops, and many rows: plh_lsr_saves_lse, plh_lsr_pays_planes16) the forward keeps it,
+    4 bytes per pixel or 6 with 16-bit planes, if a gradient will be asked for."""
 
     @staticmethod
     def forward(ctx, logits, labels, lb_smooth, lb_ignore, mean):
         ctx.args = args = _native.lsr_args(logits, labels)
         lse = None
-        if ctx.needs_input_grad[0]:
+        if ctx.needs_input_grad[0] and _native.lsr_lse_pays(args):
             loss, n_valid, lse = _native.lsr_forward_reduced_lse(logits, labels, lb_ignore, lb_smooth, mean, args=args)
         else:
             loss, n_valid = _native.lsr_forward_reduced(logits, labels, lb_ignore, lb_smooth, mean, args=args)

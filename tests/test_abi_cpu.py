@@ -101,6 +101,15 @@ def test_arguments_are_rejected_before_any_launch(native):
     assert lib.plh_taylor_ce_saves_sums(2, 8192, 1100, 1) == 1 and lib.plh_taylor_ce_saves_sums(2, 8192, 1000, 1) == 0 and lib.plh_taylor_ce_saves_sums(2, 8192, 2049, 1) == 1 and lib.plh_taylor_ce_saves_sums(2, 8192, 48, 1) == 1
     assert lib.plh_lmargin_saves_stats(1, 8192, 32000, 1) == 1 and lib.plh_lmargin_saves_stats(0, 8192, 1024, 1) == 0 and lib.plh_lmargin_saves_stats(0, 8192, 1000, 1) == 1 and lib.plh_lmargin_saves_stats(2, 8192, 1024, 1) == 1 and lib.plh_lmargin_saves_stats(2, 8192, 1100, 1) == 1 and lib.plh_lmargin_saves_stats(2, 8192, 4096, 1) == 1
     assert lib.plh_lmargin_saves_stats(0, 8, 5000, 64) == 0 and lib.plh_lmargin_saves_stats(9, 8192, 32000, 1) == 0
+    # 16-bit planes: what pays lies inside what is possible
+    for dims, lsr, taylor in [((16, 19, 769 * 769), 1, 1), ((14, 19, 769 * 769), 0, 0), ((32, 19, 767 * 767), 0, 0), ((16, 19, 1024 * 1024), 0, 0),
+                              ((2, 16, 257 * 257), 0, 0), ((33, 20, 513 * 513), 0, 0), ((16, 40, 513 * 513), 1, 1), ((15, 40, 513 * 513), 0, 0),
+                              ((16, 96, 383 * 385), 0, 1), ((300, 96, 65 * 67), 0, 0), ((5, 104, 181 * 181), 1, 1), ((5, 105, 181 * 181), 0, 1),
+                              ((5, 128, 181 * 181), 0, 1), ((5, 129, 181 * 181), 1, 0), ((5, 160, 181 * 181), 1, 0), ((5, 161, 181 * 181), 1, 1),
+                              ((1, 256, 256 * 257 - 2), 1, 1), ((1, 256, 254 * 257), 0, 0), ((1, 257, 513 * 513), 0, 0)]:
+        for tag in (1, 2):
+            assert lib.plh_lsr_pays_planes16(tag, *dims) == lsr and lib.plh_taylor_ce_pays_planes16(tag, *dims) == taylor, dims
+        assert lib.plh_lsr_pays_planes16(0, *dims) == 0 and lib.plh_taylor_ce_pays_planes16(7, *dims) == 0
     assert lib.plh_lsr_saves_lse(0, 16, 19, 63 * 65) == 0 and lib.plh_lsr_saves_lse(7, 16, 19, 769 * 769) == 0
     assert lib.plh_lsr_forward_reduced_lse(p, 0, lp, p, p, None, 1, p, 1 << 20, 2, 19, 4096, 255, 0.1, None) == -2
     assert lib.plh_lsr_forward_reduced_lse(p, 0, lp, None, p, None, 1, p, 1 << 20, 2, 19, 4097, 255, 0.1, None) == -1
