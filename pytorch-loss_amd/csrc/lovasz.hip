@@ -993,7 +993,7 @@ __global__ __launch_bounds__(kSortThreads) void lov_final(const SortArgs a, floa
             if ((k & 0x7FFFFFFFu) != kIgnoredKey) {
                 const uint32_t pos = out_base[d] + counts[wave][d] + rank[r];            // rank in the descending order
                 const uint32_t cs = hot_base[d] + counts_hot[wave][d] + hrank[r];      // positives before it
-                dj = jaccard_step(npos, pos, cs, hot);
+                dj = jaccard_step<true>(npos, pos, cs, hot);
                 part = add_loss(part, key_error(k), dj);
             }
             if constexpr (Binned) {

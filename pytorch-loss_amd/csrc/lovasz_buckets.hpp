@@ -101,12 +101,15 @@ __device__ __forceinline__ float jaccard(float npos, uint32_t k, uint32_t cs) {
     return k == 0 ? 0.f : 1.f - whole_ratio(inter, inter + (float)k);
 }
 
-// Jaccard difference of the key at rank `pos`, with `cs` of the class's npos positives before it.
+// Jaccard difference of the key at rank `pos`, with `cs` of the class's npos positives before it. kAnyRow: rows of more than
+// kBkMaxRow pixels too, by all of the division operator's steps (whole numbers below 2^31 need none of its scaling).
+template <bool kAnyRow = false>
 __device__ __forceinline__ float jaccard_step(float npos, uint32_t pos, uint32_t cs, uint32_t hot) {
+    auto ratio = [](float a, float b) { return kAnyRow ? DivideBy(b)(a) : whole_ratio(a, b); };
     const float inter_prev = npos - (float)cs;                             // csrc/lovasz_softmax.cu:124-127
     const float inter = npos - (float)(cs + hot);
-    const float j_now = 1.f - whole_ratio(inter, inter + (float)(pos + 1));
-    const float j_prev = (pos == 0) ? 0.f : 1.f - whole_ratio(inter_prev, inter_prev + (float)pos);
+    const float j_now = 1.f - ratio(inter, inter + (float)(pos + 1));
+    const float j_prev = (pos == 0) ? 0.f : 1.f - ratio(inter_prev, inter_prev + (float)pos);
     return j_now - j_prev;                                                 // csrc/lovasz_softmax.cu:141-147
 }
 
