@@ -1207,30 +1207,33 @@ struct LovaszPlan {
 
 static int64_t round_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
-// Whether rows of P keys in C classes go by value buckets. Steps of radix passes -> buckets, us, captured, of ten kinds of
-// logits (soft, a new network's, all equal, confident by 8 / 14 / 20, trained, bf16, in steps of 1/16): the ordinary one and the
-// one that buckets like least, mostly a network so sure that thousands of keys share a value (multiples of 2^-24 below 1)
+// Whether rows of P keys in C classes go by value buckets. Steps of radix passes -> buckets, us, captured, of eleven kinds of
+// logits (soft, a new network's, all equal, confident by 8 / 14 / 17 / 20 / 24, trained, bf16, in steps of 1/16): the ordinary one
+// and the one that buckets like least, mostly a network so sure that thousands of keys share a value (multiples of 2^-24 below 1)
 // and have to be sorted apart in LDS, by few blocks if the classes are few.
 //   one block per row: always (two classes of 7680 pixels 86 -> 39, at worst 87 -> 60)
 //   P C^2 >= 2^26, or C >= 32:
-//   16 of 262144 164 -> 124, at worst 203 -> 199; of 524288 226 -> 162, 320 -> 245; 12 of 524288 202 -> 147, 239 -> 219
-//   24 of 131072 147 -> 106, 187 -> 183; 8 of 1048576 262 -> 183, 295 -> 269; 6 of 2097152 356 -> 231, 405 -> 365
-//   32 of 8192 108 -> 70, 127 -> 103; of 65536 135 -> 98, 157 -> 151; 64 of 8192 179 -> 125, 165 -> 127
-//   19 of 2097152 751 -> 443, 415 -> 322
-//   below that, 12 classes and more of 131072 pixels and more where P C^2 >= 5 2^23:
-//   13 of 262144 158 -> 121, 192 -> 195; 14 of 342000 182 -> 142, 231 -> 217; 12 of 448000 192 -> 147, 225 -> 196
-//   16 of 200704 148 -> 119, 183 -> 184; 18 of 147456 145 -> 117, 174 -> 179; 19 of 131072 144 -> 108, 178 -> 169
-//   left out, for what they lose at worst: 2 of 262144 94 -> 89, 100 -> 159; 4 of 263169 115 -> 95, 115 -> 155; 8 of 262144
-//   128 -> 106, 136 -> 169; 8 of 524288 168 -> 133, 184 -> 212; 10 of 524288 195 -> 143, 221 -> 232; 12 of 262144 151 -> 118,
-//   184 -> 193; 14 of 200000 147 -> 121, 172 -> 188; 16 of 65536 108 -> 87, 127 -> 150; of 131072 125 -> 102, 149 -> 155
-// (The worst cases by buckets are those of bk_ranks_crowded, which has become some 8 us faster since.)
+//   15 of 298262 165 -> 123, at worst 219 -> 214; 16 of 262145 164 -> 120, 196 -> 206; of 524288 226 -> 162, 320 -> 245;
+//   12 of 466034 196 -> 144, 234 -> 222; 24 of 131072 140 -> 106, 179 -> 179; 8 of 1048576 257 -> 178, 281 -> 255;
+//   6 of 2097152 354 -> 226, 391 -> 331; 32 of 8192 108 -> 70, 127 -> 103; of 65536 135 -> 98, 157 -> 151
+//   64 of 8192 179 -> 125, 165 -> 127; 19 of 2097152 751 -> 443, 415 -> 322
+//   below that, 131072 pixels and more in 18 classes and more:
+//   18 of 131072 135 -> 102, 165 -> 164; of 194181 139 -> 107, 184 -> 185; 20 of 131072 139 -> 105, 171 -> 169; 22 of 131072
+//   137 -> 106, 175 -> 178; 28 of 131072 153 -> 110, 195 -> 183
+//   and in 12 and more where P C >= 9 2^19: 12 of 393216 175 -> 136, 217 -> 212; 13 of 362970 176 -> 134, 219 -> 214
+//   left out, for what they lose at worst: 12 of 291272 152 -> 117, 179 -> 195; 13 of 273003 155 -> 115, 179 -> 194; 14 of 213996
+//   141 -> 111, 170 -> 186; of 278194 150 -> 118, 186 -> 203; 15 of 242338 151 -> 123, 186 -> 202; 17 of 200000 145 -> 115, 183 -> 188;
+//   2 of 262144 94 -> 89, 100 -> 159; 4 of 263169 115 -> 95, 115 -> 155; 8 of 262144 122 -> 103, 131 -> 153;
+//   16 of 65536 108 -> 87, 127 -> 150; of 131072 118 -> 97, 143 -> 156; 19 of 100000 124 -> 96, 154 -> 157
 // Rows of more than kBkMaxRow pixels take the radix passes: with 1024 buckets there are 7.5 sampled keys per bucket, and
 // 8 keys of a tile. With 2048 buckets of 3072 (rows of 6.3 M pixels) the sample left some 30 buckets of a class larger than LDS,
 // and two classes took 0.63 ms against 0.39 of the radix passes.
 static bool bk_pays(int64_t P, int64_t C) {
     if (P <= kBkCap) return true;
     const int64_t work = P * C * C;
-    return P <= kBkMaxRow && (C >= 32 || work >= (int64_t)8 << 23 || (C >= 12 && P >= 131072 && work >= (int64_t)5 << 23));
+    if (P > kBkMaxRow) return false;
+    return C >= 32 || work >= (int64_t)8 << 23 ||
+           (P >= 131072 && (C >= 18 || (C >= 12 && P * C >= (int64_t)9 << 19)));
 }
 
 static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan &pl, bool look_back = false) {
