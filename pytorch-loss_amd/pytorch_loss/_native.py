@@ -357,11 +357,6 @@ def lsr_backward_scaled(logits, labels, ignore_index, smooth, grad_scalar, divid
                                   grad_scalar, divide_by)
 
 
-def _planes16(a):
-    """What the entry points for 16-bit channel planes are called beside those for fp32 planes and rows."""
-    return "_planes16" if a.tag != 0 and a.m > 1 else ""
-
-
 def lsr_lse_pays(a):
     """Whether a step that keeps the log-sum-exp (lsr_forward_reduced_lse) is no slower than one that recomputes."""
     return a.tag == 0 or a.m == 1 or load().plh_lsr_pays_planes16(a.tag, a.n, a.c, a.m) != 0
@@ -819,8 +814,9 @@ def taylor_ce_forward_reduced_sums(logits, labels, n, ignore_index, mean, args=N
     -> (loss, n_valid, sums or None)."""
     _check_order(n)
     a = args or taylor_args(logits, labels)
-    planes = _planes16(a)
-    if a.x.numel() == 0 or not getattr(load(), "plh_taylor_ce_saves_sums" + planes)(a.tag, a.n, a.c, a.m):
+    planes16 = a.tag != 0 and a.m > 1
+    saves = load().plh_taylor_ce_saves_sums_planes16 if planes16 else load().plh_taylor_ce_saves_sums
+    if a.x.numel() == 0 or not saves(a.tag, a.n, a.c, a.m):
         loss, n_valid = taylor_ce_forward(logits, labels, n, ignore_index, "mean" if mean else "sum", args=a)
         return loss, n_valid, None
     dev = a.x.device
@@ -828,8 +824,8 @@ def taylor_ce_forward_reduced_sums(logits, labels, n, ignore_index, mean, args=N
     n_valid = torch.empty((), dtype=torch.int64, device=dev)
     sums = torch.empty((a.n * a.m,), dtype=torch.float32, device=dev)
     ws, ws_bytes = _reduce_workspace(a.n * a.m, dev)
-    _call(a.x, "plh_taylor_ce_forward_reduced_sums" + planes, _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(loss), _ptr(n_valid),
-          1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m, int(n), int(ignore_index))
+    _call(a.x, "plh_taylor_ce_forward_reduced_sums_planes16" if planes16 else "plh_taylor_ce_forward_reduced_sums", _ptr(a.x), a.tag,
+          _ptr(a.lb), _ptr(sums), _ptr(loss), _ptr(n_valid), 1 if mean else 0, _ptr(ws), ws_bytes, a.n, a.c, a.m, int(n), int(ignore_index))
     return _back_to(loss, _loss_dtype(a.dtype)), n_valid, sums
 
 
@@ -838,8 +834,8 @@ def taylor_ce_backward_scaled_sums(sums, n, ignore_index, grad_scalar, divide_by
     a = args
     grad = torch.empty_like(a.x)
     go = _scalar_f32(grad_scalar)
-    _call(a.x, "plh_taylor_ce_backward_scaled_sums" + _planes16(a), _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(go), 1.0,
-          _ptr(divide_by), _ptr(grad), a.n, a.c, a.m, int(n), int(ignore_index))
+    _call(a.x, "plh_taylor_ce_backward_scaled_sums_planes16" if a.tag != 0 and a.m > 1 else "plh_taylor_ce_backward_scaled_sums",
+          _ptr(a.x), a.tag, _ptr(a.lb), _ptr(sums), _ptr(go), 1.0, _ptr(divide_by), _ptr(grad), a.n, a.c, a.m, int(n), int(ignore_index))
     return _back_to(grad, a.dtype)
 
 
