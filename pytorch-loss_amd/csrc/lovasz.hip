@@ -1248,7 +1248,7 @@ static int make_plan(int64_t n_size, int64_t dimsize, int64_t m_size, LovaszPlan
     pl.tiles_pad = (int)round_up(pl.tiles, kSortWaves);
     int64_t off = 0;
     pl.off_class = off;       off += round_up(4 * dimsize * 4, 256);      // pos_max[C], kept[C], all_min[C], key_bits[C]
-    pl.off_block_max = off;   off += round_up(4 * dimsize * ceil_div(pl.P, 256), 256);   // [key blocks][C]
+    pl.off_block_max = off;   off += round_up(4 * dimsize * ceil_div(pl.P, 256), 256);   // [C][key blocks]
     pl.buckets = !look_back && bk_pays(pl.P, dimsize);
     if (pl.buckets) {
         pl.bk_tiles = (int)ceil_div(pl.P, kBkTile);
@@ -1336,7 +1336,7 @@ static int lovasz_buckets(const LovaszPlan &pl, char *ws, BucketArgs a, float *l
     a.loss_part = reinterpret_cast<double *>(ws + pl.off_loss_part);
     const dim3 tiles((unsigned)pl.bk_tiles, (unsigned)C), threads(kBkThreads);
     const unsigned most = (unsigned)ceil_div(pl.P, kBkTarget) + 1;  // buckets a class can have
-    // two blocks fit a CU; each takes every so many of the class's crowded runs
+    // some 1024 blocks in all, of which a CU runs one at a time (bk_rank_rest); each takes every so many of its class's crowded runs
     const unsigned crowded_blocks = (unsigned)(ceil_div(1024, C) < most ? ceil_div(1024, C) : most);
     hipLaunchKernelGGL(bk_sample, dim3(1 + kBkItems, (unsigned)C), threads, 0, st, a);
     hipLaunchKernelGGL(bk_split, dim3((1 + kAbsentBlocks) * (unsigned)C), threads, 0, st, a);

@@ -17,8 +17,8 @@
 // A key moves 28 bytes: read and written by bk_cut, bk_rank and bk_restore, and a place of 2 bytes. The form before this one
 // wrote the buckets out one after the other: that takes a histogram first (6 bytes a key more, buckets kept for the second
 // pass) and writes of some 10 keys, where a segment of a run has 24 here. (4,19,512,1024) fp32: histogram and scatter
-// 67 + 117 us against 96 now, rank 119 against 111, gather 72 against 57, step 557 -> 436 us; (8,21,513,513) bf16 trained
-// 77 + 154 against 127, 217 against 224, 116 against 68, step 792 -> 608. Which rows come here: bk_pays.
+// 67 + 117 us against 93 now, rank 119 against 105, gather 72 against 56, step 557 -> 437 us; (8,21,513,513) bf16 trained
+// 77 + 154 against 130, 217 against 231, 116 against 70, step 792 -> 618. Which rows come here: bk_pays.
 #pragma once
 
 namespace plh {

@@ -6,8 +6,9 @@
 // every plane its 256 threads move the 32 whole lines that begin at the tile's first pixel shifted back by the plane's offset
 // into its line: 16 aligned bytes per lane, loads and stores alike, four planes in flight. The pixels' values and labels are
 // staged in LDS, transposed by pixel mod 8, so that a lane's window of 8 pixels reads without bank conflicts from one
-// address and constants per plane. Bound by memory: the walk alone, a copy, takes 148 of the 150 us at (16,19,769,769) bf16
-// (5.5 TB/s; a copy in the order of the addresses 6.2), with LSR's 6 bytes per pixel 168.
+// address and constants per plane. Bound by memory: of LSR's 160 us at (16,19,769,769) bf16 the walk alone, a copy with nothing
+// staged, takes 122 (5.9 TB/s; a copy in the order of the addresses 113), with labels and 4 bytes per pixel staged 149, with
+// LSR's 6 bytes 154.
 #pragma once
 #include "plh_common.hpp"
 
