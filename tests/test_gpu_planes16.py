@@ -1,4 +1,4 @@
-"""The backward of 16-bit channel planes from one float per pixel that the forward left (csrc/planes16.hpp): LSR and Taylor cross
+"""The backward of 16-bit channel planes from what the forward left per pixel (csrc/planes16.hpp): LSR and Taylor cross
 entropy against the same gradient in 64 bits and against the kernels that recompute. The first and last channel counts of both
 forward forms, tiles that end inside a plane, planes shared out over blocks, views at other offsets into their lines."""
 import pytest
